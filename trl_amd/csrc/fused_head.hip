@@ -1304,45 +1304,75 @@ __global__ __launch_bounds__(256) void split_bf16x3_kernel(const float* in, int6
     for (int sl = 0; sl < 6; ++sl) E::store1(o + int64_t(sl) * cpad, p[side == 0 ? a_map[sl] : b_map[sl]]);
 }
 
-// Largest magnitude of a bf16 [R, C8 * 8] matrix (row stride ld) as the bit pattern of that float, through an atomic
-// maximum on `out` (non-negative floats order like unsigned integers; the caller clears `out`).
-__global__ __launch_bounds__(256) void maxabs_bf16_kernel(const uint16_t* in, int64_t ld, int R, int C8, uint32_t* out) {
+// Largest magnitudes of the backward's operands in one launch: out[0] of the fp32 vector g [n_g], out[1] of hidden, out[2]
+// of the weight (bf16 matrices of C8 * 8 columns; no workgroups are launched for them in an fp16 problem), as the bit
+// patterns of those floats (non-negative floats order like unsigned integers; the caller clears `out`).
+//
+// Bound by the read of the weight.  Workgroups of 1024 lanes, at most two per CU for a matrix, eight 16-byte loads in
+// flight per lane, one atomic per workgroup and only when it would raise the maximum: atomics on one address retire
+// about one per 15 ns, so one per wave of 4096 small workgroups took 250 us whatever the size of the matrix.
+// Weights of 206 / 525 / 1089 MB (50257 x 2048, 128256 x 2048, 151936 x 3584) with 1400 / 1400 / 9700 tokens: the three
+// launches 263 / 279 / 355 us -> 34 / 96 / 201 us (5.6-6.1 TB/s).
+constexpr int kMaxThreads = 1024, kMaxBlocks = 512;
+struct MaxAbsArgs {
+    const float* g;
+    int64_t n_g;
+    const uint16_t *hidden, *weight;
+    int64_t ld_hidden, ld_weight;
+    int n_hidden, n_weight, C8;         // rows; 16-byte vectors per row
+    int blocks_g, blocks_h, blocks_w;   // workgroups of each
+    uint32_t* out;
+};
+__global__ __launch_bounds__(kMaxThreads) void head_maxabs_kernel(MaxAbsArgs a) {
+    __shared__ uint32_t part[kMaxThreads / kWave];
+    int block = blockIdx.x, slot;
     uint32_t m = 0;
-    auto take = [&](u32x4 q) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t lo = (q[i] << 16) & 0x7fff0000u, hi = q[i] & 0x7fff0000u;
-            m = max(m, max(lo, hi));
-        }
-    };
-    if (ld == int64_t(C8) * 8) {  // dense rows: one flat sweep, four loads in flight per lane
-        const u32x4* p = reinterpret_cast<const u32x4*>(in);
-        const int64_t n = int64_t(R) * C8, step = int64_t(gridDim.x) * 256;
-        int64_t v = int64_t(blockIdx.x) * 256 + threadIdx.x;
-        for (; v + 3 * step < n; v += 4 * step) {
-            const u32x4 q0 = __builtin_nontemporal_load(p + v), q1 = __builtin_nontemporal_load(p + v + step),
-                        q2 = __builtin_nontemporal_load(p + v + 2 * step), q3 = __builtin_nontemporal_load(p + v + 3 * step);
-            take(q0), take(q1), take(q2), take(q3);
-        }
-        for (; v < n; v += step) take(__builtin_nontemporal_load(p + v));
+    if (block >= a.blocks_w + a.blocks_h) {
+        slot = 0;
+        block -= a.blocks_w + a.blocks_h;
+        for (int64_t i = int64_t(block) * kMaxThreads + threadIdx.x; i < a.n_g; i += int64_t(a.blocks_g) * kMaxThreads)
+            m = max(m, __float_as_uint(a.g[i]) & 0x7fffffffu);
     } else {
-        for (int r = blockIdx.x; r < R; r += gridDim.x) {
-            const u32x4* row = reinterpret_cast<const u32x4*>(in + int64_t(r) * ld);
-            for (int c = threadIdx.x; c < C8; c += 256) take(row[c]);
+        const bool is_w = block < a.blocks_w;
+        slot = is_w ? 2 : 1;
+        const int blocks = is_w ? a.blocks_w : a.blocks_h;
+        block -= is_w ? 0 : a.blocks_w;
+        const uint16_t* in = is_w ? a.weight : a.hidden;
+        const int64_t ld = is_w ? a.ld_weight : a.ld_hidden;
+        const int R = is_w ? a.n_weight : a.n_hidden;
+        auto take = [&](u32x4 q) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m = max(m, max((q[i] << 16) & 0x7fff0000u, q[i] & 0x7fff0000u));
+        };
+        if (ld == int64_t(a.C8) * 8) {  // dense rows: one flat sweep
+            const u32x4* p = reinterpret_cast<const u32x4*>(in);
+            const int64_t n = int64_t(R) * a.C8, step = int64_t(blocks) * kMaxThreads;
+            int64_t v = int64_t(block) * kMaxThreads + threadIdx.x;
+            for (; v + 7 * step < n; v += 8 * step) {
+                u32x4 q[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) q[k] = p[v + k * step];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) take(q[k]);
+            }
+            for (; v < n; v += step) take(p[v]);
+        } else {
+            for (int r = block; r < R; r += blocks) {
+                const u32x4* row = reinterpret_cast<const u32x4*>(in + int64_t(r) * ld);
+                for (int c = threadIdx.x; c < a.C8; c += kMaxThreads) take(row[c]);
+            }
         }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off, 64)));
-    if ((threadIdx.x & 63) == 0 && m != 0) atomicMax(out, m);
-}
-// The same for an fp32 vector.
-__global__ __launch_bounds__(256) void maxabs_f32_kernel(const float* in, int64_t n, uint32_t* out) {
-    uint32_t m = 0;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
-        m = max(m, __float_as_uint(in[i]) & 0x7fffffffu);
+    if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off, 64)));
-    if ((threadIdx.x & 63) == 0 && m != 0) atomicMax(out, m);
+        for (int w = 0; w < kMaxThreads / kWave; ++w) m = max(m, part[w]);
+        // (a stale value only costs an atomic that changes nothing)
+        if (m > __hip_atomic_load(a.out + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a.out + slot, m);
+    }
 }
 
 // [R, C] (ld) -> [C, ldo] with columns >= R zero-filled up to `fill`: 64 x 64 tiles through LDS.
@@ -1682,14 +1712,28 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
     const uint32_t* max_h = from_bf16 ? maxima + 1 : nullptr;
     hipLaunchKernelGGL(head_fill_kernel, dim3(unsigned((2 + l.n_chunks + 255) / 256)), dim3(256), 0, s,
                        reinterpret_cast<float*>(maxima), 2 + l.n_chunks, 0.f);
-    hipLaunchKernelGGL(maxabs_f32_kernel, dim3(unsigned(N < 65536 ? (N + 255) / 256 : 256)), dim3(256), 0, s, d_g_logp,
-                       n_tokens, maxima);
+    MaxAbsArgs ma{};
+    ma.g = d_g_logp;
+    ma.n_g = n_tokens;
+    ma.blocks_g = int(N < 32 * kMaxThreads ? (N + kMaxThreads - 1) / kMaxThreads : 32);
+    ma.out = maxima;
+    if (from_bf16) {  // (one scale for the whole weight: a single sweep over it instead of one per chunk)
+        const auto blocks = [&](int64_t rows) {
+            const int64_t b = (rows * (H / 8) + 8 * kMaxThreads - 1) / (8 * kMaxThreads);
+            return int(b < kMaxBlocks ? b : kMaxBlocks);
+        };
+        ma.hidden = static_cast<const uint16_t*>(d_hidden);
+        ma.weight = static_cast<const uint16_t*>(d_weight);
+        ma.ld_hidden = hidden_stride;
+        ma.ld_weight = weight_stride;
+        ma.n_hidden = N;
+        ma.n_weight = V;
+        ma.C8 = H / 8;
+        ma.blocks_h = blocks(N);
+        ma.blocks_w = blocks(V);
+    }
+    hipLaunchKernelGGL(head_maxabs_kernel, dim3(unsigned(ma.blocks_w + ma.blocks_h + ma.blocks_g)), dim3(kMaxThreads), 0, s, ma);
     if (from_bf16) {
-        hipLaunchKernelGGL(maxabs_bf16_kernel, dim3(unsigned(N < 2048 ? N : 2048)), dim3(256), 0, s,
-                           static_cast<const uint16_t*>(d_hidden), hidden_stride, N, H / 8, maxima + 1);
-        // one scale for the whole weight: a single sweep over it instead of one per chunk
-        hipLaunchKernelGGL(maxabs_bf16_kernel, dim3(unsigned(V < 4096 ? V : 4096)), dim3(256), 0, s,
-                           static_cast<const uint16_t*>(d_weight), weight_stride, V, H / 8, maxima + 2);
         hipLaunchKernelGGL((transpose16_kernel<true, true>), dim3((H + 63) / 64, unsigned((l.npad + 63) / 64)), dim3(256), 0, s,
                            static_cast<const uint16_t*>(d_hidden), hidden_stride, N, H, ht, l.ld_n, l.npad, max_h, d_g_logp,
                            max_g, logit_scale / temperature);
