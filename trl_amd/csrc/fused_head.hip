@@ -864,22 +864,32 @@ __global__ void head_fill_kernel(float* p, int64_t n, float v) {
     if (i < n) p[i] = v;
 }
 
-// merges the vocabulary splits of every token: logp, entropy, log_z
-__global__ void head_merge_kernel(const float* partial, const float* tgt, const int64_t* targets, int N, int V,
-                                  int v_splits, float* logp, float* entropy, float* log_z, float* target_is_max,
-                                  int32_t* error_flag, float* stash_zt) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+// Merges the vocabulary splits of every token: logp, entropy, log_z.  One wave per token, lane s on splits s, s + 64, ...:
+// bound by the latency of a couple of dependent loads (a token's partials are one contiguous piece of memory), where a
+// thread per token walked the splits one after the other with the grid nearly empty: 459 tokens x 119 splits 40 -> 4.7 us.
+constexpr int kMergeTokens = 4;  // tokens per workgroup
+__global__ __launch_bounds__(kMergeTokens * kWave) void head_merge_kernel(
+    const float* partial, const float* tgt, const int64_t* targets, int N, int V, int v_splits, float* logp, float* entropy,
+    float* log_z, float* target_is_max, int32_t* error_flag, float* stash_zt) {
+    const int n = blockIdx.x * kMergeTokens + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     if (n >= N) return;
-    const float* p = partial + int64_t(n) * v_splits * 4;
-    float R = -INFINITY;
-    for (int s = 0; s < v_splits; ++s) R = fmaxf(R, p[s * 4]);
-    float S = 0.f, U = 0.f, zm = -INFINITY;
-    for (int s = 0; s < v_splits; ++s) {
-        zm = fmaxf(zm, p[s * 4 + 3]);
-        const float sc = (p[s * 4] == -INFINITY) ? 0.f : fast_exp2(p[s * 4] - R);
-        S += p[s * 4 + 1] * sc;
-        U += p[s * 4 + 2] * sc;
+    const f32x4* p = reinterpret_cast<const f32x4*>(partial) + int64_t(n) * v_splits;
+    float R = -INFINITY, S = 0.f, U = 0.f, zm = -INFINITY;
+    for (int s = lane; s < v_splits; s += kWave) {
+        const f32x4 q = p[s];
+        zm = fmaxf(zm, q[3]);
+        const float r = fmaxf(R, q[0]);
+        const float keep = R == -INFINITY ? 0.f : fast_exp2(R - r), add = q[0] == -INFINITY ? 0.f : fast_exp2(q[0] - r);
+        S = S * keep + q[1] * add;  // (the references are integers: the factors are powers of two)
+        U = U * keep + q[2] * add;
+        R = r;
     }
+    const float r = wave_max(R), sc = R == -INFINITY ? 0.f : fast_exp2(R - r);
+    R = r;
+    S = wave_sum(S * sc);
+    U = wave_sum(U * sc);
+    zm = wave_max(zm);
+    if (lane != 0) return;
     constexpr float kLn2Hi = 0.693145751953125f, kLn2Lo = 1.42860677e-06f;
     const float lz = fmaf(R, kLn2Hi, fmaf(R, kLn2Lo, logf(S)));
     const int64_t t = targets[n];
@@ -1491,19 +1501,32 @@ BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     return l;
 }
 
-// Vocabulary splits of the forward.  A workgroup keeps one token block and walks over 1/splits of the
-// vocabulary tiles, so the grid is token blocks x splits workgroups of equal length, one per CU at a
-// time: the splits are chosen so that they fill whole rounds of the 256 CUs (65 token blocks x 8 splits
-// would run 3 rounds for 2.03 rounds of work), preferring few splits.
-constexpr int kCus = 256, kMinFwdSplits = 8, kMaxFwdSplits = 128;
-int fwd_splits(int64_t n_tokens) {
+// Vocabulary splits of the forward.  A workgroup keeps one token block and walks over its share of the vocabulary tiles,
+// one workgroup per CU at a time, so a launch takes (rounds of 256 workgroups) x (tiles per share) tile times; the number
+// of splits is the one that makes this smallest, the fewest on a tie.  Any number is allowed, not only powers of two with
+// at least four tiles each: 6 token blocks x 197 (501) vocabulary tiles run 42 splits of 5 (12) tiles in one round, where
+// 32 (64) splits took 1 round of 7 (2 rounds of 8) tiles, 384 -> 290 us (896 -> 713 us), both
+// with H = 2048 and the stash.  Long launches are bound by power and gain nothing: 38 token blocks x 594 tiles run 3 rounds
+// of 30 where they ran 5 of 19, 8.6 ms either way.
+constexpr int kCus = 256, kMinFwdSplits = 8, kMaxFwdSplits = 256;
+int max_fwd_splits(int64_t n_tokens) {  // bounds the workspace, which is sized before the vocabulary is known
+    const int64_t n_tb = (n_tokens + BN - 1) / BN, most = 2048 / n_tb;
+    return int(most < kMinFwdSplits ? kMinFwdSplits : (most > kMaxFwdSplits ? kMaxFwdSplits : most));
+}
+int fwd_splits(int64_t n_tokens, int n_vt, int64_t H) {
     const int64_t n_tb = (n_tokens + BN - 1) / BN;
-    int best = kMinFwdSplits;
-    double best_cost = 1e30;
-    for (int sp = kMinFwdSplits; sp <= kMaxFwdSplits; sp *= 2) {
-        const double rounds = double(n_tb * sp) / kCus;
-        const double cost = double((n_tb * sp + kCus - 1) / kCus) / rounds;
-        if (cost < best_cost - 0.02) {  // more splits only for a gain of 2 % or more
+    // in k steps of the tile loop: a tile's own steps plus its reduction, and a workgroup's start and final merge
+    const double tile = double(H) / BK + 3., start = 4.;
+    const int most = max_fwd_splits(n_tokens) < n_vt ? max_fwd_splits(n_tokens) : n_vt;
+    int best = 1;
+    double best_cost = 1e300;
+    // (fewer than 8 splits would leave an XCD's 32 workgroups with fewer than 8 vocabulary tiles to share)
+    for (int sp = most < kMinFwdSplits ? most : kMinFwdSplits; sp <= most; ++sp) {
+        const int tps = (n_vt + sp - 1) / sp;
+        if (sp > kMinFwdSplits && (n_vt + tps - 1) / tps != sp) continue;  // some splits would be empty
+        const int64_t per_xcd = (n_tb * sp + 7) / 8, rounds = (per_xcd + kCus / 8 - 1) / (kCus / 8);
+        const double cost = double(rounds) * (tps * tile + start);
+        if (cost < best_cost * 0.99) {
             best_cost = cost;
             best = sp;
         }
@@ -1579,7 +1602,7 @@ int reserve_head_lds(Kern kern, const char* what) {
 using namespace trlk;
 
 extern "C" size_t trlk_fused_head_fwd_workspace_bytes(int64_t n_tokens) {
-    return n_tokens > 0 ? size_t(n_tokens) * (fwd_splits(n_tokens) * 4 + 1) * sizeof(float) : 0;
+    return n_tokens > 0 ? size_t(n_tokens) * (max_fwd_splits(n_tokens) * 4 + 1) * sizeof(float) : 0;
 }
 
 extern "C" size_t trlk_fused_head_stash_bytes(int64_t n_tokens, int64_t vocab, int64_t* out_ld) {
@@ -1632,8 +1655,7 @@ extern "C" int trlk_fused_head_fwd(const void* d_hidden, const void* d_weight, c
     a.inv_t = 1.f / temperature;
     a.softcap = final_logit_softcapping > 0.f ? final_logit_softcapping : 0.f;
     const int n_vt = int((vocab + BM - 1) / BM);
-    int splits = fwd_splits(n_tokens);  // what the workspace was sized for
-    while (splits > 1 && n_vt < 4 * splits) splits /= 2;  // at least 4 vocabulary tiles per workgroup
+    const int splits = fwd_splits(n_tokens, n_vt, hidden_size);
     a.v_splits = splits;
     a.tiles_per_split = (n_vt + splits - 1) / splits;
     a.partial = static_cast<float*>(d_workspace);
@@ -1659,7 +1681,8 @@ extern "C" int trlk_fused_head_fwd(const void* d_hidden, const void* d_weight, c
     else
         rc = general ? launch_fwd(std::false_type{}, std::true_type{}) : launch_fwd(std::false_type{}, std::false_type{});
     if (rc) return rc;
-    hipLaunchKernelGGL(head_merge_kernel, dim3(unsigned((n_tokens + 255) / 256)), dim3(256), 0, s, a.partial, a.tgt,
+    hipLaunchKernelGGL(head_merge_kernel, dim3(unsigned((n_tokens + kMergeTokens - 1) / kMergeTokens)),
+                       dim3(kMergeTokens * kWave), 0, s, a.partial, a.tgt,
                        d_targets, int(n_tokens), int(vocab), splits, d_out_logp, d_out_entropy, d_out_log_z,
                        d_out_target_is_max, d_error_flag, d_out_stash != nullptr ? a.stash.zt() : nullptr);
     return launch_status("fused_head_fwd (merge)");
