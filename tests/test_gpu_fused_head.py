@@ -705,3 +705,29 @@ def test_target_logit_every_tile_position(amd):
         out = ops.fused_head_fwd(hidden.to(DEV), weight.to(DEV), labels.to(DEV), 1.0, 0.0, 1.0, None, stash)
         torch.testing.assert_close(out[0].cpu(), want, atol=2e-3, rtol=0)
     amd.check_device_errors()  # no index was out of range
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,h,v,chunk", [
+    (40, 72, 9300, 9300),    # one chunk of 148 k steps for one dHidden tile: 9 slices, the last one shorter
+    (40, 72, 9001, 4096),    # three chunks of 64 k steps, the last of 16: its rows reach fewer slices
+    (300, 520, 5000, 5000),  # two token blocks x three hidden tiles, both ragged
+    (257, 264, 1024, 1024),  # 16 k steps: too few to cut
+    (3, 8, 2048, 2048),      # the smallest tile with two slices
+])
+def test_backward_with_the_dhidden_contraction_cut_into_slices(amd, dtype, n, h, v, chunk):
+    """Few tokens: the dHidden product's contraction over the vocabulary is cut into slices with fp32 sums of their
+    own.  Both gradients against fp32 products of the same operands, at the bounds of an uncut contraction."""
+    g = torch.Generator().manual_seed(n + v + chunk)
+    hidden = torch.randn(n, h, generator=g).to(dtype)
+    weight = (torch.randn(v, h, generator=g) * (2.0 / h**0.5)).to(dtype)
+    labels = torch.randint(0, v, (n,), generator=g)
+    gout = torch.randn(n, generator=g)
+    _, _, want_h, want_w = _fp32_reference(hidden, weight, labels, 0.9, None, 1.0, gout)
+    args = (hidden.to(DEV), weight.to(DEV), labels.to(DEV), 0.9, 0.0, 1.0)
+    for stash in (False, True):
+        out = amd.ops.fused_head_fwd(*args, None, stash)
+        got_h, got_w, _ = amd.ops.fused_head_bwd(*args, out[2], gout.to(DEV), chunk, None, out[4])
+        bound = 1.5e-3 if dtype == torch.bfloat16 else 5e-4
+        for got, want in ((got_h, want_h), (got_w, want_w)):
+            assert _rel_l2(got.float(), want.to(dtype).float()) < bound, (stash, _rel_l2(got.float(), want.to(dtype).float()))

@@ -1149,6 +1149,9 @@ struct GemmArgs {
     const uint32_t* max_b;
     const float* g_rows;
     float mult_a;
+    // K-major A, epilogue 1: the contraction cut into `slices` pieces of `kslice` (a multiple of the k step), each
+    // with its own fp32 sum at out_f32 + slice * M * ld_f32; slice i takes workgroups [i, i + 1) * slice_grid.
+    int slices, kslice, slice_grid;
 };
 
 // DT: dtype of the operands (the matrix-core instruction), ODT: storage dtype of `out_lp`.
@@ -1157,6 +1160,20 @@ template <int DT, int MODE, int ODT, bool AKM = false>
 __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char* smem) {
     typedef Elem<ODT> E;
     const int n_mt = (a.M + BM - 1) / BM, n_nt = (a.N + BN - 1) / BN;
+    Operand A = a.A, B = a.B;
+    int K = a.K;
+    float* out_f32 = a.out_f32;
+    if constexpr (AKM && MODE == 1) {
+        if (a.slices > 1) {
+            const int slice = block / a.slice_grid;
+            block -= slice * a.slice_grid;
+            const int k0 = slice * a.kslice;
+            A.p += int64_t(k0) * A.ld;
+            B.p += k0;
+            K = min(a.kslice, K - k0);
+            out_f32 += int64_t(slice) * a.M * a.ld_f32;
+        }
+    }
     int tm, tn;
     xcd_patch(block, n_mt, n_nt, tm, tn);
     if (tm >= n_mt || tn >= n_nt) return;
@@ -1164,7 +1181,7 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     const int wm = wave / WGN, wn = wave % WGN;
     const int m0 = tm * BM, n0 = tn * BN;
     f32x16 acc[MB][NB];
-    gemm_tile_nt<DT, TRLK_HEAD_BK_GEMM, AKM>(a.A, m0, a.B, n0, a.K, acc, smem);
+    gemm_tile_nt<DT, TRLK_HEAD_BK_GEMM, AKM>(A, m0, B, n0, K, acc, smem);
     const float inv_b = 1.f / slot_scale(a.max_b, 1.f);
     const float inv_common = inv_b / slot_scale(a.max_a, a.mult_a);
     // A tile inside the output (nearly every tile): no per-element predicates, addresses as a uniform base plus one
@@ -1195,7 +1212,7 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
             for (int nb = 0; nb < NB; ++nb) {
                 float v[16];
                 if constexpr (MODE != 0) {
-                    float* blk = a.out_f32 + int64_t(row0 + mb * 32) * a.ld_f32 + (col0 + nb * 32);  // uniform
+                    float* blk = out_f32 + int64_t(row0 + mb * 32) * a.ld_f32 + (col0 + nb * 32);  // uniform
                     const uint32_t lane_off = uint32_t(half * 4) * uint32_t(a.ld_f32) + uint32_t(l31);
                     float prev[16];
 #pragma unroll
@@ -1248,7 +1265,7 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int row = m0 + acc_row(wm, mb, r, lane);
-                prev[r] = (MODE != 0 && !a.first && row < a.M) ? a.out_f32[int64_t(row) * a.ld_f32 + col] : 0.f;
+                prev[r] = (MODE != 0 && !a.first && row < a.M) ? out_f32[int64_t(row) * a.ld_f32 + col] : 0.f;
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -1256,7 +1273,7 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
                 if (row >= a.M) continue;
                 const float v = fmaf(acc[mb][nb][r], inv[r], prev[r]);
                 if (MODE == 1)
-                    a.out_f32[int64_t(row) * a.ld_f32 + col] = v;
+                    out_f32[int64_t(row) * a.ld_f32 + col] = v;
                 else
                     E::store1(a.out_lp + int64_t(row) * a.ld_lp + col, v);
             }
@@ -1274,6 +1291,25 @@ TRLK_HEAD_KERNEL void gemm_nt_pair_kernel(GemmArgs a, int grid_a, GemmArgs b) {
         gemm_nt_body<TRLK_F16, MODE_A, ODT, true>(a, blockIdx.x, smem);
     else
         gemm_nt_body<TRLK_F16, 0, ODT>(b, int(blockIdx.x) - grid_a, smem);
+}
+
+// dHidden from the sums of the slices of its contraction, in slice order: out[i] = sum_s parts[s][i], 8 values per lane
+// (n is a multiple of 8).
+template <int ODT>
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float* parts, int slices, int64_t n, uint16_t* out) {
+    const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 8;
+    if (i >= n) return;
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < slices; ++s) {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(parts + s * n + i);
+        const f32x4 hi = *reinterpret_cast<const f32x4*>(parts + s * n + i + 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[k] += lo[k];
+            x[4 + k] += hi[k];
+        }
+    }
+    *reinterpret_cast<u32x4*>(out + i) = Elem<ODT>::pack(x);
 }
 
 // A single product (epilogue 1: fp32 output, overwritten or accumulated into).
@@ -1476,7 +1512,31 @@ struct BwdLayout {
     int64_t ld_v, ld_n, ld_c;    // row strides of [*, vpad], [*, npad], [*, cpad] matrices
     size_t off_wt, off_ht, off_dzt, off_dh, off_max, total;
     int64_t n_chunks;
+    int slices, kslice;  // of the dHidden product's contraction over a chunk
 };
+// Slices of the contraction of the dHidden product.  Its tiles (token blocks x hidden tiles) contract over the whole
+// chunk, tens of times longer than the dW tiles of the same launch, and they are few when there are few tokens: 48 tiles of
+// 788 k steps beside 1576 tiles of 24 for 1396 tokens, H = 2048 and one chunk of 50257 rows, so the launch lasts as long as
+// one of them.  The fewest slices (each costs a write and a read of [N, H] in fp32) that make the tiles' chain shorter than
+// an even share of the whole launch.  Measured there (whole backward): 1 / 2 / 3 / 6 / 16
+// slices 1331 / 854 / 765 / 776 / 858 us, the rule takes 3; 240 tokens, H = 3584, V = 151936: 1 / 3 / 8 / 16 slices 4496 /
+// 2208 / 1478 / 1519 us, the rule takes 7; 2500 tokens: 1 slice, 5.67 ms (3: 5.64, 8: 5.77).
+int dh_slices(int64_t n_tb, int64_t n_ht, int64_t kpad, int64_t npad) {
+    constexpr int64_t kEpilogue = 4, kCuCount = 256;  // a tile's start and epilogue in k steps
+    const int64_t steps = kpad / BK, tiles = n_tb * n_ht;
+    int best = 1;
+    int64_t best_chain = INT64_MAX;
+    for (int64_t s = 1; s <= 32 && steps / s >= 16; ++s) {
+        const int64_t chain = (tiles * s + kCuCount - 1) / kCuCount * ((steps + s - 1) / s + kEpilogue);
+        const int64_t share = (tiles * (steps + s * kEpilogue) + kpad / BM * n_ht * (npad / BK + kEpilogue)) / kCuCount;
+        if (chain < best_chain) {
+            best_chain = chain;
+            best = int(s);
+        }
+        if (chain * 10 <= share * 9) break;
+    }
+    return best;
+}
 BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     BwdLayout l;
     l.vpad = round_up(V, BK);
@@ -1494,7 +1554,10 @@ BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     l.off_wt = take(size_t(H) * l.ld_c * 2);
     l.off_ht = take(size_t(H) * l.ld_n * 2);
     l.off_dzt = take(size_t(l.cpad) * l.ld_n * 2);
-    l.off_dh = take(size_t(N) * H * 4);
+    const int want = dh_slices(l.npad / BN, (H + BN - 1) / BN, l.cpad, l.npad);
+    l.kslice = int(round_up((l.cpad + want - 1) / want, BK));
+    l.slices = int((l.cpad + l.kslice - 1) / l.kslice);
+    l.off_dh = take(size_t(l.slices) * N * H * 4);
     l.n_chunks = (V + l.cpad - 1) / l.cpad;
     l.off_max = take(size_t(2 + l.n_chunks) * 4);  // largest magnitudes: g, hidden, each chunk of W
     l.total = o;
@@ -1727,7 +1790,7 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
     uint16_t* wt = reinterpret_cast<uint16_t*>(ws + l.off_wt);    // [H, cpad], row stride ld_c (one chunk at a time)
     uint16_t* ht = reinterpret_cast<uint16_t*>(ws + l.off_ht);    // [H, npad], row stride ld_n
     uint16_t* dzt = reinterpret_cast<uint16_t*>(ws + l.off_dzt);  // [cpad, npad], row stride ld_n
-    float* dh = reinterpret_cast<float*>(ws + l.off_dh);          // [N, H]
+    float* dh = reinterpret_cast<float*>(ws + l.off_dh);          // [slices][N, H]
     uint32_t* maxima = reinterpret_cast<uint32_t*>(ws + l.off_max);  // [0] g, [1] hidden, [2] W
     const int H = int(hidden_size), N = int(n_tokens), V = int(vocab);
     const bool from_bf16 = dtype == TRLK_BF16;  // the products' operands are fp16: bf16 inputs are converted on the way
@@ -1853,7 +1916,11 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         gh.g_rows = d_g_logp;
         gh.mult_a = zs;
         gh.max_b = max_w;
-        const int ghgrid = xcd_patch_grid(n_tb, n_ht);
+        gh.slices = l.slices;  // (of the last, possibly shorter chunk those that its rows reach)
+        while (gh.slices > 1 && int64_t(gh.slices - 1) * l.kslice >= kpad) --gh.slices;
+        gh.kslice = l.kslice;
+        gh.slice_grid = xcd_patch_grid(n_tb, n_ht);
+        const int ghgrid = gh.slice_grid * gh.slices;
         // dW[chunk, H] = dz^T[chunk, N] * (hidden^T[H, N])^T
         GemmArgs gw{};
         gw.A = Operand{dzt, l.ld_n, kpad};
@@ -1871,13 +1938,23 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         // both products of the chunk in one launch (dHidden's workgroups first)
         const int gwgrid = xcd_patch_grid(n_vt, n_ht);
         const char* what = "fused_head_bwd (dHidden, dW)";
-        if (last)
+        if (last && l.slices == 1)
             rc = from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<2, TRLK_BF16>, ghgrid, gh, gwgrid, gw, s, what)
                            : launch_head_pair(gemm_nt_pair_kernel<2, TRLK_F16>, ghgrid, gh, gwgrid, gw, s, what);
         else
             rc = from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<1, TRLK_BF16>, ghgrid, gh, gwgrid, gw, s, what)
                            : launch_head_pair(gemm_nt_pair_kernel<1, TRLK_F16>, ghgrid, gh, gwgrid, gw, s, what);
         if (rc) return rc;
+    }
+    if (l.slices > 1) {
+        const int64_t n = int64_t(N) * H;
+        const dim3 grid(unsigned((n / 8 + 255) / 256));
+        uint16_t* out = static_cast<uint16_t*>(d_out_dhidden);
+        if (from_bf16)
+            hipLaunchKernelGGL(sum_slices_kernel<TRLK_BF16>, grid, dim3(256), 0, s, dh, l.slices, n, out);
+        else
+            hipLaunchKernelGGL(sum_slices_kernel<TRLK_F16>, grid, dim3(256), 0, s, dh, l.slices, n, out);
+        return launch_status("fused_head_bwd (dHidden)");
     }
     return TRLK_OK;
 }

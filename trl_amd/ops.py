@@ -856,6 +856,20 @@ def gemm_nt(a: Tensor, b: Tensor, out: Optional[Tensor] = None, accumulate: bool
     return out
 
 
+# Vocabulary rows per backward chunk.  Callers' chunk sizes come from a scheme that holds fp32 logits of a chunk; here a
+# chunk costs 2 bytes per row and token (dz) and 2 per row and hidden column (the weight's fp16 copy), and the smaller the
+# chunk the more the products lose in partial rounds of workgroups and in passes over dHidden.  So the caller's size is
+# raised to what this much scratch holds, and the vocabulary is cut into equal chunks.  1396 tokens, H = 2048, V = 50257,
+# chunk_size 8192: one chunk instead of seven, products 1136 -> 575 us (with the slices of the dHidden product), sweeps
+# and transposes 189 -> 126 us.
+_HEAD_SCRATCH_BYTES = 1 << 30
+
+
+def _backward_chunk(n_tokens: int, vocab: int, hidden_size: int, chunk_size: int) -> int:
+    rows = max(int(chunk_size), _HEAD_SCRATCH_BYTES // (2 * ((n_tokens + 255) // 256 * 256 + hidden_size)))
+    return -(-vocab // -(-vocab // rows))
+
+
 def head_backward(hidden: Tensor, weight: Tensor, targets: Tensor, temperature: float, softcap: float,
                   logit_scale: float, log_z: Tensor, g_logp: Tensor, chunk_size: int, bias: Optional[Tensor] = None,
                   stash: Optional[Tensor] = None) -> tuple[Tensor, Tensor, Tensor]:
@@ -865,6 +879,7 @@ def head_backward(hidden: Tensor, weight: Tensor, targets: Tensor, temperature: 
     dropped when at least a tenth of them can go."""
     n = hidden.shape[0]
     g = g_logp.reshape(-1)
+    chunk_size = _backward_chunk(n, weight.shape[0], hidden.shape[-1], chunk_size) if chunk_size >= 1 else chunk_size
     if n == 0 or os.environ.get("TRL_AMD_HEAD_DROP_ZERO_GRAD", "1") == "0":
         return fused_head_bwd(hidden, weight, targets, temperature, softcap, logit_scale, log_z, g, chunk_size, bias, stash)
     active = g != 0
