@@ -319,6 +319,26 @@ int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, const int64_
                         void* d_out_dweight, float* d_out_dbias, void* d_workspace, size_t workspace_bytes,
                         trlk_stream_t stream);
 
+/* Row selection around the fused head: the boolean indexing of hidden states, labels and log-probs by a completion mask
+ * or by labels with an ignored value (trl/trainer/utils.py:1461-1481, sft_trainer.py:160-184) without its scans and sorts.
+ * trlk_select_rows: position e = r * n_cols + c is kept when keep[r * row_stride + c] != skip; d_out_index[j] = the j-th
+ *   kept position (room for n_rows * n_cols), d_out_position[e] = its number or -1, *d_out_count = how many.
+ * trlk_gather_rows: d_out[j] = the row of position d_index[j] = b * n_cols + t, which starts at byte b * seq_stride_bytes +
+ *   t * row_stride_bytes of d_src; d_out_targets[j] = d_targets[b * target_stride + t].
+ * trlk_scatter_rows: row (b, s) of d_out [n_seq, out_cols] = row d_position[b * n_cols + s] of d_src, zero where that is
+ *   -1 and for s >= n_cols.
+ * trlk_scatter_values: the same for one or two fp32 vectors (d_out_b may be null). */
+enum trlk_keep_type { TRLK_KEEP_U8 = 0, TRLK_KEEP_I32 = 1, TRLK_KEEP_I64 = 2, TRLK_KEEP_F32 = 3 };
+int trlk_select_rows(const void* d_keep, int keep_type, int64_t n_rows, int64_t n_cols, int64_t row_stride, int64_t skip,
+                     int32_t* d_out_index, int32_t* d_out_position, int64_t* d_out_count, trlk_stream_t stream);
+int trlk_gather_rows(const void* d_src, int64_t row_bytes, int64_t seq_stride_bytes, int64_t row_stride_bytes, int64_t n_cols,
+                     const int32_t* d_index, int64_t n, void* d_out, const int64_t* d_targets, int64_t target_stride,
+                     int64_t* d_out_targets, trlk_stream_t stream);
+int trlk_scatter_rows(const void* d_src, int64_t row_bytes, const int32_t* d_position, int64_t n_seq, int64_t n_cols,
+                      int64_t out_cols, void* d_out, trlk_stream_t stream);
+int trlk_scatter_values(const float* d_a, const float* d_b, const int32_t* d_position, int64_t n, float* d_out_a,
+                        float* d_out_b, trlk_stream_t stream);
+
 /* fp32 operands of the fused head (the dtype of the reference's own unit test of _ChunkedLogProbFunction,
  * tests/test_utils.py:1161-1232; the reference runs `torch.mm(last_hidden, w_chunk.t())` in the operands'
  * dtype and the two backward products in fp32, trl/trainer/utils.py:1327-1328,1421-1422).  The matrix cores take 16-bit operands, so an

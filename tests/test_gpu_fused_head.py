@@ -731,3 +731,38 @@ def test_backward_with_the_dhidden_contraction_cut_into_slices(amd, dtype, n, h,
         bound = 1.5e-3 if dtype == torch.bfloat16 else 5e-4
         for got, want in ((got_h, want_h), (got_w, want_w)):
             assert _rel_l2(got.float(), want.to(dtype).float()) < bound, (stash, _rel_l2(got.float(), want.to(dtype).float()))
+
+
+@pytest.mark.parametrize("rows,cols,skip,dtype", [
+    (1, 1, 0, torch.bool), (3, 341, 0, torch.int64), (1, 1024, 0, torch.uint8), (5, 205, 0, torch.float32),
+    (7, 2049, -100, torch.int64), (2, 12300, 0, torch.int32), (3, 700, 0, torch.bfloat16),
+])
+@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
+def test_row_selection_gather_and_scatter(amd, rows, cols, skip, dtype, share):
+    """The selection kernels against boolean indexing, exactly: workgroup edges (1024 positions), strided views (the
+    columns 1: of a wider tensor), every element type, nothing and everything kept; rows of 16-byte pieces and not."""
+    g = torch.Generator().manual_seed(rows * cols)
+    wide = (torch.rand(rows, cols + 1, generator=g) < share)
+    if skip:
+        wide = torch.where(wide, torch.randint(0, 9, wide.shape, generator=g), torch.full(wide.shape, skip))
+    keep = wide.to(DEV).to(dtype)[:, 1:]
+    want = (keep != skip).reshape(-1)
+    index, position, count = amd.ops.select_rows(keep, skip)
+    n = int(count)
+    flat = want.nonzero().squeeze(1)
+    assert n == flat.numel() and torch.equal(index[:n].long(), flat)
+    assert torch.equal(position.long(), torch.where(want, want.cumsum(0) - 1, torch.full_like(want, -1, dtype=torch.long)))
+    targets = torch.randint(0, 99, (rows, cols + 1), generator=g).to(DEV)[:, 1:]
+    for h, kind in ((16, torch.bfloat16), (13, torch.float16), (6, torch.float32)):
+        hidden = torch.randn(rows, cols + 2, h, generator=g).to(DEV).to(kind)[:, 1:]
+        got, picked = amd.ops.gather_rows(hidden, targets, index, n)
+        assert torch.equal(got, hidden[:, :cols].reshape(-1, h)[want]) and torch.equal(picked, targets.reshape(-1)[want])
+        back = amd.ops.scatter_rows(got, position, (rows, cols + 1, h), cols)
+        full = torch.zeros(rows, cols + 1, h, dtype=kind, device=DEV)
+        full[:, :cols].view(rows, cols, h)[want.view(rows, cols)] = got
+        assert torch.equal(back, full)
+    v = torch.randn(n, device=DEV)
+    a, b = amd.ops.scatter_values(v, 2 * v, position, (rows, cols))
+    full = torch.zeros(rows * cols, device=DEV)
+    full[want] = v
+    assert torch.equal(a.reshape(-1), full) and torch.equal(b.reshape(-1), 2 * full)

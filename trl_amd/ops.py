@@ -856,6 +856,73 @@ def gemm_nt(a: Tensor, b: Tensor, out: Optional[Tensor] = None, accumulate: bool
     return out
 
 
+# ---- which rows of the hidden states enter the head, and the way back
+_KEEP_TYPES = {torch.bool: 0, torch.uint8: 0, torch.int32: 1, torch.int64: 2, torch.float32: 3}
+
+
+def select_rows(keep: Tensor, skip: int = 0) -> tuple[Tensor, Tensor, Tensor]:
+    """Positions of `keep` `[B, T]` (the last axis contiguous) whose value is not `skip`, in order: `(index, position,
+    count)`, int32 `[B * T]` flat positions of the kept ones (the first `count` entries), int32 `[B * T]` number of every
+    position among them or -1, and the int64 count `[]`, all on the device (`trlk_select_rows`)."""
+    if keep.dtype not in _KEEP_TYPES:
+        keep = keep != skip
+        skip = 0
+    if keep.stride(1) != 1:
+        keep = keep.contiguous()
+    rows, cols = keep.shape
+    n, dev = rows * cols, keep.device
+    if n == 0:
+        none = torch.empty((0,), dtype=torch.int32, device=dev)
+        return none, none, torch.zeros((), dtype=torch.int64, device=dev)
+    buf = torch.empty((2 + 2 * n,), dtype=torch.int32, device=dev)
+    count, index, position = buf[:2].view(torch.int64)[0], buf[2 : 2 + n], buf[2 + n :]
+    with torch.cuda.device(dev):
+        check(lib.trlk_select_rows(ptr(keep), _KEEP_TYPES[keep.dtype], rows, cols, keep.stride(0), skip, ptr(index),
+                                   ptr(position), ptr(count), current_stream(dev)))
+    return index, position, count
+
+
+def gather_rows(hidden: Tensor, targets: Tensor, index: Tensor, n: int) -> tuple[Tensor, Tensor]:
+    """The first `n` positions of `index` out of `hidden[:, :T]` (`[B, S, H]`, S >= T) and `targets` `[B, T]`, packed:
+    `([n, H], [n])` (`trlk_gather_rows`)."""
+    if hidden.stride(2) != 1:
+        hidden = hidden.contiguous()
+    if targets.dtype != torch.int64 or targets.stride(1) != 1:
+        targets = targets.long().contiguous()
+    h, size, dev = hidden.shape[2], hidden.element_size(), hidden.device
+    rows = torch.empty((n, h), dtype=hidden.dtype, device=dev)
+    picked = torch.empty((n,), dtype=torch.int64, device=dev)
+    if n:
+        with torch.cuda.device(dev):
+            check(lib.trlk_gather_rows(ptr(hidden), h * size, hidden.stride(0) * size, hidden.stride(1) * size,
+                                       targets.shape[1], ptr(index), n, ptr(rows), ptr(targets), targets.stride(0),
+                                       ptr(picked), current_stream(dev)))
+    return rows, picked
+
+
+def scatter_rows(rows: Tensor, position: Tensor, shape: tuple[int, int, int], cols: int) -> Tensor:
+    """`[B, S, H] = shape`: packed `rows` `[n, H]` at the places `position` (`[B * cols]`) gives them, zeros elsewhere
+    (`trlk_scatter_rows`)."""
+    out = torch.empty(shape, dtype=rows.dtype, device=rows.device)
+    if position.numel() == 0 or rows.numel() == 0:
+        return out.zero_()
+    with torch.cuda.device(rows.device):
+        check(lib.trlk_scatter_rows(ptr(rows), shape[2] * rows.element_size(), ptr(position), shape[0], cols, shape[1],
+                                    ptr(out), current_stream(rows.device)))
+    return out
+
+
+def scatter_values(a: Tensor, b: Optional[Tensor], position: Tensor, shape: tuple[int, int]) -> tuple[Tensor, Optional[Tensor]]:
+    """Packed fp32 `[n]` vectors at the places `position` gives them, zeros elsewhere, as `shape` (`trlk_scatter_values`)."""
+    out_a = torch.empty(shape, dtype=torch.float32, device=a.device)
+    out_b = None if b is None else torch.empty(shape, dtype=torch.float32, device=a.device)
+    if position.numel():
+        with torch.cuda.device(a.device):
+            check(lib.trlk_scatter_values(ptr(a), ptr(b), ptr(position), position.numel(), ptr(out_a), ptr(out_b),
+                                          current_stream(a.device)))
+    return out_a, out_b
+
+
 # Vocabulary rows per backward chunk.  Callers' chunk sizes come from a scheme that holds fp32 logits of a chunk; here a
 # chunk costs 2 bytes per row and token (dz) and 2 per row and hidden column (the weight's fp16 copy), and the smaller the
 # chunk the more the products lose in partial rounds of workgroups and in passes over dHidden.  So the caller's size is
@@ -872,15 +939,16 @@ def _backward_chunk(n_tokens: int, vocab: int, hidden_size: int, chunk_size: int
 
 def head_backward(hidden: Tensor, weight: Tensor, targets: Tensor, temperature: float, softcap: float,
                   logit_scale: float, log_z: Tensor, g_logp: Tensor, chunk_size: int, bias: Optional[Tensor] = None,
-                  stash: Optional[Tensor] = None) -> tuple[Tensor, Tensor, Tensor]:
+                  stash: Optional[Tensor] = None, look_for_zeros: bool = True) -> tuple[Tensor, Tensor, Tensor]:
     """`fused_head_bwd` that first drops the tokens whose upstream gradient is exactly zero (masked positions of
     a policy loss): their dz row is zero, so they add nothing to d weight and their d hidden row is zero.  Both
     products shrink with the share of such tokens; one host synchronisation (the count) per call.  Tokens are only
-    dropped when at least a tenth of them can go."""
+    dropped when at least a tenth of them can go.  `look_for_zeros=False`: the caller knows that
+    its loss leaves no token without a gradient."""
     n = hidden.shape[0]
     g = g_logp.reshape(-1)
     chunk_size = _backward_chunk(n, weight.shape[0], hidden.shape[-1], chunk_size) if chunk_size >= 1 else chunk_size
-    if n == 0 or os.environ.get("TRL_AMD_HEAD_DROP_ZERO_GRAD", "1") == "0":
+    if n == 0 or not look_for_zeros or os.environ.get("TRL_AMD_HEAD_DROP_ZERO_GRAD", "1") == "0":
         return fused_head_bwd(hidden, weight, targets, temperature, softcap, logit_scale, log_z, g, chunk_size, bias, stash)
     active = g != 0
     n_active = int(active.sum())

@@ -18,24 +18,16 @@ from torch import Tensor
 
 from .. import ops
 from .grpo_trainer import _METRIC_INDEX, grpo_loss
-from .utils import _ChunkedLogProbFunction
+from .utils import _masked_head
 
 __all__ = ["FusedLinearGRPOLoss", "FusedLinearDPOLoss", "FusedLinearKTOLoss"]
 
 
 def _head_logps(hidden: Tensor, weight: Tensor, targets: Tensor, keep: Tensor, temperature: float,
-                chunk_size: int, bias: Tensor | None = None) -> Tensor:
+                chunk_size: int, bias: Tensor | None = None, skip: int = 0, may_clip: bool = False) -> Tensor:
     """fp32 log-probs of `targets` `[B, T]` under `softmax((hidden @ weight.T + bias) / temperature)`; only the
-    rows with `keep != 0` go through the head, the others are 0 (and receive no gradient)."""
-    b, t, h = hidden.shape
-    sel = keep.reshape(b * t) != 0
-    flat_h = hidden.reshape(b * t, h)[sel]
-    flat_t = targets.reshape(b * t)[sel]
-    lp_v, _ = _ChunkedLogProbFunction.apply(flat_h, weight, flat_t, float(temperature), int(chunk_size), None, 1.0,
-                                            bias)
-    lp = torch.zeros(b * t, dtype=torch.float32, device=hidden.device)
-    lp[sel] = lp_v
-    return lp.view(b, t)
+    rows with `keep != skip` go through the head, the others are 0 (and receive no gradient)."""
+    return _masked_head(hidden, weight, targets, keep, temperature, chunk_size, bias=bias, skip=skip, may_clip=may_clip)[0]
 
 
 class FusedLinearGRPOLoss(torch.nn.Module):
@@ -77,7 +69,8 @@ class FusedLinearGRPOLoss(torch.nn.Module):
         if self.beta != 0.0 and ref_per_token_logps is None:
             raise ValueError("ref_per_token_logps is required when beta != 0")
         mask = attention_mask
-        logps = _head_logps(_input, lin_weight, selected_token_ids, mask, self.temperature, self.chunk_size, bias)
+        logps = _head_logps(_input, lin_weight, selected_token_ids, mask, self.temperature, self.chunk_size, bias,
+                            may_clip=True)
         n_items = mask.sum().float()
         n_proc = 1
         if torch.distributed.is_available() and torch.distributed.is_initialized():
@@ -134,14 +127,13 @@ class FusedLinearDPOLoss(torch.nn.Module):
             raise ValueError("_input must be [2P, T, H]: chosen sequences first, rejected second")
         pairs = _input.shape[0] // 2
         keep = target != self.ignore_index
-        labels = torch.where(keep, target, torch.zeros_like(target))
-        logps = _head_logps(_input, lin_weight, labels, keep, 1.0, self.chunk_size, bias)
+        logps = _head_logps(_input, lin_weight, target, target, 1.0, self.chunk_size, bias, self.ignore_index)
         if self.use_ref_model:
             if ref_input is None:
                 raise ValueError("ref_input is required when use_ref_model=True")
             with torch.no_grad():
-                ref_logps = _head_logps(ref_input, lin_weight if ref_weight is None else ref_weight, labels, keep, 1.0,
-                                        self.chunk_size, bias if ref_weight is None else ref_bias)
+                ref_logps = _head_logps(ref_input, lin_weight if ref_weight is None else ref_weight, target, target, 1.0,
+                                        self.chunk_size, bias if ref_weight is None else ref_bias, self.ignore_index)
                 ref_seq = (ref_logps * keep).sum(-1)
         else:
             ref_seq = torch.zeros(2 * pairs, dtype=torch.float32, device=_input.device)
@@ -198,14 +190,14 @@ class FusedLinearKTOLoss(torch.nn.Module):
             raise ValueError("preference_labels must hold one entry per sequence")
         dev = _input.device
         keep = target != self.ignore_index
-        labels = torch.where(keep, target, torch.zeros_like(target))
-        seq = (_head_logps(_input, lin_weight, labels, keep, 1.0, self.chunk_size, bias) * keep).sum(-1)
+        seq = (_head_logps(_input, lin_weight, target, target, 1.0, self.chunk_size, bias, self.ignore_index) * keep).sum(-1)
         if self.use_ref_model:
             if ref_input is None:
                 raise ValueError("ref_input is required when use_ref_model=True")
             with torch.no_grad():
-                ref_seq = (_head_logps(ref_input, lin_weight if ref_weight is None else ref_weight, labels, keep, 1.0,
-                                       self.chunk_size, bias if ref_weight is None else ref_bias) * keep).sum(-1)
+                ref_seq = (_head_logps(ref_input, lin_weight if ref_weight is None else ref_weight, target, target, 1.0,
+                                       self.chunk_size, bias if ref_weight is None else ref_bias,
+                                       self.ignore_index) * keep).sum(-1)
         else:
             ref_seq = torch.zeros_like(seq)
         chosen = torch.as_tensor(preference_labels, dtype=torch.bool, device=dev)

@@ -214,38 +214,98 @@ class _ChunkedLogProbFunction(torch.autograd.Function):
     def forward(ctx, last_hidden, weight, targets, temperature, chunk_size, final_logit_softcapping=None,
                 logit_scale=1.0, bias=None):
         cap = 0.0 if final_logit_softcapping is None else float(final_logit_softcapping)
-        if last_hidden.dtype == torch.float32:
-            if not last_hidden.is_cuda:
-                raise NotImplementedError("the fused head runs on the GPU only")
-            w32 = weight.float()
-            logp, ent, log_z = _fp32_head_forward(last_hidden, w32, targets.long(), float(temperature), cap,
-                                                  float(logit_scale), None if bias is None else bias.float())
-            ctx.save_for_backward(last_hidden, weight, targets, log_z, bias, None)
-            ctx.cfg = (float(temperature), int(chunk_size), cap, float(logit_scale))
-            ctx.mark_non_differentiable(ent)
-            return logp, ent
-        stash = any(ctx.needs_input_grad[:2]) and ops.head_stash_fits(last_hidden.shape[0], weight.shape[0])
-        logp, ent, log_z, _, saved = ops.fused_head_fwd(last_hidden, weight, targets, float(temperature), cap,
-                                                        float(logit_scale), bias, stash)
+        cfg = (float(temperature), int(chunk_size), cap, float(logit_scale))
+        logp, ent, log_z, _, saved = _head_forward(last_hidden, weight, targets, bias, cfg, any(ctx.needs_input_grad[:2]))
         ctx.save_for_backward(last_hidden, weight, targets, log_z, bias, saved)
-        ctx.cfg = (float(temperature), int(chunk_size), cap, float(logit_scale))
+        ctx.cfg = cfg
         ctx.mark_non_differentiable(ent)
         return logp, ent
 
     @staticmethod
     def backward(ctx, grad_logprobs, grad_entropy):
-        hidden, weight, targets, log_z, bias, saved = ctx.saved_tensors
-        temperature, chunk_size, cap, logit_scale = ctx.cfg
-        if hidden.dtype == torch.float32:
-            d_hidden, d_weight, d_bias = _fp32_head_backward(hidden, weight.float(), targets.long(), temperature, cap,
-                                                             logit_scale, None if bias is None else bias.float(), log_z,
-                                                             grad_logprobs)
-            return (d_hidden, d_weight.to(weight.dtype), None, None, None, None, None,
-                    None if bias is None else d_bias.to(bias.dtype))
+        d_hidden, d_weight, d_bias = _head_backward(*ctx.saved_tensors, ctx.cfg, grad_logprobs)
+        return d_hidden, d_weight, None, None, None, None, None, d_bias
+
+
+def _head_forward(hidden, weight, targets, bias, cfg, keep_products):
+    """`(logp, entropy, log_z, target_is_max, stash or None)`, fp32 `[N]` each; `cfg` = (temperature, chunk size, soft
+    cap or 0, logit scale).  `keep_products`: a backward will follow."""
+    temperature, _, cap, logit_scale = cfg
+    if hidden.dtype == torch.float32:  # fp32 operands: three bf16 pieces each through the same kernels
+        if not hidden.is_cuda:
+            raise NotImplementedError("the fused head runs on the GPU only")
+        return (*_fp32_head_forward(hidden, weight.float(), targets.long(), temperature, cap, logit_scale,
+                                    None if bias is None else bias.float(), True), None)
+    stash = keep_products and ops.head_stash_fits(hidden.shape[0], weight.shape[0])
+    return ops.fused_head_fwd(hidden, weight, targets, temperature, cap, logit_scale, bias, stash)
+
+
+def _head_backward(hidden, weight, targets, log_z, bias, saved, cfg, grad_logprobs, look_for_zeros=True):
+    """`(d hidden, d weight, d bias or None)` in the operands' dtypes."""
+    temperature, chunk_size, cap, logit_scale = cfg
+    if hidden.dtype == torch.float32:
+        d_hidden, d_weight, d_bias = _fp32_head_backward(hidden, weight.float(), targets.long(), temperature, cap,
+                                                         logit_scale, None if bias is None else bias.float(), log_z,
+                                                         grad_logprobs)
+        d_weight = d_weight.to(weight.dtype)
+    else:
         d_hidden, d_weight, d_bias = ops.head_backward(hidden, weight, targets, temperature, cap, logit_scale,
-                                                        log_z, grad_logprobs, chunk_size, bias, saved)
-        return (d_hidden, d_weight, None, None, None, None, None,
-                None if bias is None else d_bias.to(bias.dtype))
+                                                        log_z, grad_logprobs, chunk_size, bias, saved, look_for_zeros)
+    return d_hidden, d_weight, None if bias is None else d_bias.to(bias.dtype)
+
+
+class _MaskedHeadFunction(torch.autograd.Function):
+    """The head on some of the positions of `hidden` `[B, S, H]`: `targets` `[B, T]` (T <= S) belong to its first T
+    positions, those whose `keep` `[B, T]` is not `skip` go through it.  Returns fp32 log-probs, entropies (both `[B, T]`,
+    0 at the other positions, or packed `[n]` with `packed`) and argmax hits (packed), and the count as a device scalar.
+    Only the log-probs are differentiable."""
+
+    @staticmethod
+    def forward(ctx, hidden, weight, bias, targets, keep, skip, cfg, packed, may_clip, with_grad):
+        index, position, count = ops.select_rows(keep, skip)
+        n = int(count)  # (the one synchronisation: the packed tensors' size)
+        rows, picked = ops.gather_rows(hidden, targets, index, n)
+        logp, ent, log_z, hit, saved = _head_forward(rows, weight, picked, bias, cfg,
+                                                     with_grad and any(ctx.needs_input_grad[:2]))
+        ctx.save_for_backward(rows, weight, picked, log_z, bias, saved, index, position)
+        ctx.cfg, ctx.shape, ctx.cols, ctx.packed = cfg, tuple(hidden.shape), targets.shape[1], packed
+        # tokens that a loss clipped are worth looking for (a synchronisation, about 50 us) where the backward takes
+        # some milliseconds; masked ones are not among the packed rows
+        ctx.look_for_zeros = may_clip and 4 * n * weight.numel() > 2e12
+        if not packed:
+            logp, ent = ops.scatter_values(logp, ent, position, tuple(targets.shape))
+        ctx.mark_non_differentiable(ent, hit, count)
+        ctx.set_materialize_grads(False)
+        return logp, ent, hit, count
+
+    @staticmethod
+    def backward(ctx, g_logp, g_ent, g_hit, g_count):
+        if g_logp is None:
+            return (None,) * 10
+        *operands, index, position = ctx.saved_tensors
+        n = operands[0].shape[0]
+        g = g_logp if ctx.packed else g_logp.reshape(-1).index_select(0, index[:n])
+        d_rows, d_weight, d_bias = _head_backward(*operands, ctx.cfg, g, ctx.look_for_zeros)
+        d_hidden = ops.scatter_rows(d_rows, position, ctx.shape, ctx.cols) if ctx.needs_input_grad[0] else None
+        return d_hidden, d_weight, d_bias, None, None, None, None, None, None, None
+
+
+def _masked_head(hidden: Tensor, weight: Tensor, targets: Tensor, keep: Tensor, temperature: float, chunk_size: int,
+                 softcap: float | None = None, logit_scale: float = 1.0, bias: Tensor | None = None, skip: int = 0,
+                 packed: bool = False, may_clip: bool = True):
+    """See `_MaskedHeadFunction`; the products are kept for a backward only where one can follow (under `no_grad` the
+    operands may still be parameters).  `may_clip=False`: the loss gives every token that enters a gradient."""
+    if not hidden.is_cuda:
+        raise NotImplementedError("the fused head runs on the GPU only")
+    if keep.shape != targets.shape or targets.shape[0] != hidden.shape[0] or targets.shape[1] > hidden.shape[1]:
+        raise ValueError(f"fused head: hidden {tuple(hidden.shape)}, targets {tuple(targets.shape)} and mask "
+                         f"{tuple(keep.shape)} do not match")
+    if any(t.device != hidden.device for t in (weight, targets, keep)):
+        raise ValueError("fused head: the operands are on different devices")
+    cap = 0.0 if softcap is None else float(softcap)
+    return _MaskedHeadFunction.apply(hidden, weight, bias, targets, keep, skip,
+                                     (float(temperature), int(chunk_size), cap, float(logit_scale)), packed,
+                                     may_clip, torch.is_grad_enabled())
 
 
 def chunked_logprobs_from_hidden(hidden_states: Tensor, lm_head_weight: Tensor, labels: Tensor,
@@ -254,25 +314,15 @@ def chunked_logprobs_from_hidden(hidden_states: Tensor, lm_head_weight: Tensor, 
     """The tensor part of the reference's patched forward (utils.py:1449-1484): shift by one, keep only
     completion rows, run the fused head on them, scatter into zero-filled `[B, S-1]` outputs.
     Returns `(log_probs, entropy)`."""
-    hs = hidden_states[:, :-1, :]
     lab = labels[:, 1:]
-    b, s, h = hs.shape
-    flat_h = hs.reshape(b * s, h)
-    flat_t = lab.reshape(b * s)
-    keep = None
     if completion_mask is not None:
-        keep = completion_mask[:, 1:].bool().reshape(b * s)
-        flat_h = flat_h[keep]
-        flat_t = flat_t[keep]
-    lp_v, ent_v = _ChunkedLogProbFunction.apply(flat_h, lm_head_weight, flat_t, temperature, chunk_size,
-                                                final_logit_softcapping, logit_scale)
-    if keep is None:
-        return lp_v.reshape(b, s), ent_v.reshape(b, s)
-    lp = torch.zeros(b * s, device=lp_v.device, dtype=lp_v.dtype)
-    ent = torch.zeros(b * s, device=ent_v.device, dtype=ent_v.dtype)
-    lp[keep] = lp_v
-    ent[keep] = ent_v
-    return lp.reshape(b, s), ent.reshape(b, s)
+        return _masked_head(hidden_states, lm_head_weight, lab, completion_mask[:, 1:], temperature, chunk_size,
+                            final_logit_softcapping, logit_scale)[:2]
+    hs = hidden_states[:, :-1, :]
+    b, s, h = hs.shape
+    lp_v, ent_v = _ChunkedLogProbFunction.apply(hs.reshape(b * s, h), lm_head_weight, lab.reshape(b * s), temperature,
+                                                chunk_size, final_logit_softcapping, logit_scale)
+    return lp_v.reshape(b, s), ent_v.reshape(b, s)
 
 
 def patch_chunked_lm_head(model: torch.nn.Module, chunk_size: int, temperature: float,
