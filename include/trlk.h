@@ -339,6 +339,15 @@ int trlk_scatter_rows(const void* d_src, int64_t row_bytes, const int32_t* d_pos
 int trlk_scatter_values(const float* d_a, const float* d_b, const int32_t* d_position, int64_t n, float* d_out_a,
                         float* d_out_b, trlk_stream_t stream);
 
+/* Mean logit of every sequence over its rows and the whole vocabulary, without logits (the logged mean logits of the
+ * fused-linear preference losses, trl/trainer/dpo_trainer.py:1293-1301): d_out [n_seq, trlk_mean_logits_chunks(rows)] sums
+ * to it over its second axis.  hidden [n_seq, rows_per_seq, hidden_size] (strides in elements), weight [vocab, hidden_size]. */
+size_t trlk_mean_logits_workspace_bytes(int64_t hidden_size);
+int64_t trlk_mean_logits_chunks(int64_t rows_per_seq);
+int trlk_mean_logits(const void* d_hidden, const void* d_weight, int dtype, int64_t n_seq, int64_t rows_per_seq, int64_t vocab,
+                     int64_t hidden_size, int64_t seq_stride, int64_t row_stride, int64_t weight_stride, float* d_out,
+                     void* d_workspace, size_t workspace_bytes, trlk_stream_t stream);
+
 /* fp32 operands of the fused head (the dtype of the reference's own unit test of _ChunkedLogProbFunction,
  * tests/test_utils.py:1161-1232; the reference runs `torch.mm(last_hidden, w_chunk.t())` in the operands'
  * dtype and the two backward products in fp32, trl/trainer/utils.py:1327-1328,1421-1422).  The matrix cores take 16-bit operands, so an

@@ -175,3 +175,19 @@ def test_fused_linear_kto_loss(amd, kl):
         assert abs(float(got) - float(want)) <= 2e-3 * max(1.0, abs(float(want))), (float(got), float(want))
     for got, want in ((dh, oh), (dw, ow), (db, ob)):
         assert _rel_l2(got.grad.float(), want.grad) < 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,t,h,v", [(1, 1, 8, 1), (3, 17, 72, 513), (2, 130, 2056, 4103), (2, 16, 264, 512)])
+def test_mean_logits(amd, dtype, b, t, h, v):
+    """Column sums and row products against float64: hidden sizes around 2048 columns and 64-lane waves, row counts around
+    the 16 of a workgroup, vocabularies around the 512 partial sums.  fp32 sums: 1e-6 of the terms' magnitudes."""
+    g = torch.Generator().manual_seed(b + t + h + v)
+    wide = torch.randn(b, t + 1, h, generator=g).to(dtype)
+    weight = torch.randn(v, h, generator=g).to(dtype)
+    got = amd.ops.mean_logits(wide.to(DEV)[:, 1:], weight.to(DEV))
+    terms = wide[:, 1:].double(), weight.double()
+    want = (terms[0] @ terms[1].sum(0)).mean(1) / v
+    scale = (terms[0].abs() @ terms[1].abs().sum(0)).mean(1) / v
+    assert got.dtype == torch.float32 and got.shape == (b,)
+    assert bool(((got.cpu().double() - want).abs() <= 1e-6 * scale).all())

@@ -108,6 +108,13 @@ SIGNATURES = {
     ),
     "trlk_scatter_rows": (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
     "trlk_scatter_values": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
+    "trlk_mean_logits_workspace_bytes": (c_size_t, [c_int64]),
+    "trlk_mean_logits_chunks": (c_int64, [c_int64]),
+    "trlk_mean_logits": (
+        c_int32,
+        [c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+         c_size_t, c_void_p],
+    ),
     "trlk_rloo_loss": (
         c_int32,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_float, c_float, c_void_p, c_void_p, c_void_p,

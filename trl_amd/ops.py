@@ -923,6 +923,25 @@ def scatter_values(a: Tensor, b: Optional[Tensor], position: Tensor, shape: tupl
     return out_a, out_b
 
 
+def mean_logits(hidden: Tensor, weight: Tensor) -> Tensor:
+    """`(hidden @ weight.T).mean((1, 2))` in fp32 for `hidden` `[B, T, H]`, `weight` `[V, H]`, without the logits
+    (`trlk_mean_logits`; operands it does not take, fp32 ones among them, go through a torch product)."""
+    b, t, h = hidden.shape
+    if (hidden.dtype not in (torch.bfloat16, torch.float16) or weight.dtype != hidden.dtype or h % 8 or not b * t
+            or hidden.stride(2) != 1 or weight.stride(1) != 1 or (hidden.stride(0) | hidden.stride(1) | weight.stride(0)) % 8
+            or weight.stride(0) < h or (hidden.data_ptr() | weight.data_ptr()) % 16):
+        return (hidden.float() @ weight.float().sum(0)).mean(dim=1) / weight.shape[0]
+    dev = hidden.device
+    ws_bytes = lib.trlk_mean_logits_workspace_bytes(h)
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+    out = torch.empty((b, lib.trlk_mean_logits_chunks(t)), dtype=torch.float32, device=dev)
+    with torch.cuda.device(dev):
+        check(lib.trlk_mean_logits(ptr(hidden), ptr(weight), dtype_code(hidden.dtype), b, t, weight.shape[0], h,
+                                   hidden.stride(0), hidden.stride(1), weight.stride(0), ptr(out), ptr(ws), ws_bytes,
+                                   current_stream(dev)))
+    return out.sum(dim=1)
+
+
 # Vocabulary rows per backward chunk.  Callers' chunk sizes come from a scheme that holds fp32 logits of a chunk; here a
 # chunk costs 2 bytes per row and token (dz) and 2 per row and hidden column (the weight's fp16 copy), and the smaller the
 # chunk the more the products lose in partial rounds of workgroups and in passes over dHidden.  So the caller's size is

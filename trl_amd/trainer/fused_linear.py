@@ -154,8 +154,7 @@ class FusedLinearDPOLoss(torch.nn.Module):
             loss = per_pair.mean()
         with torch.no_grad():
             seq = seq.detach()
-            wsum = lin_weight.float().sum(0)
-            logits_mean = (_input.float() @ wsum).mean(dim=1) / lin_weight.shape[0]  # [2P], over T and V
+            logits_mean = ops.mean_logits(_input, lin_weight)  # [2P], over T and V
             if bias is not None:
                 logits_mean = logits_mean + bias.float().mean()
             rewards = self.beta * (seq - ref_seq)
@@ -208,8 +207,7 @@ class FusedLinearKTOLoss(torch.nn.Module):
         loss = per_example.mean()
         with torch.no_grad():
             c = chosen.to(torch.float32)
-            wsum = lin_weight.float().sum(0)
-            logits_mean = (_input.float() @ wsum).mean(dim=1) / lin_weight.shape[0]
+            logits_mean = ops.mean_logits(_input, lin_weight)
             if bias is not None:
                 logits_mean = logits_mean + bias.float().mean()
             rewards = self.beta * lr.detach()
