@@ -339,6 +339,20 @@ int trlk_scatter_rows(const void* d_src, int64_t row_bytes, const int32_t* d_pos
 int trlk_scatter_values(const float* d_a, const float* d_b, const int32_t* d_position, int64_t n, float* d_out_a,
                         float* d_out_b, trlk_stream_t stream);
 
+/* What a trainer logs of trlk_grpo_loss's metrics, in one vector of TRLK_GRPO_LOG_VALUES floats: the sums that processes add
+ * up (KL, entropy, mask, clip count, aux, aux count, and the low / high / region clip sums), the smallest low and the largest
+ * high clip ratio of a sequence, the policy loss, the error word (trl/trainer/grpo_trainer.py:3212-3258). */
+#define TRLK_GRPO_LOG_VALUES 13
+int trlk_grpo_log_values(const float* d_metrics, const int32_t* d_error_flag, float* d_out, trlk_stream_t stream);
+
+/* The completion mask as fp32 [n_seq, seq_len] (d_out_mask may be null) and the factor that trlk_grpo_fused_fwd_bwd takes as
+ * d_row_scale: numerator / max(active tokens of the sequence, 1) for TRLK_GRPO, of the batch for TRLK_BNPO, numerator /
+ * max(*d_n_items, 1) for TRLK_DAPO, the numerator itself for TRLK_DR_GRPO; times *d_upstream unless that is null.
+ * mask_type: enum trlk_keep_type; strides in elements. */
+int trlk_grpo_row_scale(const void* d_mask, int mask_type, int64_t n_seq, int64_t seq_len, int64_t stride_b, int64_t stride_t,
+                        int loss_type, float numerator, const float* d_n_items, const float* d_upstream, float* d_out_mask,
+                        float* d_out_scale, trlk_stream_t stream);
+
 /* Mean logit of every sequence over its rows and the whole vocabulary, without logits (the logged mean logits of the
  * fused-linear preference losses, trl/trainer/dpo_trainer.py:1293-1301): d_out [n_seq, trlk_mean_logits_chunks(rows)] sums
  * to it over its second axis.  hidden [n_seq, rows_per_seq, hidden_size] (strides in elements), weight [vocab, hidden_size]. */

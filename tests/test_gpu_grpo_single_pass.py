@@ -1010,3 +1010,40 @@ def test_trainer_divisor_is_folded_into_the_forward(amd, monkeypatch, grad_accum
                 assert torch.equal(leaf.grad, before), (divides, grad_accum, loss_type)
             grads[single] = leaf.grad
         assert _rel_l2(grads[True], grads[False]) < 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8, torch.int32, torch.int64, torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 255), (5, 257), (300, 7), (2, 0)])
+def test_row_scale_and_fp32_mask(amd, dtype, shape):
+    """Mask in fp32 and per-sequence factor of every normalisation, for mask types, strided masks and sequence counts on
+    both sides of a workgroup, against float64 (sums of zeros and ones are exact: two roundings)."""
+    from trl_amd import _lib, ops
+
+    B, T = shape
+    g = torch.Generator().manual_seed(B * 1000 + T)
+    wide = (torch.rand(B, 2 * T + 3, generator=g) < 0.6).to(dtype).to(DEV)
+    if B > 1:
+        wide[1] = 0  # a sequence without active tokens: its count is taken as 1
+    for mask in (wide[:, :T].contiguous(), wide[:, 3 : 3 + T], wide[:, : 2 * T : 2]):
+        want = mask.double()
+        n_items = torch.tensor(float(want.sum()) + 0.5, device=DEV)
+        up = torch.tensor(8.0, device=DEV)
+        rows = {_lib.GRPO: 0.25 / want.sum(1).clamp(min=1), _lib.BNPO: (0.25 / want.sum().clamp(min=1)).expand(B),
+                _lib.DR_GRPO: torch.full((B,), 0.25, device=DEV, dtype=torch.float64),
+                _lib.DAPO: (0.25 / n_items.double().clamp(min=1)).expand(B)}
+        for code, scale in rows.items():
+            for factor in (None, up):
+                got_mask, got = ops.grpo_row_scale(mask, code, 0.25, n_items, factor)
+                assert got_mask.dtype == torch.float32 and torch.equal(got_mask.double(), want)
+                torch.testing.assert_close(got.double(), scale * (1.0 if factor is None else 8.0), rtol=1.5e-7, atol=0)
+
+
+def test_log_values_are_the_metrics(amd):
+    from trl_amd import _lib, ops
+
+    m = torch.arange(_lib.GRPO_NUM_METRICS, dtype=torch.float32, device=DEV) + 0.5
+    for count in (0.0, 12.5):
+        m[12] = count
+        got = ops.grpo_log_values(m).tolist()
+        c = max(count, 1.0)
+        assert got == [9.5, 10.5, 8.5, count, 13.5, 14.5, 2.5 * c, 3.5 * c, 4.5 * c, 5.5, 6.5, 7.5, 0.0]

@@ -22,6 +22,7 @@ TERM_CLIP, TERM_CISPO, TERM_SAPO, TERM_WEIGHTED_LOGP = 0, 1, 2, 3
 SCALE_GROUP, SCALE_BATCH, SCALE_NONE = 0, 1, 2
 FLAG_INDEX_OUT_OF_RANGE = 1
 GRPO_NUM_METRICS = 16
+GRPO_LOG_VALUES = 13
 DPO_NUM_METRICS = 8
 RLOO_NUM_METRICS = 8
 
@@ -108,6 +109,12 @@ SIGNATURES = {
     ),
     "trlk_scatter_rows": (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
     "trlk_scatter_values": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
+    "trlk_grpo_log_values": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p]),
+    "trlk_grpo_row_scale": (
+        c_int32,
+        [c_void_p, c_int32, c_int64, c_int64, c_int64, c_int64, c_int32, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p],
+    ),
     "trlk_mean_logits_workspace_bytes": (c_size_t, [c_int64]),
     "trlk_mean_logits_chunks": (c_int64, [c_int64]),
     "trlk_mean_logits": (

@@ -62,6 +62,28 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     return r;
 }
 
+// N block-wide sums at once: two barriers in all instead of two each, every sum with the combination order (and so the
+// bits) of block_sum.  `scratch` holds [N][NT/64] floats.
+template <int NT, int N>
+__device__ __forceinline__ void block_sums(float (&v)[N], float (*scratch)[NT / kWave]) {
+    constexpr int NW = NT / kWave;
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = wave_sum(v[j]);
+    __syncthreads();  // protects scratch against the previous use
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) scratch[j][threadIdx.x / kWave] = v[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        float r = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) r += scratch[j][w];
+        v[j] = r;
+    }
+}
+
 // Storage-dtype traits: EPV = elements in one 16-byte vector.
 template <int DT>
 struct Elem;

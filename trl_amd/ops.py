@@ -572,6 +572,36 @@ def scale_unless_one_(data: Tensor, scale: Tensor) -> Tensor:
 # --------------------------------------------------------------------------------------------
 # DPO / RLOO sequence losses (K4)
 # --------------------------------------------------------------------------------------------
+def grpo_log_values(metrics: Tensor) -> Tensor:
+    """What `_compute_loss` logs of the loss kernel's `metrics`, as one fp32 device vector (`trlk_grpo_log_values`): nine
+    sums to be added over the processes, the smallest and the largest clip ratio, the policy loss, the error word."""
+    dev = metrics.device
+    out = torch.empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32, device=dev)
+    with torch.cuda.device(dev):
+        check(lib.trlk_grpo_log_values(ptr(metrics), ptr(_error_flag(dev)), ptr(out), current_stream(dev)))
+    return out
+
+
+def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Optional[Tensor] = None,
+                   upstream: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
+    """`(mask in fp32, d loss / d masked token loss [B])` of a `[B, T]` mask (`trlk_grpo_row_scale`); `n_items` and
+    `upstream` are fp32 device scalars."""
+    B, T = mask.shape
+    dev = mask.device
+    if not mask.is_cuda or any(t is not None and t.device != dev for t in (n_items, upstream)):
+        raise ValueError("grpo_row_scale: the mask and the scalars must be on one GPU")
+    if mask.dtype not in _KEEP_TYPES:
+        mask = mask.float()
+    as_is = mask.dtype == torch.float32 and mask.is_contiguous()
+    mask_f = mask if as_is else torch.empty((B, T), dtype=torch.float32, device=dev)
+    scale = torch.empty((B,), dtype=torch.float32, device=dev)
+    with torch.cuda.device(dev):
+        check(lib.trlk_grpo_row_scale(ptr(mask), _KEEP_TYPES[mask.dtype], B, T, mask.stride(0), mask.stride(1), loss_type,
+                                      numerator, ptr(n_items), ptr(upstream), None if as_is else ptr(mask_f), ptr(scale),
+                                      current_stream(dev)))
+    return mask_f, scale
+
+
 @torch.library.custom_op("trl_amd::dpo_loss", mutates_args=(), device_types="cuda")
 def dpo_loss_op(token_logp: Tensor, mask: Tensor, ref_chosen: Tensor, ref_rejected: Tensor, beta: float
                 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:

@@ -278,28 +278,10 @@ class _GRPOFromLogits(torch.autograd.Function):
             if keep_start < 0 or keep_start + keep_len > length:
                 raise ValueError("grpo_loss_from_logits: keep_start + K exceeds the logits' rows")
         ids = completion_ids[:, -keep_len:] if keep_len > 0 else completion_ids[:, :0]
-        mask_f = mask[:, -keep_len:].float() if keep_len > 0 else mask[:, :0].float()
+        mask = mask[:, -keep_len:] if keep_len > 0 else mask[:, :0]
         n_seq = logits.shape[0]
         reduce_code, term_code = ops.LOSS_TYPES[kw["loss_type"]]
         ga = 1.0 if reduce_code == _lib.DAPO else float(kw["grad_accum_steps"])
-        # d loss / d (masked token loss of sequence b): what the loss kernel's second pass applies to its rows
-        if reduce_code == _lib.GRPO:
-            row_scale = (1.0 / n_seq) / ga / mask_f.sum(dim=1).clamp(min=1.0)
-        elif reduce_code == _lib.BNPO:
-            row_scale = ((1.0 / mask_f.sum().clamp(min=1.0)) / ga).expand(n_seq)
-        elif reduce_code == _lib.DR_GRPO:
-            row_scale = torch.full((n_seq,), (1.0 / float(n_seq * kw["max_completion_length"])) / ga, device=logits.device)
-        else:  # DAPO
-            n_items = kw["num_items_in_batch"]
-            n_items = (n_items.to(device=logits.device, dtype=torch.float32) if torch.is_tensor(n_items)
-                       else torch.tensor(float(n_items), dtype=torch.float32, device=logits.device))
-            row_scale = (float(kw["num_processes"]) / n_items.clamp(min=1.0)).reshape(1).expand(n_seq)
-        ent_weight = None
-        if kw["entropy_coef"] != 0.0:  # d loss / d entropy = -coef * mask / normaliser (grpo_trainer.py:3155-3181)
-            if reduce_code == _lib.DAPO:
-                ent_weight = mask_f * (-float(kw["entropy_coef"]) * row_scale[0])
-            else:
-                ent_weight = mask_f * (-float(kw["entropy_coef"]) / mask_f.sum().clamp(min=1.0) / ga)
         up = kw.get("upstream_scale")
         if up is not None:
             # the caller will multiply the loss by this factor before backward (a gradient scaler's scale, a loss
@@ -307,9 +289,26 @@ class _GRPOFromLogits(torch.autograd.Function):
             # and `backward` has nothing left to do
             up = (up.to(device=logits.device, dtype=torch.float32).reshape(()) if torch.is_tensor(up)
                   else torch.tensor(float(up), dtype=torch.float32, device=logits.device))
-            row_scale = row_scale * up
-            if ent_weight is not None:
-                ent_weight = ent_weight * up
+        n_items = kw["num_items_in_batch"]
+        # d loss / d (masked token loss of sequence b), times the announced factor: what the loss kernel's second pass
+        # applies to its rows
+        if reduce_code == _lib.DAPO:
+            n_items = (n_items.to(device=logits.device, dtype=torch.float32).reshape(()) if torch.is_tensor(n_items)
+                       else torch.tensor(float(n_items), dtype=torch.float32, device=logits.device))
+            numerator = float(kw["num_processes"])
+        elif reduce_code == _lib.DR_GRPO:
+            numerator = 1.0 / float(n_seq * kw["max_completion_length"]) / ga
+        else:
+            numerator = 1.0 / (n_seq if reduce_code == _lib.GRPO else 1) / ga
+        mask_f, row_scale = ops.grpo_row_scale(mask, reduce_code, numerator, n_items if reduce_code == _lib.DAPO else None, up)
+        ent_weight = None
+        if kw["entropy_coef"] != 0.0:  # d loss / d entropy = -coef * mask / normaliser (grpo_trainer.py:3155-3181)
+            if reduce_code == _lib.DAPO:
+                ent_weight = mask_f * (-float(kw["entropy_coef"]) * row_scale[0])
+            else:
+                ent_weight = mask_f * (-float(kw["entropy_coef"]) / mask_f.sum().clamp(min=1.0) / ga)
+                if up is not None:
+                    ent_weight = ent_weight * up
         delta = kw["delta"]
         logp, ent, _, dlogits = ops.grpo_fused_fwd_bwd(
             logits, ids, float(temperature), keep_start, keep_len, mask_f, advantages, row_scale,
@@ -330,7 +329,7 @@ class _GRPOFromLogits(torch.autograd.Function):
             logp, advantages, mask_f, entropies=ent, old_per_token_logps=kw["old_per_token_logps"],
             ref_per_token_logps=kw["ref_per_token_logps"], loss_type=kw["loss_type"], epsilon_low=kw["epsilon_low"],
             epsilon_high=kw["epsilon_high"], beta=kw["beta"], delta=delta,
-            max_completion_length=kw["max_completion_length"], num_items_in_batch=kw["num_items_in_batch"],
+            max_completion_length=kw["max_completion_length"], num_items_in_batch=n_items,
             num_processes=kw["num_processes"], grad_accum_steps=kw["grad_accum_steps"],
             use_bias_correction_kl=kw["use_bias_correction_kl"], token_weight=kw["token_weight"],
             entropy_coef=kw["entropy_coef"],
@@ -692,18 +691,22 @@ class GRPOLossMixin:
             self._metrics[mode]["aux_loss"].append(self.accelerator.gather_for_metrics(aux_loss).mean().item())
 
         # metrics: cross-process sums of (sum, count) pairs, then one host copy
-        m = metrics.detach()
-        i = _METRIC_INDEX
-        sums = m[[i["KL_SUM"], i["ENTROPY_SUM"], i["MASK_SUM"], i["CLIP_COUNT"], i["AUX_SUM"], i["AUX_COUNT"]]]
-        clip = m[2:5] * m[i["CLIP_COUNT"]].clamp(min=1.0)
-        totals = self.accelerator.reduce(torch.cat([sums, clip]), reduction="sum")
-        low_min = nanmin(self.accelerator.gather(m[5:6]))
-        high_max = nanmax(self.accelerator.gather(m[6:7]))
         # (the kernels' error word rides along: a token id outside the vocabulary raises here, as the reference's
         # gather would, instead of surfacing as a NaN loss)
-        host = torch.cat([totals, low_min.reshape(1), high_max.reshape(1), m[7:8], ops.device_error_bits(m.device)]).tolist()
-        kl_sum, ent_sum, cnt, clip_cnt, aux_sum, aux_cnt, low, high, region, lmin, hmax, policy_loss, bits = host
-        ops.raise_for_error_bits(bits, m.device)
+        values = ops.grpo_log_values(metrics.detach())
+        sums, low_min, high_max = values[:9], values[9:10], values[10:11]
+        totals = self.accelerator.reduce(sums, reduction="sum")
+        lows, highs = self.accelerator.gather(low_min), self.accelerator.gather(high_max)
+        if totals is sums and lows is low_min and highs is high_max:
+            host = values.tolist()
+        else:
+            host = torch.cat([totals, lows.reshape(-1), highs.reshape(-1), values[11:]]).tolist()
+        n = lows.numel()
+        kl_sum, ent_sum, cnt, clip_cnt, aux_sum, aux_cnt, low, high, region = host[:9]
+        lmin = min((x for x in host[9 : 9 + n] if x == x), default=math.nan)
+        hmax = max((x for x in host[9 + n : -2] if x == x), default=math.nan)
+        policy_loss, bits = host[-2:]
+        ops.raise_for_error_bits(bits, values.device)
         cnt, clip_cnt, aux_cnt = max(cnt, 1.0), max(clip_cnt, 1.0), max(aux_cnt, 1.0)
         log = self._metrics[mode]
         if bonus:

@@ -58,7 +58,7 @@ def logps_and_entropies(
         idx = idx.long()
     rm = None
     if row_mask is not None:
-        rm = (row_mask.reshape(-1) != 0).to(torch.uint8).contiguous()
+        rm = (row_mask != 0).reshape(-1).view(torch.uint8).contiguous()
     logp, ent, _ = ops.logp_entropy_forward(logits, idx, float(temperature), keep_start, keep_len, rm)
     logp = logp.view(n_seq, keep_len) if squeeze else logp.view(n_seq, keep_len, index.shape[-1])
     return logp, ent.view(n_seq, keep_len)
