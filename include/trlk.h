@@ -345,6 +345,15 @@ int trlk_scatter_values(const float* d_a, const float* d_b, const int32_t* d_pos
 #define TRLK_GRPO_LOG_VALUES 13
 int trlk_grpo_log_values(const float* d_metrics, const int32_t* d_error_flag, float* d_out, trlk_stream_t stream);
 
+/* What a trainer logs of a DPO step (trl/trainer/dpo_trainer.py:1587-1653), in one vector of 8 + 2 n_seq floats, P = n_seq / 2:
+ * masked sums of the entropy and the mask, of the mean logit and the mask over the chosen and over the rejected sequences,
+ * arg-max hits of the chosen ones, the error word, then P chosen rewards beta * (seq - ref), P rejected ones, and the
+ * sequence log-probs.  d_row_stats [n_seq, seq_len, 4] and d_entropy as trlk_logp_entropy_fwd writes them (16-byte aligned);
+ * workspace: 4 n_seq floats. */
+int trlk_dpo_log_values(const float* d_entropy, const float* d_row_stats, const float* d_mask, int64_t n_seq, int64_t seq_len,
+                        const float* d_seq_logps, const float* d_ref_chosen, const float* d_ref_rejected, float beta,
+                        const int32_t* d_error_flag, float* d_out, float* d_workspace, trlk_stream_t stream);
+
 /* The completion mask as fp32 [n_seq, seq_len] (d_out_mask may be null) and the factor that trlk_grpo_fused_fwd_bwd takes as
  * d_row_scale: numerator / max(active tokens of the sequence, 1) for TRLK_GRPO, of the batch for TRLK_BNPO, numerator /
  * max(*d_n_items, 1) for TRLK_DAPO, the numerator itself for TRLK_DR_GRPO; times *d_upstream unless that is null.

@@ -732,3 +732,27 @@ def test_trainer_method_raises_on_a_token_id_outside_the_vocabulary(amd, single_
         tr._compute_loss(model, bad)
     assert math.isfinite(float(tr._compute_loss(model, inputs).detach()))
     amd.check_device_errors()
+
+
+@pytest.mark.parametrize("pairs,T", [(1, 1), (2, 257), (3, 64), (300, 5), (1, 0)])
+def test_dpo_log_values(amd, pairs, T):
+    """The packed DPO log values against float64, sequence counts and lengths on both sides of a workgroup; sums of
+    T * pairs fp32 terms in trees and chains of at most T / 256 + pairs / 256 + 16 steps."""
+    from trl_amd import ops
+
+    g = torch.Generator().manual_seed(pairs * 1000 + T)
+    B = 2 * pairs
+    ent, stats = torch.rand(B, T, generator=g), torch.randn(B, T, 4, generator=g)
+    mask = (torch.rand(B, T, generator=g) < 0.6).float()
+    seq, rc, rr = torch.randn(B, generator=g), torch.randn(pairs, generator=g), torch.randn(pairs, generator=g)
+    got = ops.dpo_log_values(*(t.to(DEV) for t in (ent, stats, mask, seq, rc, rr)), 0.1).cpu().double()
+    m = mask.double()
+    sums = [((x.double() * m).view(2, -1)).sum(1) for x in (ent, stats[..., 0], stats[..., 2], torch.ones(B, T))]
+    want = torch.stack([sums[0].sum(), sums[3].sum(), sums[1][0], sums[3][0], sums[1][1], sums[3][1], sums[2][0],
+                        torch.zeros((), dtype=torch.float64)])
+    scale = 2.0 + stats.abs().double().sum() + ent.double().sum()
+    assert ((got[:8] - want).abs() <= 24 * 6e-8 * scale).all()
+    seq64 = seq.double()
+    rewards = torch.cat([0.1 * (seq64[:pairs] - rc.double()), 0.1 * (seq64[pairs:] - rr.double())])
+    torch.testing.assert_close(got[8 : 8 + B], rewards, rtol=1e-6, atol=1e-7)
+    assert torch.equal(got[8 + B :], seq64)

@@ -447,6 +447,58 @@ __global__ __launch_bounds__(kThreads) void dpo_finish_kernel(const float* __res
     for (int64_t t = tid; t < T; t += kThreads) out_dlogp[off + t] = (mask[off + t] != 0.f) ? g : 0.f;
 }
 
+// The logged DPO values: masked sums of the entropies, the mean logits and the arg-max hits, one workgroup per sequence,
+// then their sums per half of the batch and the rewards, in one vector for one copy to the host.  Two launches in place
+// of two dozen [2P, T]-sized ones.
+constexpr int kDpoSums = 4;  // entropy, mean logit, arg-max hits, tokens
+__global__ __launch_bounds__(kThreads) void dpo_log_rows_kernel(const float* entropy, const float* row_stats, const float* mask,
+                                                                int64_t T, float* ws) {
+    __shared__ float scratch[kDpoSums][kThreads / kWave];
+    const int64_t off = int64_t(blockIdx.x) * T;
+    float v[kDpoSums] = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t t = threadIdx.x; t < T; t += kThreads) {
+        const float m = mask[off + t];
+        const float4 st = reinterpret_cast<const float4*>(row_stats)[off + t];
+        v[0] += entropy[off + t] * m;
+        v[1] += st.x * m;
+        v[2] += st.z * m;
+        v[3] += m;
+    }
+    block_sums<kThreads>(v, scratch);
+    if (threadIdx.x < kDpoSums) ws[int64_t(blockIdx.x) * kDpoSums + threadIdx.x] = v[threadIdx.x];
+}
+
+__global__ __launch_bounds__(kThreads) void dpo_log_finish_kernel(const float* ws, const float* seq, const float* ref_c,
+                                                                  const float* ref_r, int64_t P, float beta,
+                                                                  const int32_t* flag, float* out) {
+    __shared__ float scratch[2 * kDpoSums][kThreads / kWave];
+    float v[2 * kDpoSums] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // chosen, then rejected
+    float* const parts = out + 8;
+    for (int64_t p = threadIdx.x; p < P; p += kThreads) {
+#pragma unroll
+        for (int j = 0; j < kDpoSums; ++j) {
+            v[j] += ws[p * kDpoSums + j];
+            v[kDpoSums + j] += ws[(P + p) * kDpoSums + j];
+        }
+        const float c = seq[p], r = seq[P + p];
+        parts[p] = beta * (c - ref_c[p]);
+        parts[P + p] = beta * (r - ref_r[p]);
+        parts[2 * P + p] = c;
+        parts[3 * P + p] = r;
+    }
+    block_sums<kThreads>(v, scratch);
+    if (threadIdx.x == 0) {
+        out[0] = v[0] + v[4];
+        out[1] = v[3] + v[7];
+        out[2] = v[1];
+        out[3] = v[3];
+        out[4] = v[5];
+        out[5] = v[7];
+        out[6] = v[2];
+        out[7] = float(*flag);
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void rloo_finish_kernel(const float* __restrict__ seq,
                                                                const float* __restrict__ old_seq,
                                                                const float* __restrict__ adv,
@@ -739,6 +791,24 @@ extern "C" int trlk_dpo_loss(const float* d_token_logp, const float* d_mask, con
     hipLaunchKernelGGL(dpo_finish_kernel, dim3((unsigned)n_seq), dim3(kThreads), 0, s, d_out_seq_logps, d_ref_chosen,
                        d_ref_rejected, d_mask, n_seq, seq_len, beta, d_out_loss, d_out_metrics, d_out_dlogp);
     return launch_status("dpo_loss (finish)");
+}
+
+extern "C" int trlk_dpo_log_values(const float* d_entropy, const float* d_row_stats, const float* d_mask, int64_t n_seq,
+                                   int64_t seq_len, const float* d_seq_logps, const float* d_ref_chosen,
+                                   const float* d_ref_rejected, float beta, const int32_t* d_error_flag, float* d_out,
+                                   float* d_workspace, trlk_stream_t stream) {
+    clear_error();
+    TRLK_REQUIRE(n_seq >= 2 && n_seq % 2 == 0 && n_seq < (int64_t(1) << 31) && seq_len >= 0, TRLK_ERR_BAD_SHAPE,
+                 "dpo_log_values: n_seq must be even and >= 2 ([chosen; rejected] layout), got %lld", (long long)n_seq);
+    TRLK_REQUIRE((seq_len == 0 || (d_entropy && d_row_stats && d_mask)) && d_seq_logps && d_ref_chosen && d_ref_rejected &&
+                     d_error_flag && d_out && d_workspace,
+                 TRLK_ERR_NULL_POINTER, "dpo_log_values: a required pointer is null");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(dpo_log_rows_kernel, dim3((unsigned)n_seq), dim3(kThreads), 0, s, d_entropy, d_row_stats, d_mask, seq_len,
+                       d_workspace);
+    hipLaunchKernelGGL(dpo_log_finish_kernel, dim3(1), dim3(kThreads), 0, s, d_workspace, d_seq_logps, d_ref_chosen,
+                       d_ref_rejected, n_seq / 2, beta, d_error_flag, d_out);
+    return launch_status("dpo_log_values");
 }
 
 extern "C" int trlk_rloo_loss(const float* d_token_logp, const float* d_mask, const float* d_old_seq_logps,

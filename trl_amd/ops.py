@@ -602,6 +602,27 @@ def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Opti
     return mask_f, scale
 
 
+def dpo_log_values(entropy: Tensor, row_stats: Tensor, mask: Tensor, seq_logps: Tensor, ref_chosen: Tensor,
+                   ref_rejected: Tensor, beta: float) -> Tensor:
+    """What a DPO step logs, as one fp32 device vector `[8 + 4 P]` (`trlk_dpo_log_values`): `entropy`, `mask` `[2P, T]`,
+    `row_stats` `[2P, T, 4]` (contiguous), `seq_logps` `[2P]`, the reference's log-probs `[P]` or broadcast to it."""
+    B, T = mask.shape
+    P, dev = B // 2, mask.device
+    if B % 2 or entropy.numel() != B * T or row_stats.numel() != 4 * B * T or seq_logps.numel() != B:
+        raise ValueError("dpo_log_values: the shapes do not match")
+    mask, seq_logps, row_stats = _f32c(mask), _f32c(seq_logps), row_stats.contiguous()
+    ref_chosen, ref_rejected = _f32c(ref_chosen.expand(P)), _f32c(ref_rejected.expand(P))
+    out = torch.empty((8 + 2 * B,), dtype=torch.float32, device=dev)
+    if B == 0:
+        return out.zero_()
+    ws = torch.empty((4 * B,), dtype=torch.float32, device=dev)
+    with torch.cuda.device(dev):
+        check(lib.trlk_dpo_log_values(ptr(entropy.contiguous()), ptr(row_stats), ptr(mask), B, T, ptr(seq_logps),
+                                      ptr(ref_chosen), ptr(ref_rejected), beta, ptr(_error_flag(dev)), ptr(out), ptr(ws),
+                                      current_stream(dev)))
+    return out
+
+
 @torch.library.custom_op("trl_amd::dpo_loss", mutates_args=(), device_types="cuda")
 def dpo_loss_op(token_logp: Tensor, mask: Tensor, ref_chosen: Tensor, ref_rejected: Tensor, beta: float
                 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:

@@ -3,6 +3,7 @@ the fused sigmoid path (`dpo_sigmoid_loss`, one loss kernel) and the general one
 loss types, `ld_alpha`, WPO weighting, f-divergences, every logged metric from one pass over the logits)."""
 from __future__ import annotations
 
+import math
 from contextlib import contextmanager
 
 import torch
@@ -85,15 +86,35 @@ def dpo_compute_loss(
     passes for those); everything after that is `[2P, L]`- or `[P]`-sized torch arithmetic in fp32.  Rows outside
     the completion mask contribute to nothing and are not read unless `skip_masked_rows=False`.
     Returns `(loss, metrics)`, `metrics` a dict of device scalars keyed like the reference's log."""
+    loss, values = _dpo_loss_and_log_values(
+        logits, input_ids, completion_mask, ref_chosen_logps, ref_rejected_logps, beta, loss_types, loss_weights,
+        label_smoothing, ld_alpha, use_weighting, f_divergence_type, f_alpha_divergence_coef, discopop_tau,
+        skip_masked_rows)
+    c_rew, r_rew, chosen, rejected = values[8:].view(4, logits.shape[0] // 2).unbind(0)
+    return loss, {
+        "entropy_sum": values[0], "n_tokens": values[1],
+        "logits_chosen_sum": values[2], "n_chosen_tokens": values[3],
+        "logits_rejected_sum": values[4], "n_rejected_tokens": values[5],
+        "correct_tokens": values[6],
+        "chosen_rewards": c_rew, "rejected_rewards": r_rew, "chosen_logps": chosen, "rejected_logps": rejected,
+    }
+
+
+def _dpo_loss_and_log_values(logits, input_ids, completion_mask, ref_chosen_logps, ref_rejected_logps, beta, loss_types,
+                             loss_weights, label_smoothing, ld_alpha, use_weighting, f_divergence_type,
+                             f_alpha_divergence_coef, discopop_tau, skip_masked_rows):
+    """See `dpo_compute_loss`; the metrics as the one vector that `ops.dpo_log_values` makes."""
     if logits.dim() != 3 or logits.shape[0] % 2:
         raise ValueError("logits must be [2P, L, V]: chosen sequences first, rejected second")
     n_seq, length, _ = logits.shape
     labels = input_ids[:, 1:]
     smask = completion_mask[:, 1:]
+    if tuple(smask.shape) != (n_seq, length - 1):
+        raise ValueError(f"completion_mask {tuple(completion_mask.shape)} does not match logits {tuple(logits.shape)}")
     idx = labels.reshape(n_seq * (length - 1), 1)
     if idx.dtype != torch.int64:
         idx = idx.long()
-    rm = (smask.reshape(-1) != 0).to(torch.uint8).contiguous() if skip_masked_rows else None
+    rm = (smask != 0).reshape(-1).view(torch.uint8).contiguous() if skip_masked_rows else None
     # (the sum of squared probabilities is wanted by the WPO weights only)
     logp, ent, _, stats = ops.logp_entropy_stats_fwd(logits, idx, 1.0, 0, length - 1, rm, bool(use_weighting))
     m = smask.to(torch.float32)
@@ -105,8 +126,7 @@ def dpo_compute_loss(
             and f_divergence_type == "reverse_kl" and (loss_weights is None or [float(x) for x in loss_weights] == [1.0])):
         # the default configuration: masked sequence sums, loss and d loss / d log-prob from one loss kernel
         loss, seq, _, _ = ops.dpo_loss_op(logp.view(n_seq, length - 1), m, ref_c, ref_r, float(beta))
-        chosen, rejected = seq.detach().chunk(2)
-        return loss, _dpo_metric_parts(ent, stats, m, chosen, rejected, ref_c, ref_r, beta)
+        return loss, ops.dpo_log_values(ent, stats, m, seq.detach(), ref_c, ref_r, float(beta))
     tok = logp.view(n_seq, length - 1) * m
 
     if ld_alpha is None:
@@ -176,7 +196,7 @@ def dpo_compute_loss(
             term = term * pair_weight
         loss = loss + term.mean() * lw
 
-    return loss, _dpo_metric_parts(ent, stats, m, chosen.detach(), rejected.detach(), ref_c, ref_r, beta)
+    return loss, ops.dpo_log_values(ent, stats, m, seq.detach(), ref_c, ref_r, float(beta))
 
 
 def _masked_row_sums(token_logps: Tensor, mask: Tensor) -> Tensor:
@@ -187,24 +207,6 @@ def _masked_row_sums(token_logps: Tensor, mask: Tensor) -> Tensor:
         return (token_logps.float() * (mask != 0)).sum(dim=1)
     zero = token_logps.new_zeros((token_logps.shape[0] // 2,), dtype=torch.float32)
     return ops.dpo_loss_op(token_logps, mask, zero, zero, 1.0)[1]
-
-
-@torch.no_grad()
-def _dpo_metric_parts(ent, stats, m, chosen, rejected, ref_c, ref_r, beta):
-    """The parts of the logged metrics (dpo_trainer.py:1587-1653) as device scalars / `[P]` vectors: masked sums of
-    the entropies, the mean logits and the arg-max hits per half of the batch, from one stacked reduction."""
-    n_seq = m.shape[0]
-    vals = torch.stack((ent, stats[..., 0], stats[..., 2], torch.ones_like(ent)), dim=0)  # [4, 2P, L-1]
-    halves = (vals * m).view(4, 2, (n_seq // 2) * m.shape[1]).sum(dim=2)  # [quantity, chosen | rejected]
-    both = halves.sum(dim=1)
-    return {
-        "entropy_sum": both[0], "n_tokens": both[3],
-        "logits_chosen_sum": halves[1, 0], "n_chosen_tokens": halves[3, 0],
-        "logits_rejected_sum": halves[1, 1], "n_rejected_tokens": halves[3, 1],
-        "correct_tokens": halves[2, 0],
-        "chosen_rewards": beta * (chosen - ref_c), "rejected_rewards": beta * (rejected - ref_r),
-        "chosen_logps": chosen, "rejected_logps": rejected,
-    }
 
 
 def dpo_metrics_to_dict(metrics: dict) -> dict[str, float]:
@@ -279,31 +281,47 @@ class DPOLossMixin:
                         ref_logits = self.model(**ref_kwargs).logits
                 ref_seq = dpo_sequence_logps(ref_logits, input_ids, completion_mask, self.ld_alpha)
             ref_c, ref_r = ref_seq.chunk(2)
-        loss, parts = dpo_compute_loss(
+        loss, values = _dpo_loss_and_log_values(
             outputs.logits, input_ids, completion_mask, ref_c, ref_r, beta=self.beta, loss_types=self.loss_types,
             loss_weights=self.loss_weights, label_smoothing=self.label_smoothing, use_weighting=self.use_weighting,
-            discopop_tau=getattr(getattr(self, "args", None), "discopop_tau", 0.05), **cfg)
+            discopop_tau=getattr(getattr(self, "args", None), "discopop_tau", 0.05), skip_masked_rows=True, **cfg)
         log = self._metrics[mode]
+        n_pairs = input_ids.shape[0] // 2
         if aux_enabled:
             loss = loss + self.router_aux_loss_coef * outputs.aux_loss
             log["aux_loss"].append(self.accelerator.gather_for_metrics(outputs.aux_loss).mean().item())
         acc = self.accelerator
-        counts = torch.stack([parts[k] for k in ("entropy_sum", "n_tokens", "logits_chosen_sum", "n_chosen_tokens",
-                                                  "logits_rejected_sum", "n_rejected_tokens", "correct_tokens")])
-        bits = ops.device_error_bits(counts.device)  # (a token id outside the vocabulary raises here)
-        c_rew, r_rew = acc.gather(parts["chosen_rewards"]), acc.gather(parts["rejected_rewards"])
-        means = torch.stack([c_rew.mean(), r_rew.mean(), (c_rew > r_rew).float().mean(), (c_rew - r_rew).mean(),
-                             acc.gather(parts["chosen_logps"]).mean(), acc.gather(parts["rejected_logps"]).mean()])
-        n_train = (acc.gather_for_metrics(inputs["attention_mask"].sum()).sum().reshape(1) if mode == "train"
-                   else counts.new_zeros(1))
-        # every logged number in ONE copy to the host (each `.item()` would make the host wait for the device again)
-        (ent_sum, n_tok, lc, nc, lr, nr, correct, bits, rew_c, rew_r, rew_acc, rew_margin, logp_c, logp_r,
-         n_train) = torch.cat([acc.gather_for_metrics(counts.unsqueeze(0)).sum(dim=0).double(), bits.double(),
-                               means.double(), n_train.double()]).tolist()
-        ops.raise_for_error_bits(bits, counts.device)
+        # every logged number in ONE copy to the host (each `.item()` would make the host wait for the device again; a
+        # token id outside the vocabulary raises here, through the error word), the last sums and means there.  As 32-bit
+        # words, so that the token count keeps its 64 bits.
+        local = [values[:7].unsqueeze(0), *values[8:].view(4, n_pairs).unbind(0)]
+        counts, *vectors = parts = [acc.gather_for_metrics(local[0]), *(acc.gather(v) for v in local[1:])]
+        if any(p is not own for p, own in zip(parts, local)):
+            values = torch.cat([counts.reshape(-1), values[7:8], *(v.reshape(-1) for v in vectors)])
+        words = [values.view(torch.int32)]
+        if mode == "train":
+            tokens = acc.gather_for_metrics(inputs["attention_mask"].sum()).reshape(-1)
+            words.insert(0, tokens.to(device=values.device, dtype=torch.int64).view(torch.int32))
+        host = torch.cat(words).cpu()
+        # (plain Python from here on: the device has nothing to do until this method returns)
+        split = host.numel() - values.numel()
+        n_train = sum(host[:split].view(torch.int64).tolist())
+        numbers = host[split:].view(torch.float32).tolist()
+        n_counts, p = counts.numel(), vectors[0].numel()
+        ent_sum, n_tok, lc, nc, lr, nr, correct = (sum(numbers[j:n_counts:7]) for j in range(7))
+        bits = numbers[n_counts]
+        c_rew, r_rew, c_logp, r_logp = (numbers[n_counts + 1 + j * p : n_counts + 1 + (j + 1) * p] for j in range(4))
+
+        def mean(x):
+            return sum(x) / len(x) if x else math.nan
+
+        rew_c, rew_r, logp_c, logp_r = mean(c_rew), mean(r_rew), mean(c_logp), mean(r_logp)
+        rew_margin = mean([c - r for c, r in zip(c_rew, r_rew)])
+        rew_acc = mean([float(c > r) for c, r in zip(c_rew, r_rew)])
+        ops.raise_for_error_bits(bits, values.device)
         log["entropy"].append(ent_sum / n_tok if n_tok > 0 else 0.0)
         if mode == "train":
-            self._total_train_tokens += int(n_train)
+            self._total_train_tokens += n_train
         log["num_tokens"] = [self._total_train_tokens]
         log["logits/chosen"].append(lc / nc if nc > 0 else 0.0)
         log["logits/rejected"].append(lr / nr if nr > 0 else 0.0)
