@@ -1047,3 +1047,37 @@ def test_log_values_are_the_metrics(amd):
         got = ops.grpo_log_values(m).tolist()
         c = max(count, 1.0)
         assert got == [9.5, 10.5, 8.5, count, 13.5, 14.5, 2.5 * c, 3.5 * c, 4.5 * c, 5.5, 6.5, 7.5, 0.0]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_rows_at_the_edges_of_the_builds(amd, dtype):
+    """Rows around the sizes at which the kernel changes its number of vectors per lane or its workgroup (256 lanes of
+    4 .. 36 vectors, then 1024), whole and ragged, rows that begin in the middle of a 128-byte line among them: the
+    gradient of every row, the untouched ones included, against float64.  A bf16 gradient is rounded once: at most 2^-8 of
+    each entry, and so of the norm."""
+    epv = 16 // torch.empty((), dtype=dtype).element_size()
+    vectors = [256 * 4 * k + d for k in (1, 2, 5, 6, 9) for d in (-8, -7, 0, 1)] + [10240, 10241, 12288 - 7]
+    for i, n in enumerate(vectors):
+        for V in (n * epv, n * epv + 1 + i % (epv - 1)):
+            logits, ids, mask, adv, _ = _inputs(2, 3, V, dtype=dtype, seed=i, extra_rows=1)
+            mask[:] = 1
+            mask[1, 2:] = 0
+            ids[0, 0], ids[0, 1], ids[0, 2] = 0, V - 1, 9 % V
+            leaf = logits.detach().clone().requires_grad_(True)
+            loss, _, logp, ent = amd.grpo_loss_from_logits(leaf, ids, adv, mask, temperature=0.9, loss_type="bnpo")
+            loss.backward()
+            start = logits.shape[1] - 1 - ids.shape[1]
+            rows = logits[:, start : start + 3].double() / 0.9
+            lsm = rows.log_softmax(-1)
+            want_lp = lsm.gather(-1, ids[..., None]).squeeze(-1)
+            on = mask.bool()
+            torch.testing.assert_close(logp.double()[on], want_lp[on], rtol=0, atol=1e-5)
+            torch.testing.assert_close(ent.double()[on], -(lsm.exp() * lsm).sum(-1)[on], rtol=0, atol=1e-5)
+            # d loss / d logp = -advantage / active tokens (no old log-probs: the ratio is 1)
+            g = -adv.double()[:, None] * mask.double() / mask.double().sum()
+            want = torch.zeros(logits.shape, dtype=torch.float64, device=DEV)
+            want[:, start : start + 3] = -g[..., None] * lsm.exp() / 0.9
+            want[:, start : start + 3].scatter_add_(-1, ids[..., None], (g / 0.9)[..., None])
+            assert _rel_l2(leaf.grad.double(), want) < (2e-5 if dtype == torch.float32 else 2.0**-8), V
+            assert float(leaf.grad[1, start + 2 :].float().abs().max()) == 0.0
+    amd.check_device_errors()

@@ -19,7 +19,12 @@ namespace trlk {
 namespace {
 
 constexpr int kFThreads = 1024;
-constexpr int kFWaves = kFThreads / kWave;
+// Rows of up to kNarrowVec vectors per lane of a 256-lane workgroup (73728 16-bit logits) take one: three or more of them
+// fit a CU, and one row's loads run beside another's reduction and stores.  One 1024-lane workgroup fills the CU from 8
+// vectors (76 registers) on.  8144 rows, 53 % of them read, bf16: V = 20480 119 -> 80 us, 32000 178 -> 155 us, 50257 312 ->
+// 280 us, 65536 360 -> 340 us; 512 lanes lie between, 128 lanes are slower from 40960 on.
+constexpr int kNarrowThreads = 256, kNarrowVec = 36;
+constexpr int kSkew = 7;  // most vectors by which a row's vectors are shifted to 128-byte lines (see the kernel)
 constexpr int kMaxVec = 20;  // 16-byte vectors of a row per lane in registers: rows of up to 20 * 1024 * 8 = 163840 logits
 constexpr int kVecStep = 4;  // the kernel is built for 4, 8, ... kMaxVec vectors per lane; the host picks the smallest that holds the row
 // Longer rows keep what the registers cannot hold in the CU's LDS: up to kMaxLdsVec more vectors per lane (16 KiB of
@@ -69,7 +74,7 @@ __device__ __forceinline__ void lds_transfer(const u32x4* src, uint32_t lds) {
 }
 #pragma clang diagnostic pop
 
-// One workgroup of 1024 lanes per output row; NVEC = 16-byte vectors of the row a lane holds (the last kVecStep of
+// One workgroup of TH lanes per output row; NVEC = 16-byte vectors of the row a lane holds (the last kVecStep + 1 of
 // them may lie beyond the row's end for some lanes).  A workgroup fills its CU's register file, so nothing else
 // runs beside it: the arithmetic has to overlap the row's own memory traffic.  Hence
 //   * the per-row scalars are loaded first, from uniform addresses before any store: scalar loads, which return
@@ -90,16 +95,19 @@ __device__ __forceinline__ void lds_transfer(const u32x4* src, uint32_t lds) {
 //     after the last whole vector belong to one lane each, which reads its element ahead of the row for the sums
 //     and again after the row's stores for its gradient.  The gradient row may sit at another alignment than the
 //     logits row: its vectors are stored through accesses that need none.
-template <int DT, int NVEC, int NLDS, bool EXTRA = false, bool RAGGED = false>
-__global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
+template <int DT, int NVEC, int NLDS, bool EXTRA = false, bool RAGGED = false, int TH = kFThreads>
+__global__ __launch_bounds__(TH) void grpo_fused_kernel(FusedArgs a) {
     typedef Elem<DT> E;
     typedef typename E::type T;
     constexpr int EPV = E::EPV;
     // (the last register vectors keep their end-of-row test in the builds with vectors in LDS too, where it is always
     // true: without it the compiler unpacks every register vector ahead of its use and spills a hundred registers)
-    constexpr int kTail = NVEC - kVecStep;
+    // (one vector more than the step between builds: the build is picked for the largest shift to whole lines, and a row
+    // may hold kSkew + 1 vectors less; the builds with vectors in LDS start beyond NVEC * TH - kSkew)
+    constexpr int kTail = NLDS > 0 ? NVEC - kVecStep : NVEC - kVecStep - 1;
+    static_assert(TH > kSkew + 1, "a row holds more than (NVEC - kVecStep - 1) * TH vectors");
     extern __shared__ __attribute__((aligned(16))) char overflow[];  // [NLDS][1024 lanes] 16-byte vectors
-    __shared__ float red[7][kFWaves];
+    __shared__ float red[7][(TH / kWave)];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     // The hardware deals consecutive workgroups to the eight XCDs in turn.  Each XCD takes one contiguous eighth of
     // the rows and walks it in order, instead of every eighth row of the whole tensor: eight separate streams of reads
@@ -142,10 +150,19 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         else if (tid - head < int(a.vocab) - tail0)
             edge = tail0 + (tid - head);
     }
+    // Vectors are numbered from the 128-byte line in which the gradient row begins: its first whole vector has number
+    // `skew`, `nv` ends behind its last one, and a wave's stores cover whole lines.  (Numbered from the row's own start,
+    // every 1 KiB store of a row that begins inside a line leaves two lines half written: 8144 rows of 50264 against
+    // 50304 bf16 logits 281 against 259 us; both 260 us from whole lines, 8192 rows of 128257 715 -> 678 us.)  Lanes below `skew` have no vector 0; they load the row's first one, for its
+    // reference exponent, and leave it out of the sums and the stores.
     OutVec* op = reinterpret_cast<OutVec*>(out + head);
+    const int skew = int((reinterpret_cast<uintptr_t>(op) >> 4) & kSkew);
+    op -= skew;
+    nv += skew;
     if (m == 0.f) {  // no gradient reaches this row: zero-fill
         const u32x4 z = {0u, 0u, 0u, 0u};
-        for (int v = tid; v < nv; v += kFThreads) __builtin_nontemporal_store(z, op + v);
+        for (int v = tid; v < nv; v += TH)
+            if (v >= skew) __builtin_nontemporal_store(z, op + v);
         if (RAGGED && edge >= 0) E::store1(out + edge, 0.f);
     }
     if (m == 0.f && !(inside && a.all_rows)) {  // and nothing is read
@@ -157,7 +174,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         return;
     }
     const T* base = static_cast<const T*>(a.logits) + b * a.seq_stride + t * a.row_stride;
-    const u32x4* vp = reinterpret_cast<const u32x4*>(base + head);
+    const u32x4* vp = reinterpret_cast<const u32x4*>(base + head) - skew;
     const float inv_t = 1.f / a.temperature, c = kLog2e * inv_t;
     // sums of 2^(x c - r0) and of the same times x
     float r0 = 0.f, s = 0.f, u = 0.f;
@@ -171,15 +188,15 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
             u = s * x;
         }
     }
-    constexpr int kOnChip = (NVEC + NLDS) * kFThreads;  // vectors of the row the workgroup holds
+    constexpr int kOnChip = (NVEC + NLDS) * TH;  // vectors of the row the workgroup holds
     if constexpr (EXTRA) {
-        for (int v0 = kOnChip; v0 < nv; v0 += 4 * kFThreads) {
+        for (int v0 = kOnChip; v0 < nv; v0 += 4 * TH) {
             u32x4 e4[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) e4[k] = vp[min(v0 + k * kFThreads + tid, nv - 1)];
+            for (int k = 0; k < 4; ++k) e4[k] = vp[min(v0 + k * TH + tid, nv - 1)];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                if (v0 + k * kFThreads + tid < nv) {
+                if (v0 + k * TH + tid < nv) {
                     float x[EPV];
                     E::unpack(e4[k], x);
                     if (!have_r0) {
@@ -204,10 +221,10 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
                               uint32_t(__builtin_amdgcn_readfirstlane(wave)) * (kWave * 16);
 #pragma unroll
         for (int jl = 0; jl < NLDS; ++jl) {
-            const int v0 = (NVEC + jl) * kFThreads;
+            const int v0 = (NVEC + jl) * TH;
             if (v0 < nv) {  // (uniform over the workgroup; lanes beyond the row's end re-read its last vector)
                 const int tj = min(tid, nv - 1 - v0);
-                lds_transfer(vp + v0 + tj, lds0 + uint32_t(jl) * (kFThreads * 16));
+                lds_transfer(vp + v0 + tj, lds0 + uint32_t(jl) * (TH * 16));
             }
         }
     }
@@ -218,10 +235,11 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         // serves all NVEC loads and stores instead of one offset register each.  (Pointers that pass through the
         // empty asm must say that they point to global memory, or the accesses become flat ones, whose waits are
         // all-or-nothing.)
-        GlobalVecIn* vj = (GlobalVecIn*)vp + j * kFThreads;
+        GlobalVecIn* vj = (GlobalVecIn*)vp + j * TH;
         asm volatile("" : "+s"(vj));
         int tj = tid;
-        if (j >= kTail) tj = min(tid, nv - 1 - j * kFThreads);  // (a lane beyond the row's end re-reads the last vector and ignores it)
+        if (j == 0) tj = max(tid, skew);
+        if (j >= kTail) tj = min(tj, nv - 1 - j * TH);  // (a lane beyond the row's end re-reads the last vector and ignores it)
         q[j] = vj[tj];  // (plain loads: non-temporal ones measure the same to 1 % either way)
     }
     const bool idx_ok = idx >= 0 && idx < a.vocab;
@@ -231,15 +249,17 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
 #pragma unroll
     for (int j = 0; j < NVEC; ++j) {
         asm volatile("" : "+v"(q[j]));  // (pins the order: vector j is waited for and consumed before vector j + 1)
-        if (j < kTail || j * kFThreads + tid < nv) {
+        if (j == 0 && !((EXTRA || RAGGED) && have_r0)) {
             float x[EPV];
             E::unpack(q[j], x);
-            if (j == 0 && !((EXTRA || RAGGED) && have_r0)) {
-                float mx = x[0];
+            float mx = x[0];
 #pragma unroll
-                for (int i = 1; i < EPV; ++i) mx = fmaxf(mx, x[i]);
-                r0 = ceilf(mx * c);
-            }
+            for (int i = 1; i < EPV; ++i) mx = fmaxf(mx, x[i]);
+            r0 = ceilf(mx * c);
+        }
+        if ((j > 0 || tid >= skew) && (j < kTail || j * TH + tid < nv)) {
+            float x[EPV];
+            E::unpack(q[j], x);
 #pragma unroll
             for (int i = 0; i < EPV; ++i) {
                 const float e = fast_exp2(fmaf(x[i], c, -r0));
@@ -248,15 +268,15 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
             }
         }
     }
-    const u32x4* lds_q = reinterpret_cast<const u32x4*>(overflow) + tid;  // + jl * kFThreads
+    const u32x4* lds_q = reinterpret_cast<const u32x4*>(overflow) + tid;  // + jl * TH
     if constexpr (NLDS > 0) {
         // the transfers were issued before every register load and loads return in order: they have landed
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll 1  // (one vector at a time: the registers are full of the row)
         for (int jl = 0; jl < NLDS; ++jl) {
-            if ((NVEC + jl) * kFThreads + tid < nv) {
+            if ((NVEC + jl) * TH + tid < nv) {
                 float x[EPV];
-                E::unpack(lds_q[jl * kFThreads], x);
+                E::unpack(lds_q[jl * TH], x);
 #pragma unroll
                 for (int i = 0; i < EPV; ++i) {
                     const float e = fast_exp2(fmaf(x[i], c, -r0));
@@ -269,7 +289,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
     // bring the lanes' sums to a common exponent K >= r0 + log2(s) of every lane
     int es = 0;
     (void)frexpf(s, &es);
-    const bool has_data = tid < nv || (RAGGED && edge >= 0);
+    const bool has_data = (tid >= skew ? tid : tid + TH) < nv || (RAGGED && edge >= 0);
     const float key = has_data ? r0 + float(es) : -INFINITY;
     const bool bad = !(s < INFINITY) || !(fabsf(u) < INFINITY);  // overflow of a term, or inf / NaN in the row
     const float wk = wave_max(key);
@@ -281,7 +301,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
     __syncthreads();
     float K = -INFINITY, any_bad = 0.f;
 #pragma unroll
-    for (int k = 0; k < kFWaves; ++k) {
+    for (int k = 0; k < (TH / kWave); ++k) {
         K = fmaxf(K, red[0][k]);
         any_bad += red[3][k];
     }
@@ -297,7 +317,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kFWaves; ++k) {
+        for (int k = 0; k < (TH / kWave); ++k) {
             S += red[1][k];
             U += red[2][k];
         }
@@ -306,7 +326,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         // the exact reduction: the row's maximum first, then the sums relative to it.  Rare, so it re-reads the row
         // from memory instead of competing with the fast path for the registers that hold it.
         float lm = -INFINITY;
-        for (int v = tid; v < nv; v += kFThreads) {
+        for (int v = tid >= skew ? tid : tid + TH; v < nv; v += TH) {
             float x[EPV];
             E::unpack(vp[v], x);
 #pragma unroll
@@ -317,11 +337,11 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         if (lane == 0) red[4][wave] = M;
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kFWaves; ++k) M = fmaxf(M, red[4][k]);
+        for (int k = 0; k < (TH / kWave); ++k) M = fmaxf(M, red[4][k]);
         const float mc = M * c;
         s = 0.f;
         u = 0.f;
-        for (int v = tid; v < nv; v += kFThreads) {
+        for (int v = tid >= skew ? tid : tid + TH; v < nv; v += TH) {
             float x[EPV];
             E::unpack(vp[v], x);
 #pragma unroll
@@ -345,7 +365,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kFWaves; ++k) {
+        for (int k = 0; k < (TH / kWave); ++k) {
             S += red[5][k];
             U += red[6][k];
         }
@@ -383,8 +403,8 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
     const float b0 = with_h ? -h * kLn2 * inv_t : 0.f;
 #pragma unroll
     for (int j = 0; j < NVEC; ++j) {
-        const int v = j * kFThreads + tid;
-        if (j < kTail || v < nv) {
+        const int v = j * TH + tid;
+        if ((j > 0 || tid >= skew) && (j < kTail || v < nv)) {
             float x[EPV], d[EPV];
             E::unpack(q[j], x);
 #pragma unroll
@@ -393,7 +413,7 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
                 d[i] = fast_exp2(tt) * (with_h ? fmaf(b0, tt, a0) : a0);
             }
             typedef typename std::conditional<RAGGED, GlobalVecOutU, GlobalVecOut>::type GOut;
-            GOut* oj = (GOut*)op + j * kFThreads;
+            GOut* oj = (GOut*)op + j * TH;
             asm volatile("" : "+s"(oj));
             __builtin_nontemporal_store(E::pack(d), oj + tid);  // (streaming stores: 2-3 % faster than plain ones here)
         }
@@ -401,10 +421,10 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
     if constexpr (NLDS > 0) {
 #pragma unroll 1
         for (int jl = 0; jl < NLDS; ++jl) {
-            const int v = (NVEC + jl) * kFThreads + tid;
+            const int v = (NVEC + jl) * TH + tid;
             if (v < nv) {
                 float x[EPV], d[EPV];
-                E::unpack(lds_q[jl * kFThreads], x);
+                E::unpack(lds_q[jl * TH], x);
 #pragma unroll
                 for (int i = 0; i < EPV; ++i) {
                     const float tt = fmaf(x[i], c, -lse2);
@@ -415,13 +435,13 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
         }
     }
     if constexpr (EXTRA) {
-        for (int v0 = kOnChip; v0 < nv; v0 += 4 * kFThreads) {
+        for (int v0 = kOnChip; v0 < nv; v0 += 4 * TH) {
             u32x4 e4[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) e4[k] = vp[min(v0 + k * kFThreads + tid, nv - 1)];
+            for (int k = 0; k < 4; ++k) e4[k] = vp[min(v0 + k * TH + tid, nv - 1)];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int v = v0 + k * kFThreads + tid;
+                const int v = v0 + k * TH + tid;
                 if (v < nv) {
                     float x[EPV], d[EPV];
                     E::unpack(e4[k], x);
@@ -443,10 +463,10 @@ __global__ __launch_bounds__(kFThreads) void grpo_fused_kernel(FusedArgs a) {
     }
     // one-hot term: the lane that stored the target's vector (or edge element) rewrites that element (same lane,
     // same address: ordered after its first store)
-    int owner = int((idx / EPV) % kFThreads);
+    int owner = int((idx / EPV + skew) % TH);
     if constexpr (RAGGED) {
-        const int64_t tail0 = head + int64_t(nv) * EPV;
-        owner = idx < head ? int(idx) : idx >= tail0 ? head + int(idx - tail0) : int(((idx - head) / EPV) % kFThreads);
+        const int64_t tail0 = head + int64_t(nv - skew) * EPV;
+        owner = idx < head ? int(idx) : idx >= tail0 ? head + int(idx - tail0) : int(((idx - head) / EPV + skew) % TH);
     }
     if (idx_ok && owner == tid) {
         const float tt = fmaf(x_t, c, -lse2);
@@ -498,7 +518,8 @@ int launch_fused_wide(const FusedArgs& a, unsigned rows, hipStream_t s) {
 
 // R: rows that are not whole aligned vectors
 template <int DT, bool R>
-int launch_fused(const FusedArgs& a, int nvec, unsigned rows, hipStream_t s) {
+int launch_fused(const FusedArgs& a, int vectors, unsigned rows, hipStream_t s) {
+    const int nvec = (vectors + kFThreads - 1) / kFThreads;  // per lane of a wide workgroup
     if (nvec > kWideVec + kMaxLdsVec) return launch_fused_wide<DT, kMaxLdsVec, true, R>(a, rows, s);
     if (nvec > kMaxVec) {
         switch ((nvec - kWideVec + kLdsStep - 1) / kLdsStep) {
@@ -507,19 +528,33 @@ int launch_fused(const FusedArgs& a, int nvec, unsigned rows, hipStream_t s) {
             default: return launch_fused_wide<DT, 9, false, R>(a, rows, s);
         }
     }
-    switch ((nvec + kVecStep - 1) / kVecStep) {
-        case 1: hipLaunchKernelGGL((grpo_fused_kernel<DT, 4, 0, false, R>), dim3((rows + 7) / 8 * 8), dim3(kFThreads), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((grpo_fused_kernel<DT, 8, 0, false, R>), dim3((rows + 7) / 8 * 8), dim3(kFThreads), 0, s, a); break;
-        case 3: hipLaunchKernelGGL((grpo_fused_kernel<DT, 12, 0, false, R>), dim3((rows + 7) / 8 * 8), dim3(kFThreads), 0, s, a); break;
-        case 4: hipLaunchKernelGGL((grpo_fused_kernel<DT, 16, 0, false, R>), dim3((rows + 7) / 8 * 8), dim3(kFThreads), 0, s, a); break;
-        default: hipLaunchKernelGGL((grpo_fused_kernel<DT, 20, 0, false, R>), dim3((rows + 7) / 8 * 8), dim3(kFThreads), 0, s, a); break;
+#define TRLK_LAUNCH_FUSED(NVEC, TH) \
+    hipLaunchKernelGGL((grpo_fused_kernel<DT, NVEC, 0, false, R, TH>), dim3((rows + 7) / 8 * 8), dim3(TH), 0, s, a)
+    const int narrow = (vectors + kNarrowThreads - 1) / kNarrowThreads;
+    switch (narrow <= kNarrowVec ? (narrow + kVecStep - 1) / kVecStep : 0) {
+        case 1: TRLK_LAUNCH_FUSED(4, kNarrowThreads); return TRLK_OK;
+        case 2: TRLK_LAUNCH_FUSED(8, kNarrowThreads); return TRLK_OK;
+        case 3: TRLK_LAUNCH_FUSED(12, kNarrowThreads); return TRLK_OK;
+        case 4: TRLK_LAUNCH_FUSED(16, kNarrowThreads); return TRLK_OK;
+        case 5: TRLK_LAUNCH_FUSED(20, kNarrowThreads); return TRLK_OK;
+        case 6: TRLK_LAUNCH_FUSED(24, kNarrowThreads); return TRLK_OK;
+        case 7: TRLK_LAUNCH_FUSED(28, kNarrowThreads); return TRLK_OK;
+        case 8: TRLK_LAUNCH_FUSED(32, kNarrowThreads); return TRLK_OK;
+        case 9: TRLK_LAUNCH_FUSED(36, kNarrowThreads); return TRLK_OK;
+        default: break;
     }
+    switch ((nvec + kVecStep - 1) / kVecStep) {  // (ten vectors at least: see kNarrowVec)
+        case 3: TRLK_LAUNCH_FUSED(12, kFThreads); break;
+        case 4: TRLK_LAUNCH_FUSED(16, kFThreads); break;
+        default: TRLK_LAUNCH_FUSED(20, kFThreads); break;
+    }
+#undef TRLK_LAUNCH_FUSED
     return TRLK_OK;
 }
 
 template <int DT>
-int launch_fused_any(const FusedArgs& a, int nvec, bool ragged, unsigned rows, hipStream_t s) {
-    return ragged ? launch_fused<DT, true>(a, nvec, rows, s) : launch_fused<DT, false>(a, nvec, rows, s);
+int launch_fused_any(const FusedArgs& a, int vectors, bool ragged, unsigned rows, hipStream_t s) {
+    return ragged ? launch_fused<DT, true>(a, vectors, rows, s) : launch_fused<DT, false>(a, vectors, rows, s);
 }
 
 // data *= *scale over 16-byte vectors, unless the scale is exactly 1 (then nothing is read or written, and what the
@@ -696,10 +731,13 @@ extern "C" int trlk_grpo_fused_fwd_bwd(const void* d_logits, int dtype, int64_t 
     a.all_rows = compute_masked_rows != 0;
     a.total_rows = orows;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int nvec = int((vocab / epv + kFThreads - 1) / kFThreads);  // 16-byte vectors of the row per lane
-    if (int rc = dtype == TRLK_BF16  ? launch_fused_any<TRLK_BF16>(a, nvec, ragged, unsigned(orows), s)
-                 : dtype == TRLK_F16 ? launch_fused_any<TRLK_F16>(a, nvec, ragged, unsigned(orows), s)
-                                     : launch_fused_any<TRLK_F32>(a, nvec, ragged, unsigned(orows), s))
+    // 16-byte vectors of a row, and those that the shift to whole lines may add
+    const bool lines = !ragged && reinterpret_cast<uintptr_t>(d_dlogits) % 128 == 0 && (out_seq_stride * es) % 128 == 0 &&
+                       (out_row_stride * es) % 128 == 0;
+    const int vectors = int(vocab / epv) + (lines ? 0 : kSkew);
+    if (int rc = dtype == TRLK_BF16  ? launch_fused_any<TRLK_BF16>(a, vectors, ragged, unsigned(orows), s)
+                 : dtype == TRLK_F16 ? launch_fused_any<TRLK_F16>(a, vectors, ragged, unsigned(orows), s)
+                                     : launch_fused_any<TRLK_F32>(a, vectors, ragged, unsigned(orows), s))
         return rc;
     return launch_status("grpo_fused");
 }

@@ -234,9 +234,10 @@ def grpo_loss(
 _SINGLE_PASS_LOSS_TYPES = ("grpo", "bnpo", "dr_grpo", "dapo", "cispo", "sapo")
 
 
-# Rows shorter than this go through the two-pass kernels by default: on bf16 [64, 1024, V] logits with half of the
-# rows masked the one pass takes 0.70 / 0.78 / 0.82 / 1.15 ms at V = 8192 / 16384 / 20480 / 32000, the two passes
-# 0.51 / 0.79 / 0.94 / 1.41 ms.
+# Rows shorter than this go through the two-pass kernels by default.  The line lies where the one pass won when a row took a
+# 1024-lane workgroup whatever its length; since short rows take 256 lanes it wins below too (bf16 [64, 1024, V] logits with
+# half of the rows masked, whole step at V = 8192 / 16384 / 20480: 0.31 / 0.62 / 0.71 against 0.42 / 0.77 / 0.84 ms), but its
+# backward can run only once, and short rows keep the path that has no such limit.
 _SINGLE_PASS_MIN_ROW_BYTES = 40960
 
 
