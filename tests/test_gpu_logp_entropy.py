@@ -480,3 +480,35 @@ def test_rows_that_are_not_whole_vectors(amd, dtype):
         want_hit = (x.argmax(-1) == index[:, :, 0]).reshape(-1)
         assert torch.equal(stats[:, 2] != 0, want_hit), V
     amd.check_device_errors()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("vocab", [8, 56, 63, 64, 65, 72, 127, 1032, 4088, 4096 + 8, 8192 + 56, 12289])
+def test_rows_walked_from_their_first_line(amd, dtype, vocab):
+    """Rows that begin inside a 128-byte line (whole vectors or not, and rows with no line of their own): targets before
+    the first line, at its edge and at the row's end, forward and backward with both upstream gradients against float64.
+    A bf16 gradient is rounded once, at most 2^-8 of an entry; the fp32 chain holds 1e-5."""
+    g = torch.Generator().manual_seed(vocab)
+    n, L, T = 2, 5, 0.9
+    logits = (2.0 * torch.randn(n, L, vocab, generator=g)).to(dtype)
+    line = 128 // logits.element_size()
+    idx = torch.randint(0, vocab, (n, L), generator=g)
+    for b in range(n):
+        for t in range(L):  # the last element before the row's first line, the first one of it, the row's ends
+            at = ((b * L + t) * vocab) % line
+            idx[b, t] = (0, line - at - 1, line - at, vocab - 1, idx[b, t])[t] % vocab
+    glp, gent = torch.randn(n, L, generator=g), torch.randn(n, L, generator=g)
+    want = logits.double().requires_grad_(True)
+    lsm = (want / T).log_softmax(-1)
+    wlp, went = lsm.gather(-1, idx[..., None]).squeeze(-1), -(lsm.exp() * lsm).sum(-1)
+    leaf = logits.to(DEV).requires_grad_(True)
+    lp, ent = amd.trainer.utils.logps_and_entropies(leaf, idx.to(DEV), T)
+    torch.testing.assert_close(lp.detach().cpu().double(), wlp.detach(), rtol=0, atol=1e-5)
+    torch.testing.assert_close(ent.detach().cpu().double(), went.detach(), rtol=0, atol=1e-5)
+    for with_entropy in (False, True):
+        loss = (wlp * glp).sum() + ((went * gent).sum() if with_entropy else 0.0)
+        (w,) = torch.autograd.grad(loss, want, retain_graph=True)
+        loss = (lp * glp.to(DEV)).sum() + ((ent * gent.to(DEV)).sum() if with_entropy else 0.0)
+        (got,) = torch.autograd.grad(loss, leaf, retain_graph=True)
+        assert _rel_l2(got, w) < (1e-5 if dtype == torch.float32 else 2.0**-8)
+    amd.check_device_errors()

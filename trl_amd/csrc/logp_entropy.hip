@@ -67,6 +67,7 @@ __device__ __forceinline__ void stream_store(u32x4 v, V* p) {
 }
 constexpr bool kFwdNt = TRLK_FWD_NT_LOAD != 0;
 constexpr bool kBwdNt = TRLK_BWD_NT_LOAD != 0;
+constexpr int kLine = 128;  // bytes of a cache line
 constexpr int kMaxIndex = 64;  // most indices per row the backward accepts
 
 struct FwdArgs {
@@ -141,7 +142,7 @@ __device__ __forceinline__ float max_of(const float* x) {
 }
 
 // VEC: rows are 16-byte aligned and vocab is a multiple of the vector width.  Otherwise a row is read in aligned
-// vectors from its first 16-byte boundary on, and the few elements before that and after the last whole vector one by one.
+// vectors from its first 128-byte line on, and the few elements before that and after the last whole vector one by one.
 // STATS: 1 or 2 also produce the row statistics of `out_stats`; only 2 accumulates the sum of squared probabilities
 // (one more multiply-add per logit in a loop that is bound by its arithmetic: 5.14 against 4.95 ms on 33.6 GB of bf16
 // logits), 1 reports 0 in its place.
@@ -224,10 +225,12 @@ __global__ __launch_bounds__(TH) void logp_entropy_fwd_kernel(FwdArgs a) {
     };
     {
         constexpr int EPV = E::EPV;
-        // Rows that are not whole aligned vectors (not VEC): the `head` elements before the row's first 16-byte
-        // boundary go one by one (first: a lane's positions must come in increasing order), then aligned vectors,
-        // then what is left after the last whole one.
-        const int head = VEC ? 0 : int(min(V, int64_t(((16 - (reinterpret_cast<uintptr_t>(base) & 15)) & 15) / sizeof(T))));
+        // Rows that are not whole aligned vectors (not VEC): the `head` elements before the row's first 128-byte
+        // line go one by one (first: a lane's positions must come in increasing order), then aligned vectors,
+        // then what is left after the last whole one.  (From the first 16-byte boundary on, a wave's 1 KiB load touches
+        // nine lines: 8700 rows of 128257 bf16 logits 377 against 362 us, with statistics 391 against 372.)
+        const int head = VEC ? 0 : int(min(V, int64_t(((kLine - (reinterpret_cast<uintptr_t>(base) & (kLine - 1))) & (kLine - 1)) / sizeof(T))));
+        static_assert(kLine / sizeof(T) <= TH, "one lane per element before the first line");
         if constexpr (!VEC) {
             if (tid < head) {
                 const float x = E::load1(base + tid);
@@ -421,11 +424,14 @@ __global__ __launch_bounds__(kThreads) void logp_entropy_bwd_kernel(BwdArgs a, i
     const int64_t to = orow - b * a.out_rows_per_seq;
     const int64_t t = to - a.out_row_offset;
     T* out = static_cast<T*>(a.dlogits) + b * a.out_seq_stride + to * a.out_row_stride;
-    // Rows that are not whole aligned vectors (not VEC) are walked from the first 16-byte boundary of the OUTPUT row:
+    // Rows that do not all begin on a 128-byte line (not VEC) are walked from the first line boundary of the OUTPUT row:
     // the `head` elements before it and what is left after the last whole vector go one by one, the vectors between
     // through accesses that need no alignment (when the logits row sits like the gradient row -- two contiguous
-    // tensors of one shape -- both sides are in fact aligned).  The chunks count from that boundary.
-    const int head = VEC ? 0 : int(min(a.vocab, int64_t(((16 - (reinterpret_cast<uintptr_t>(out) & 15)) & 15) / sizeof(T))));
+    // tensors of one shape -- both sides are in fact aligned).  The chunks count from that boundary, so that a wave's
+    // stores cover whole lines: from the first 16-byte boundary on, two lines of every 1 KiB were written in halves
+    // (16384 rows of 128257 bf16 logits, 53 % of them read, 1203 against 1147 us; of 128264 1230 against 1158).
+    const int head = VEC ? 0 : int(min(a.vocab, int64_t(((kLine - (reinterpret_cast<uintptr_t>(out) & (kLine - 1))) & (kLine - 1)) / sizeof(T))));
+    static_assert(kLine / sizeof(T) <= kThreads, "one lane per element before the first line");
     const int body = int(a.vocab) - head;
     const int e0 = chunk * CE;                                   // first element of this chunk, counted from `head`
     const int e1 = max(e0, body < e0 + CE ? body : e0 + CE);     // (an empty range in a last chunk that the head made superfluous)
@@ -526,10 +532,10 @@ __global__ __launch_bounds__(kThreads) void logp_entropy_bwd_kernel(BwdArgs a, i
     }
 }
 
-bool aligned16(const void* p, size_t es, std::initializer_list<int64_t> strides) {
-    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+bool aligned_to(int bytes, const void* p, size_t es, std::initializer_list<int64_t> strides) {
+    if (reinterpret_cast<uintptr_t>(p) % unsigned(bytes) != 0) return false;
     for (int64_t s : strides)
-        if ((s * int64_t(es)) % 16 != 0) return false;
+        if ((s * int64_t(es)) % bytes != 0) return false;
     return true;
 }
 
@@ -583,7 +589,7 @@ extern "C" int trlk_logp_entropy_fwd(const void* d_logits, int dtype, int64_t n_
               n_index,     temperature,  d_row_mask,    d_out_logp, d_out_entropy, d_out_lse,
               d_out_row_stats, d_error_flag};
     const size_t es = elem_size(dtype);
-    const bool vec = aligned16(d_logits, es, {seq_stride, row_stride}) && vocab % int64_t(16 / es) == 0;
+    const bool vec = aligned_to(16, d_logits, es, {seq_stride, row_stride}) && vocab % int64_t(16 / es) == 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 grid((unsigned)rows), block(kThreads);
     const int stats = d_out_row_stats == nullptr ? 0 : (row_stats_sum_p2 ? 2 : 1);
@@ -650,8 +656,8 @@ extern "C" int trlk_logp_entropy_bwd(const void* d_logits, int dtype, int64_t n_
               temperature, d_lse,     d_entropy, d_g_logp,   d_g_entropy, d_dlogits,       out_rows_per_seq,
               out_row_offset, out_seq_stride, out_row_stride};
     const size_t es = elem_size(dtype);
-    const bool vec = aligned16(d_logits, es, {seq_stride, row_stride}) &&
-                     aligned16(d_dlogits, es, {out_seq_stride, out_row_stride}) && vocab % int64_t(16 / es) == 0;
+    const bool vec = aligned_to(16, d_logits, es, {seq_stride, row_stride}) &&
+                     aligned_to(kLine, d_dlogits, es, {out_seq_stride, out_row_stride}) && vocab % int64_t(16 / es) == 0;
     const bool has_h = d_g_entropy != nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t chunk = kChunkBytes / int64_t(es);
