@@ -227,7 +227,9 @@ struct DirectLoader {
 
 // `prefetched`: the caller has already run DirectLoader::prologue for this tile (and nothing has
 // touched the LDS since).
-template <int DT, int BKT, bool AKM = false>
+// IDLE: waves whose rows or columns all lie beyond the operands skip the matrix work (the products of the backward; in the
+// forward the second path costs registers that it does not have).
+template <int DT, int BKT, bool AKM = false, bool IDLE = false>
 __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, const Operand B, int n0, int K,
                                                     f32x16 (&acc)[MB][NB], char* smem, bool prefetched) {
     typedef DirectCfg<BKT> C;
@@ -305,6 +307,29 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
     else
         __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    constexpr int kLoadsPost = (kStageLoads + 1) / 2, kLoadsPre = kStageLoads - kLoadsPost;
+    // A wave whose rows or columns all lie beyond the operands (the last tile of either) moves its share of the tiles
+    // and nothing else.  Waves that differ in their rows only share a SIMD, so a last row tile that is at most half full
+    // takes half the matrix time.  (Exactly the transfers and barriers of the loop below.)
+    if (IDLE && (m0 + wm * WM >= A.rows || n0 + wn * WN >= B.rows)) {
+#pragma unroll 1
+        for (int kt = 0; kt < nk; ++kt) {
+            if (kt > 0 && kt - 1 + kStages < nk) {
+#pragma unroll
+                for (int j = kLoadsPost; j < kStageLoads; ++j)
+                    loader.issue_one((kt - 1) & (kStages - 1), (kt - 1 + kStages) * BKT, j);
+            }
+            __builtin_amdgcn_s_waitcnt(0);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (kt + kStages < nk) {
+#pragma unroll
+                for (int j = 0; j < kLoadsPost; ++j) loader.issue_one(kt & (kStages - 1), (kt + kStages) * BKT, j);
+            }
+        }
+        return;
+    }
     load_frags(0, 0, fa[0], fb[0]);
     // Exact issue order, pinned instruction by instruction (sched_barrier(0) between the groups):
     // MFMA i of the slice, then at most one fragment read of the next slice and at most one tile
@@ -313,7 +338,6 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
     // of a stage is split: the first half of its transfers goes behind the barrier that frees it, the
     // second half into the first slice of the following step.
     constexpr int M = MB * NB, R = MB + NB;
-    constexpr int kLoadsPost = (kStageLoads + 1) / 2, kLoadsPre = kStageLoads - kLoadsPost;
     auto slice = [&](u32x4(&ca)[MB], u32x4(&cb)[NB], auto read_tag, int rbuf, int rks, u32x4(&na)[MB], u32x4(&nb_)[NB],
                      auto nload_tag, int lbuf, int lk0, int lfirst) {
         constexpr bool READ = decltype(read_tag)::value;
@@ -492,15 +516,15 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
     }
 }
 
-template <int DT, int BKT, bool AKM = false>
+template <int DT, int BKT, bool AKM = false, bool IDLE = false>
 __device__ __forceinline__ void gemm_tile_nt(const Operand A, int m0, const Operand B, int n0, int K,
                                              f32x16 (&acc)[MB][NB], char* smem, bool prefetched = false) {
     if constexpr (AKM) {  // (callers of this form pad K to whole steps)
         static_assert(BKT == 64, "k-major left operands need the direct-to-LDS loop with 64-wide steps");
-        gemm_tile_nt_direct<DT, BKT, true>(A, m0, B, n0, K, acc, smem, prefetched);
+        gemm_tile_nt_direct<DT, BKT, true, IDLE>(A, m0, B, n0, K, acc, smem, prefetched);
     } else {
         if ((K & (BKT - 1)) == 0)
-            gemm_tile_nt_direct<DT, BKT>(A, m0, B, n0, K, acc, smem, prefetched);
+            gemm_tile_nt_direct<DT, BKT, false, IDLE>(A, m0, B, n0, K, acc, smem, prefetched);
         else
             gemm_tile_nt_staged<DT>(A, m0, B, n0, K, acc, smem);
     }
@@ -1181,7 +1205,7 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     const int wm = wave / WGN, wn = wave % WGN;
     const int m0 = tm * BM, n0 = tn * BN;
     f32x16 acc[MB][NB];
-    gemm_tile_nt<DT, TRLK_HEAD_BK_GEMM, AKM>(A, m0, B, n0, K, acc, smem);
+    gemm_tile_nt<DT, TRLK_HEAD_BK_GEMM, AKM, true>(A, m0, B, n0, K, acc, smem);
     const float inv_b = 1.f / slot_scale(a.max_b, 1.f);
     const float inv_common = inv_b / slot_scale(a.max_a, a.mult_a);
     // A tile inside the output (nearly every tile): no per-element predicates, addresses as a uniform base plus one
@@ -1927,7 +1951,7 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         gw.B = Operand{ht, l.ld_n, H};
         gw.M = rows;
         gw.N = H;
-        gw.K = int(l.npad);
+        gw.K = int(round_up(N, BK));  // (dz is zero from there to npad)
         gw.out_lp = static_cast<uint16_t*>(d_out_dweight) + c0 * hidden_size;
         gw.ld_lp = hidden_size;
         gw.first = 1;
