@@ -190,5 +190,24 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
-def current_stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+def current_stream(device: torch.device) -> int:
+    """The current stream of `device` as the raw handle that the library takes (without the Python stream object that
+    `torch.cuda.current_stream` builds around it; with `on_device` 26.5 -> 23.5 us for the smallest scoring call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+class on_device:
+    """`torch.cuda.device(device)` for a tensor's own device, which needs no parsing."""
+
+    __slots__ = ("index", "previous")
+
+    def __init__(self, device: torch.device):
+        self.index = -1 if device.index is None else device.index
+
+    def __enter__(self):
+        self.previous = torch.cuda._exchange_device(self.index)
+
+    def __exit__(self, *exc):
+        torch.cuda._maybe_exchange_device(self.previous)
+        return False

@@ -20,7 +20,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from ._lib import check, current_stream, dtype_code, lib, ptr
+from ._lib import check, current_stream, dtype_code, lib, on_device, ptr
 
 _SYNC_CHECKS = os.environ.get("TRL_AMD_SYNC_CHECKS", "0") == "1"
 _error_flags: dict[int, Tensor] = {}
@@ -93,7 +93,7 @@ def _run_logp_entropy_fwd(logits, index, temperature, keep_start, keep_len, row_
         return logp, ent, lse, stats
     index = index.contiguous()
     view = logits[:, keep_start : keep_start + keep_len]
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(
             lib.trlk_logp_entropy_fwd(
                 view.data_ptr(), dtype_code(logits.dtype), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
@@ -159,7 +159,7 @@ def logp_entropy_bwd(
     index = index.contiguous()
     g_logp = None if g_logp is None else g_logp.contiguous().float()
     g_entropy = None if g_entropy is None else g_entropy.contiguous().float()
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(
             lib.trlk_logp_entropy_bwd(
                 view.data_ptr(), dtype_code(logits.dtype), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
@@ -221,7 +221,7 @@ def logp_entropy_fwd_f64(
         return logp, ent, lse
     index = index.contiguous()
     view = logits[:, keep_start : keep_start + keep_len]
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_logp_entropy_fwd_f64(view.data_ptr(), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
                                             ptr(index), k, temperature, ptr(row_mask), ptr(logp), ptr(ent), ptr(lse),
                                             ptr(_error_flag(dev)), current_stream(dev)))
@@ -254,7 +254,7 @@ def logp_entropy_bwd_f64(
     index = index.contiguous()
     g_logp = None if g_logp is None else g_logp.contiguous().double()
     g_entropy = None if g_entropy is None else g_entropy.contiguous().double()
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_logp_entropy_bwd_f64(view.data_ptr(), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
                                             ptr(index), k, temperature, ptr(lse),
                                             ptr(entropy if g_entropy is not None else None), ptr(g_logp), ptr(g_entropy),
@@ -300,7 +300,7 @@ def _group_advantages(rewards: Tensor, group_size: int, scale_mode: int) -> Tens
     rewards = rewards.contiguous().float()
     out = torch.empty_like(rewards)
     dev = rewards.device
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_group_advantages(ptr(rewards), rewards.numel(), group_size, scale_mode, ptr(out), current_stream(dev)))
     return out
 
@@ -380,7 +380,7 @@ def grpo_loss_op(
     dent = torch.empty((B, T), dtype=torch.float32, device=dev) if entropy_coef != 0.0 else None
     ws_bytes = lib.trlk_grpo_workspace_bytes(B)
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(
             lib.trlk_grpo_loss(
                 ptr(logp), ptr(old_logp), ptr(ref_logp), ptr(entropy), ptr(advantages), sb, st, ptr(mask),
@@ -477,7 +477,7 @@ def grpo_loss_static_(
                     ("out_metrics", out_metrics), ("out_dlogp", out_dlogp), ("out_dentropy", out_dentropy)):
         if t is not None and t.device != dev:
             raise ValueError(f"grpo_loss_static_: {name} is on {t.device}, logp on {dev}")
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(
             lib.trlk_grpo_loss_static(
                 ptr(logp), ptr(old_logp), ptr(ref_logp), ptr(entropy), ptr(advantages), sb, st, ptr(mask),
@@ -541,7 +541,7 @@ def grpo_fused_fwd_bwd(
     if dlogits.numel() == 0:
         return logp, ent, lse, dlogits
     view = logits[:, keep_start : keep_start + keep_len]
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(
             lib.trlk_grpo_fused_fwd_bwd(
                 view.data_ptr(), dtype_code(logits.dtype), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
@@ -563,7 +563,7 @@ def scale_unless_one_(data: Tensor, scale: Tensor) -> Tensor:
     if not data.is_contiguous() or data.dtype not in (torch.bfloat16, torch.float16, torch.float32):
         raise ValueError("scale_unless_one_: contiguous bf16 / fp16 / fp32 data expected")
     scale = scale.reshape(1).to(device=data.device, dtype=torch.float32)
-    with torch.cuda.device(data.device):
+    with on_device(data.device):
         check(lib.trlk_scale_unless_one(data.data_ptr(), dtype_code(data.dtype), data.numel(), ptr(scale),
                                         current_stream(data.device)))
     return data
@@ -577,7 +577,7 @@ def grpo_log_values(metrics: Tensor) -> Tensor:
     sums to be added over the processes, the smallest and the largest clip ratio, the policy loss, the error word."""
     dev = metrics.device
     out = torch.empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_grpo_log_values(ptr(metrics), ptr(_error_flag(dev)), ptr(out), current_stream(dev)))
     return out
 
@@ -595,7 +595,7 @@ def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Opti
     as_is = mask.dtype == torch.float32 and mask.is_contiguous()
     mask_f = mask if as_is else torch.empty((B, T), dtype=torch.float32, device=dev)
     scale = torch.empty((B,), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_grpo_row_scale(ptr(mask), _KEEP_TYPES[mask.dtype], B, T, mask.stride(0), mask.stride(1), loss_type,
                                       numerator, ptr(n_items), ptr(upstream), None if as_is else ptr(mask_f), ptr(scale),
                                       current_stream(dev)))
@@ -616,7 +616,7 @@ def dpo_log_values(entropy: Tensor, row_stats: Tensor, mask: Tensor, seq_logps: 
     if B == 0:
         return out.zero_()
     ws = torch.empty((4 * B,), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_dpo_log_values(ptr(entropy.contiguous()), ptr(row_stats), ptr(mask), B, T, ptr(seq_logps),
                                       ptr(ref_chosen), ptr(ref_rejected), beta, ptr(_error_flag(dev)), ptr(out), ptr(ws),
                                       current_stream(dev)))
@@ -641,7 +641,7 @@ def dpo_loss_op(token_logp: Tensor, mask: Tensor, ref_chosen: Tensor, ref_reject
     seq = torch.empty((B,), dtype=torch.float32, device=dev)
     metrics = torch.empty((_lib.DPO_NUM_METRICS,), dtype=torch.float32, device=dev)
     dlogp = torch.empty((B, T), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_dpo_loss(ptr(token_logp), ptr(mask), ptr(ref_chosen), ptr(ref_rejected), B, T, beta, ptr(seq),
                                 ptr(loss), ptr(metrics), ptr(dlogp), current_stream(dev)))
     return loss, seq, metrics, dlogp
@@ -692,7 +692,7 @@ def rloo_loss_op(token_logp: Tensor, mask: Tensor, old_seq_logps: Tensor, advant
     seq = torch.empty((B,), dtype=torch.float32, device=dev)
     metrics = torch.empty((_lib.RLOO_NUM_METRICS,), dtype=torch.float32, device=dev)
     dlogp = torch.empty((B, T), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_rloo_loss(ptr(token_logp), ptr(mask), ptr(old_seq_logps), ptr(advantages), B, T, epsilon_low,
                                  epsilon_high, ptr(seq), ptr(loss), ptr(metrics), ptr(dlogp), current_stream(dev)))
     return loss, seq, metrics, dlogp
@@ -798,7 +798,7 @@ def fused_head_fwd(hidden: Tensor, weight: Tensor, targets: Tensor, temperature:
         saved = torch.empty((0, 0, 4), dtype=torch.float16, device=dev)
     ws_bytes = lib.trlk_fused_head_fwd_workspace_bytes(n)
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_fused_head_fwd(ptr(hidden), ptr(weight), ptr(targets), dtype_code(hidden.dtype), n, v, h,
                                       hidden.stride(0), weight.stride(0), temperature, softcap, logit_scale,
                                       ptr(bias32), ptr(logp), ptr(ent), ptr(log_z), ptr(hit),
@@ -850,7 +850,7 @@ def fused_head_bwd(hidden: Tensor, weight: Tensor, targets: Tensor, temperature:
         raise ValueError("fused head: the stash does not belong to these operands")
     ws_bytes = lib.trlk_fused_head_bwd_workspace_bytes(max(n, 1), v, h, chunk_size)
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_fused_head_bwd(ptr(hidden), ptr(weight), ptr(targets), dtype_code(hidden.dtype), n, v, h,
                                       hidden.stride(0), weight.stride(0), temperature, softcap, logit_scale,
                                       ptr(bias32), ptr(log_z), ptr(g), chunk_size, ptr(stash),
@@ -880,7 +880,7 @@ def split_bf16x3(x: Tensor, side: int) -> Tensor:
     rows, cols = x.shape
     cpad = (cols + 7) // 8 * 8
     out = torch.empty((rows, 6 * cpad), dtype=torch.bfloat16, device=x.device)
-    with torch.cuda.device(x.device):
+    with on_device(x.device):
         check(lib.trlk_split_bf16x3(ptr(x), rows, cols, x.stride(0) if rows > 1 else cols, side, ptr(out), 6 * cpad,
                                     current_stream(x.device)))
     return out
@@ -901,7 +901,7 @@ def gemm_nt(a: Tensor, b: Tensor, out: Optional[Tensor] = None, accumulate: bool
         out = torch.empty((m, n), dtype=torch.float32, device=a.device)
     elif out.shape != (m, n) or out.dtype != torch.float32 or out.stride(1) != 1:
         raise ValueError("gemm_nt: out must be a float32 [M, N] tensor with contiguous rows")
-    with torch.cuda.device(a.device):
+    with on_device(a.device):
         check(lib.trlk_gemm_nt(ptr(a), a.stride(0), ptr(b), b.stride(0), dtype_code(a.dtype), m, n, k, ptr(out),
                                out.stride(0), int(accumulate), current_stream(a.device)))
     return out
@@ -927,7 +927,7 @@ def select_rows(keep: Tensor, skip: int = 0) -> tuple[Tensor, Tensor, Tensor]:
         return none, none, torch.zeros((), dtype=torch.int64, device=dev)
     buf = torch.empty((2 + 2 * n,), dtype=torch.int32, device=dev)
     count, index, position = buf[:2].view(torch.int64)[0], buf[2 : 2 + n], buf[2 + n :]
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_select_rows(ptr(keep), _KEEP_TYPES[keep.dtype], rows, cols, keep.stride(0), skip, ptr(index),
                                    ptr(position), ptr(count), current_stream(dev)))
     return index, position, count
@@ -944,7 +944,7 @@ def gather_rows(hidden: Tensor, targets: Tensor, index: Tensor, n: int) -> tuple
     rows = torch.empty((n, h), dtype=hidden.dtype, device=dev)
     picked = torch.empty((n,), dtype=torch.int64, device=dev)
     if n:
-        with torch.cuda.device(dev):
+        with on_device(dev):
             check(lib.trlk_gather_rows(ptr(hidden), h * size, hidden.stride(0) * size, hidden.stride(1) * size,
                                        targets.shape[1], ptr(index), n, ptr(rows), ptr(targets), targets.stride(0),
                                        ptr(picked), current_stream(dev)))
@@ -957,7 +957,7 @@ def scatter_rows(rows: Tensor, position: Tensor, shape: tuple[int, int, int], co
     out = torch.empty(shape, dtype=rows.dtype, device=rows.device)
     if position.numel() == 0 or rows.numel() == 0:
         return out.zero_()
-    with torch.cuda.device(rows.device):
+    with on_device(rows.device):
         check(lib.trlk_scatter_rows(ptr(rows), shape[2] * rows.element_size(), ptr(position), shape[0], cols, shape[1],
                                     ptr(out), current_stream(rows.device)))
     return out
@@ -968,7 +968,7 @@ def scatter_values(a: Tensor, b: Optional[Tensor], position: Tensor, shape: tupl
     out_a = torch.empty(shape, dtype=torch.float32, device=a.device)
     out_b = None if b is None else torch.empty(shape, dtype=torch.float32, device=a.device)
     if position.numel():
-        with torch.cuda.device(a.device):
+        with on_device(a.device):
             check(lib.trlk_scatter_values(ptr(a), ptr(b), ptr(position), position.numel(), ptr(out_a), ptr(out_b),
                                           current_stream(a.device)))
     return out_a, out_b
@@ -986,7 +986,7 @@ def mean_logits(hidden: Tensor, weight: Tensor) -> Tensor:
     ws_bytes = lib.trlk_mean_logits_workspace_bytes(h)
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
     out = torch.empty((b, lib.trlk_mean_logits_chunks(t)), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check(lib.trlk_mean_logits(ptr(hidden), ptr(weight), dtype_code(hidden.dtype), b, t, weight.shape[0], h,
                                    hidden.stride(0), hidden.stride(1), weight.stride(0), ptr(out), ptr(ws), ws_bytes,
                                    current_stream(dev)))
