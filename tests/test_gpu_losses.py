@@ -756,3 +756,15 @@ def test_dpo_log_values(amd, pairs, T):
     rewards = torch.cat([0.1 * (seq64[:pairs] - rc.double()), 0.1 * (seq64[pairs:] - rr.double())])
     torch.testing.assert_close(got[8 : 8 + B], rewards, rtol=1e-6, atol=1e-7)
     assert torch.equal(got[8 + B :], seq64)
+
+
+def test_log_and_scale_ops_can_be_traced(amd):
+    """Schema and shapes of the ops inside the loss functions that a tracer calls with fake tensors."""
+    from trl_amd import _lib, ops
+
+    f = lambda *s: torch.rand(s, device=DEV)  # noqa: E731
+    checks = ("test_schema", "test_faketensor")
+    for with_mask in (True, False):
+        args = (torch.ones((3, 5), device=DEV), _lib.DAPO, 1.0, f(1).reshape(()), None, with_mask)
+        torch.library.opcheck(ops._grpo_row_scale, args, test_utils=checks)
+    torch.library.opcheck(ops.dpo_log_values, (f(4, 6), f(4, 6, 4), f(4, 6), f(4), f(2), f(2), 0.1), test_utils=checks)

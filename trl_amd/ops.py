@@ -582,45 +582,64 @@ def grpo_log_values(metrics: Tensor) -> Tensor:
     return out
 
 
-def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Optional[Tensor] = None,
-                   upstream: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
-    """`(mask in fp32, d loss / d masked token loss [B])` of a `[B, T]` mask (`trlk_grpo_row_scale`); `n_items` and
-    `upstream` are fp32 device scalars."""
+@torch.library.custom_op("trl_amd::grpo_row_scale", mutates_args=(), device_types="cuda")
+def _grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Optional[Tensor], upstream: Optional[Tensor],
+                    with_mask: bool) -> tuple[Tensor, Tensor]:
     B, T = mask.shape
     dev = mask.device
-    if not mask.is_cuda or any(t is not None and t.device != dev for t in (n_items, upstream)):
+    if any(t is not None and t.device != dev for t in (n_items, upstream)):
         raise ValueError("grpo_row_scale: the mask and the scalars must be on one GPU")
-    if mask.dtype not in _KEEP_TYPES:
-        mask = mask.float()
-    as_is = mask.dtype == torch.float32 and mask.is_contiguous()
-    mask_f = mask if as_is else torch.empty((B, T), dtype=torch.float32, device=dev)
+    mask_f = torch.empty((B, T) if with_mask else (0,), dtype=torch.float32, device=dev)
     scale = torch.empty((B,), dtype=torch.float32, device=dev)
     with on_device(dev):
         check(lib.trlk_grpo_row_scale(ptr(mask), _KEEP_TYPES[mask.dtype], B, T, mask.stride(0), mask.stride(1), loss_type,
-                                      numerator, ptr(n_items), ptr(upstream), None if as_is else ptr(mask_f), ptr(scale),
+                                      numerator, ptr(n_items), ptr(upstream), ptr(mask_f) if with_mask else None, ptr(scale),
                                       current_stream(dev)))
     return mask_f, scale
 
 
+@_grpo_row_scale.register_fake
+def _(mask, loss_type, numerator, n_items, upstream, with_mask):
+    f = lambda *s: torch.empty(s, dtype=torch.float32, device=mask.device)  # noqa: E731
+    return (f(*mask.shape) if with_mask else f(0)), f(mask.shape[0])
+
+
+def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Optional[Tensor] = None,
+                   upstream: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
+    """`(mask in fp32, d loss / d masked token loss [B])` of a `[B, T]` mask (`trlk_grpo_row_scale`); `n_items` and
+    `upstream` are fp32 device scalars."""
+    if mask.dtype not in _KEEP_TYPES:
+        mask = mask.float()
+    as_is = mask.dtype == torch.float32 and mask.is_contiguous()
+    mask_f, scale = _grpo_row_scale(mask, loss_type, numerator, n_items, upstream, not as_is)
+    return (mask if as_is else mask_f), scale
+
+
+@torch.library.custom_op("trl_amd::dpo_log_values", mutates_args=(), device_types="cuda")
 def dpo_log_values(entropy: Tensor, row_stats: Tensor, mask: Tensor, seq_logps: Tensor, ref_chosen: Tensor,
                    ref_rejected: Tensor, beta: float) -> Tensor:
     """What a DPO step logs, as one fp32 device vector `[8 + 4 P]` (`trlk_dpo_log_values`): `entropy`, `mask` `[2P, T]`,
-    `row_stats` `[2P, T, 4]` (contiguous), `seq_logps` `[2P]`, the reference's log-probs `[P]` or broadcast to it."""
+    `row_stats` `[2P, T, 4]`, `seq_logps` `[2P]`, the reference's log-probs `[P]` or broadcast to it."""
     B, T = mask.shape
     P, dev = B // 2, mask.device
     if B % 2 or entropy.numel() != B * T or row_stats.numel() != 4 * B * T or seq_logps.numel() != B:
         raise ValueError("dpo_log_values: the shapes do not match")
-    mask, seq_logps, row_stats = _f32c(mask), _f32c(seq_logps), row_stats.contiguous()
+    entropy, row_stats, mask, seq_logps = _f32c(entropy), _f32c(row_stats), _f32c(mask), _f32c(seq_logps)
     ref_chosen, ref_rejected = _f32c(ref_chosen.expand(P)), _f32c(ref_rejected.expand(P))
     out = torch.empty((8 + 2 * B,), dtype=torch.float32, device=dev)
     if B == 0:
         return out.zero_()
     ws = torch.empty((4 * B,), dtype=torch.float32, device=dev)
     with on_device(dev):
-        check(lib.trlk_dpo_log_values(ptr(entropy.contiguous()), ptr(row_stats), ptr(mask), B, T, ptr(seq_logps),
-                                      ptr(ref_chosen), ptr(ref_rejected), beta, ptr(_error_flag(dev)), ptr(out), ptr(ws),
+        check(lib.trlk_dpo_log_values(ptr(entropy), ptr(row_stats), ptr(mask), B, T, ptr(seq_logps), ptr(ref_chosen),
+                                      ptr(ref_rejected), beta, ptr(_error_flag(dev)), ptr(out), ptr(ws),
                                       current_stream(dev)))
     return out
+
+
+@dpo_log_values.register_fake
+def _(entropy, row_stats, mask, seq_logps, ref_chosen, ref_rejected, beta):
+    return torch.empty((8 + 2 * mask.shape[0],), dtype=torch.float32, device=mask.device)
 
 
 @torch.library.custom_op("trl_amd::dpo_loss", mutates_args=(), device_types="cuda")
