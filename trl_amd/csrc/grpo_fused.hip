@@ -3,8 +3,8 @@
 // The two-pass path reads the logits twice (K1 for the log-probs, K3 for the gradient) because the loss sits
 // between them.  For the token-level GRPO losses the gradient coefficient of a token depends only on that
 // token's own log-prob, on per-token inputs (old / reference log-probs, advantage, mask, weight) and on
-// normalisers that are known from the mask before any logit is read.  A 1024-lane workgroup can hold a whole
-// vocabulary row of logits in registers (up to kMaxVec 16-byte vectors per lane: 8 16-bit or 4 fp32 logits each), so one workgroup
+// normalisers that are known from the mask before any logit is read.  A workgroup can hold a whole vocabulary row of
+// logits in registers (a lane up to kNarrowVec or kMaxVec 16-byte vectors: 8 16-bit or 4 fp32 logits each), so one workgroup
 // per row loads the row once, reduces it to (lse, entropy, target logit), evaluates the token's loss terms
 // with the same device functions as the [B, T]-sized loss kernel, and writes the row's dlogits from the
 // registers.  Rows outside the completion mask are never read: their gradient row is zero-filled and their
@@ -75,8 +75,8 @@ __device__ __forceinline__ void lds_transfer(const u32x4* src, uint32_t lds) {
 #pragma clang diagnostic pop
 
 // One workgroup of TH lanes per output row; NVEC = 16-byte vectors of the row a lane holds (the last kVecStep + 1 of
-// them may lie beyond the row's end for some lanes).  A workgroup fills its CU's register file, so nothing else
-// runs beside it: the arithmetic has to overlap the row's own memory traffic.  Hence
+// them may lie beyond the row's end for some lanes).  A workgroup of 1024 lanes fills its CU's register file, so nothing
+// else runs beside it: the arithmetic has to overlap the row's own memory traffic.  Hence
 //   * the per-row scalars are loaded first, from uniform addresses before any store: scalar loads, which return
 //     long before (and independently of) the row's vector loads; the target's logit is requested right behind the row;
 //   * the exponentials are summed while the row arrives: a lane takes its reference exponent r0 from its FIRST
