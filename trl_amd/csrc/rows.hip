@@ -111,12 +111,18 @@ __global__ __launch_bounds__(256) void scatter_values_kernel(const float* a, con
 }
 
 // ---- mean logits of whole sequences without logits: mean over t and v of hidden[b, t] . weight[v] =
-// (sum_t hidden[b, t] . wsum) / (T V) with wsum = sum_v weight[v].  Bound by the read of the weight (525 MB and 2048 hidden rows: 90 us, 5.8 TB/s, of
-// 112 us for all three launches);
-// converting it to fp32 first and summing that copy moved five times the bytes, 470 us.
+// (sum_t hidden[b, t] . wsum) / (T V) with wsum = sum_v weight[v].  Bound by the read of the weight (525 MB and 2048 hidden
+// rows: 89 us, 5.9 TB/s, of 113 us for all three launches; the same with fp32 sums); converting it to fp32 first and summing
+// that copy moved five times the bytes, 470 us.
 //
-// Column sums: workgroup (x, y) sums rows y, y + gridDim.y, ... of 2048 columns, 8 columns per lane in fp32, eight rows in
-// flight; the partial sums of the gridDim.y row sets are added in order by the second kernel.
+// A mean logit is small against the terms it is made of, and a chain of 250 fp32 additions per column (what 128256 rows in
+// 512 partial sums make) left it four times as far from 64 bits as the torch product (5e-7 against 1.3e-7 of its value on
+// [2, 512] positions).  So sums are exact or in fp64 on the chip and rounded to fp32 once on their way to memory: in 2^-24 of
+// the size that such a sum of random terms has, 0.7 to 1.3 where the torch product is 2.7 to 3.6 away (32000 to 202048 rows).
+//
+// Column sums: workgroup (x, y) sums rows y, y + gridDim.y, ... of 2048 columns, 8 columns per lane, eight rows in flight:
+// those are added up in pairs in fp32 (their 16-bit values leave 13 bits and more to spare), then to the fp64 sum; the
+// partial sums of the gridDim.y row sets are added in order by the second kernel.
 constexpr int kColBlock = 256, kColParts = 512;
 template <int DT>
 __global__ __launch_bounds__(kColBlock) void column_sum_kernel(const uint16_t* w, int64_t ld, int rows, int cols8, float* parts) {
@@ -124,64 +130,69 @@ __global__ __launch_bounds__(kColBlock) void column_sum_kernel(const uint16_t* w
     if (c >= cols8) return;
     const u32x4* p = reinterpret_cast<const u32x4*>(w) + c;
     const int64_t ld8 = ld / 8;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    auto add = [&](u32x4 q) {
-        float x[8];
-        Elem<DT>::unpack(q, x);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += x[i];
-    };
+    double acc[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
     int r = blockIdx.y;
     for (; r + 7 * step < rows; r += 8 * step) {
         u32x4 q[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) q[k] = p[int64_t(r + k * step) * ld8];
+        float x[8][8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) add(q[k]);
+        for (int k = 0; k < 8; ++k) Elem<DT>::unpack(q[k], x[k]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            acc[i] += double(((x[0][i] + x[1][i]) + (x[2][i] + x[3][i])) + ((x[4][i] + x[5][i]) + (x[6][i] + x[7][i])));
     }
-    for (; r < rows; r += step) add(p[int64_t(r) * ld8]);
+    for (; r < rows; r += step) {
+        float x[8];
+        Elem<DT>::unpack(p[int64_t(r) * ld8], x);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] += double(x[i]);
+    }
     float* o = parts + (int64_t(blockIdx.y) * cols8 + c) * 8;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = acc[i];
+    for (int i = 0; i < 8; ++i) o[i] = float(acc[i]);
 }
 // One workgroup per 64 columns: its 16 waves add every 16th partial, then each other.
 __global__ __launch_bounds__(1024) void column_sum_finish_kernel(const float* parts, int n_parts, int cols, float* out) {
-    __shared__ float sum[16][kWave];
+    __shared__ double sum[16][kWave];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, c = blockIdx.x * kWave + lane;
-    float s = 0.f;
+    double s = 0.;
     if (c < cols)
-        for (int p = wave; p < n_parts; p += 16) s += parts[int64_t(p) * cols + c];
+        for (int p = wave; p < n_parts; p += 16) s += double(parts[int64_t(p) * cols + c]);
     sum[wave][lane] = s;
     __syncthreads();
     if (wave == 0 && c < cols) {
-        float t = 0.f;
+        double t = 0.;
 #pragma unroll
         for (int k = 0; k < 16; ++k) t += sum[k][lane];
-        out[c] = t;
+        out[c] = float(t);
     }
 }
 // out[b][chunk] = scale * sum over the chunk's rows of hidden[b, t] . wsum, one wave per row at a time.
 constexpr int kDotRows = 16;  // rows per workgroup
 template <int DT>
 __global__ __launch_bounds__(256) void row_dot_kernel(const uint16_t* hidden, int64_t seq_stride, int64_t row_stride, int T,
-                                                      int cols8, const float* wsum, float scale, float* out) {
-    __shared__ float part[4];
+                                                      int cols8, const float* wsum, double scale, float* out) {
+    __shared__ double part[4];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int t0 = blockIdx.x * kDotRows, t1 = min(T, t0 + kDotRows);
-    float s = 0.f;
+    double s = 0.;
     for (int t = t0 + wave; t < t1; t += 4) {
         const u32x4* row = reinterpret_cast<const u32x4*>(hidden + int64_t(blockIdx.y) * seq_stride + int64_t(t) * row_stride);
         for (int c = lane; c < cols8; c += kWave) {
             float x[8];
             Elem<DT>::unpack(row[c], x);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s = fmaf(x[i], wsum[c * 8 + i], s);
+            for (int i = 0; i < 8; ++i) s = fma(double(x[i]), double(wsum[c * 8 + i]), s);
         }
     }
-    s = wave_sum(s);
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane == 0) part[wave] = s;
     __syncthreads();
-    if (threadIdx.x == 0) out[int64_t(blockIdx.y) * gridDim.x + blockIdx.x] = scale * (part[0] + part[1] + part[2] + part[3]);
+    if (threadIdx.x == 0)
+        out[int64_t(blockIdx.y) * gridDim.x + blockIdx.x] = float(scale * (part[0] + part[1] + part[2] + part[3]));
 }
 
 bool whole_pieces(const void* a, const void* b, int64_t bytes) {
@@ -309,7 +320,7 @@ extern "C" int trlk_mean_logits(const void* d_hidden, const void* d_weight, int 
     const int cols8 = int(hidden_size / 8), n_parts = int(vocab < kColParts ? vocab : kColParts);
     float* parts = static_cast<float*>(d_workspace);
     float* wsum = parts + int64_t(n_parts) * hidden_size;
-    const float scale = float(1.0 / (double(rows_per_seq) * double(vocab)));
+    const double scale = 1.0 / (double(rows_per_seq) * double(vocab));
     auto go = [&](auto tag) {
         constexpr int DT = decltype(tag)::value;
         hipLaunchKernelGGL(column_sum_kernel<DT>, dim3(unsigned((cols8 + kColBlock - 1) / kColBlock), unsigned(n_parts)),
