@@ -207,3 +207,24 @@ def test_mean_logits_lose_nothing_to_long_sums(amd, b, t, h, v, seed):
     size = (h64.square() @ w64.square().sum(0)).sqrt() / (t * v)
     error = (got - want) / size * 2.0**24
     assert float(error.square().mean().sqrt()) < 1.6 and float(error.abs().max()) < 4.5, error
+
+
+def test_targets_of_another_shape(amd):
+    """What the length checks let through and what not: flat targets that hold one entry per position are the same as
+    targets of the hidden states' shape; reference hidden states of another length are refused."""
+    from trl_amd.trainer.sft_trainer import _chunked_cross_entropy_loss
+
+    _, hidden, weight, _, _ = _problem(4, 2, 6, 64, 300)
+    hidden, weight = hidden.to(DEV), weight.to(DEV)
+    ids = torch.arange(12, device=DEV).view(2, 6)
+    mask, adv = torch.ones_like(ids), torch.tensor([1.0, -1.0], device=DEV)
+    op = amd.FusedLinearGRPOLoss(beta=0.0)
+    assert torch.equal(op(hidden, weight, ids, mask, adv)[0], op(hidden, weight, ids.reshape(-1), mask, adv)[0])
+    sft = lambda **kw: torch.stack([x.double() for x in _chunked_cross_entropy_loss(hidden, weight, 64, **kw)])  # noqa: E731
+    assert torch.equal(sft(shift_labels=ids), sft(shift_labels=ids.reshape(-1)))
+    assert torch.equal(sft(shift_labels=ids.view(3, 4)), sft(shift_labels=ids))
+    for short in (hidden[:, :5], hidden[:1]):
+        with pytest.raises(ValueError, match="do not match"):
+            amd.FusedLinearDPOLoss()(weight, hidden, ids, None, short)
+        with pytest.raises(ValueError, match="do not match"):
+            amd.FusedLinearKTOLoss()(hidden, weight, ids, None, [True, False], short)

@@ -1,5 +1,6 @@
 """Host-side logic that needs no GPU: how the model call's keyword arguments are built for a sub-batch of a multimodal
 batch (trl/trainer/grpo_trainer.py:1463-1510), and when the fused head keeps its stash."""
+import pytest
 import torch
 
 
@@ -87,3 +88,29 @@ def test_head_stash_budget_and_shape(monkeypatch):
     monkeypatch.delenv("TRL_AMD_HEAD_STASH_GIB")
     assert ops.head_stash_fits(32768, 151936) and not ops.head_stash_fits(0, v)  # 10.3 GB of the default 24 GiB
     assert not ops.head_stash_fits(131072, 151936)  # 41 GB
+
+
+@pytest.mark.parametrize("shape", [(2, 5), (2, 7), (2, 4), (1, 6), (3, 6)])
+def test_head_entry_points_refuse_targets_of_another_length(shape):
+    """Hidden states [2, 6, H] with targets (or a mask) of another length: a target paired with another position's
+    hidden state gives a loss without an error, so every entry point refuses them, on the host."""
+    import trl_amd
+    from trl_amd.trainer.sft_trainer import _chunked_cross_entropy_loss
+
+    hidden, weight = torch.randn(2, 6, 8), torch.randn(16, 8)
+    ids, ok, adv = torch.ones(shape, dtype=torch.long), torch.ones(2, 6, dtype=torch.long), torch.randn(2)
+    grpo = trl_amd.FusedLinearGRPOLoss(beta=0.0)
+    calls = {
+        "sft labels": lambda: _chunked_cross_entropy_loss(hidden, weight, 8, labels=ids),
+        "sft shift_labels": lambda: _chunked_cross_entropy_loss(hidden, weight, 8, shift_labels=ids),
+        "scoring labels": lambda: trl_amd.chunked_logprobs_from_hidden(hidden, weight, ids, ok, 1.0),
+        "scoring mask": lambda: trl_amd.chunked_logprobs_from_hidden(hidden, weight, ok, ids, 1.0),
+        "grpo ids": lambda: grpo(hidden, weight, ids, ok, adv),
+        "grpo mask": lambda: grpo(hidden, weight, ok, ids, adv),
+        "dpo": lambda: trl_amd.FusedLinearDPOLoss(use_ref_model=False)(weight, hidden, ids),
+        "kto": lambda: trl_amd.FusedLinearKTOLoss(use_ref_model=False)(hidden, weight, ids, None, [True, False]),
+    }
+    for name, call in calls.items():
+        with pytest.raises(ValueError, match="do not match"):
+            call()
+            pytest.fail(name)

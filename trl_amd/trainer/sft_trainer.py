@@ -2,6 +2,8 @@
 (`_chunked_cross_entropy_loss`, trl/trainer/sft_trainer.py:117-234)."""
 from __future__ import annotations
 
+import math
+
 import torch
 from torch import Tensor
 
@@ -30,14 +32,17 @@ def _chunked_cross_entropy_loss(
     the kernels need no token chunking).  `correct_count` counts tokens whose label holds the row maximum."""
     if labels is None and shift_labels is None:
         raise ValueError("At least one of `labels` or `shift_labels` must be provided.")
-    h = hidden_states.size(-1)
-    if shift_labels is not None:
+    h = hidden_states.shape[-1]
+    shifted = shift_labels is None and labels.shape == hidden_states.shape[:-1]
+    if shifted:  # label t + 1 belongs to position t; the last position has none
+        shape = math.prod(labels.shape[:-1]), labels.shape[-1]
+        hidden, targets = hidden_states.reshape(*shape, h), labels.reshape(shape)[:, 1:]
+    elif shift_labels is not None:
         hidden, targets = hidden_states.reshape(1, -1, h), shift_labels.reshape(1, -1)
-    else:  # label t + 1 belongs to position t; the last position has none
-        hidden = hidden_states.reshape(-1, hidden_states.shape[-2], h)
-        targets = labels.reshape(-1, labels.shape[-1])[:, 1:]
+    else:  # (labels of another shape that leave one label per remaining position)
+        hidden, targets = hidden_states[..., :-1, :].reshape(1, -1, h), labels[..., 1:].reshape(1, -1)
     logp, ent, hit, n_valid = _masked_head(hidden, lm_head_weight, targets, targets, 1.0, chunk_size,
-                                           final_logit_softcapping, logit_scale, lm_head_bias, -100, True, False)
+                                           final_logit_softcapping, logit_scale, lm_head_bias, -100, True, False, shifted)
     if logp.numel() == 0:
         # whole micro-batch masked: keep the loss attached to every trainable input (sft_trainer.py:186-195)
         loss = (hidden_states.float().sum() + lm_head_weight.float().sum()) * 0.0

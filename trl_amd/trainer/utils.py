@@ -292,14 +292,18 @@ class _MaskedHeadFunction(torch.autograd.Function):
 
 def _masked_head(hidden: Tensor, weight: Tensor, targets: Tensor, keep: Tensor, temperature: float, chunk_size: int,
                  softcap: float | None = None, logit_scale: float = 1.0, bias: Tensor | None = None, skip: int = 0,
-                 packed: bool = False, may_clip: bool = True):
-    """See `_MaskedHeadFunction`; the products are kept for a backward only where one can follow (under `no_grad` the
-    operands may still be parameters).  `may_clip=False`: the loss gives every token that enters a gradient."""
-    if not hidden.is_cuda:
-        raise NotImplementedError("the fused head runs on the GPU only")
-    if keep.shape != targets.shape or targets.shape[0] != hidden.shape[0] or targets.shape[1] > hidden.shape[1]:
+                 packed: bool = False, may_clip: bool = True, shifted: bool = False):
+    """See `_MaskedHeadFunction`; every position has a target, or with `shifted` all but the last one of a sequence.  The
+    products are kept for a backward only where one can follow (under `no_grad` the operands may still be parameters).
+    `may_clip=False`: the loss gives every token that enters a gradient."""
+    shape = (hidden.shape[0], max(0, hidden.shape[1] - 1) if shifted else hidden.shape[1])
+    # (targets and masks may come flat, or in any other shape of as many entries)
+    targets, keep = (t.reshape(shape) if t.shape != shape and t.numel() == shape[0] * shape[1] else t for t in (targets, keep))
+    if targets.shape != shape or keep.shape != shape:
         raise ValueError(f"fused head: hidden {tuple(hidden.shape)}, targets {tuple(targets.shape)} and mask "
                          f"{tuple(keep.shape)} do not match")
+    if not hidden.is_cuda:
+        raise NotImplementedError("the fused head runs on the GPU only")
     if any(t.device != hidden.device for t in (weight, targets, keep)):
         raise ValueError("fused head: the operands are on different devices")
     cap = 0.0 if softcap is None else float(softcap)
@@ -317,7 +321,7 @@ def chunked_logprobs_from_hidden(hidden_states: Tensor, lm_head_weight: Tensor, 
     lab = labels[:, 1:]
     if completion_mask is not None:
         return _masked_head(hidden_states, lm_head_weight, lab, completion_mask[:, 1:], temperature, chunk_size,
-                            final_logit_softcapping, logit_scale)[:2]
+                            final_logit_softcapping, logit_scale, shifted=True)[:2]
     hs = hidden_states[:, :-1, :]
     b, s, h = hs.shape
     lp_v, ent_v = _ChunkedLogProbFunction.apply(hs.reshape(b * s, h), lm_head_weight, lab.reshape(b * s), temperature,
