@@ -321,8 +321,9 @@ int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, const int64_
 
 /* Row selection around the fused head: the boolean indexing of hidden states, labels and log-probs by a completion mask
  * or by labels with an ignored value (trl/trainer/utils.py:1461-1481, sft_trainer.py:160-184) without its scans and sorts.
- * trlk_select_rows: position e = r * n_cols + c is kept when keep[r * row_stride + c] != skip; d_out_index[j] = the j-th
- *   kept position (room for n_rows * n_cols), d_out_position[e] = its number or -1, *d_out_count = how many.
+ * trlk_select_rows: position e = r * n_cols + c is kept when keep[r * row_stride + c] != skip (rows may overlap or be one
+ *   and the same, row_stride 0); d_out_index[j] = the j-th kept position (room for n_rows * n_cols),
+ *   d_out_position[e] = its number or -1, *d_out_count = how many.
  * trlk_gather_rows: d_out[j] = the row of position d_index[j] = b * n_cols + t, which starts at byte b * seq_stride_bytes +
  *   t * row_stride_bytes of d_src; d_out_targets[j] = d_targets[b * target_stride + t].
  * trlk_scatter_rows: row (b, s) of d_out [n_seq, out_cols] = row d_position[b * n_cols + s] of d_src, zero where that is

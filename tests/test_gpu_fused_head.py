@@ -766,3 +766,23 @@ def test_row_selection_gather_and_scatter(amd, rows, cols, skip, dtype, share):
     full = torch.zeros(rows * cols, device=DEV)
     full[want] = v
     assert torch.equal(a.reshape(-1), full) and torch.equal(b.reshape(-1), 2 * full)
+
+
+@pytest.mark.parametrize("rows,cols", [(2, 1), (3, 341), (5, 2049)])
+def test_selection_from_a_mask_that_is_broadcast(amd, rows, cols):
+    """A mask or labels expanded over the batch (row stride 0) or with overlapping rows select as their copies do."""
+    one = (torch.rand(1, cols + rows, generator=torch.Generator().manual_seed(cols)) < 0.5).long().to(DEV)
+    for keep in (one[:, 1 : cols + 1].expand(rows, cols), one[:, :cols].bool().expand(rows, cols),
+                 one.as_strided((rows, cols), (1, 1))):
+        (index, position, count), copy = amd.ops.select_rows(keep), amd.ops.select_rows(keep.contiguous())
+        assert int(count) == int(keep.sum()) and torch.equal(index[: int(count)], copy[0][: int(count)])
+        assert torch.equal(position, copy[1])
+
+
+def test_scoring_with_a_broadcast_mask(amd):
+    g = torch.Generator().manual_seed(8)
+    hidden, weight = torch.randn(3, 9, 64, generator=g).bfloat16().to(DEV), torch.randn(200, 64, generator=g).bfloat16().to(DEV)
+    labels = torch.randint(0, 200, (3, 9), generator=g).to(DEV)
+    mask = torch.tensor([[0, 0, 1, 1, 0, 1, 1, 1, 0]], device=DEV).expand(3, 9)
+    got, want = (amd.chunked_logprobs_from_hidden(hidden, weight, labels, m, 0.8) for m in (mask, mask.contiguous()))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and int((got[0] != 0).sum()) == 15

@@ -210,8 +210,7 @@ extern "C" int trlk_select_rows(const void* d_keep, int keep_type, int64_t n_row
     clear_error();
     TRLK_REQUIRE(n_rows >= 1 && n_cols >= 1 && n_rows < (int64_t(1) << 31) / n_cols - kScan, TRLK_ERR_BAD_SHAPE,
                  "select_rows: bad shape %lld x %lld", (long long)n_rows, (long long)n_cols);
-    TRLK_REQUIRE(n_rows == 1 || row_stride >= n_cols, TRLK_ERR_BAD_STRIDE, "select_rows: row_stride %lld < %lld columns",
-                 (long long)row_stride, (long long)n_cols);
+    TRLK_REQUIRE(n_rows == 1 || row_stride >= 0, TRLK_ERR_BAD_STRIDE, "select_rows: row_stride %lld", (long long)row_stride);
     TRLK_REQUIRE(d_keep && d_out_index && d_out_position && d_out_count, TRLK_ERR_NULL_POINTER, "select_rows: null pointer");
     const int n = int(n_rows * n_cols), cols = int(n_cols);
     const dim3 grid(unsigned((n + kScan - 1) / kScan));
