@@ -786,3 +786,11 @@ def test_scoring_with_a_broadcast_mask(amd):
     mask = torch.tensor([[0, 0, 1, 1, 0, 1, 1, 1, 0]], device=DEV).expand(3, 9)
     got, want = (amd.chunked_logprobs_from_hidden(hidden, weight, labels, m, 0.8) for m in (mask, mask.contiguous()))
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and int((got[0] != 0).sum()) == 15
+
+
+def test_selection_of_one_long_row(amd):
+    """A flat row of more than 2^31 / 1025 positions (the form that aligned labels arrive in)."""
+    keep = (torch.arange(2_100_001, device=DEV) % 3 == 0).view(1, -1)
+    index, position, count = amd.ops.select_rows(keep)
+    assert int(count) == 700_001 and torch.equal(index[:700_001], torch.arange(0, 2_100_001, 3, device=DEV, dtype=torch.int32))
+    assert torch.equal(position, torch.where(keep[0], torch.arange(2_100_001, device=DEV) // 3, -1).int())

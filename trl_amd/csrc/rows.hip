@@ -208,7 +208,8 @@ extern "C" int trlk_select_rows(const void* d_keep, int keep_type, int64_t n_row
                                 int64_t skip, int32_t* d_out_index, int32_t* d_out_position, int64_t* d_out_count,
                                 trlk_stream_t stream) {
     clear_error();
-    TRLK_REQUIRE(n_rows >= 1 && n_cols >= 1 && n_rows < (int64_t(1) << 31) / n_cols - kScan, TRLK_ERR_BAD_SHAPE,
+    // (the kernel counts positions in 32 bits, up to eight workgroups' shares ahead of its own)
+    TRLK_REQUIRE(n_rows >= 1 && n_cols >= 1 && n_rows <= ((int64_t(1) << 31) - 1 - 8 * kScan) / n_cols, TRLK_ERR_BAD_SHAPE,
                  "select_rows: bad shape %lld x %lld", (long long)n_rows, (long long)n_cols);
     TRLK_REQUIRE(n_rows == 1 || row_stride >= 0, TRLK_ERR_BAD_STRIDE, "select_rows: row_stride %lld", (long long)row_stride);
     TRLK_REQUIRE(d_keep && d_out_index && d_out_position && d_out_count, TRLK_ERR_NULL_POINTER, "select_rows: null pointer");
@@ -261,7 +262,7 @@ extern "C" int trlk_gather_rows(const void* d_src, int64_t row_bytes, int64_t se
 extern "C" int trlk_scatter_rows(const void* d_src, int64_t row_bytes, const int32_t* d_position, int64_t n_seq, int64_t n_cols,
                                  int64_t out_cols, void* d_out, trlk_stream_t stream) {
     clear_error();
-    TRLK_REQUIRE(n_seq >= 1 && n_cols >= 1 && out_cols >= n_cols && n_seq < ((int64_t(1) << 31) - kRowsPerBlock) / out_cols &&
+    TRLK_REQUIRE(n_seq >= 1 && n_cols >= 1 && out_cols >= n_cols && n_seq <= ((int64_t(1) << 31) - 1 - kRowsPerBlock) / out_cols &&
                      row_bytes >= 2 && row_bytes < (int64_t(1) << 31) && row_bytes % 2 == 0,
                  TRLK_ERR_BAD_SHAPE, "scatter_rows: bad sizes n_seq=%lld cols=%lld of %lld row bytes=%lld", (long long)n_seq,
                  (long long)n_cols, (long long)out_cols, (long long)row_bytes);
