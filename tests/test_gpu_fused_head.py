@@ -794,3 +794,12 @@ def test_selection_of_one_long_row(amd):
     index, position, count = amd.ops.select_rows(keep)
     assert int(count) == 700_001 and torch.equal(index[:700_001], torch.arange(0, 2_100_001, 3, device=DEV, dtype=torch.int32))
     assert torch.equal(position, torch.where(keep[0], torch.arange(2_100_001, device=DEV) // 3, -1).int())
+
+
+def test_scoring_with_a_mask_on_the_host(amd):
+    """A completion mask in host memory selects rows of device tensors, as boolean indexing lets it."""
+    g = torch.Generator().manual_seed(9)
+    hidden, weight = torch.randn(2, 9, 64, generator=g).bfloat16().to(DEV), torch.randn(200, 64, generator=g).bfloat16().to(DEV)
+    labels, mask = torch.randint(0, 200, (2, 9), generator=g).to(DEV), torch.rand(2, 9, generator=g) < 0.5
+    got, want = (amd.chunked_logprobs_from_hidden(hidden, weight, labels, m, 0.8) for m in (mask, mask.to(DEV)))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -320,7 +320,8 @@ def chunked_logprobs_from_hidden(hidden_states: Tensor, lm_head_weight: Tensor, 
     Returns `(log_probs, entropy)`."""
     lab = labels[:, 1:]
     if completion_mask is not None:
-        return _masked_head(hidden_states, lm_head_weight, lab, completion_mask[:, 1:], temperature, chunk_size,
+        mask = completion_mask[:, 1:].to(hidden_states.device)  # (a mask in host memory selects rows as well)
+        return _masked_head(hidden_states, lm_head_weight, lab, mask, temperature, chunk_size,
                             final_logit_softcapping, logit_scale, shifted=True)[:2]
     hs = hidden_states[:, :-1, :]
     b, s, h = hs.shape
