@@ -228,3 +228,13 @@ def test_targets_of_another_shape(amd):
             amd.FusedLinearDPOLoss()(weight, hidden, ids, None, short)
         with pytest.raises(ValueError, match="do not match"):
             amd.FusedLinearKTOLoss()(hidden, weight, ids, None, [True, False], short)
+
+
+def test_mean_logits_of_very_many_sequences(amd):
+    """More sequences than a grid's second axis holds (65535)."""
+    g = torch.Generator().manual_seed(2)
+    hidden, weight = torch.randn(65537, 2, 8, generator=g).bfloat16(), torch.randn(24, 8, generator=g).bfloat16()
+    got = amd.ops.mean_logits(hidden.to(DEV), weight.to(DEV)).cpu().double()
+    want = (hidden.double() @ weight.double().sum(0)).mean(1) / 24
+    scale = (hidden.double().abs() @ weight.double().abs().sum(0)).mean(1) / 24
+    assert bool(((got - want).abs() <= 1e-6 * scale).all())

@@ -999,7 +999,7 @@ def mean_logits(hidden: Tensor, weight: Tensor) -> Tensor:
     b, t, h = hidden.shape
     if (hidden.dtype not in (torch.bfloat16, torch.float16) or weight.dtype != hidden.dtype or h % 8 or not b * t
             or hidden.stride(2) != 1 or weight.stride(1) != 1 or (hidden.stride(0) | hidden.stride(1) | weight.stride(0)) % 8
-            or weight.stride(0) < h or (hidden.data_ptr() | weight.data_ptr()) % 16):
+            or weight.stride(0) < h or (hidden.data_ptr() | weight.data_ptr()) % 16 or b > 65535):  # (a grid's second axis)
         return (hidden.float() @ weight.float().sum(0)).mean(dim=1) / weight.shape[0]
     dev = hidden.device
     ws_bytes = lib.trlk_mean_logits_workspace_bytes(h)
