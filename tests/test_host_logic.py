@@ -114,3 +114,22 @@ def test_head_entry_points_refuse_targets_of_another_length(shape):
         with pytest.raises(ValueError, match="do not match"):
             call()
             pytest.fail(name)
+
+
+def test_a_batch_without_labels_needs_no_kernel():
+    """A micro-batch whose labels are all ignored has a zero loss attached to its inputs whatever else holds of it: on the
+    host, in a type that the head does not take, or cut to another length (the reference returns before its head,
+    trl/trainer/sft_trainer.py:186-195)."""
+    from trl_amd.trainer.sft_trainer import _chunked_cross_entropy_loss
+
+    for dtype, cols in ((torch.float32, 6), (torch.bfloat16, 6), (torch.float64, 6), (torch.float32, 5)):
+        hidden = torch.randn(2, 6, 8, dtype=dtype, requires_grad=True)
+        weight = torch.randn(16, 8, dtype=dtype, requires_grad=True)
+        for name in ("labels", "shift_labels"):
+            loss, correct, entropy, n_valid = _chunked_cross_entropy_loss(
+                hidden, weight, 8, **{name: torch.full((2, cols), -100)})
+            assert float(loss.detach()) == float(correct) == float(entropy) == int(n_valid) == 0 and n_valid.dtype == torch.int64
+            for grad in torch.autograd.grad(loss, (hidden, weight)):
+                assert not grad.any()
+            with pytest.raises((NotImplementedError, ValueError, TypeError)):
+                _chunked_cross_entropy_loss(hidden, weight, 8, **{name: torch.zeros((2, cols), dtype=torch.long)})

@@ -41,8 +41,13 @@ def _chunked_cross_entropy_loss(
         hidden, targets = hidden_states.reshape(1, -1, h), shift_labels.reshape(1, -1)
     else:  # (labels of another shape that leave one label per remaining position)
         hidden, targets = hidden_states[..., :-1, :].reshape(1, -1, h), labels[..., 1:].reshape(1, -1)
-    logp, ent, hit, n_valid = _masked_head(hidden, lm_head_weight, targets, targets, 1.0, chunk_size,
-                                           final_logit_softcapping, logit_scale, lm_head_bias, -100, True, False, shifted)
+    try:
+        logp, ent, hit, n_valid = _masked_head(hidden, lm_head_weight, targets, targets, 1.0, chunk_size,
+                                               final_logit_softcapping, logit_scale, lm_head_bias, -100, True, False, shifted)
+    except (ValueError, TypeError, NotImplementedError):
+        if bool((targets != -100).any()):
+            raise
+        logp, n_valid = targets.new_empty(0), targets.new_zeros((), dtype=torch.int64)  # nothing enters the head
     if logp.numel() == 0:
         # whole micro-batch masked: keep the loss attached to every trainable input (sft_trainer.py:186-195)
         loss = (hidden_states.float().sum() + lm_head_weight.float().sum()) * 0.0
