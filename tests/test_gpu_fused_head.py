@@ -803,3 +803,18 @@ def test_scoring_with_a_mask_on_the_host(amd):
     labels, mask = torch.randint(0, 200, (2, 9), generator=g).to(DEV), torch.rand(2, 9, generator=g) < 0.5
     got, want = (amd.chunked_logprobs_from_hidden(hidden, weight, labels, m, 0.8) for m in (mask, mask.to(DEV)))
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 65536), (1, 65537), (3, 43691), (7, 40961), (2, 524289)])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.bool])
+def test_selection_of_many_positions(amd, rows, cols, dtype):
+    """Both forms of the selection (one launch up to 65536 positions, three beyond), whole and ragged last workgroups,
+    rows of a wider tensor; against boolean indexing, exactly."""
+    g = torch.Generator(device=DEV).manual_seed(rows + cols)
+    for share in (0.4, 0.0, 1.0):
+        keep = (torch.rand(rows, cols + 1, generator=g, device=DEV) < share).to(dtype)[:, 1:]
+        index, position, count = amd.ops.select_rows(keep)
+        want = (keep != 0).reshape(-1)
+        flat = want.nonzero().squeeze(1)
+        assert int(count) == flat.numel() and torch.equal(index[: flat.numel()].long(), flat)
+        assert torch.equal(position.long(), torch.where(want, want.cumsum(0) - 1, -1))

@@ -1,9 +1,9 @@
 // Row selection for the fused head: which token rows a caller wants (a mask, or labels with an ignored value), their
 // hidden states and targets packed together, and results and gradients spread out again.  What boolean indexing needs a
 // scan of several launches, a host synchronisation per indexed tensor and a sort for (its backward) is one launch each
-// here and one synchronisation in all (the count, which the sizes of the packed tensors depend on).
+// here (the selection from more than 65536 positions takes three) and one synchronisation in all (the count, which the sizes of the packed tensors depend on).
 //
-// All four kernels are bound by launch latency at a few thousand tokens and by their bytes beyond that.
+// Bound by launch latency at a few thousand tokens and by their bytes beyond that.
 // An SFT step on 2052 positions, 1396 of them kept (H = 2048): 63 -> 27 launches, the selection 5.2, gather 6.6 and gradient
 // scatter 5.1 us, the step 1549 -> 1187 us.
 #include "common.hpp"
@@ -13,32 +13,48 @@
 namespace trlk {
 namespace {
 
-constexpr int kScan = 1024;  // positions per workgroup of the selection
+constexpr int kScan = 1024, kScanWaves = kScan / kWave;  // positions per workgroup of the selection
 
-// keep(r, c) = p[r * stride + c] != skip, positions numbered e = r * cols + c.  idx[j] = the j-th kept position, pos[e] =
-// its number or -1, *count = how many.  Workgroup b needs the number of kept positions before its own 1024: it counts them
-// itself (at most 8 bytes per position out of the L2, eight loads in flight per lane) instead of waiting for the others.
+// keep(r, c) = p[r * stride + c] != skip, positions numbered e = r * cols + c.
 template <typename T>
-__global__ __launch_bounds__(kScan) void select_rows_kernel(const T* p, int n, int cols, int64_t stride, T skip, int32_t* idx,
-                                                            int32_t* pos, int64_t* count) {
-    constexpr int kWaves = kScan / kWave;
-    __shared__ int before_wave[kWaves], in_wave[kWaves];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    auto kept = [&](int e) {
+struct Keep {
+    const T* p;
+    int64_t stride;
+    int cols;
+    T skip;
+    __device__ __forceinline__ bool operator()(int e) const {
         const int r = e / cols;
         return p[int64_t(r) * stride + (e - r * cols)] != skip;
-    };
+    }
+};
+
+// idx[j] = the j-th kept position, pos[e] = its number or -1, *count = how many.  Workgroup b needs the number of kept
+// positions before its own 1024.  Up to kOneLaunch positions it counts them itself (at most 8 bytes per position out of the
+// L2, eight loads in flight per lane) instead of waiting for the others; that reads n^2 / 2048 positions in all, so beyond
+// that (BASE) pos[1024 b] holds the number already, from the two kernels below.  One launch against three, int64 labels: 49152
+// positions 13.8 us against about 15 (three launches), 65536 17.3, 81920 20.8 against 16.0, 131072 31 against 15.7, 1048576
+// 523 against 15.3 us.
+constexpr int kOneLaunch = 65536;
+template <typename T, bool BASE>
+__global__ __launch_bounds__(kScan) void select_rows_kernel(Keep<T> kept, int n, int32_t* idx, int32_t* pos, int64_t* count) {
+    __shared__ int before_wave[kScanWaves], in_wave[kScanWaves];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int first = blockIdx.x * kScan, e = first + tid;
     const bool mine = e < n && kept(e);
-    int before = 0, k = tid;
-    for (; k + 7 * kScan < first; k += 8 * kScan) {
-        bool q[8];
+    int before = 0;
+    if constexpr (BASE) {
+        before = tid == 0 ? pos[first] : 0;  // (read before the barrier below, overwritten after it, by this workgroup alone)
+    } else {
+        int k = tid;
+        for (; k + 7 * kScan < first; k += 8 * kScan) {
+            bool q[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) q[i] = kept(k + i * kScan);
+            for (int i = 0; i < 8; ++i) q[i] = kept(k + i * kScan);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) before += q[i];
+            for (int i = 0; i < 8; ++i) before += q[i];
+        }
+        for (; k < first; k += kScan) before += kept(k);
     }
-    for (; k < first; k += kScan) before += kept(k);
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) before += __shfl_xor(before, o);
     const uint64_t vote = __ballot(mine);
@@ -49,7 +65,7 @@ __global__ __launch_bounds__(kScan) void select_rows_kernel(const T* p, int n, i
     __syncthreads();
     int at = __popcll(vote & ((uint64_t(1) << lane) - 1)), total = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
+    for (int w = 0; w < kScanWaves; ++w) {
         total += before_wave[w] + in_wave[w];
         at += before_wave[w] + (w < wave ? in_wave[w] : 0);
     }
@@ -58,6 +74,49 @@ __global__ __launch_bounds__(kScan) void select_rows_kernel(const T* p, int n, i
         if (mine) idx[at] = e;
     }
     if (tid == 0 && int(blockIdx.x) == int(gridDim.x) - 1) *count = total;
+}
+
+// pos[1024 b] = kept positions among the 1024 from there on
+template <typename T>
+__global__ __launch_bounds__(kScan) void count_rows_kernel(Keep<T> kept, int n, int32_t* pos) {
+    __shared__ int in_wave[kScanWaves];
+    const int tid = threadIdx.x, e = blockIdx.x * kScan + tid;
+    const uint64_t vote = __ballot(e < n && kept(e));
+    if ((tid & (kWave - 1)) == 0) in_wave[tid / kWave] = __popcll(vote);
+    __syncthreads();
+    if (tid == 0) {
+        int s = 0;
+#pragma unroll
+        for (int w = 0; w < kScanWaves; ++w) s += in_wave[w];
+        pos[blockIdx.x * kScan] = s;
+    }
+}
+
+// pos[1024 b] -> the sum of those before it, for b < blocks: one workgroup, 1024 of them at a time
+__global__ __launch_bounds__(kScan) void count_prefix_kernel(int blocks, int32_t* pos) {
+    __shared__ int in_wave[kScanWaves];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    int carry = 0;
+    for (int b0 = 0; b0 < blocks; b0 += kScan) {
+        const int b = b0 + tid;
+        const int own = b < blocks ? pos[int64_t(b) * kScan] : 0;
+        int upto = own;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int other = __shfl_up(upto, o);
+            if (lane >= o) upto += other;
+        }
+        if (lane == kWave - 1) in_wave[wave] = upto;
+        __syncthreads();
+        int before = carry;
+#pragma unroll
+        for (int w = 0; w < kScanWaves; ++w) {
+            before += w < wave ? in_wave[w] : 0;
+            carry += in_wave[w];
+        }
+        if (b < blocks) pos[int64_t(b) * kScan] = before + upto - own;
+        __syncthreads();  // (in_wave is written again)
+    }
 }
 
 // One wave per row, 16 bytes per lane (VEC) or 2 where rows, strides or pointers are not whole 16-byte pieces.
@@ -208,8 +267,8 @@ extern "C" int trlk_select_rows(const void* d_keep, int keep_type, int64_t n_row
                                 int64_t skip, int32_t* d_out_index, int32_t* d_out_position, int64_t* d_out_count,
                                 trlk_stream_t stream) {
     clear_error();
-    // (the kernel counts positions in 32 bits, up to eight workgroups' shares ahead of its own)
-    TRLK_REQUIRE(n_rows >= 1 && n_cols >= 1 && n_rows <= ((int64_t(1) << 31) - 1 - 8 * kScan) / n_cols, TRLK_ERR_BAD_SHAPE,
+    // (the kernels count positions in 32 bits, up to a workgroup's share beyond the last one)
+    TRLK_REQUIRE(n_rows >= 1 && n_cols >= 1 && n_rows <= ((int64_t(1) << 31) - 1 - kScan) / n_cols, TRLK_ERR_BAD_SHAPE,
                  "select_rows: bad shape %lld x %lld", (long long)n_rows, (long long)n_cols);
     TRLK_REQUIRE(n_rows == 1 || row_stride >= 0, TRLK_ERR_BAD_STRIDE, "select_rows: row_stride %lld", (long long)row_stride);
     TRLK_REQUIRE(d_keep && d_out_index && d_out_position && d_out_count, TRLK_ERR_NULL_POINTER, "select_rows: null pointer");
@@ -218,8 +277,16 @@ extern "C" int trlk_select_rows(const void* d_keep, int keep_type, int64_t n_row
     hipStream_t s = static_cast<hipStream_t>(stream);
     auto go = [&](auto tag) {
         typedef decltype(tag) T;
-        hipLaunchKernelGGL(select_rows_kernel<T>, grid, dim3(kScan), 0, s, static_cast<const T*>(d_keep), n, cols, row_stride,
-                           T(skip), d_out_index, d_out_position, d_out_count);
+        const Keep<T> kept{static_cast<const T*>(d_keep), row_stride, cols, T(skip)};
+        if (n <= kOneLaunch) {
+            hipLaunchKernelGGL((select_rows_kernel<T, false>), grid, dim3(kScan), 0, s, kept, n, d_out_index, d_out_position,
+                               d_out_count);
+            return;
+        }
+        hipLaunchKernelGGL(count_rows_kernel<T>, grid, dim3(kScan), 0, s, kept, n, d_out_position);
+        hipLaunchKernelGGL(count_prefix_kernel, dim3(1), dim3(kScan), 0, s, int(grid.x), d_out_position);
+        hipLaunchKernelGGL((select_rows_kernel<T, true>), grid, dim3(kScan), 0, s, kept, n, d_out_index, d_out_position,
+                           d_out_count);
     };
     switch (keep_type) {
         case TRLK_KEEP_U8: go(uint8_t{}); break;
