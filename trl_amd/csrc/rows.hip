@@ -1,7 +1,8 @@
 // Row selection for the fused head: which token rows a caller wants (a mask, or labels with an ignored value), their
 // hidden states and targets packed together, and results and gradients spread out again.  What boolean indexing needs a
 // scan of several launches, a host synchronisation per indexed tensor and a sort for (its backward) is one launch each
-// here (the selection from more than 65536 positions takes three) and one synchronisation in all (the count, which the sizes of the packed tensors depend on).
+// here (the selection from more than 65536 positions takes three) and one synchronisation in all (the count, which the sizes
+// of the packed tensors depend on).
 //
 // Bound by launch latency at a few thousand tokens and by their bytes beyond that.
 // An SFT step on 2052 positions, 1396 of them kept (H = 2048): 63 -> 27 launches, the selection 5.2, gather 6.6 and gradient
