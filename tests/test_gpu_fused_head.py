@@ -818,3 +818,36 @@ def test_selection_of_many_positions(amd, rows, cols, dtype):
         flat = want.nonzero().squeeze(1)
         assert int(count) == flat.numel() and torch.equal(index[: flat.numel()].long(), flat)
         assert torch.equal(position.long(), torch.where(want, want.cumsum(0) - 1, -1))
+
+
+@pytest.mark.parametrize("n,v,h,flat,products", [
+    (2048, 32000, 2048, 2, [1024, 2048]),  # 4 n V H of 4e11 and more: the products hold the tokens with a gradient only
+    (64, 50257, 2048, 2, [64, 64]),        # 1e8 weights, few tokens: packing some of them costs more than it gains,
+    (64, 50257, 2048, 4, [64]),            # but a micro-batch of one group whose rewards are all equal needs no products
+    (64, 4096, 256, 4, [64, 64]),          # not even searched
+])
+def test_tokens_without_gradient_leave_the_backward(amd, monkeypatch, n, v, h, flat, products):
+    """Groups whose rewards are all equal have no gradient: `products` lists the tokens of every call of the products,
+    with the search and with TRL_AMD_HEAD_DROP_ZERO_GRAD=0; the gradients are the same."""
+    from trl_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    hidden = torch.randn(4, n // 4, h, generator=g, device=DEV).bfloat16().requires_grad_(True)
+    weight = (torch.randn(v, h, generator=g, device=DEV) * 0.02).bfloat16().requires_grad_(True)
+    ids = torch.randint(0, v, (4, n // 4), generator=g, device=DEV)
+    adv = torch.tensor([0.0] * flat + [1.0, -1.0], device=DEV)[:4]
+    seen, real = [], ops.fused_head_bwd
+
+    def counted(hid, *args):
+        seen.append(hid.shape[0])
+        return real(hid, *args)
+
+    grads = []
+    monkeypatch.setattr(ops, "fused_head_bwd", counted)
+    for drop in ("1", "0"):
+        monkeypatch.setenv("TRL_AMD_HEAD_DROP_ZERO_GRAD", drop)
+        loss, _ = amd.FusedLinearGRPOLoss(beta=0.0)(hidden, weight, ids, torch.ones_like(ids), adv)
+        grads.append(torch.autograd.grad(loss, (hidden, weight)))
+    assert seen == products
+    for a, b in zip(*grads):  # (each rounded once to bf16; the products sum in another order)
+        assert _rel_l2(a, b) < 2.0**-8 if flat < 4 else not a.any() and not b.any()

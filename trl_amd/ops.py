@@ -1028,12 +1028,12 @@ def _backward_chunk(n_tokens: int, vocab: int, hidden_size: int, chunk_size: int
 
 def head_backward(hidden: Tensor, weight: Tensor, targets: Tensor, temperature: float, softcap: float,
                   logit_scale: float, log_z: Tensor, g_logp: Tensor, chunk_size: int, bias: Optional[Tensor] = None,
-                  stash: Optional[Tensor] = None, look_for_zeros: bool = True) -> tuple[Tensor, Tensor, Tensor]:
+                  stash: Optional[Tensor] = None, look_for_zeros: bool = True, pack: bool = True) -> tuple[Tensor, Tensor, Tensor]:
     """`fused_head_bwd` that first drops the tokens whose upstream gradient is exactly zero (masked positions of
     a policy loss): their dz row is zero, so they add nothing to d weight and their d hidden row is zero.  Both
     products shrink with the share of such tokens; one host synchronisation (the count) per call.  Tokens are only
-    dropped when at least a tenth of them can go.  `look_for_zeros=False`: the caller knows that
-    its loss leaves no token without a gradient."""
+    dropped when at least a tenth of them can go.  `look_for_zeros=False`: the caller knows that its loss leaves no token
+    without a gradient, or that the search costs more than it gains; `pack=False`: dropping some does (not all of them)."""
     n = hidden.shape[0]
     g = g_logp.reshape(-1)
     chunk_size = _backward_chunk(n, weight.shape[0], hidden.shape[-1], chunk_size) if chunk_size >= 1 else chunk_size
@@ -1041,7 +1041,7 @@ def head_backward(hidden: Tensor, weight: Tensor, targets: Tensor, temperature: 
         return fused_head_bwd(hidden, weight, targets, temperature, softcap, logit_scale, log_z, g, chunk_size, bias, stash)
     active = g != 0
     n_active = int(active.sum())
-    if n_active > 0.9 * n:
+    if n_active > 0.9 * n or (n_active and not pack):
         return fused_head_bwd(hidden, weight, targets, temperature, softcap, logit_scale, log_z, g, chunk_size, bias, stash)
     idx = active.nonzero().squeeze(1)
     d_hidden = torch.zeros_like(hidden)

@@ -240,7 +240,7 @@ def _head_forward(hidden, weight, targets, bias, cfg, keep_products):
     return ops.fused_head_fwd(hidden, weight, targets, temperature, cap, logit_scale, bias, stash)
 
 
-def _head_backward(hidden, weight, targets, log_z, bias, saved, cfg, grad_logprobs, look_for_zeros=True):
+def _head_backward(hidden, weight, targets, log_z, bias, saved, cfg, grad_logprobs, look_for_zeros=True, pack=True):
     """`(d hidden, d weight, d bias or None)` in the operands' dtypes."""
     temperature, chunk_size, cap, logit_scale = cfg
     if hidden.dtype == torch.float32:
@@ -250,7 +250,7 @@ def _head_backward(hidden, weight, targets, log_z, bias, saved, cfg, grad_logpro
         d_weight = d_weight.to(weight.dtype)
     else:
         d_hidden, d_weight, d_bias = ops.head_backward(hidden, weight, targets, temperature, cap, logit_scale,
-                                                        log_z, grad_logprobs, chunk_size, bias, saved, look_for_zeros)
+                                                        log_z, grad_logprobs, chunk_size, bias, saved, look_for_zeros, pack)
     return d_hidden, d_weight, None if bias is None else d_bias.to(bias.dtype)
 
 
@@ -269,9 +269,13 @@ class _MaskedHeadFunction(torch.autograd.Function):
                                                      with_grad and any(ctx.needs_input_grad[:2]))
         ctx.save_for_backward(rows, weight, picked, log_z, bias, saved, index, position)
         ctx.cfg, ctx.shape, ctx.cols, ctx.packed = cfg, tuple(hidden.shape), targets.shape[1], packed
-        # tokens that a loss clipped are worth looking for (a synchronisation, about 50 us) where the backward takes
-        # some milliseconds; masked ones are not among the packed rows
-        ctx.look_for_zeros = may_clip and 4 * n * weight.numel() > 2e12
+        # Tokens without gradient (masked ones are not among the packed rows) are those that a loss clipped and, far more
+        # of them, whole groups whose rewards are all equal.  The search costs a synchronisation, 35 to 80 us, and packing
+        # the others 80 us more.  A micro-batch that is one such group needs no products at all: 1320 of 2000 us for 113
+        # tokens of a 151936 x 3584 head, 200 of 655 at 50257 x 2048, 30 of 490 at 32000 x 1024 -- the passes over the
+        # weight, so it is searched for from 1e8 weights on.  With half of the tokens in such groups packing gains 60 of 940
+        # us at 4 n V H = 4.9e11 (32000 x 1024), nothing at 3e11 to 4e11 (128256 and 50257 x 2048), 600 of 3300 at 2e12.
+        ctx.drop = may_clip and (weight.numel() >= 1e8 or 4 * n * weight.numel() >= 4e11), 4 * n * weight.numel() >= 4e11
         if not packed:
             logp, ent = ops.scatter_values(logp, ent, position, tuple(targets.shape))
         ctx.mark_non_differentiable(ent, hit, count)
@@ -285,7 +289,7 @@ class _MaskedHeadFunction(torch.autograd.Function):
         *operands, index, position = ctx.saved_tensors
         n = operands[0].shape[0]
         g = g_logp if ctx.packed else g_logp.reshape(-1).index_select(0, index[:n])
-        d_rows, d_weight, d_bias = _head_backward(*operands, ctx.cfg, g, ctx.look_for_zeros)
+        d_rows, d_weight, d_bias = _head_backward(*operands, ctx.cfg, g, *ctx.drop)
         d_hidden = ops.scatter_rows(d_rows, position, ctx.shape, ctx.cols) if ctx.needs_input_grad[0] else None
         return d_hidden, d_weight, d_bias, None, None, None, None, None, None, None
 
