@@ -133,3 +133,32 @@ def test_a_batch_without_labels_needs_no_kernel():
                 assert not grad.any()
             with pytest.raises((NotImplementedError, ValueError, TypeError)):
                 _chunked_cross_entropy_loss(hidden, weight, 8, **{name: torch.zeros((2, cols), dtype=torch.long)})
+
+
+def test_backward_falls_back_to_the_callers_chunk_when_memory_is_short(monkeypatch):
+    """The head's backward raises the caller's chunk of vocabulary rows to what 1 GiB of scratch holds; where that cannot
+    be allocated it runs with the caller's own chunk, as a caller with little memory left has sized it."""
+    from trl_amd import ops
+
+    asked, free = [], [1 << 40]
+
+    def backward(hidden, weight, targets, t, cap, scale, log_z, g, chunk, *rest):
+        asked.append(chunk)
+        if chunk > free[0]:
+            raise torch.OutOfMemoryError("no room")
+        return hidden, weight, None
+
+    monkeypatch.setattr(ops, "fused_head_bwd", backward)
+    n, v, h = 64, 50257, 16
+    hidden, weight, g = torch.ones(n, h), torch.ones(1, h).expand(v, h), torch.ones(n)
+    run = lambda chunk, g: ops.head_backward(hidden, weight, torch.zeros(n, dtype=torch.long), 1.0, 0.0, 1.0, g, g, chunk)  # noqa: E731
+    run(4096, g)
+    assert asked == [v]  # (64 rows of 2 bytes per vocabulary row: all of it fits)
+    for grad in (g, torch.cat([g[:32], torch.zeros(32)])):  # every token, and the ones with a gradient
+        asked.clear()
+        free[0] = 4096
+        run(4096, grad)
+        assert asked == [v, 4096]
+        free[0] = 1
+        with pytest.raises(torch.OutOfMemoryError):
+            run(4096, g)

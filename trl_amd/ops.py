@@ -1017,7 +1017,7 @@ def mean_logits(hidden: Tensor, weight: Tensor) -> Tensor:
 # chunk the more the products lose in partial rounds of workgroups and in passes over dHidden.  So the caller's size is
 # raised to what this much scratch holds, and the vocabulary is cut into equal chunks.  1396 tokens, H = 2048, V = 50257,
 # chunk_size 8192: one chunk instead of seven, products 1136 -> 575 us (with the slices of the dHidden product), sweeps
-# and transposes 189 -> 126 us.
+# and transposes 189 -> 126 us.  Where that scratch cannot be allocated, the caller's own size is what it can have.
 _HEAD_SCRATCH_BYTES = 1 << 30
 
 
@@ -1036,22 +1036,32 @@ def head_backward(hidden: Tensor, weight: Tensor, targets: Tensor, temperature: 
     without a gradient, or that the search costs more than it gains; `pack=False`: dropping some does (not all of them)."""
     n = hidden.shape[0]
     g = g_logp.reshape(-1)
-    chunk_size = _backward_chunk(n, weight.shape[0], hidden.shape[-1], chunk_size) if chunk_size >= 1 else chunk_size
+
+    def products(hidden, targets, log_z, g, cols=None):
+        chunk = _backward_chunk(n, weight.shape[0], hidden.shape[-1], chunk_size) if chunk_size >= 1 else chunk_size
+        rest = () if cols is None else (cols,)
+        args = (hidden, weight, targets, temperature, softcap, logit_scale, log_z, g)
+        try:
+            return fused_head_bwd(*args, chunk, bias, stash, *rest)
+        except torch.OutOfMemoryError:
+            if chunk <= chunk_size:
+                raise
+        return fused_head_bwd(*args, chunk_size, bias, stash, *rest)  # (what the first try allocated is free by now)
+
     if n == 0 or not look_for_zeros or os.environ.get("TRL_AMD_HEAD_DROP_ZERO_GRAD", "1") == "0":
-        return fused_head_bwd(hidden, weight, targets, temperature, softcap, logit_scale, log_z, g, chunk_size, bias, stash)
+        return products(hidden, targets, log_z, g)
     active = g != 0
     n_active = int(active.sum())
     if n_active > 0.9 * n or (n_active and not pack):
-        return fused_head_bwd(hidden, weight, targets, temperature, softcap, logit_scale, log_z, g, chunk_size, bias, stash)
+        return products(hidden, targets, log_z, g)
     idx = active.nonzero().squeeze(1)
     d_hidden = torch.zeros_like(hidden)
     if n_active == 0:
         d_bias = torch.zeros((weight.shape[0] if bias is not None else 0,), dtype=torch.float32, device=hidden.device)
         return d_hidden, torch.zeros_like(weight), d_bias
     cols = idx.to(torch.int32) if stash is not None and stash.numel() else None
-    d_h, d_weight, d_bias = fused_head_bwd(
-        hidden.index_select(0, idx), weight, targets.index_select(0, idx), temperature, softcap, logit_scale,
-        log_z.index_select(0, idx), g.index_select(0, idx), chunk_size, bias, stash, cols)
+    d_h, d_weight, d_bias = products(hidden.index_select(0, idx), targets.index_select(0, idx), log_z.index_select(0, idx),
+                                     g.index_select(0, idx), cols)
     d_hidden.index_copy_(0, idx, d_h)
     return d_hidden, d_weight, d_bias
 

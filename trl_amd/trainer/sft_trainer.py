@@ -28,7 +28,8 @@ def _chunked_cross_entropy_loss(
     Same arguments and return value as the reference: `(loss, correct_count, entropy_sum, n_valid)` over the
     local batch; `labels` are shifted here, `shift_labels` are taken as already aligned; `-100` positions are
     dropped before the matmul; the loss is `sum / num_items_in_batch` if that is given, else the mean over
-    valid tokens.  `chunk_size` sizes the backward's vocabulary-chunk workspace (the reference chunks tokens;
+    valid tokens.  `chunk_size` is the number of vocabulary rows that the backward takes at a time where memory is
+    short: it is raised to what 1 GiB of workspace holds where that much can be allocated (the reference chunks tokens;
     the kernels need no token chunking).  `correct_count` counts tokens whose label holds the row maximum."""
     if labels is None and shift_labels is None:
         raise ValueError("At least one of `labels` or `shift_labels` must be provided.")

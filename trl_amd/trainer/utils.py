@@ -200,8 +200,9 @@ class _ChunkedLogProbFunction(torch.autograd.Function):
     (utils.py:1298-1307): `apply(last_hidden [N, H], weight [V, H], targets [N], temperature,
     chunk_size, final_logit_softcapping=None, logit_scale=1.0) -> (logprobs fp32 [N], entropy fp32 [N])`.
 
-    The forward is one matrix-core kernel sweep (no vocabulary chunking is needed, `chunk_size` only
-    sizes the backward's dz workspace).  When a gradient is required and the fp32 `[V, N]` products fit
+    The forward is one matrix-core kernel sweep (no vocabulary chunking is needed; `chunk_size` is
+    the number of vocabulary rows that the backward takes at a time where memory is short: it is raised to what 1 GiB of
+    workspace holds where that much can be allocated).  When a gradient is required and the fp32 `[V, N]` products fit
     `ops.head_stash_fits` (24 GiB by default), the forward keeps them and the backward skips the
     reference's recompute of the logits; otherwise it recomputes them chunk by chunk as the reference does.
     fp32 operands run through the same kernels as three bf16 pieces each (`ops.split_bf16x3`: the matrix cores take
