@@ -851,3 +851,20 @@ def test_tokens_without_gradient_leave_the_backward(amd, monkeypatch, n, v, h, f
     assert seen == products
     for a, b in zip(*grads):  # (each rounded once to bf16; the products sum in another order)
         assert _rel_l2(a, b) < 2.0**-8 if flat < 4 else not a.any() and not b.any()
+
+
+def test_row_selection_and_mean_logits_can_be_traced(amd):
+    """Schema and shapes of the ops around the head that a tracer calls with fake tensors."""
+    ops, checks = torch.ops.trl_amd, ("test_schema", "test_faketensor")
+    keep = torch.tensor([[1, 0, 1], [0, 1, 1]], device=DEV)
+    table, (index, position, _) = ops.select_rows(keep, 0), amd.ops.select_rows(keep)
+    assert table.dtype == torch.int32 and table.numel() == 14
+    hidden, ids = torch.randn(2, 4, 8, device=DEV).bfloat16(), torch.arange(6, device=DEV).view(2, 3)
+    values = torch.randn(4, device=DEV)
+    for op, args in (
+        (ops.select_rows, (keep, 0)), (ops.gather_rows, (hidden, ids, index, 4)),
+        (ops.scatter_rows, (hidden[0].contiguous(), position, [2, 4, 8], 3)),
+        (ops.scatter_values, (values, values, position, [2, 3])), (ops.mean_logits, (hidden, hidden[1])),
+        (ops.mean_logits, (hidden.float(), hidden[1].float())), (ops.grpo_log_values, (torch.rand(16, device=DEV),)),
+    ):
+        torch.library.opcheck(op.default, args, test_utils=checks)

@@ -69,6 +69,25 @@ def raise_for_error_bits(bits: float, device: torch.device) -> None:
         raise RuntimeError(f"trl_amd: device error flag {bits:#x}")
 
 
+# Ops without a gradient of their own (their callers' autograd functions have it) that run several times per step: no Python
+# autograd layer around them, as `custom_op` would put there.
+_library = torch.library.Library("trl_amd", "FRAGMENT")
+
+
+def _plain_op(schema: str, fake):
+    """Registers the decorated function as `trl_amd::<schema>` for GPU tensors, `fake` as its shapes for tracers; returns
+    the op."""
+    name = schema[: schema.index("(")]
+    _library.define(schema)
+    torch.library.register_fake(f"trl_amd::{name}", fake, lib=_library)
+
+    def register(fn):
+        _library.impl(name, fn, "CUDA")
+        return getattr(torch.ops.trl_amd, name).default
+
+    return register
+
+
 # --------------------------------------------------------------------------------------------
 # log-prob + entropy (K1 / K3)
 # --------------------------------------------------------------------------------------------
@@ -572,7 +591,9 @@ def scale_unless_one_(data: Tensor, scale: Tensor) -> Tensor:
 # --------------------------------------------------------------------------------------------
 # DPO / RLOO sequence losses (K4)
 # --------------------------------------------------------------------------------------------
-def grpo_log_values(metrics: Tensor) -> Tensor:
+@_plain_op("grpo_log_values(Tensor metrics) -> Tensor",
+           lambda metrics: metrics.new_empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32))
+def grpo_log_values(metrics):
     """What `_compute_loss` logs of the loss kernel's `metrics`, as one fp32 device vector (`trlk_grpo_log_values`): nine
     sums to be added over the processes, the smallest and the largest clip ratio, the policy loss, the error word."""
     dev = metrics.device
@@ -930,29 +951,39 @@ def gemm_nt(a: Tensor, b: Tensor, out: Optional[Tensor] = None, accumulate: bool
 _KEEP_TYPES = {torch.bool: 0, torch.uint8: 0, torch.int32: 1, torch.int64: 2, torch.float32: 3}
 
 
+@_plain_op("select_rows(Tensor keep, int skip) -> Tensor",
+           lambda keep, skip: keep.new_empty((2 + 2 * keep.shape[0] * keep.shape[1],), dtype=torch.int32))
+def _select_rows(keep, skip):
+    """The count as two words, then the index, then the position (see `select_rows`)."""
+    rows, cols = keep.shape
+    n, dev = rows * cols, keep.device
+    buf = torch.empty((2 + 2 * n,), dtype=torch.int32, device=dev)
+    if n == 0:
+        return buf.zero_()
+    with on_device(dev):
+        check(lib.trlk_select_rows(ptr(keep), _KEEP_TYPES[keep.dtype], rows, cols, keep.stride(0), skip, ptr(buf) + 8,
+                                   ptr(buf) + 8 + 4 * n, ptr(buf), current_stream(dev)))
+    return buf
+
+
 def select_rows(keep: Tensor, skip: int = 0) -> tuple[Tensor, Tensor, Tensor]:
-    """Positions of `keep` `[B, T]` (the last axis contiguous) whose value is not `skip`, in order: `(index, position,
-    count)`, int32 `[B * T]` flat positions of the kept ones (the first `count` entries), int32 `[B * T]` number of every
-    position among them or -1, and the int64 count `[]`, all on the device (`trlk_select_rows`)."""
+    """Positions of `keep` `[B, T]` whose value is not `skip`, in order: `(index, position, count)`, int32 `[B * T]` flat
+    positions of the kept ones (the first `count` entries), int32 `[B * T]` number of every position among them or -1, and
+    the int64 count `[]`, all on the device (`trlk_select_rows`)."""
     if keep.dtype not in _KEEP_TYPES:
         keep = keep != skip
         skip = 0
     if keep.stride(1) != 1:
         keep = keep.contiguous()
-    rows, cols = keep.shape
-    n, dev = rows * cols, keep.device
-    if n == 0:
-        none = torch.empty((0,), dtype=torch.int32, device=dev)
-        return none, none, torch.zeros((), dtype=torch.int64, device=dev)
-    buf = torch.empty((2 + 2 * n,), dtype=torch.int32, device=dev)
-    count, index, position = buf[:2].view(torch.int64)[0], buf[2 : 2 + n], buf[2 + n :]
-    with on_device(dev):
-        check(lib.trlk_select_rows(ptr(keep), _KEEP_TYPES[keep.dtype], rows, cols, keep.stride(0), skip, ptr(index),
-                                   ptr(position), ptr(count), current_stream(dev)))
-    return index, position, count
+    n = keep.shape[0] * keep.shape[1]
+    buf = _select_rows(keep, skip)
+    return buf[2 : 2 + n], buf[2 + n :], buf[:2].view(torch.int64)[0]
 
 
-def gather_rows(hidden: Tensor, targets: Tensor, index: Tensor, n: int) -> tuple[Tensor, Tensor]:
+@_plain_op("gather_rows(Tensor hidden, Tensor targets, Tensor index, SymInt n) -> (Tensor, Tensor)",
+           lambda hidden, targets, index, n: (hidden.new_empty((n, hidden.shape[2])),
+                                              targets.new_empty((n,), dtype=torch.int64)))
+def gather_rows(hidden, targets, index, n):
     """The first `n` positions of `index` out of `hidden[:, :T]` (`[B, S, H]`, S >= T) and `targets` `[B, T]`, packed:
     `([n, H], [n])` (`trlk_gather_rows`)."""
     if hidden.stride(2) != 1:
@@ -970,7 +1001,9 @@ def gather_rows(hidden: Tensor, targets: Tensor, index: Tensor, n: int) -> tuple
     return rows, picked
 
 
-def scatter_rows(rows: Tensor, position: Tensor, shape: tuple[int, int, int], cols: int) -> Tensor:
+@_plain_op("scatter_rows(Tensor rows, Tensor position, SymInt[] shape, SymInt cols) -> Tensor",
+           lambda rows, position, shape, cols: rows.new_empty(shape))
+def scatter_rows(rows, position, shape, cols):
     """`[B, S, H] = shape`: packed `rows` `[n, H]` at the places `position` (`[B * cols]`) gives them, zeros elsewhere
     (`trlk_scatter_rows`)."""
     out = torch.empty(shape, dtype=rows.dtype, device=rows.device)
@@ -982,18 +1015,25 @@ def scatter_rows(rows: Tensor, position: Tensor, shape: tuple[int, int, int], co
     return out
 
 
-def scatter_values(a: Tensor, b: Optional[Tensor], position: Tensor, shape: tuple[int, int]) -> tuple[Tensor, Optional[Tensor]]:
-    """Packed fp32 `[n]` vectors at the places `position` gives them, zeros elsewhere, as `shape` (`trlk_scatter_values`)."""
-    out_a = torch.empty(shape, dtype=torch.float32, device=a.device)
-    out_b = None if b is None else torch.empty(shape, dtype=torch.float32, device=a.device)
+def _scatter_values_fake(a, b, position, shape):
+    return a.new_empty(shape, dtype=torch.float32), a.new_empty(shape if b is not None else (0,), dtype=torch.float32)
+
+
+@_plain_op("scatter_values(Tensor a, Tensor? b, Tensor position, SymInt[] shape) -> (Tensor, Tensor)", _scatter_values_fake)
+def scatter_values(a, b, position, shape):
+    """Packed fp32 `[n]` vectors at the places `position` gives them, zeros elsewhere, as `shape` (`trlk_scatter_values`);
+    the second result is empty without `b`."""
+    out_a, out_b = _scatter_values_fake(a, b, position, shape)
     if position.numel():
         with on_device(a.device):
-            check(lib.trlk_scatter_values(ptr(a), ptr(b), ptr(position), position.numel(), ptr(out_a), ptr(out_b),
-                                          current_stream(a.device)))
+            check(lib.trlk_scatter_values(ptr(a), ptr(b), ptr(position), position.numel(), ptr(out_a),
+                                          ptr(out_b if b is not None else None), current_stream(a.device)))
     return out_a, out_b
 
 
-def mean_logits(hidden: Tensor, weight: Tensor) -> Tensor:
+@_plain_op("mean_logits(Tensor hidden, Tensor weight) -> Tensor",
+           lambda hidden, weight: hidden.new_empty((hidden.shape[0],), dtype=torch.float32))
+def mean_logits(hidden, weight):
     """`(hidden @ weight.T).mean((1, 2))` in fp32 for `hidden` `[B, T, H]`, `weight` `[V, H]`, without the logits
     (`trlk_mean_logits`; operands it does not take, fp32 ones among them, go through a torch product)."""
     b, t, h = hidden.shape
