@@ -768,3 +768,24 @@ def test_log_and_scale_ops_can_be_traced(amd):
         args = (torch.ones((3, 5), device=DEV), _lib.DAPO, 1.0, f(1).reshape(()), None, with_mask)
         torch.library.opcheck(ops._grpo_row_scale, args, test_utils=checks)
     torch.library.opcheck(ops.dpo_log_values, (f(4, 6), f(4, 6, 4), f(4, 6), f(4), f(2), f(2), 0.1), test_utils=checks)
+
+
+def _finish(amd, accelerator, metrics, loss_type="dapo"):
+    """What `_finish_loss` logs of a vector of kernel metrics."""
+    tr = _fake_trainer(amd, dict(loss_type=loss_type, beta=0.04, eps_low=0.2, eps_high=0.2), 4)
+    tr.accelerator = accelerator
+    tr._finish_loss(torch.zeros((), device=DEV), metrics, None, None, None, None, False, 1.0, "train", False)
+    return {k: v[-1] for k, v in tr._metrics["train"].items()}
+
+
+def test_one_process_logs_without_a_concatenation(amd, monkeypatch):
+    """accelerate's `reduce` returns a copy even in a single process; the log values then still go to the host as the
+    one vector that the kernel wrote."""
+    class Accelerator(_Identity):
+        def reduce(self, x, reduction="sum"):
+            return x.clone()
+
+    metrics = torch.arange(16, dtype=torch.float32, device=DEV) + 0.5
+    want = _finish(amd, _Identity(), metrics)
+    monkeypatch.setattr(torch, "cat", lambda *a, **k: pytest.fail("log values put together from parts"))
+    assert _finish(amd, Accelerator(), metrics) == want

@@ -696,11 +696,11 @@ class GRPOLossMixin:
         # gather would, instead of surfacing as a NaN loss)
         values = ops.grpo_log_values(metrics.detach())
         sums, low_min, high_max = values[:9], values[9:10], values[10:11]
-        totals = self.accelerator.reduce(sums, reduction="sum")
-        lows, highs = self.accelerator.gather(low_min), self.accelerator.gather(high_max)
-        if totals is sums and lows is low_min and highs is high_max:
-            host = values.tolist()
+        if self.accelerator.num_processes == 1:  # (accelerate's `reduce` would return a copy)
+            lows, highs, host = low_min, high_max, values.tolist()
         else:
+            totals = self.accelerator.reduce(sums, reduction="sum")
+            lows, highs = self.accelerator.gather(low_min), self.accelerator.gather(high_max)
             host = torch.cat([totals, lows.reshape(-1), highs.reshape(-1), values[11:]]).tolist()
         n = lows.numel()
         kl_sum, ent_sum, cnt, clip_cnt, aux_sum, aux_cnt, low, high, region = host[:9]
