@@ -789,3 +789,85 @@ def test_one_process_logs_without_a_concatenation(amd, monkeypatch):
     want = _finish(amd, _Identity(), metrics)
     monkeypatch.setattr(torch, "cat", lambda *a, **k: pytest.fail("log values put together from parts"))
     assert _finish(amd, Accelerator(), metrics) == want
+
+
+class _TwoProcesses(_Identity):
+    """Two processes: the other one's tensors are `other` of this one's."""
+
+    num_processes = 2
+
+    def __init__(self, other):
+        self.other = other
+
+    def gather(self, x):
+        return torch.cat([x.reshape(1) if x.dim() == 0 else x, self.other(x).reshape(1) if x.dim() == 0 else self.other(x)])
+
+    gather_for_metrics = gather
+
+    def reduce(self, x, reduction="sum"):
+        return x + self.other(x)
+
+
+@pytest.mark.parametrize("low,high", [((0.25, 0.5), (0.75, 0.5)), ((math.nan, 0.5), (0.25, math.nan)),
+                                      ((math.nan, math.nan), (math.nan, math.nan))])
+def test_grpo_log_of_two_processes(amd, low, high):
+    """Sums added over the processes, means of the sums, the smallest and the largest clip ratio over both (a process
+    whose sequences were all masked has none)."""
+    m = torch.arange(16, dtype=torch.float32, device=DEV) + 0.5
+    m[5], m[6] = low[0], high[0]
+    calls = []
+
+    def other(x):
+        calls.append(x.numel())
+        return 3 * x if x.numel() > 1 else torch.full_like(x, (low, high)[len(calls) - 2][1])
+
+    got = _finish(amd, _TwoProcesses(other), m)
+    assert calls == [9, 1, 1]  # one reduction, two gathers
+    mask, clip = 4 * 8.5, 4 * 12.5
+    want = {"kl": 4 * 9.5 / mask, "entropy": 4 * 10.5 / mask, "clip_ratio/low_mean": 4 * 2.5 * 12.5 / clip,
+            "clip_ratio/high_mean": 4 * 3.5 * 12.5 / clip, "clip_ratio/region_mean": 4 * 4.5 * 12.5 / clip}
+    for k, v in want.items():
+        assert abs(got[k] - v) <= 1e-6 * v, k
+    for k, values, best in (("low_min", low, min), ("high_max", high, max)):
+        there = [x for x in values if x == x]
+        assert got["clip_ratio/" + k] == best(there) if there else math.isnan(got["clip_ratio/" + k])
+
+
+def test_dpo_log_of_two_processes(amd):
+    """Every logged value of a DPO step over two processes against plain arithmetic on both processes' parts."""
+    class Trainer(amd.DPOLossMixin):
+        pass
+
+    g = torch.Generator().manual_seed(12)
+    P, L, V = 3, 9, 50
+    ids = torch.randint(0, V, (2 * P, L), generator=g).to(DEV)
+    mask = (torch.rand(2 * P, L, generator=g) < 0.7).long().to(DEV)
+    ref_c, ref_r = torch.randn(P, generator=g).to(DEV) - 25, torch.randn(P, generator=g).to(DEV) - 25
+    leaf = torch.randn(2 * P, L, V, generator=g).to(DEV).requires_grad_(True)
+    other = lambda x: x + 5 if x.dtype == torch.int64 else 0.5 * x + 1  # noqa: E731
+    tr = Trainer()
+    tr.accelerator, tr.model, tr.aux_loss_enabled, tr.precompute_ref_logps = _TwoProcesses(other), SimpleNamespace(training=True), False, True
+    tr.beta, tr.loss_types, tr.loss_weights, tr.label_smoothing, tr.ld_alpha, tr.use_weighting = 0.1, ["sigmoid"], [1.0], 0.0, None, False
+    tr.f_divergence_type, tr.f_alpha_divergence_coef, tr.args = "reverse_kl", 1.0, SimpleNamespace(discopop_tau=0.05)
+    tr._metrics, tr._total_train_tokens = {"train": defaultdict(list), "eval": defaultdict(list)}, 2**33 + 1
+    tr._compute_loss(lambda **kw: SimpleNamespace(logits=leaf, aux_loss=None),
+                     dict(input_ids=ids, attention_mask=torch.ones_like(ids), completion_mask=mask, ref_chosen_logps=ref_c,
+                          ref_rejected_logps=ref_r), False)
+    got = {k: v[-1] for k, v in tr._metrics["train"].items()}
+    _, parts = amd.dpo_compute_loss(leaf, ids, mask, ref_c, ref_r, beta=0.1)
+    assert not any(v.requires_grad for v in parts.values())
+    both = {k: torch.cat([v.reshape(-1), other(v).reshape(-1)]).double().cpu() for k, v in parts.items()}
+    total = {k: float(v.sum()) for k, v in both.items()}
+    mean = {k: float(v.mean()) for k, v in both.items()}
+    c, r = both["chosen_rewards"], both["rejected_rewards"]
+    want = {
+        "entropy": total["entropy_sum"] / total["n_tokens"], "num_tokens": 2**33 + 1 + 2 * ids.numel() + 5,
+        "logits/chosen": total["logits_chosen_sum"] / total["n_chosen_tokens"],
+        "logits/rejected": total["logits_rejected_sum"] / total["n_rejected_tokens"],
+        "mean_token_accuracy": total["correct_tokens"] / total["n_chosen_tokens"], "rewards/chosen": mean["chosen_rewards"],
+        "rewards/rejected": mean["rejected_rewards"], "rewards/accuracies": float((c > r).double().mean()),
+        "rewards/margins": float((c - r).mean()), "logps/chosen": mean["chosen_logps"], "logps/rejected": mean["rejected_logps"],
+    }
+    assert got.keys() == want.keys() and got["num_tokens"] == want["num_tokens"]
+    for k, v in want.items():
+        assert abs(got[k] - v) <= 1e-6 * max(1.0, abs(v)), k
