@@ -486,8 +486,9 @@ def test_rows_that_are_not_whole_vectors(amd, dtype):
 @pytest.mark.parametrize("vocab", [8, 56, 63, 64, 65, 72, 127, 1032, 4088, 4096 + 8, 8192 + 56, 12289])
 def test_rows_walked_from_their_first_line(amd, dtype, vocab):
     """Rows that begin inside a 128-byte line (whole vectors or not, and rows with no line of their own): targets before
-    the first line, at its edge and at the row's end, forward and backward with both upstream gradients against float64.
-    A bf16 gradient is rounded once, at most 2^-8 of an entry; the fp32 chain holds 1e-5."""
+    the first line, at its edge and at the row's end, forward and backward with both upstream gradients against float64,
+    every entry: the fp32 chain holds 1e-5 of the terms that an entry is the sum of, and a bf16 gradient is rounded once
+    (2^-8 of an entry).  The buffer that the gradient is likely to get holds NaN beforehand."""
     g = torch.Generator().manual_seed(vocab)
     n, L, T = 2, 5, 0.9
     logits = (2.0 * torch.randn(n, L, vocab, generator=g)).to(dtype)
@@ -505,10 +506,18 @@ def test_rows_walked_from_their_first_line(amd, dtype, vocab):
     lp, ent = amd.trainer.utils.logps_and_entropies(leaf, idx.to(DEV), T)
     torch.testing.assert_close(lp.detach().cpu().double(), wlp.detach(), rtol=0, atol=1e-5)
     torch.testing.assert_close(ent.detach().cpu().double(), went.detach(), rtol=0, atol=1e-5)
+    p, one = lsm.detach().exp(), torch.zeros(n, L, vocab, dtype=torch.float64).scatter_(-1, idx[..., None], 1.0)
     for with_entropy in (False, True):
         loss = (wlp * glp).sum() + ((went * gent).sum() if with_entropy else 0.0)
         (w,) = torch.autograd.grad(loss, want, retain_graph=True)
+        poison = torch.full_like(leaf, float("nan"))
+        del poison
         loss = (lp * glp.to(DEV)).sum() + ((ent * gent.to(DEV)).sum() if with_entropy else 0.0)
         (got,) = torch.autograd.grad(loss, leaf, retain_graph=True)
+        terms = glp.abs().double()[..., None] * (p + one)
+        if with_entropy:
+            terms = terms + gent.abs().double()[..., None] * p * (lsm.detach().abs() + went.detach()[..., None])
+        bound = 1e-5 * terms / T + (0.0 if dtype == torch.float32 else 2.0**-8) * w.abs()
+        assert bool(((got.cpu().double() - w).abs() <= bound).all())
         assert _rel_l2(got, w) < (1e-5 if dtype == torch.float32 else 2.0**-8)
     amd.check_device_errors()
