@@ -19,10 +19,13 @@ namespace trlk {
 namespace {
 
 constexpr int kFThreads = 1024;
-// Rows of up to kNarrowVec vectors per lane of a 256-lane workgroup (73728 16-bit logits) take one: three or more of them
-// fit a CU, and one row's loads run beside another's reduction and stores.  One 1024-lane workgroup fills the CU from 8
-// vectors (76 registers) on.  8144 rows, 53 % of them read, bf16: V = 20480 119 -> 80 us, 32000 178 -> 155 us, 50257 312 ->
-// 280 us, 65536 360 -> 340 us; 512 lanes lie between, 128 lanes are slower from 40960 on.
+// Rows of up to kNarrowVec vectors per lane of a 256-lane workgroup (73728 16-bit logits) take one.  By their registers
+// eight of them fit a CU with 4 vectors per lane, seven with 8, five with 12, four with 16 to 24 (three with 24 where rows are
+// not whole vectors), three with 28 and 32, two with 36, and one row's loads run beside another's reduction and stores; one
+// 1024-lane workgroup fills the CU from 8 vectors (76 registers) on.  8144 rows, 53 % of them read, bf16, against 1024 lanes
+// and vectors numbered from the row's own start (see `skew`): V = 20480 123 -> 84 us, 32000 178 -> 154, 50257 315 -> 262,
+// 65536 364 -> 341, 73728 412 -> 383.  Of that the lanes, in the widest build: 69632 388 -> 364, 73728 407 -> 383, fp32 of
+// 36864 374 -> 371.  512 lanes lie between, 128 lanes are slower from 40960 on.
 constexpr int kNarrowThreads = 256, kNarrowVec = 36;
 constexpr int kSkew = 7;  // most vectors by which a row's vectors are shifted to 128-byte lines (see the kernel)
 constexpr int kMaxVec = 20;  // 16-byte vectors of a row per lane in registers: rows of up to 20 * 1024 * 8 = 163840 logits
@@ -171,8 +174,9 @@ __global__ __launch_bounds__(TH) void grpo_fused_kernel(FusedArgs a) {
     // Vectors are numbered from the 128-byte line in which the gradient row begins: its first whole vector has number
     // `skew`, `nv` ends behind its last one, and a wave's stores cover whole lines.  (Numbered from the row's own start,
     // every 1 KiB store of a row that begins inside a line leaves two lines half written: 8144 rows of 50264 against
-    // 50304 bf16 logits 281 against 259 us; both 260 us from whole lines, 8192 rows of 128257 715 -> 678 us.)  Lanes below `skew` have no vector 0; they load the row's first one, for its
-    // reference exponent, and leave it out of the sums and the stores.
+    // 50304 bf16 logits 281 against 259 us with 256 lanes; both 260 us from whole lines, 8192 rows of 128257 687 -> 656 us.)
+    // Lanes below `skew` have no vector 0; they load the row's first one, for its reference exponent, and leave it out of the
+    // sums and the stores.
     OutVec* op = reinterpret_cast<OutVec*>(out + head);
     const int skew = int((reinterpret_cast<uintptr_t>(op) >> 4) & kSkew);
     op -= skew;
