@@ -223,6 +223,7 @@ def test_targets_of_another_shape(amd):
     sft = lambda **kw: torch.stack([x.double() for x in _chunked_cross_entropy_loss(hidden, weight, 64, **kw)])  # noqa: E731
     assert torch.equal(sft(shift_labels=ids), sft(shift_labels=ids.reshape(-1)))
     assert torch.equal(sft(shift_labels=ids.view(3, 4)), sft(shift_labels=ids))
+    assert torch.equal(sft(labels=torch.cat([ids[:1, :1], ids[:, 1:].reshape(1, 10)], 1)), sft(labels=ids))
     for short in (hidden[:, :5], hidden[:1]):
         with pytest.raises(ValueError, match="do not match"):
             amd.FusedLinearDPOLoss()(weight, hidden, ids, None, short)
