@@ -868,3 +868,24 @@ def test_row_selection_and_mean_logits_can_be_traced(amd):
         (ops.mean_logits, (hidden.float(), hidden[1].float())), (ops.grpo_log_values, (torch.rand(16, device=DEV),)),
     ):
         torch.library.opcheck(op.default, args, test_utils=checks)
+
+
+@pytest.mark.parametrize("stash", [True, False])
+@pytest.mark.parametrize("n,h,v", [(1, 64, 256), (64, 128, 257), (65, 64, 384), (128, 192, 385), (129, 64, 100), (193, 128, 513),
+                                   (255, 64, 640), (257, 64, 255), (320, 128, 129), (450, 320, 1000)])
+def test_partly_filled_tiles(amd, monkeypatch, n, h, v, stash):
+    """Token and vocabulary counts around the 64-column and 128-row pieces of a tile that one wave owns: waves whose tokens
+    lie beyond the last one do no matrix work, the others' results must not notice."""
+    if not stash:
+        monkeypatch.setenv("TRL_AMD_HEAD_STASH_GIB", "0")
+    g = torch.Generator().manual_seed(n + v)
+    hidden = torch.randn(n, h, generator=g).bfloat16()
+    weight = (torch.randn(v, h, generator=g) * (2.0 / h**0.5)).bfloat16()
+    labels = torch.randint(0, v, (n,), generator=g)
+    gout = torch.randn(n, generator=g)
+    lp, ent, dh, dw = _run_device(amd, hidden, weight, labels, 0.9, 256, None, 1.0, gout)
+    rlp, rent, rdh, rdw = _fp32_reference(hidden, weight, labels, 0.9, None, 1.0, gout)
+    # fp32 sums of h products and v exponentials: a few 1e-6 of values of up to about 20
+    torch.testing.assert_close(lp, rlp, atol=5e-5, rtol=0)
+    torch.testing.assert_close(ent, rent, atol=5e-5, rtol=0)
+    _check_beyond_output_rounding(dh, dw, rdh, rdw, torch.bfloat16)

@@ -1,16 +1,16 @@
 // K5 / K6: lm_head fused with the log-prob / entropy reduction (forward) and its backward.
 //
-// All contractions run on the matrix cores (v_mfma_f32_32x32x16_{bf16,f16}, fp32 accumulate)
+// All contractions run on the matrix cores (v_mfma_f32_16x16x32_{bf16,f16}, fp32 accumulate)
 // through ONE "NT" tile loop: C[256 x 256] += A[256 x K] * B[256 x K]^T with both operands
 // row-major and K contiguous, which is the layout the MFMA A/B fragments want (a lane holds 8
 // consecutive k of one row), so fragments come straight out of LDS with 16-byte reads and nothing
-// is ever transposed on the fly.  512 threads = 8 waves as 2 (M) x 4 (N); a wave owns 128 x 64 of
-// the tile = 4 x 2 MFMA blocks = 128 accumulator registers per lane.  Tiles go from memory
-// straight into a ring of LDS stages (global_load_lds_dwordx4) when K is a multiple of the k step,
+// is ever transposed on the fly.  512 threads = 8 waves, 2 along M x 4 along N; a wave owns 128 x 64 of
+// the tile = 8 x 4 MFMA blocks = 128 accumulator registers per lane.  Tiles go from memory
+// straight into two LDS stages (global_load_lds_dwordx4) when K is a multiple of the k step,
 // through registers otherwise.
 //
 // Forward (K5): the tile is computed TRANSPOSED -- M = vocabulary rows of W, N = tokens -- so that
-// a lane of the accumulator layout holds 16 vocabulary entries of ONE token per block.  The online
+// a lane of the accumulator layout holds 4 vocabulary entries of ONE token per block.  The online
 // log-sum-exp state of a token therefore lives in the lane's own registers and the per-tile
 // epilogue needs no cross-lane traffic; a workgroup keeps 256 tokens and walks over its share of
 // the vocabulary tiles, the logits exist only as accumulators.
@@ -18,10 +18,11 @@
 // Backward (K6), per vocabulary chunk: (1) dz = dL/dlogits as scaled fp16 [chunk, tokens] (vocabulary-major, each
 // token's column in that token's own power-of-two scale) -- from a recompute of the chunk's logits (same tile loop),
 // or, when the forward was asked to stash its softmax numerators, from one elementwise sweep over that stash;
-// (2) dHidden += dz * W_chunk: the tile loop with dz as a K-MAJOR left operand (its k rows go to LDS as they lie in
+// (2) dHidden += dz * W_chunk: the tile loop with dz as a K-MAJOR operand (its k rows go to LDS as they lie in
 // memory and the MFMA fragments come out through the LDS transpose loads, ds_read_b64_tr_b16) against W_chunk^T;
 // (3) dW_chunk = dz^T * hidden as an NT product against hidden^T, whose columns carry the inverse of the tokens'
-// scales; all on fp16 operands (bf16 inputs are converted while they are transposed).  The contraction of (2)/(3)
+// scales; all on fp16 operands (bf16 inputs are converted while they are transposed).  Both are computed transposed too
+// (M = columns of the output), so that a lane of the accumulator layout holds 4 consecutive columns of one output row.  The contraction of (2)/(3)
 // is over a different axis than the recompute, and with H in the thousands the output tile of a fused kernel cannot
 // stay in registers, so dz goes through a chunk-sized workspace (never the whole [N, V] matrix).
 #include "common.hpp"
@@ -31,62 +32,60 @@
 namespace trlk {
 namespace {
 
-// Tile configuration (overridable with -D for experiments).
-#ifndef TRLK_HEAD_BM
-#define TRLK_HEAD_BM 256
-#endif
-#ifndef TRLK_HEAD_BN
-#define TRLK_HEAD_BN 256
-#endif
-#ifndef TRLK_HEAD_BK
-#define TRLK_HEAD_BK 64
-#endif
-#ifndef TRLK_HEAD_WGM
-#define TRLK_HEAD_WGM 2
-#endif
-#ifndef TRLK_HEAD_WGN
-#define TRLK_HEAD_WGN 4
-#endif
-constexpr int BM = TRLK_HEAD_BM, BN = TRLK_HEAD_BN, BK = TRLK_HEAD_BK;
-constexpr int WGM = TRLK_HEAD_WGM, WGN = TRLK_HEAD_WGN;  // waves along M and N
+constexpr int BM = 256, BN = 256, BK = 64;  // a workgroup's tile, the k step
+constexpr int WGM = 2, WGN = 4;               // waves along M and N
 constexpr int kHeadThreads = WGM * WGN * 64;
-#ifndef TRLK_HEAD_WAVES_PER_EU
-#define TRLK_HEAD_WAVES_PER_EU 2
-#endif
-#define TRLK_HEAD_KERNEL __global__ __launch_bounds__(kHeadThreads) __attribute__((amdgpu_waves_per_eu(TRLK_HEAD_WAVES_PER_EU, TRLK_HEAD_WAVES_PER_EU)))
-constexpr int kLdsRow = BK + 8;  // elements per LDS row: 16 bytes of padding keep 16-byte reads conflict-free
+#define TRLK_HEAD_KERNEL __global__ __launch_bounds__(kHeadThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 constexpr int WM = BM / WGM, WN = BN / WGN;  // per-wave tile
-constexpr int MB = WM / 32, NB = WN / 32;
+constexpr int MI = WM / 16, NI = WN / 16;    // MFMA blocks of it
+constexpr int kLdsRow = BK + 8;  // register-staged loop: elements per LDS row (16 bytes of padding keep 16-byte reads conflict-free)
 constexpr int kCpr = BK / 8;                        // 16-byte chunks per tile row
 constexpr int kRowStep = kHeadThreads / kCpr;       // rows staged per pass of the workgroup
 constexpr int kLoadsA = BM / kRowStep, kLoadsB = BN / kRowStep;
 constexpr int kTileABytes = BM * kLdsRow * 2, kTileBBytes = BN * kLdsRow * 2;
 constexpr int kStageBytes = kTileABytes + kTileBBytes;
-constexpr int kDirectLdsBytesDecl = 2 * (BM + BN) * 64 * 2;  // direct-to-LDS tile ring: 4 x 32-wide or 2 x 64-wide stages
+constexpr int kRowBytes = BK * 2;                    // direct-to-LDS loop: a dense LDS row
+constexpr int kDenseA = BM * kRowBytes, kDenseStage = (BM + BN) * kRowBytes;
 constexpr int kDzLdsRow = BN * 2 + 16;     // bytes per vocabulary row of the dz tile staged in LDS by the backward
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-constexpr int kHeadLdsBytes = cmax(cmax(2 * kStageBytes, kDirectLdsBytesDecl), BM * kDzLdsRow);
-static_assert(BM * kDzLdsRow <= kHeadLdsBytes, "dz staging tile");
-static_assert(2 * WGM * BN * 4 * 4 <= kHeadLdsBytes && BN <= kHeadThreads, "merge scratch");
-static_assert(BM % kRowStep == 0 && BN % kRowStep == 0 && WM % 32 == 0 && WN % 32 == 0 && BK % 16 == 0, "tile shape");
+constexpr int kHeadLdsBytes = cmax(cmax(2 * kStageBytes, 2 * kDenseStage), BM * kDzLdsRow);
+static_assert(4 * WGM * BN * 4 * 4 <= kHeadLdsBytes && BN <= kHeadThreads, "merge scratch");
+static_assert(BM % kRowStep == 0 && BN % kRowStep == 0, "tile shape");
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// The 16x16x32 shape reads and writes half as many accumulators per multiply-add as 32x32x16 does.  The part is limited by
+// power under matrix load, so that shows as speed: a bare loop of MFMAs on random bf16 operands runs at 2020-2060 TFLOP/s
+// (2.05-2.12 GHz) against 1830-1880 TFLOP/s (1.87-1.90 GHz), on zeros both at 2450-2490 TFLOP/s (2.4 GHz).
 template <int DT>
-__device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
+__device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
     if constexpr (DT == TRLK_BF16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
                                                        0, 0, 0);
     else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
                                                       0, 0);
 }
 
-// One operand of the NT product: `rows` x K, row-major with leading dimension ld (elements).  The left operand may
-// instead be given "k-major" (AKM below): K x `rows`, row-major with leading dimension ld -- the transpose of what the
+// The same value, but nothing computed from it is kept across loop iterations: what the compiler hoists out of the
+// forward's tile loop it spills, and a reload waits for every tile transfer in flight.
+__device__ __forceinline__ int fresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// A value that is the same in every lane, in a scalar register.
+__device__ __forceinline__ float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+
+// Where a wave sits in the tile.  A SIMD runs waves w and w + 4: they differ in their columns (N) by half the tile, so
+// that a tile of at most 128 columns leaves every SIMD one wave with work, not two of them both.
+__device__ __forceinline__ int wave_m(int wave) { return (wave >> 1) & 1; }
+__device__ __forceinline__ int wave_n(int wave) { return (wave & 1) | ((wave >> 2) << 1); }
+
+// One operand of the NT product: `rows` x K, row-major with leading dimension ld (elements).  The right operand may
+// instead be given "k-major" (BKM below): K x `rows`, row-major with leading dimension ld -- the transpose of what the
 // product wants, read through the LDS transpose loads; its columns must be readable (and zero) up to the next
 // multiple of the tile size.
 struct Operand {
@@ -97,94 +96,63 @@ struct Operand {
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-// k-step width of the direct-to-LDS loop per kernel.  All three use 64-wide steps (two 64 KiB stages, half as
-// many barriers, whole 128-byte lines per row and step); the 32-wide, four-stage ring was only ahead for the
-// short contraction over the hidden size while the forward's workgroups still ran out of step with each other.
-#ifndef TRLK_HEAD_BK_FWD
-#define TRLK_HEAD_BK_FWD 64
-#endif
-#ifndef TRLK_HEAD_BK_DZ
-#define TRLK_HEAD_BK_DZ 64
-#endif
-#ifndef TRLK_HEAD_BK_GEMM
-#define TRLK_HEAD_BK_GEMM 64
-#endif
-
 // Direct-to-LDS variant of the tile loop (K % BK == 0): `global_load_lds_dwordx4` moves 16 bytes per
-// lane from memory straight into LDS, 1 KiB contiguous per wave instruction = 1024 / (2 BK) tile
-// rows, with no register staging and no ds_write.  Rows are dense (no padding is possible inside a
-// wave's 1 KiB), so bank conflicts are avoided by an XOR swizzle of the 16-byte chunk index: the
-// chunk at physical position pc of row r holds logical chunk pc ^ swz(r), with
-//   BK = 64 (128-byte rows): swz(r) = (r & 7) ^ ((r >> 3) & 1),   BK = 32 (64-byte rows): swz(r) = (r >> 2) & 3,
+// lane from memory straight into LDS, 1 KiB contiguous per wave instruction = 8 tile rows of 64 k, with no register
+// staging and no ds_write.  Rows are dense (no padding is possible inside a wave's 1 KiB), so bank conflicts are avoided
+// by an XOR swizzle of the 16-byte chunk index: the chunk at physical position pc of row r holds logical chunk
+//   pc ^ swz(r),  swz(r) = (r & 7) ^ ((r >> 3) & 1),
 // which makes the 16 rows that one ds_read_b128 phase touches cover all 64 banks once.  The lane
 // fetches that logical chunk from memory (a permutation inside one row, still coalesced) and the
 // fragment reads apply the same XOR.
 //
-// The loop keeps kStages tiles in LDS (4 x 32 KiB for BK = 32, 2 x 64 KiB for BK = 64).  A stage is
-// refilled as soon as the barrier that ends its last use has passed, kStages - 1 steps before it
-// is needed again: the transfer of one stage through the CU's vector memory path (64 bytes per
-// clock) takes longer than half a k step of MFMAs, so with only two stages every barrier waits
-// for data in flight.
-template <int BKT>
-struct DirectCfg {
-    static_assert(BKT == 32 || BKT == 64, "direct-to-LDS layouts exist for 32- and 64-wide k steps");
-    static constexpr int kStages = BKT == 32 ? 4 : 2;
-    static constexpr int kRowBytes = BKT * 2;                // dense LDS row
-    static constexpr int kRowsPerBlk = 1024 / kRowBytes;     // rows one wave instruction fills
-    static constexpr int kChunks = kRowBytes / 16;
-    static constexpr int kDenseA = BM * kRowBytes, kDenseStage = (BM + BN) * kRowBytes;
-    static constexpr int kLdsBytes = kStages * kDenseStage;
-    static __device__ __forceinline__ int swizzle(int r) {
-        return BKT == 64 ? ((r & 7) ^ ((r >> 3) & 1)) : ((r >> 2) & 3);
-    }
-};
-static_assert(DirectCfg<32>::kLdsBytes <= kHeadLdsBytes && DirectCfg<64>::kLdsBytes <= kHeadLdsBytes, "LDS budget");
+// The loop keeps two 64 KiB stages in LDS; a stage is refilled as soon as the barrier that ends its last use has passed,
+// one step before it is needed again.
+__device__ __forceinline__ int tile_swizzle(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 // Loader side of the direct-to-LDS loop: per-lane source offsets of the wave's tile blocks and the
 // transfer of one stage.
-// AKM: the left operand is k-major.  Its stage is then 64 k rows of 512 bytes (256 columns); one transfer fills two
-// k rows; the 16-byte unit at physical position pu of k row r holds logical unit pu ^ ((r & 3) << 1), which spreads
-// the four k rows that one group of 16 lanes reads with a transpose load over all banks.
-template <int BKT, bool AKM = false>
+// BKM: the right operand is k-major.  Its stage is then 64 k rows of 512 bytes (256 columns); one transfer fills two
+// k rows; the 16-byte unit at physical position pu of k row r holds logical unit pu ^ ((r & 3) << 1) ^ (r & 8), which
+// spreads the eight k rows that two neighbouring groups of 16 lanes read with a transpose load over all banks.
+template <bool BKM = false>
 struct DirectLoader {
-    typedef DirectCfg<BKT> C;
-    static_assert(!AKM || (BKT == 64 && BM == 256), "k-major left operands: 64-wide steps of 256 columns");
-    static constexpr int kWaves = kHeadThreads / 64;
-    static constexpr int kBlkA = BM / C::kRowsPerBlk / kWaves, kBlkB = BN / C::kRowsPerBlk / kWaves;  // per wave and stage
+    static constexpr int kWaves = kHeadThreads / 64, kRowsPerBlk = 1024 / kRowBytes;
+    static constexpr int kBlkA = BM / kRowsPerBlk / kWaves, kBlkB = BN / kRowsPerBlk / kWaves;  // per wave and stage
     static constexpr int kStageLoads = kBlkA + kBlkB;
-    static_assert(BM % (C::kRowsPerBlk * kWaves) == 0 && BN % (C::kRowsPerBlk * kWaves) == 0, "blocks per wave");
+    static_assert(BM % (kRowsPerBlk * kWaves) == 0 && BN % (kRowsPerBlk * kWaves) == 0 && BN == 256, "blocks per wave");
     const char *abase, *bbase;
     char* smem;
     int wave;
-    int64_t akstep;  // bytes between two k of the left operand
+    int64_t bkstep;  // bytes between two k of the right operand
     uint32_t ao[kBlkA], bo[kBlkB];
 
     __device__ __forceinline__ DirectLoader(const Operand A, int m0, const Operand B, int n0, char* lds) : smem(lds) {
-        const int lane = threadIdx.x & 63;
+        const int lane = fresh(threadIdx.x & 63);
         wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: LDS targets stay scalar
-        const int rr = lane / C::kChunks, pc = lane % C::kChunks;  // row inside a block, chunk position
-        abase = reinterpret_cast<const char*>(AKM ? A.p + m0 : A.p + int64_t(m0) * A.ld);
-        bbase = reinterpret_cast<const char*>(B.p + int64_t(n0) * B.ld);
-        akstep = AKM ? A.ld * 2 : 2;
+        const int rr = lane / kCpr, pc = lane % kCpr;  // row inside a block, chunk position
+        abase = reinterpret_cast<const char*>(A.p + int64_t(m0) * A.ld);
+        bbase = reinterpret_cast<const char*>(BKM ? B.p + n0 : B.p + int64_t(n0) * B.ld);
+        bkstep = BKM ? B.ld * 2 : 2;
+        const uint32_t lda = uint32_t(A.ld * 2), ldb = uint32_t(B.ld * 2);  // (a tile spans less than 4 GiB)
 #pragma unroll
         for (int j = 0; j < kBlkA; ++j) {
-            if constexpr (AKM) {
-                const int krow = (wave + kWaves * j) * 2 + (lane >> 5);
-                const int lu = (lane & 31) ^ ((krow & 3) << 1);  // the logical 16-byte unit this lane fetches
-                ao[j] = uint32_t((int64_t(krow) * A.ld + lu * 8) * 2);
-                continue;
-            }
-            const int row = (wave + kWaves * j) * C::kRowsPerBlk + rr;
-            const int kc = pc ^ C::swizzle(row);  // the logical chunk this lane fetches
+            const int row = (wave + kWaves * j) * kRowsPerBlk + rr;
+            const int kc = pc ^ tile_swizzle(row);  // the logical chunk this lane fetches
             const int r = m0 + row < A.rows ? row : A.rows - 1 - m0;
-            ao[j] = uint32_t((int64_t(r) * A.ld + kc * 8) * 2);
+            ao[j] = uint32_t(r) * lda + uint32_t(kc * 16);
         }
 #pragma unroll
         for (int j = 0; j < kBlkB; ++j) {
-            const int row = (wave + kWaves * j) * C::kRowsPerBlk + rr;
-            const int kc = pc ^ C::swizzle(row);
+            if constexpr (BKM) {
+                const int krow = (wave + kWaves * j) * 2 + (lane >> 5);
+                const int lu = (lane & 31) ^ ((krow & 3) << 1) ^ (krow & 8);  // the logical 16-byte unit this lane fetches
+                bo[j] = uint32_t(krow) * ldb + uint32_t(lu * 16);
+                continue;
+            }
+            const int row = (wave + kWaves * j) * kRowsPerBlk + rr;
+            const int kc = pc ^ tile_swizzle(row);
             const int r = n0 + row < B.rows ? row : B.rows - 1 - n0;
-            bo[j] = uint32_t((int64_t(r) * B.ld + kc * 8) * 2);
+            bo[j] = uint32_t(r) * ldb + uint32_t(kc * 16);
         }
     }
     // One 1 KiB transfer: 16 bytes per lane from `src` to LDS offset `lds` + 16 * lane.  Issued as
@@ -203,229 +171,187 @@ struct DirectLoader {
     }
 #pragma clang diagnostic pop
     __device__ __forceinline__ uint32_t lds_base(int buf) const {
-        return uint32_t(reinterpret_cast<uintptr_t>(smem)) + uint32_t(buf * C::kDenseStage);
+        return uint32_t(reinterpret_cast<uintptr_t>(smem)) + uint32_t(buf * kDenseStage);
     }
     // transfer j of a stage (A blocks first, then B blocks)
     __device__ __forceinline__ void issue_one(int buf, int k0, int j) const {
         if (j < kBlkA)
-            transfer(abase + int64_t(k0) * akstep, ao[j], lds_base(buf) + (wave + kWaves * j) * 1024);
+            transfer(abase + int64_t(k0) * 2, ao[j], lds_base(buf) + (wave + kWaves * j) * 1024);
         else
-            transfer(bbase + int64_t(k0) * 2, bo[j - kBlkA], lds_base(buf) + C::kDenseA + (wave + kWaves * (j - kBlkA)) * 1024);
+            transfer(bbase + int64_t(k0) * bkstep, bo[j - kBlkA], lds_base(buf) + kDenseA + (wave + kWaves * (j - kBlkA)) * 1024);
     }
     __device__ __forceinline__ void issue(int buf, int k0) const {
 #pragma unroll
         for (int j = 0; j < kStageLoads; ++j) issue_one(buf, k0, j);
     }
-    // the first kStages tiles of a product; every stage must be free (all reads of the LDS done)
+    // the first two stages of a product; both must be free (all reads of the LDS done)
     __device__ __forceinline__ void prologue(int K) const {
-        const int nk = K / BKT;
-#pragma unroll
-        for (int st = 0; st < C::kStages; ++st)
-            if (st < nk) issue(st, st * BKT);
+        issue(0, 0);
+        if (K > BK) issue(1, BK);
+    }
+    __device__ __forceinline__ void first_stage_landed(int nk) const {
+        if (nk >= 2)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStageLoads) : "memory");
+        else
+            __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
     }
 };
 
+// What a wave whose rows or columns all lie beyond the operands does in place of the tile loop: it moves its share of the
+// tiles (exactly the transfers, waits and barriers of the loop) and spends nothing on matrix work.
+template <bool BKM>
+__device__ __forceinline__ void move_tiles_only(const DirectLoader<BKM>& loader, int K, bool prefetched) {
+    const int nk = K / BK;
+    if (!prefetched) loader.prologue(K);
+    loader.first_stage_landed(nk);
+#pragma unroll 1
+    for (int kt = 0; kt < nk; ++kt) {
+        __builtin_amdgcn_s_waitcnt(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (kt + 2 < nk) loader.issue(kt & 1, (kt + 2) * BK);
+    }
+}
+
 // `prefetched`: the caller has already run DirectLoader::prologue for this tile (and nothing has
 // touched the LDS since).
-// IDLE: waves whose rows or columns all lie beyond the operands skip the matrix work (the products of the backward; in the
-// forward the second path costs registers that it does not have).
-template <int DT, int BKT, bool AKM = false, bool IDLE = false>
+template <int DT, bool BKM = false>
 __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, const Operand B, int n0, int K,
-                                                    f32x16 (&acc)[MB][NB], char* smem, bool prefetched) {
-    typedef DirectCfg<BKT> C;
-    constexpr int kStages = C::kStages, kRowBytes = C::kRowBytes;
-    constexpr int kDenseA = C::kDenseA, kDenseStage = C::kDenseStage;
-    const DirectLoader<BKT, AKM> loader(A, m0, B, n0, smem);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = loader.wave;
-    const int wm = wave / WGN, wn = wave % WGN;
+                                                    f32x4 (&acc)[MI][NI], char* smem, bool prefetched) {
+    const DirectLoader<BKM> loader(A, m0, B, n0, smem);
+    constexpr int kStageLoads = DirectLoader<BKM>::kStageLoads;
+    const int lane = threadIdx.x & 63, wave = loader.wave;
+    const int wm = wave_m(wave), wn = wave_n(wave);
 
-    // --- fragment side (tile rows of a wave start at multiples of 32, so the swizzle depends on the lane only)
-    const int swz = C::swizzle(lane & 31);
-    const int hl = lane >> 5;
-    const int fa_row = (wm * WM + (lane & 31)) * kRowBytes, fb_row = (wn * WN + (lane & 31)) * kRowBytes;
-    constexpr int KS = BKT / 16;
-    int koff[KS];
+    // --- fragment side (blocks start at multiples of 16 rows, so the swizzle depends on the lane only).  A fragment is
+    // 16 rows x 32 k: lane l holds the 8 k from 8 (l / 16) on of row l % 16.
+    const int g = lane >> 4, l15 = lane & 15;
+    const int koff[2] = {(g ^ tile_swizzle(l15)) * 16, ((4 + g) ^ tile_swizzle(l15)) * 16};
+    const int fa_row = (wm * WM + l15) * kRowBytes, fb_row = (wn * WN + l15) * kRowBytes;
+    // k-major right operand: a fragment is two transpose loads of 8 bytes.  The lanes work in groups of 16: lane t of a
+    // group points at the 8 bytes that hold columns 4 (t % 4) .. + 3 of k row t / 4 (of the group's 4 k rows), and
+    // receives column t of those 4 k rows.  Group g takes the block's 16 columns at k 8 g .. + 3 (second load: + 4 .. + 7).
+    int fb_km[NI];
+    if constexpr (BKM) {
+        const int f = ((l15 >> 2) << 1) ^ ((g & 1) << 3);  // the unit swizzle of this lane's k rows
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) koff[ks] = ((ks * 2 + hl) ^ swz) * 16;
-    // k-major left operand: a fragment (32 rows x 16 k, 8 k per lane) is two transpose loads of 8 bytes.  The lanes
-    // work in groups of 16: lane t of a group points at the 8 bytes that hold columns 4 (t % 4) .. + 3 of k row t / 4
-    // (of the group's 4 k rows), and receives column t of those 4 k rows.  Groups 0, 1 take columns 0-15, 16-31 of the
-    // block at k 0-3 (second load: 4-7), groups 2, 3 the same columns at k 8-11 (12-15).
-    int fa_km[MB];
-    if constexpr (AKM) {
-        const int t = lane & 15, g = lane >> 4;
-        const int f = (t >> 2) << 1;  // the unit swizzle of this lane's k row ((k row & 3) << 1)
-        const int lu0 = (wm * WM + 16 * (g & 1)) / 8 + ((t & 3) >> 1);
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-            fa_km[mb] = (8 * (g >> 1) + (t >> 2)) * 512 + ((lu0 + 4 * mb) ^ f) * 16 + (t & 1) * 8;
+        for (int j = 0; j < NI; ++j)
+            fb_km[j] = (8 * g + (l15 >> 2)) * (BN * 2) + (((wn * WN + j * 16) / 8 + ((l15 & 3) >> 1)) ^ f) * 16 + (l15 & 1) * 8;
     }
-    auto read_a = [&](const char* sa, int mb, int ks) -> u32x4 {
-        if constexpr (AKM) {
-            const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(sa)) + uint32_t(fa_km[mb] + ks * 16 * 512);
+    auto read_a = [&](const char* sa, int i, int ks) -> u32x4 {
+        return *reinterpret_cast<const u32x4*>(sa + fa_row + i * 16 * kRowBytes + koff[ks]);
+    };
+    auto read_b = [&](const char* sb, int j, int ks) -> u32x4 {
+        if constexpr (BKM) {
+            const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(sb)) + uint32_t(fb_km[j] + ks * 32 * (BN * 2));
             const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at + 4 * 512));
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at + 4 * (BN * 2)));
             typedef short s16x8 __attribute__((ext_vector_type(8)));
             const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
             return __builtin_bit_cast(u32x4, both);
         } else {
-            return *reinterpret_cast<const u32x4*>(sa + fa_row + mb * 32 * kRowBytes + koff[ks]);
+            return *reinterpret_cast<const u32x4*>(sb + fb_row + j * 16 * kRowBytes + koff[ks]);
         }
     };
 
+    const int nk = K / BK;
+    if (!prefetched) loader.prologue(K);
+    loader.first_stage_landed(nk);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
+        for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Software pipeline.  Fragment loads run one 16-wide k slice ahead of the MFMAs that consume them,
-    // across the barrier too: the last slice of a stage is already in registers when the workgroup
-    // synchronises, so its MFMAs cover the refill of the freed stage and the first fragment reads of
-    // the next one.  The compiler's own scheduler sinks every ds_read next to its first use (one
-    // exposed LDS latency per MFMA pair), so the issue order is pinned explicitly below.
-    constexpr int kStageLoads = DirectLoader<BKT, AKM>::kStageLoads;
-    auto load_frags = [&](int buf, int ks, u32x4(&fa)[MB], u32x4(&fb)[NB]) {
-        const char* sa = smem + buf * kDenseStage;
-        const char* sb = sa + kDenseA;
+    // Software pipeline over slices of 32 k, two per step.  A slice runs over the wave's blocks twice, first with the
+    // column blocks 0, 1, then with 2, 3.  Every fragment register is loaded again, for the next slice, right behind its
+    // last use: a row fragment in the second half, a pair of column fragments at the end of its half -- 14 to 16 MFMAs
+    // before the next use, with one set of fragment registers (48; a second set would not fit beside the epilogues).
+    // The compiler's own scheduler sinks every ds_read next to its first use (one exposed LDS latency per MFMA pair), so
+    // the issue order is pinned explicitly: MFMA, then at most two fragment reads and one tile transfer.
+    //
+    // The barrier that frees a stage sits inside the step's second slice, kBarAt row blocks into its first half: by then
+    // the last fragments of the stage, read at the end of the first slice, have arrived.  The stage's refill follows
+    // it, one transfer every other MFMA, and has until the same place of the next step to land.
+    //
+    // Bound by power (clock 1.5-1.7 GHz) and the arrival of the tiles.  Whole steps, forward and both products, against
+    // the loop on 32x32x16 MFMAs with two sets of fragments: 9664 tokens, H = 3584, V = 151936 28.3 -> 26.8 ms; 1396 tokens,
+    // H = 2048, V = 50257 1128 -> 1054 us; forward alone of 459 tokens, H = 3584, V = 151936 532 -> 520 us.
+    constexpr int kBarAt = 4;
+    static_assert(NI == 4 && 2 * kStageLoads <= 2 * (MI - kBarAt) + 2 * MI, "the refill fits behind the barrier");
+    u32x4 a[MI], b[NI];
+    {
+        const char* sa = smem;
+        const char* sb = smem + kDenseA;
+        b[0] = read_b(sb, 0, 0);
+        b[1] = read_b(sb, 1, 0);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) fa[mb] = read_a(sa, mb, ks);
+        for (int i = 0; i < MI; ++i) a[i] = read_a(sa, i, 0);
+        b[2] = read_b(sb, 2, 0);
+        b[3] = read_b(sb, 3, 0);
+    }
+    auto step = [&](int kt, auto refill_tag, auto next_tag) {
+        constexpr bool REFILL = decltype(refill_tag)::value, NEXT = decltype(next_tag)::value;
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-            fb[nb] = *reinterpret_cast<const u32x4*>(sb + fb_row + nb * 32 * kRowBytes + koff[ks]);
+        for (int ks = 0; ks < 2; ++ks) {
+            // the next slice: this stage's second, or the next stage's first
+            const char* na = smem + ((kt + ks) & 1) * kDenseStage;
+            const char* nb = na + kDenseA;
+            const bool load = ks == 0 || NEXT;
+            int issued = 0, slot = 0;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    if (ks == 1 && half == 0 && i == kBarAt) {
+                        // Every fragment read of this stage has returned and the next stage has landed.  A bare s_barrier:
+                        // __syncthreads() carries release / acquire fences; nothing may move across it.
+                        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                        __builtin_amdgcn_sched_barrier(0);
+                        __builtin_amdgcn_s_barrier();
+                        __builtin_amdgcn_sched_barrier(0);
+                        asm volatile("" ::: "memory");
+                    }
+#pragma unroll
+                    for (int jj = 0; jj < 2; ++jj) {
+                        const int j = half * 2 + jj;
+                        acc[i][j] = mfma<DT>(a[i], b[j], acc[i][j]);
+                        __builtin_amdgcn_sched_barrier(0);  // (a load moved above the MFMA would need registers of its own)
+                        if (load) {
+                            if (half == 1 && jj == 1) a[i] = read_a(na, i, ks ^ 1);
+                            if (i == MI - 1) b[j] = read_b(nb, j, ks ^ 1);
+                        }
+                        if (REFILL && ks == 1 && (half == 1 || i >= kBarAt)) {
+                            if ((slot & 1) && issued < kStageLoads) {
+                                loader.issue_one(kt & 1, (kt + 2) * BK, issued);
+                                ++issued;
+                            }
+                            ++slot;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
     };
-    u32x4 fa[2][MB], fb[2][NB];
-    static_assert(KS % 2 == 0 && MB * NB > MB + NB && (kStages - 2) * kStageLoads < 64, "pipeline shape");
     constexpr std::true_type T{};
     constexpr std::false_type F{};
-    const int nk = K / BKT;
-    if (!prefetched) loader.prologue(K);
-    if (nk >= kStages)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 1) * kStageLoads) : "memory");
-    else
-        __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    constexpr int kLoadsPost = (kStageLoads + 1) / 2, kLoadsPre = kStageLoads - kLoadsPost;
-    // A wave whose rows or columns all lie beyond the operands (the last tile of either) moves its share of the tiles
-    // and nothing else.  Waves that differ in their rows only share a SIMD, so a last row tile that is at most half full
-    // takes half the matrix time.  (Exactly the transfers and barriers of the loop below.)
-    if (IDLE && (m0 + wm * WM >= A.rows || n0 + wn * WN >= B.rows)) {
-#pragma unroll 1
-        for (int kt = 0; kt < nk; ++kt) {
-            if (kt > 0 && kt - 1 + kStages < nk) {
-#pragma unroll
-                for (int j = kLoadsPost; j < kStageLoads; ++j)
-                    loader.issue_one((kt - 1) & (kStages - 1), (kt - 1 + kStages) * BKT, j);
-            }
-            __builtin_amdgcn_s_waitcnt(0);
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if (kt + kStages < nk) {
-#pragma unroll
-                for (int j = 0; j < kLoadsPost; ++j) loader.issue_one(kt & (kStages - 1), (kt + kStages) * BKT, j);
-            }
-        }
-        return;
-    }
-    load_frags(0, 0, fa[0], fb[0]);
-    // Exact issue order, pinned instruction by instruction (sched_barrier(0) between the groups):
-    // MFMA i of the slice, then at most one fragment read of the next slice and at most one tile
-    // transfer.  Fragments are read in the order the mb-major MFMA sequence needs them (fa0, fb*,
-    // fa1, ...), so every read has most of a slice between its issue and its first use.  The refill
-    // of a stage is split: the first half of its transfers goes behind the barrier that frees it, the
-    // second half into the first slice of the following step.
-    constexpr int M = MB * NB, R = MB + NB;
-    auto slice = [&](u32x4(&ca)[MB], u32x4(&cb)[NB], auto read_tag, int rbuf, int rks, u32x4(&na)[MB], u32x4(&nb_)[NB],
-                     auto nload_tag, int lbuf, int lk0, int lfirst) {
-        constexpr bool READ = decltype(read_tag)::value;
-        constexpr int NL = decltype(nload_tag)::value;
-        const char* sa = smem + rbuf * kDenseStage;
-        const char* sb = sa + kDenseA;
-        int issued = 0;
-#pragma unroll
-        for (int i = 0; i < M; ++i) {
-            const int mb = i / NB, nb = i % NB;
-            acc[mb][nb] = mfma<DT>(ca[mb], cb[nb], acc[mb][nb]);
-            if (READ && i < R) {
-                // read order: fa[0], fb[0..NB-1], fa[1..MB-1]
-                if (i == 0)
-                    na[0] = read_a(sa, 0, rks);
-                else if (i <= NB)
-                    nb_[i - 1] = *reinterpret_cast<const u32x4*>(sb + fb_row + (i - 1) * 32 * kRowBytes + koff[rks]);
-                else
-                    na[i - NB] = read_a(sa, i - NB, rks);
-            }
-            if (NL > 0 && (i + 1) * NL / M > i * NL / M) {
-                loader.issue_one(lbuf, lk0, lfirst + issued);
-                ++issued;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    typedef std::integral_constant<int, kLoadsPost> post_t;
-    typedef std::integral_constant<int, kLoadsPre> pre_t;
-    typedef std::integral_constant<int, 0> zero_t;
-    // POST / PRE: this step issues the first half of the refill of the stage it frees / the second
-    // half of the refill the previous step started.  FULL, NEXT as above.
-    auto xstep = [&](int kt, auto post_tag, auto pre_tag, auto full_tag, auto next_tag) {
-        constexpr bool POST = decltype(post_tag)::value, PRE = decltype(pre_tag)::value;
-        constexpr bool FULL = decltype(full_tag)::value, NEXT = decltype(next_tag)::value;
-        const int cur = kt & (kStages - 1), prev = (kt - 1) & (kStages - 1);
-#pragma unroll
-        for (int ks = 0; ks + 1 < KS; ++ks) {
-            if (PRE && ks == 0)
-                slice(fa[ks & 1], fb[ks & 1], T, cur, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1], pre_t{}, prev,
-                      (kt - 1 + kStages) * BKT, kLoadsPost);
-            else
-                slice(fa[ks & 1], fb[ks & 1], T, cur, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1], zero_t{}, 0, 0, 0);
-        }
-        // every fragment read of this stage has returned and the next stage has landed
-        if constexpr (FULL)
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kStages - 2) * kStageLoads) : "memory");
-        else
-            __builtin_amdgcn_s_waitcnt(0);
-        // A bare s_barrier: __syncthreads() carries release/acquire fences, for which the compiler
-        // drains every outstanding transfer (vmcnt(0)), younger stages included.  The waits above
-        // are the ones this exchange needs; nothing may move across the barrier.
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("" ::: "memory");
-        constexpr int L = (KS - 1) & 1;
-        const int nxt = (kt + 1) & (kStages - 1);
-        if constexpr (NEXT && POST)
-            slice(fa[L], fb[L], T, nxt, 0, fa[0], fb[0], post_t{}, cur, (kt + kStages) * BKT, 0);
-        else if constexpr (NEXT)
-            slice(fa[L], fb[L], T, nxt, 0, fa[0], fb[0], zero_t{}, 0, 0, 0);
-        else
-            slice(fa[L], fb[L], F, 0, 0, fa[0], fb[0], zero_t{}, 0, 0, 0);
-    };
-    static_assert(((KS - 1) & 1) == 1, "the last slice of a stage sits in fragment buffer 1, the next stage's first in 0");
     int kt = 0;
-    if (nk > kStages) {
-        xstep(kt++, T, F, T, T);
-        for (; kt + kStages < nk; ++kt) xstep(kt, T, T, T, T);
-        xstep(kt++, F, T, T, T);  // kt = nk - kStages: completes the last refill
-    } else if (nk == kStages) {
-        xstep(kt++, F, F, T, T);
-    }
-    for (; kt + 1 < nk; ++kt) xstep(kt, F, F, F, T);
-    xstep(kt, F, F, F, F);
+    for (; kt + 2 < nk; ++kt) step(kt, T, T);
+    if (kt + 1 < nk) step(kt++, F, T);
+    step(kt, F, F);
     // every LDS read of this tile completed before the last barrier: the caller may reuse the LDS right away
 }
 
-// acc[mb][nb] = sum_k A[m0 + .., k] * B[n0 + .., k].  Rows beyond the operand's end are clamped to
+// acc[i][j] = sum_k A[m0 + .., k] * B[n0 + .., k].  Rows beyond the operand's end are clamped to
 // its last row (callers ignore those outputs); k beyond K reads as zero (K % 8 == 0).
 template <int DT>
 __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, const Operand B, int n0, int K,
-                                             f32x16 (&acc)[MB][NB], char* smem) {
+                                             f32x4 (&acc)[MI][NI], char* smem) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int wm = wave_m(wave), wn = wave_n(wave);
     const int kc = tid % kCpr, r0 = tid / kCpr;  // this thread stages rows r0 + kRowStep*j, 16-byte chunk kc
 
     // uniform tile base + 32-bit per-lane byte offsets (a tile spans < 4 GiB)
@@ -445,15 +371,13 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
         bo[j] = uint32_t((int64_t(rb) * B.ld + kc * 8) * 2);
     }
     const int st_off = (r0 * kLdsRow + kc * 8) * 2;        // + j * kRowStep rows
-    const int fa_off = ((wm * WM + (lane & 31)) * kLdsRow + (lane >> 5) * 8) * 2;  // + mb*32 rows, + ks*16
-    const int fb_off = ((wn * WN + (lane & 31)) * kLdsRow + (lane >> 5) * 8) * 2;
+    const int fa_off = ((wm * WM + (lane & 15)) * kLdsRow + (lane >> 4) * 8) * 2;  // + i * 16 rows, + ks * 32
+    const int fb_off = ((wn * WN + (lane & 15)) * kLdsRow + (lane >> 4) * 8) * 2;
 
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
+        for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const u32x4 zero = {0u, 0u, 0u, 0u};
     // full k steps load unconditionally; only the last, partial step (K % BK != 0) masks its chunks
@@ -485,18 +409,16 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
         const char* sa = smem + buf * kStageBytes;
         const char* sb = sa + kTileABytes;
 #pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
-            u32x4 fa[MB], fb[NB];
+        for (int ks = 0; ks < BK / 32; ++ks) {
+            u32x4 fa[MI], fb[NI];
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-                fa[mb] = *reinterpret_cast<const u32x4*>(sa + fa_off + (mb * 32 * kLdsRow + ks * 16) * 2);
+            for (int i = 0; i < MI; ++i) fa[i] = *reinterpret_cast<const u32x4*>(sa + fa_off + (i * 16 * kLdsRow + ks * 32) * 2);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-                fb[nb] = *reinterpret_cast<const u32x4*>(sb + fb_off + (nb * 32 * kLdsRow + ks * 16) * 2);
+            for (int j = 0; j < NI; ++j) fb[j] = *reinterpret_cast<const u32x4*>(sb + fb_off + (j * 16 * kLdsRow + ks * 32) * 2);
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma<DT>(fa[mb], fb[nb], acc[mb][nb]);
+                for (int j = 0; j < NI; ++j) acc[i][j] = mfma<DT>(fa[i], fb[j], acc[i][j]);
         }
     };
 
@@ -516,26 +438,23 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
     }
 }
 
-template <int DT, int BKT, bool AKM = false, bool IDLE = false>
+template <int DT, bool BKM = false>
 __device__ __forceinline__ void gemm_tile_nt(const Operand A, int m0, const Operand B, int n0, int K,
-                                             f32x16 (&acc)[MB][NB], char* smem, bool prefetched = false) {
-    if constexpr (AKM) {  // (callers of this form pad K to whole steps)
-        static_assert(BKT == 64, "k-major left operands need the direct-to-LDS loop with 64-wide steps");
-        gemm_tile_nt_direct<DT, BKT, true, IDLE>(A, m0, B, n0, K, acc, smem, prefetched);
+                                             f32x4 (&acc)[MI][NI], char* smem, bool prefetched = false) {
+    if constexpr (BKM) {  // (callers of this form pad K to whole steps)
+        gemm_tile_nt_direct<DT, true>(A, m0, B, n0, K, acc, smem, prefetched);
     } else {
-        if ((K & (BKT - 1)) == 0)
-            gemm_tile_nt_direct<DT, BKT, false, IDLE>(A, m0, B, n0, K, acc, smem, prefetched);
+        if ((K & (BK - 1)) == 0)
+            gemm_tile_nt_direct<DT>(A, m0, B, n0, K, acc, smem, prefetched);
         else
             gemm_tile_nt_staged<DT>(A, m0, B, n0, K, acc, smem);
     }
 }
 
-// Row (M index) inside the workgroup tile of accumulator element r of block mb, for this lane.
-__device__ __forceinline__ int acc_row(int wm, int mb, int r, int lane) {
-    return wm * WM + mb * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-}
-// Column (N index) inside the workgroup tile of block nb, for this lane.
-__device__ __forceinline__ int acc_col(int wn, int nb, int lane) { return wn * WN + nb * 32 + (lane & 31); }
+// Row (M index) inside the workgroup tile of accumulator element r of block i, for this lane.
+__device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) { return wm * WM + i * 16 + (lane >> 4) * 4 + r; }
+// Column (N index) inside the workgroup tile of block j, for this lane.
+__device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * WN + j * 16 + (lane & 15); }
 
 // Workgroup id -> (tile along axis `a`, tile along axis `b`) such that the workgroups that run
 // together on one XCD (ids congruent mod 8, dispatched round-robin) form 4 x 8 patches: they share
@@ -671,97 +590,109 @@ TRLK_HEAD_KERNEL void fused_head_fwd_kernel(HeadArgs a) {
     int tb, vs;
     xcd_patch(blockIdx.x, n_tb, a.v_splits, tb, vs);
     if (tb >= n_tb || vs >= a.v_splits) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave_m(wave), wn = wave_n(wave);
     const int n0 = tb * BN;
     const int n_vt = (a.V + BM - 1) / BM;
     const int vt0 = vs * a.tiles_per_split;
     const int vt1 = vt0 + a.tiles_per_split < n_vt ? vt0 + a.tiles_per_split : n_vt;
 
-    // per-lane online state of the NB tokens this lane owns (base-2, integer reference exponent)
-    float ref[NB], rr[NB], S[NB], U[NB], zmax[NB];
-    int64_t tg[NB];
+    // per-lane online state of the NI tokens this lane owns (base-2, integer reference exponent)
+    float ref[NI], S[NI], U[NI], zmax[NI];
+    int tg[NI];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        ref[nb] = -INFINITY;
-        zmax[nb] = -INFINITY;
-        rr[nb] = 0.f;
-        S[nb] = 0.f;
-        U[nb] = 0.f;
-        const int tok = n0 + acc_col(wn, nb, lane);
-        tg[nb] = tok < a.N ? a.targets[tok] : -1;
+    for (int j = 0; j < NI; ++j) {
+        ref[j] = -INFINITY;
+        zmax[j] = -INFINITY;
+        S[j] = 0.f;
+        U[j] = 0.f;
+        const int tok = n0 + acc_col(wn, j, tid & 63);
+        const int64_t t = tok < a.N ? a.targets[tok] : -1;
+        tg[j] = t >= 0 && t < a.V ? int(t) : -1;
     }
     const Operand W{a.weight, a.ldw, a.V}, Hd{a.hidden, a.ldh, a.N};
 
     if constexpr (!STAGED)
-        if (vt0 < vt1) DirectLoader<TRLK_HEAD_BK_FWD>(W, vt0 * BM, Hd, n0, smem).prologue(a.H);
-    for (int vt = vt0; vt < vt1; ++vt) {
+        if (vt0 < vt1) DirectLoader<>(W, vt0 * BM, Hd, n0, smem).prologue(a.H);
+    const float zs = uniform(a.logit_scale * a.inv_t), zs2 = uniform(zs * kLog2e);
+    const bool idle = !STAGED && n0 + wn * WN >= a.N;  // all of this wave's tokens lie beyond the last one
+    if (idle) {
+#pragma unroll 1
+        for (int vt = vt0; vt < vt1; ++vt) {
+            move_tiles_only(DirectLoader<>(W, vt * BM, Hd, n0, smem), a.H, true);
+            if (vt + 1 < vt1) DirectLoader<>(W, (vt + 1) * BM, Hd, n0, smem).prologue(a.H);
+        }
+    }
+    for (int vt = vt0; vt < vt1 && !idle; ++vt) {
         const int m0 = vt * BM;
-        f32x16 acc[MB][NB];
+        f32x4 acc[MI][NI];
         if constexpr (STAGED) {
             gemm_tile_nt_staged<DT>(W, m0, Hd, n0, a.H, acc, smem);
         } else {
-            gemm_tile_nt_direct<DT, TRLK_HEAD_BK_FWD>(W, m0, Hd, n0, a.H, acc, smem, true);
+            gemm_tile_nt_direct<DT>(W, m0, Hd, n0, a.H, acc, smem, true);
+            // What of the state did not fit beside the accumulators and fragments comes back from scratch here: behind the
+            // transfers below each reload would wait for them to land (5 of a tile's 96 us at H = 3584).
+#pragma unroll
+            for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(ref[j]), "+v"(S[j]), "+v"(U[j]), "+v"(zmax[j]), "+v"(tg[j]));
             // the next tile's first stages travel while this tile's logits are reduced (registers only)
-            if (vt + 1 < vt1) DirectLoader<TRLK_HEAD_BK_FWD>(W, m0 + BM, Hd, n0, smem).prologue(a.H);
+            if (vt + 1 < vt1) DirectLoader<>(W, m0 + BM, Hd, n0, smem).prologue(a.H);
         }
-        // Stash: for one accumulator quad (4 consecutive vocabulary rows of one token per lane) the 32 lanes of a
-        // half-wave hold 32 consecutive tokens = 256 contiguous bytes per store.  The buffer is padded to whole tiles.
+        const int lane = fresh(tid & 63), g = lane >> 4, l15 = lane & 15;
+        // Stash: for one accumulator quad (4 consecutive vocabulary rows of one token per lane) the 16 lanes of a
+        // group hold 16 consecutive tokens = 128 contiguous bytes per store.  The buffer is padded to whole tiles.
         // Addresses are a uniform pointer that walks down the quads (scalar registers, one addition per store) plus
         // the lane's byte offset (one vector register; the entry point bounds ld so that it fits 32 bits).
         char* stash_blk = nullptr;
         float* ref_blk = nullptr;
         uint32_t stash_lane = 0, ref_lane = 0;
         if constexpr (STASH) {
-            const int uw = __builtin_amdgcn_readfirstlane(wave);
-            const int uwm = uw / WGN, ucol = n0 + (uw % WGN) * WN;
-            stash_blk = reinterpret_cast<char*>(a.stash.quads() + int64_t(m0 / 4 + uwm * (WM / 4)) * a.stash.ld + ucol);
-            ref_blk = a.stash.refs() + int64_t(m0 / 128 + uwm) * 2 * a.stash.ld + ucol;
-            ref_lane = uint32_t(lane >> 5) * uint32_t(a.stash.ld) + uint32_t(lane & 31);
-            stash_lane = ref_lane * 8u;
+            const int col = n0 + wn * WN;
+            stash_blk = reinterpret_cast<char*>(a.stash.quads() + int64_t(m0 / 4 + wm * (WM / 4)) * a.stash.ld + col);
+            ref_blk = a.stash.refs() + int64_t(m0 / 128 + wm) * 2 * a.stash.ld + col;
+            ref_lane = uint32_t(g & 1) * uint32_t(a.stash.ld) + uint32_t(l15);
+            stash_lane = (uint32_t(g) * uint32_t(a.stash.ld) + uint32_t(l15)) * 8u;
         }
         const bool partial_tile = m0 + BM > a.V;
-        const float zs = a.logit_scale * a.inv_t, zs2 = zs * kLog2e;
         constexpr bool plain = !GENERAL;
         // Before the reduction, only where needed (a bias, the general form of z, or the vocabulary's last tile, whose
         // rows beyond the vocabulary count as -inf): the accumulators become y + bias (usual head) or z itself
-        // (general form).  A lane's 16 accumulators of a block are 4 quads of consecutive vocabulary rows, so the bias
-        // comes as one 16-byte load per quad, all of a block row's loads issued before the first is used.
+        // (general form).  A lane's 4 accumulators of a block are consecutive vocabulary rows, so the bias
+        // comes as one 16-byte load per block row, four of them issued before the first is used.
         if (GENERAL || a.bias != nullptr || partial_tile) {
             const float inv_cap = a.softcap > 0.f ? 1.f / a.softcap : 0.f;
             typedef float f32x4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) {
+            for (int i0 = 0; i0 < MI; i0 += 4) {
                 f32x4 bq[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int v0 = m0 + acc_row(wm, mb, q * 4, lane);
+                    const int v0 = m0 + acc_row(wm, i0 + q, 0, lane);
                     bq[q] = f32x4{0.f, 0.f, 0.f, 0.f};
                     if (a.bias != nullptr) {
                         if (v0 + 3 < a.V) {
                             bq[q] = *reinterpret_cast<const f32x4_dword_aligned*>(a.bias + v0);
                         } else {
 #pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                if (v0 + i < a.V) bq[q][i] = a.bias[v0 + i];
+                            for (int r = 0; r < 4; ++r)
+                                if (v0 + r < a.V) bq[q][r] = a.bias[v0 + r];
                         }
                     }
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int v0 = m0 + acc_row(wm, mb, q * 4, lane);
+                    const int v0 = m0 + acc_row(wm, i0 + q, 0, lane);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const bool beyond = partial_tile && v0 + i >= a.V;
+                    for (int r = 0; r < 4; ++r) {
+                        const bool beyond = partial_tile && v0 + r >= a.V;
 #pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) {
-                            float y = acc[mb][nb][q * 4 + i] + bq[q][i];
+                        for (int j = 0; j < NI; ++j) {
+                            float y = acc[i0 + q][j][r] + bq[q][r];
                             if constexpr (GENERAL) {
                                 y *= a.logit_scale;
                                 if (a.softcap > 0.f) y = head_tanh(y * inv_cap) * a.softcap;
                                 y *= a.inv_t;
                             }
-                            acc[mb][nb][q * 4 + i] = beyond ? -INFINITY : y;
+                            acc[i0 + q][j][r] = beyond ? -INFINITY : y;
                         }
                     }
                 }
@@ -770,95 +701,96 @@ TRLK_HEAD_KERNEL void fused_head_fwd_kernel(HeadArgs a) {
         // (With a stash the numerators are stored as they are produced.  Packed into registers and stored in one run
         // at the end of the epilogue they cost more: 28.6 against 27.8 ms for the benchmark's forward.)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
+        for (int j = 0; j < NI; ++j) {
             float bm = -INFINITY;
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) bm = fmaxf(bm, acc[mb][nb][r]);
+                for (int r = 0; r < 4; ++r) bm = fmaxf(bm, acc[i][j][r]);
             if constexpr (plain) bm *= zs;
             // target logit: rarely inside this wave's 128 vocabulary rows.  It is selected into one register
             // and stored once: a conditional store per accumulator held the wave for about 20 us, and a
             // workgroup that falls behind the others no longer finds the tiles they share in the L2.
-            const int64_t rel = tg[nb] - (m0 + wm * WM);
-            if (rel >= 0 && rel < WM) {
-                const int want = int(rel) - (lane >> 5) * 4;  // acc_row() without this lane's half-wave offset
+            const int rel = tg[j] - (m0 + wm * WM);
+            if (tg[j] >= 0 && rel >= 0 && rel < WM) {
+                const int want = rel - g * 4;  // acc_row() without this lane's group offset
                 float tv = 0.f;
                 bool mine = false;
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
+                for (int i = 0; i < MI; ++i)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const bool m = (mb * 32 + (r >> 2) * 8 + (r & 3)) == want;
-                        tv = m ? acc[mb][nb][r] : tv;
+                    for (int r = 0; r < 4; ++r) {
+                        const bool m = i * 16 + r == want;
+                        tv = m ? acc[i][j][r] : tv;
                         mine |= m;
                     }
-                if (mine) a.tgt[n0 + acc_col(wn, nb, lane)] = plain ? tv * zs : tv;
+                if (mine) a.tgt[n0 + acc_col(wn, j, lane)] = plain ? tv * zs : tv;
             }
-            zmax[nb] = fmaxf(zmax[nb], bm);
-            const float need = ceilf(bm * kLog2e);
-            if (need > ref[nb]) {
-                const float sc = fast_exp2(ref[nb] - need);
-                S[nb] *= sc;
-                U[nb] *= sc;
-                ref[nb] = need;
-                rr[nb] = need;
+            zmax[j] = fmaxf(zmax[j], bm);
+            // lanes l and l + 32 hold row quads of the same parity: they share a reference exponent (see StashView)
+            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(bm), __float_as_uint(bm), false, false);
+            const float need = ceilf(fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])) * kLog2e);
+            if (need > ref[j]) {
+                const float sc = fast_exp2(ref[j] - need);
+                S[j] *= sc;
+                U[j] *= sc;
+                ref[j] = need;
             }
+            const float rr = ref[j] == -INFINITY ? 0.f : ref[j];
             // numerators times 2^15 (exact; S and U carry the factor until they are written out), with or without a
             // stash: the outputs must not depend on stashing
-            int64_t stash_off = nb * 32 * 8;  // byte offset of this token block's column of quads (uniform)
-            if constexpr (STASH) ref_blk[nb * 32 + ref_lane] = rr[nb];
-            const float rsub = rr[nb] - kStashExp;
+            int64_t stash_off = j * 16 * 8;  // byte offset of this token block's column of quads (uniform)
+            if constexpr (STASH) ref_blk[j * 16 + ref_lane] = rr;
+            const float rsub = rr - kStashExp;
             float s = 0.f, u = 0.f;
             auto sum_tile = [&](auto guard_tag) {
                 constexpr bool kGuard = decltype(guard_tag)::value;  // -inf among the logits (0 * -inf in sum(e * y))
                 const float mul = plain ? zs2 : kLog2e;  // general path: the accumulators hold z itself by now
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
+                for (int i = 0; i < MI; ++i) {
+                    float e[4];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        float e[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float y = acc[mb][nb][q * 4 + i];
-                            e[i] = fast_exp2(fmaf(y, mul, -rsub));
-                            s += e[i];
-                            u = (kGuard && y == -INFINITY) ? u : fmaf(e[i], y, u);
-                        }
-                        if constexpr (STASH) {
-                            uint2 w;
-                            w.x = Elem<TRLK_F16>::pack2(e[0], e[1]);
-                            w.y = Elem<TRLK_F16>::pack2(e[2], e[3]);
-                            *reinterpret_cast<uint2*>(stash_blk + stash_off + stash_lane) = w;
-                            stash_off += a.stash.ld * 16;  // two quads down: the other parity is the other half-wave's
-                            // (one running offset, not 16 precomputed ones; an offset, because a pointer that
-                            // passed through here would no longer be known to point to global memory)
-                            asm volatile("" : "+s"(stash_off));
-                        }
+                    for (int r = 0; r < 4; ++r) {
+                        const float y = acc[i][j][r];
+                        e[r] = fast_exp2(fmaf(y, mul, -rsub));
+                        s += e[r];
+                        u = (kGuard && y == -INFINITY) ? u : fmaf(e[r], y, u);
                     }
+                    if constexpr (STASH) {
+                        uint2 w;
+                        w.x = Elem<TRLK_F16>::pack2(e[0], e[1]);
+                        w.y = Elem<TRLK_F16>::pack2(e[2], e[3]);
+                        *reinterpret_cast<uint2*>(stash_blk + stash_off + stash_lane) = w;
+                        stash_off += a.stash.ld * 32;  // four quads down: those between are the other lane groups'
+                        // (one running offset, not 8 precomputed ones; an offset, because a pointer that
+                        // passed through here would no longer be known to point to global memory)
+                        asm volatile("" : "+s"(stash_off));
+                    }
+                }
             };
             if (GENERAL || partial_tile)
                 sum_tile(std::true_type{});
             else
                 sum_tile(std::false_type{});
             if constexpr (plain) u *= zs;
-            S[nb] += s;
-            U[nb] += u;
+            S[j] += s;
+            U[j] += u;
         }
     }
 
-    // merge the partial states of every token (2 lane halves x WGM M-waves) through LDS
-    constexpr int kParts = 2 * WGM;
+    // merge the partial states of every token (4 lane groups x WGM M-waves) through LDS
+    const int lane = tid & 63, g = lane >> 4;
+    constexpr int kParts = 4 * WGM;
     float* sm = reinterpret_cast<float*>(smem);  // [kParts][BN tokens][4]
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const int col = acc_col(wn, nb, lane);
-        const int part = wm * 2 + (lane >> 5);
-        float* dst = sm + (part * BN + col) * 4;
-        dst[0] = ref[nb];
-        dst[1] = S[nb] * 0x1p-15f;
-        dst[2] = U[nb] * 0x1p-15f;
-        dst[3] = zmax[nb];
+    for (int j = 0; j < NI; ++j) {
+        const int col = acc_col(wn, j, lane);
+        const int part = wm * 4 + g;
+        // (copies of their own: joined to a 16-byte store's registers, the state would be kept as vectors through the whole
+        // tile loop, and spilled)
+        float r, z;
+        asm volatile("v_mov_b32 %0, %2\n\tv_mov_b32 %1, %3" : "=&v"(r), "=v"(z) : "v"(ref[j]), "v"(zmax[j]));
+        *reinterpret_cast<f32x4*>(sm + (part * BN + col) * 4) = f32x4{r, S[j] * 0x1p-15f, U[j] * 0x1p-15f, z};
     }
     __syncthreads();
     if (tid < BN && n0 + tid < a.N) {
@@ -942,11 +874,11 @@ TRLK_HEAD_KERNEL void fused_head_dz_kernel(HeadArgs a) {
     xcd_patch(blockIdx.x, n_tb, n_vt, tb, vt);
     if (tb >= n_tb || vt >= n_vt) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int wm = wave_m(wave), wn = wave_n(wave);
     const int n0 = tb * BN, m0 = a.c0 + vt * BM;
     const Operand W{a.weight, a.ldw, a.V}, Hd{a.hidden, a.ldh, a.N};
-    f32x16 acc[MB][NB];
-    gemm_tile_nt<DT, TRLK_HEAD_BK_DZ>(W, m0, Hd, n0, a.H, acc, smem);
+    f32x4 acc[MI][NI];
+    gemm_tile_nt<DT>(W, m0, Hd, n0, a.H, acc, smem);
 
     // Common case (no soft-capping, tile inside the chunk): dz = -(g * chain) * exp2(y * zs2 - lzc)
     // with one scale folded into the exponent; the target's one-hot term is patched afterwards.
@@ -954,30 +886,30 @@ TRLK_HEAD_KERNEL void fused_head_dz_kernel(HeadArgs a) {
     const bool plain = a.softcap <= 0.f && m0 + BM <= a.c1 && a.bias == nullptr;
     typedef Elem<TRLK_F16> EO;  // storage of dz
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const int tok = n0 + acc_col(wn, nb, lane);
+    for (int j = 0; j < NI; ++j) {
+        const int tok = n0 + acc_col(wn, j, lane);
         const bool tok_ok = tok < a.N;
         const float g = tok_ok ? a.g[tok] * pow2_scale(fabsf(a.g[tok]) * zs) : 0.f;  // g carries the token's scale
         const float lzc = tok_ok ? a.log_z[tok] * kLog2e : INFINITY;  // rows beyond N: exp2(-inf) = 0
         const int64_t tg = tok_ok ? a.targets[tok] : -1;
         const int64_t rel = tg - (m0 + wm * WM);  // target row relative to this wave's rows
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            float d[16];
+        for (int i = 0; i < MI; ++i) {
+            f32x4 d;
             if (plain) {
                 const float ngc = -g * zs;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) d[r] = ngc * fast_exp2(fmaf(acc[mb][nb][r], zs2, -lzc));
-                if (rel >= mb * 32 && rel < mb * 32 + 32) {
+                for (int r = 0; r < 4; ++r) d[r] = ngc * fast_exp2(fmaf(acc[i][j][r], zs2, -lzc));
+                if (rel >= i * 16 && rel < i * 16 + 16) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (acc_row(0, mb, r, lane) == int(rel)) d[r] -= ngc;
+                    for (int r = 0; r < 4; ++r)
+                        if (acc_row(0, i, r, lane) == int(rel)) d[r] -= ngc;
                 }
             } else {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int v = m0 + acc_row(wm, mb, r, lane);
-                    float y = acc[mb][nb][r];
+                for (int r = 0; r < 4; ++r) {
+                    const int v = m0 + acc_row(wm, i, r, lane);
+                    float y = acc[i][j][r];
                     if (a.bias != nullptr && v < a.c1) y += a.bias[v];
                     y *= a.logit_scale;
                     float chain = a.inv_t * a.logit_scale;
@@ -993,8 +925,7 @@ TRLK_HEAD_KERNEL void fused_head_dz_kernel(HeadArgs a) {
                     d[r] = (v < a.c1 && tok_ok) ? dzv * chain : 0.f;
                 }
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = d[r];
+            acc[i][j] = d;
         }
     }
     // dz^T [chunk row][token]: the lanes of a block hold consecutive tokens of one vocabulary row.
@@ -1004,18 +935,18 @@ TRLK_HEAD_KERNEL void fused_head_dz_kernel(HeadArgs a) {
     constexpr int kChunksPerRow = BN / 8;  // 16-byte pieces per row of the staged tile
     const int odd = lane & 1;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        const int tcol = (acc_col(wn, nb, lane) & ~1) * 2;  // byte offset of the token pair inside a staged row
+    for (int j = 0; j < NI; ++j) {
+        const int tcol = (acc_col(wn, j, lane) & ~1) * 2;  // byte offset of the token pair inside a staged row
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const float mine0 = acc[mb][nb][r], mine1 = acc[mb][nb][r + 1];
+            for (int r = 0; r < 4; r += 2) {
+                const float mine0 = acc[i][j][r], mine1 = acc[i][j][r + 1];
                 const float give = odd ? mine0 : mine1;
                 const float got = __builtin_bit_cast(
                     float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xB1 /* quad_perm 1,0,3,2 */, 0xf, 0xf, true));
                 const uint32_t w = odd ? EO::pack2(got, mine1) : EO::pack2(mine0, got);
-                const int vrow = acc_row(wm, mb, r, lane) + odd;
+                const int vrow = acc_row(wm, i, r, lane) + odd;
                 *reinterpret_cast<uint32_t*>(smem + vrow * kDzLdsRow + tcol) = w;
             }
     }
@@ -1161,6 +1092,7 @@ __global__ __launch_bounds__(256) void head_dz_from_stash_kernel(HeadArgs a) {
 //   The accumulators are multiplied by 1 / (scale of A * scale of B) first: the scales are powers of two derived from
 //   the maxima in `max_a` (times `mult_a`) and `max_b` (null = 1), and, when `g_rows` is given, row m of A carries its
 //   own scale pow2_scale(|g_rows[m]| * mult_a) instead of the common one.
+// The tile is computed transposed (B is the tile loop's left operand): a lane then holds 4 consecutive columns of one row.
 struct GemmArgs {
     Operand A, B;
     int M, N, K;
@@ -1183,7 +1115,7 @@ struct GemmArgs {
 template <int DT, int MODE, int ODT, bool AKM = false>
 __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char* smem) {
     typedef Elem<ODT> E;
-    const int n_mt = (a.M + BM - 1) / BM, n_nt = (a.N + BN - 1) / BN;
+    const int n_mt = (a.M + BN - 1) / BN, n_nt = (a.N + BM - 1) / BM;
     Operand A = a.A, B = a.B;
     int K = a.K;
     float* out_f32 = a.out_f32;
@@ -1202,106 +1134,78 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     xcd_patch(block, n_mt, n_nt, tm, tn);
     if (tm >= n_mt || tn >= n_nt) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave / WGN, wn = wave % WGN;
-    const int m0 = tm * BM, n0 = tn * BN;
-    f32x16 acc[MB][NB];
-    gemm_tile_nt<DT, TRLK_HEAD_BK_GEMM, AKM, true>(A, m0, B, n0, K, acc, smem);
+    const int wm = wave_m(wave), wn = wave_n(wave);
+    const int r0 = tm * BN, c0 = tn * BM;  // the tile's first row and column of the output
+    f32x4 acc[MI][NI];
+    const bool idle = r0 + wn * WN >= a.M || c0 + wm * WM >= a.N;  // all of this wave's rows or columns lie beyond the output
+    if (idle && (AKM || (K & (BK - 1)) == 0)) return move_tiles_only(DirectLoader<AKM>(B, c0, A, r0, smem), K, false);
+    gemm_tile_nt<DT, AKM>(B, c0, A, r0, K, acc, smem);
+    if (idle) return;  // (no barrier follows)
     const float inv_b = 1.f / slot_scale(a.max_b, 1.f);
     const float inv_common = inv_b / slot_scale(a.max_a, a.mult_a);
-    // A tile inside the output (nearly every tile): no per-element predicates, addresses as a uniform base plus one
-    // 32-bit lane offset, the 16 running sums of a block loaded before the first is used and its 16 results stored in
-    // one run.  (Written per element with a bounds test each, the compiler lost count of the loads in flight and
-    // waited for EVERYTHING outstanding before each accumulate, i.e. for the previous store's acknowledgement: 128
-    // store round trips per tile.)
-    const bool lp_pairs = (reinterpret_cast<uintptr_t>(a.out_lp) & 3) == 0 && (a.ld_lp & 1) == 0;
-    if (m0 + BM <= a.M && n0 + BN <= a.N && (MODE == 1 || lp_pairs) && a.ld_f32 < (int64_t(1) << 24) &&
-        a.ld_lp < (int64_t(1) << 24)) {
-        const int uw = __builtin_amdgcn_readfirstlane(wave);
-        const int row0 = m0 + (uw / WGN) * WM, col0 = n0 + (uw % WGN) * WN;  // uniform
-        const int half = lane >> 5, l31 = lane & 31, odd = lane & 1;
-        typedef float f32x4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
+    const int g = lane >> 4;
+    // The wave's 128 columns inside the output (nearly every tile), rows aligned for vector accesses: a row's 8 running
+    // sums of 16 bytes are loaded before the first is used, its results stored in one run.  (Written per element with a
+    // bounds test each, the compiler lost count of the loads in flight and waited for EVERYTHING outstanding before each
+    // accumulate, i.e. for the previous store's acknowledgement: 128 store round trips per tile.)
+    const bool f32_ok = MODE == 0 || ((reinterpret_cast<uintptr_t>(out_f32) & 15) == 0 && (a.ld_f32 & 3) == 0);
+    const bool lp_ok = MODE == 1 || ((reinterpret_cast<uintptr_t>(a.out_lp) & 15) == 0 && (a.ld_lp & 7) == 0);
+    const bool fast = c0 + (wm + 1) * WM <= a.N && f32_ok && lp_ok;
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            float inv[16];
+    for (int j = 0; j < NI; ++j) {
+        const int row = r0 + acc_col(wn, j, lane);
+        if (row >= a.M) continue;
+        const float inv = a.g_rows != nullptr ? inv_b / pow2_scale(fabsf(a.g_rows[row]) * a.mult_a) : inv_common;
+        if (fast) {
+            f32x4 v[MI];
+            if constexpr (MODE != 0) {
+                float* out = out_f32 + int64_t(row) * a.ld_f32 + (c0 + acc_row(wm, 0, 0, lane));
+                f32x4 prev[MI];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                f32x4 g4 = {0.f, 0.f, 0.f, 0.f};
-                if (a.g_rows != nullptr)
-                    g4 = *reinterpret_cast<const f32x4_dword_aligned*>(a.g_rows + row0 + mb * 32 + q * 8 + half * 4);
+                for (int i = 0; i < MI; ++i)
+                    prev[i] = a.first ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(out + i * 16);
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    inv[q * 4 + i] = a.g_rows != nullptr ? inv_b / pow2_scale(fabsf(g4[i]) * a.mult_a) : inv_common;
-            }
+                for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                float v[16];
-                if constexpr (MODE != 0) {
-                    float* blk = out_f32 + int64_t(row0 + mb * 32) * a.ld_f32 + (col0 + nb * 32);  // uniform
-                    const uint32_t lane_off = uint32_t(half * 4) * uint32_t(a.ld_f32) + uint32_t(l31);
-                    float prev[16];
+                    for (int r = 0; r < 4; ++r) v[i][r] = fmaf(acc[i][j][r], inv, prev[i][r]);
+                if constexpr (MODE == 1) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        prev[r] = a.first ? 0.f : blk[int64_t(((r >> 2) * 8 + (r & 3)) * a.ld_f32) + lane_off];
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) v[r] = fmaf(acc[mb][nb][r], inv[r], prev[r]);
-                    if constexpr (MODE == 1) {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) blk[int64_t(((r >> 2) * 8 + (r & 3)) * a.ld_f32) + lane_off] = v[r];
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) v[r] = acc[mb][nb][r] * inv[r];
+                    for (int i = 0; i < MI; ++i) *reinterpret_cast<f32x4*>(out + i * 16) = v[i];
                 }
-                if constexpr (MODE != 1) {
-                    // 16-bit outputs: neighbouring lanes swap one value, the even lane then owns two columns of row
-                    // r and the odd lane two columns of row r + 1 -- 4-byte stores, 64 contiguous bytes per row
-                    typename E::type* blk = a.out_lp + int64_t(row0 + mb * 32) * a.ld_lp + (col0 + nb * 32);  // uniform
-                    const uint32_t lane_off = uint32_t(half * 4 + odd) * uint32_t(a.ld_lp) + uint32_t(l31 & ~1);
+            } else {
 #pragma unroll
-                    for (int r = 0; r < 16; r += 2) {
-                        const float give = odd ? v[r] : v[r + 1];
-                        const float got = __builtin_bit_cast(
-                            float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xB1 /* quad_perm 1,0,3,2 */, 0xf, 0xf, true));
-                        const uint32_t w = odd ? E::pack2(got, v[r + 1]) : E::pack2(v[r], got);
-                        *reinterpret_cast<uint32_t*>(blk + int64_t(((r >> 2) * 8 + (r & 3)) * a.ld_lp) + lane_off) = w;
-                    }
+                for (int i = 0; i < MI; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[i][r] = acc[i][j][r] * inv;
+            }
+            if constexpr (MODE != 1) {
+                // 16-bit outputs: of two neighbouring blocks the lane groups 0, 2 take the first and 1, 3 the second, 8
+                // consecutive columns (16 bytes) per lane, 64 contiguous bytes per row and store
+                typename E::type* out = a.out_lp + int64_t(row) * a.ld_lp + (c0 + wm * WM + (g & 1) * 16 + (g >> 1) * 8);
+#pragma unroll
+                for (int i = 0; i < MI; i += 2) {
+                    const auto lo = __builtin_amdgcn_permlane16_swap(E::pack2(v[i][0], v[i][1]), E::pack2(v[i + 1][0], v[i + 1][1]),
+                                                                     false, false);
+                    const auto hi = __builtin_amdgcn_permlane16_swap(E::pack2(v[i][2], v[i][3]), E::pack2(v[i + 1][2], v[i + 1][3]),
+                                                                     false, false);
+                    *reinterpret_cast<u32x4*>(out + i * 16) = u32x4{lo[0], hi[0], lo[1], hi[1]};
                 }
             }
-        }
-        return;
-    }
-    // The running sum of a block is read as a whole before any of the block is written: with a load
-    // and a store of the same array per element the compiler keeps them in program order, one memory
-    // latency per element (67 us per tile instead of a few).
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-        float inv[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = m0 + acc_row(wm, mb, r, lane);
-            inv[r] = (a.g_rows != nullptr && row < a.M) ? inv_b / pow2_scale(fabsf(a.g_rows[row]) * a.mult_a) : inv_common;
+            continue;
         }
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const int col = n0 + acc_col(wn, nb, lane);
-            if (col >= a.N) continue;
-            float prev[16];
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + acc_row(wm, mb, r, lane);
-                prev[r] = (MODE != 0 && !a.first && row < a.M) ? out_f32[int64_t(row) * a.ld_f32 + col] : 0.f;
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + acc_row(wm, mb, r, lane);
-                if (row >= a.M) continue;
-                const float v = fmaf(acc[mb][nb][r], inv[r], prev[r]);
+            for (int r = 0; r < 4; ++r) {
+                const int col = c0 + acc_row(wm, i, r, lane);
+                if (col >= a.N) continue;
+                const float prev = (MODE != 0 && !a.first) ? out_f32[int64_t(row) * a.ld_f32 + col] : 0.f;
+                const float v = fmaf(acc[i][j][r], inv, prev);
                 if (MODE == 1)
                     out_f32[int64_t(row) * a.ld_f32 + col] = v;
                 else
                     E::store1(a.out_lp + int64_t(row) * a.ld_lp + col, v);
             }
-        }
     }
 }
 
@@ -1754,7 +1658,7 @@ extern "C" int trlk_fused_head_fwd(const void* d_hidden, const void* d_weight, c
     const char* what = "fused_head_fwd";
     int rc;
     const bool general = a.softcap > 0.f || !(a.logit_scale * a.inv_t > 0.f);
-    const bool staged = hidden_size % TRLK_HEAD_BK_FWD != 0;
+    const bool staged = hidden_size % BK != 0;
     auto launch_fwd = [&](auto stash_tag, auto general_tag) {
         constexpr bool kS = decltype(stash_tag)::value, kG = decltype(general_tag)::value;
         if (staged)
