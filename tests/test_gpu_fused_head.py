@@ -872,10 +872,12 @@ def test_row_selection_and_mean_logits_can_be_traced(amd):
 
 @pytest.mark.parametrize("stash", [True, False])
 @pytest.mark.parametrize("n,h,v", [(1, 64, 256), (64, 128, 257), (65, 64, 384), (128, 192, 385), (129, 64, 100), (193, 128, 513),
-                                   (255, 64, 640), (257, 64, 255), (320, 128, 129), (450, 320, 1000)])
+                                   (255, 64, 640), (257, 64, 255), (320, 128, 129), (450, 320, 1000), (2305, 64, 1500),
+                                   (4400, 320, 300), (8200, 64, 520)])
 def test_partly_filled_tiles(amd, monkeypatch, n, h, v, stash):
     """Token and vocabulary counts around the 64-column and 128-row pieces of a tile that one wave owns: waves whose tokens
-    lie beyond the last one do no matrix work, the others' results must not notice."""
+    lie beyond the last one do no matrix work, the others' results must not notice.  The larger token counts take the tile orders
+    of 8 to 31 and of 32 and more token tiles."""
     if not stash:
         monkeypatch.setenv("TRL_AMD_HEAD_STASH_GIB", "0")
     g = torch.Generator().manual_seed(n + v)

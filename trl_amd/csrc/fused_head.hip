@@ -457,19 +457,27 @@ __device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) { return 
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * WN + j * 16 + (lane & 15); }
 
 // Workgroup id -> (tile along axis `a`, tile along axis `b`) such that the workgroups that run
-// together on one XCD (ids congruent mod 8, dispatched round-robin) form 4 x 8 patches: they share
-// operand slabs through that XCD's L2.  An XCD owns the `a` tiles congruent to its number mod 8, in
-// bands of 4; inside a band it walks b with the band's a tiles innermost.  The last band holds only
-// as many a tiles per XCD as n_a needs, so that (almost) no workgroup of the grid is empty: the
-// hardware deals workgroups to the CUs in order, and with empty ones interleaved at a fixed stride
-// the real ones end up on a fraction of the CUs (measured: a third more time for 65 instead of 64
-// a tiles with a grid padded to whole bands).  The n_a % 8 a tiles that are left when every XCD has
-// the same number are not given to that many XCDs whole (one XCD in eight would then carry an a
-// tile more than the others and the launch would wait for it): their n_b tiles each are dealt out
-// in equal runs over all eight XCDs, a innermost.  The caller skips ta >= n_a or tb >= n_b.
+// together on one XCD (ids congruent mod 8, dispatched round-robin) form patches of about 4 x 8 tiles: they share
+// operand slabs through that XCD's L2.  No workgroup of the grid but a few at the end is empty: the hardware deals
+// workgroups to the CUs in order, and with empty ones interleaved at a fixed stride the real ones end up on a fraction of
+// the CUs (measured: a third more time for 65 instead of 64 a tiles with a grid padded to whole bands).
+//
+// From 32 a tiles on an XCD owns the `a` tiles congruent to its number mod 8, in bands of 4; inside a band it walks b
+// with the band's a tiles innermost.  The last band holds only as many a tiles per XCD as n_a needs.  The n_a % 8 a tiles
+// that are left when every XCD has the same number are not given to that many XCDs whole (one XCD in eight would then
+// carry an a tile more than the others and the launch would wait for it): their n_b tiles each are dealt out
+// in equal runs over all eight XCDs, a innermost.
+//
+// Fewer a tiles (token counts below 8192) are put into even bands of at most 8; inside a band b is walked with the band's a
+// tiles innermost, and each XCD takes one eighth of that sequence: 4 to 8 a tiles beside 4 to 8 b tiles at a time.  Under
+// the rule for many a tiles an XCD has ONE a tile beside 32 b tiles when there are 8 to 15, and fetches 33 slabs where
+// 12 would do: 2300 tokens, H = 2048, V = 128256 forward 1140 -> 1107 us, with backward 3720 -> 3690 us; 3000 tokens, H =
+// 3072, V = 50257 866 -> 834 and 2713 -> 2664 us; 1000 tokens, H = 2048, V = 128256 (there the slices of dHidden) 1948 -> 1918 us.
+// The same for the last few of many a tiles loses (79 a tiles: forward 3653 -> 3735 us).
+// The caller skips ta >= n_a or tb >= n_b.
 __device__ __forceinline__ void xcd_patch(int w, int n_a, int n_b, int& ta, int& tb) {
     const int xcd = w & 7, q = w >> 3;
-    const int groups = n_a >> 3;                   // a tiles every XCD owns whole
+    const int groups = n_a >= 32 ? n_a >> 3 : 0;   // a tiles every XCD owns whole
     const int bands = groups >> 2;                 // full bands of 4 of them
     const int full = bands * 4 * n_b;              // workgroups of this XCD in the full bands
     const int m = groups & 3;                      // whole a tiles per XCD in the last band
@@ -477,21 +485,31 @@ __device__ __forceinline__ void xcd_patch(int w, int n_a, int n_b, int& ta, int&
         const int rem = q % (4 * n_b);
         tb = rem >> 2;
         ta = ((q / (4 * n_b)) * 4 + (rem & 3)) * 8 + xcd;
-    } else if (q < full + m * n_b) {
+        return;
+    }
+    if (q < full + m * n_b) {
         const int qq = q - full;
         tb = qq / m;
         ta = (bands * 4 + qq % m) * 8 + xcd;
-    } else {
-        const int r = (n_a & 7) ? (n_a & 7) : 1, left = (n_a & 7) * n_b;  // the a tiles that are left, and their tiles
-        const int share = (left + 7) >> 3;
-        const int t = xcd * share + (q - full - m * n_b);
-        const bool real = q - full - m * n_b < share && t < left;
-        ta = real ? groups * 8 + t % r : n_a;      // a innermost, as in the bands: neighbours share the b slab
-        tb = real ? t / r : n_b;
+        return;
     }
+    // the a tiles that are left, from n_a - left on, dealt out in runs
+    const int left = n_a - groups * 8, share = (left * n_b + 7) >> 3, i = q - full - m * n_b, t = xcd * share + i;
+    if (i >= share || t >= left * n_b) {
+        ta = n_a;
+        tb = n_b;
+        return;
+    }
+    const int n_bands = (left + 7) >> 3, narrow = left / n_bands, wide = left % n_bands;  // `wide` bands of narrow + 1, then narrow
+    const int in_wide = wide * (narrow + 1) * n_b;
+    const int width = t < in_wide ? narrow + 1 : narrow, u = t < in_wide ? t : t - in_wide;
+    const int band = u / (width * n_b), v = u - band * (width * n_b);
+    tb = v / width;
+    ta = groups * 8 + (t < in_wide ? 0 : wide * (narrow + 1)) + band * width + (v - tb * width);
 }
 inline int xcd_patch_grid(int n_a, int n_b) {
-    return 8 * ((n_a / 8) * n_b + ((n_a % 8) * n_b + 7) / 8);
+    const int groups = n_a >= 32 ? n_a / 8 : 0, left = n_a - groups * 8;
+    return 8 * (groups * n_b + (left * n_b + 7) / 8);
 }
 
 // What a forward keeps for the backward when it is given a stash: for every logit its softmax numerator
@@ -1106,8 +1124,9 @@ struct GemmArgs {
     const float* g_rows;
     float mult_a;
     // K-major A, epilogue 1: the contraction cut into `slices` pieces of `kslice` (a multiple of the k step), each
-    // with its own fp32 sum at out_f32 + slice * M * ld_f32; slice i takes workgroups [i, i + 1) * slice_grid.
-    int slices, kslice, slice_grid;
+    // with its own fp32 sum at out_f32 + slice * M * ld_f32.  The slices are further columns of the tile grid, so that an
+    // XCD works on few of them: its tiles of one slice share their slabs of both operands.
+    int slices, kslice;
 };
 
 // DT: dtype of the operands (the matrix-core instruction), ODT: storage dtype of `out_lp`.
@@ -1119,20 +1138,19 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     Operand A = a.A, B = a.B;
     int K = a.K;
     float* out_f32 = a.out_f32;
-    if constexpr (AKM && MODE == 1) {
-        if (a.slices > 1) {
-            const int slice = block / a.slice_grid;
-            block -= slice * a.slice_grid;
-            const int k0 = slice * a.kslice;
-            A.p += int64_t(k0) * A.ld;
-            B.p += k0;
-            K = min(a.kslice, K - k0);
-            out_f32 += int64_t(slice) * a.M * a.ld_f32;
-        }
-    }
+    constexpr bool kSlices = AKM && MODE == 1;
+    const int n_cols = kSlices ? n_nt * a.slices : n_nt;
     int tm, tn;
-    xcd_patch(block, n_mt, n_nt, tm, tn);
-    if (tm >= n_mt || tn >= n_nt) return;
+    xcd_patch(block, n_mt, n_cols, tm, tn);
+    if (tm >= n_mt || tn >= n_cols) return;
+    if constexpr (kSlices) {
+        const int slice = tn / n_nt, k0 = slice * a.kslice;
+        tn -= slice * n_nt;
+        A.p += int64_t(k0) * A.ld;
+        B.p += k0;
+        K = min(a.kslice, K - k0);
+        out_f32 += int64_t(slice) * a.M * a.ld_f32;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave_m(wave), wn = wave_n(wave);
     const int r0 = tm * BN, c0 = tn * BM;  // the tile's first row and column of the output
@@ -1847,8 +1865,7 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         gh.slices = l.slices;  // (of the last, possibly shorter chunk those that its rows reach)
         while (gh.slices > 1 && int64_t(gh.slices - 1) * l.kslice >= kpad) --gh.slices;
         gh.kslice = l.kslice;
-        gh.slice_grid = xcd_patch_grid(n_tb, n_ht);
-        const int ghgrid = gh.slice_grid * gh.slices;
+        const int ghgrid = xcd_patch_grid(n_tb, n_ht * gh.slices);
         // dW[chunk, H] = dz^T[chunk, N] * (hidden^T[H, N])^T
         GemmArgs gw{};
         gw.A = Operand{dzt, l.ld_n, kpad};
