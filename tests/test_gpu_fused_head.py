@@ -891,3 +891,40 @@ def test_partly_filled_tiles(amd, monkeypatch, n, h, v, stash):
     torch.testing.assert_close(lp, rlp, atol=5e-5, rtol=0)
     torch.testing.assert_close(ent, rent, atol=5e-5, rtol=0)
     _check_beyond_output_rounding(dh, dw, rdh, rdw, torch.bfloat16)
+
+
+@pytest.mark.parametrize("stash", [True, False])
+@pytest.mark.parametrize("kind", ["outlier", "outlier_of_one_chunk", "zero_sample", "zero_weight", "just_inside"])
+def test_weight_scale_from_a_sample(amd, monkeypatch, kind, stash):
+    """The backward converts the bf16 weight to fp16 in a scale taken from every 32nd row; a chunk that reaches beyond what that
+    scale leaves room for, or whose sample holds only zeros, is converted again in its own scale."""
+    if not stash:
+        monkeypatch.setenv("TRL_AMD_HEAD_STASH_GIB", "0")
+    n, h, v = 70, 128, 900
+    g = torch.Generator().manual_seed(3)
+    hidden = torch.randn(n, h, generator=g).bfloat16() * 0.01
+    weight = torch.randn(v, h, generator=g) * 0.02
+    sample_max = weight[::32].abs().max()
+    if kind == "outlier":
+        weight[5, 7] = 300.0
+        weight[801, 0] = -2000.0
+    elif kind == "outlier_of_one_chunk":
+        weight[300, 64] = 500.0
+    elif kind == "zero_sample":
+        weight[::32] = 0.0
+    elif kind == "zero_weight":
+        weight.zero_()
+    else:  # the largest magnitude that the sample's scale still holds
+        weight[33, 1] = 3.9 * 2.0 ** torch.floor(torch.log2(sample_max))
+    weight = weight.bfloat16()
+    labels = torch.randint(0, v, (n,), generator=g)
+    labels[:4] = torch.tensor([5, 801, 300, 33])
+    gout = torch.randn(n, generator=g)
+    lp, ent, dh, dw = _run_device(amd, hidden, weight, labels, 1.0, 256, None, 1.0, gout)
+    rlp, _, rdh, rdw = _fp32_reference(hidden, weight, labels, 1.0, None, 1.0, gout)
+    torch.testing.assert_close(lp, rlp, atol=1e-4, rtol=0)
+    assert torch.isfinite(dh).all() and torch.isfinite(dw).all()
+    if kind == "zero_weight":
+        assert not dh.any()
+        rdh = dh.float()
+    _check_beyond_output_rounding(dh, dw, rdh, rdw, torch.bfloat16)

@@ -565,7 +565,7 @@ struct HeadArgs {
 // into [2^13, 2^14) (exact, undone in the products' epilogue): d logits per token (|dz[:, n]| <= |g[n]| * logit_scale
 // / T, so token n's column carries s_n = pow2_scale(|g[n]| * logit_scale / T) and a token whose upstream gradient is
 // a million times smaller than the largest keeps its own relative accuracy in dHidden, whose row n the epilogue
-// divides by s_n), W^T and hidden^T of a bf16 problem by their largest magnitude (bf16 -> fp16 is then exact down to
+// divides by s_n), W^T and hidden^T of a bf16 problem by their largest magnitude (of W's a sample decides; bf16 -> fp16 is then exact down to
 // 2^-31 of that maximum).  The dW product sums over the tokens, so it needs the columns of d logits in ONE scale: row
 // n of hidden^T's source is multiplied by s_all / s_n on its way (s_all = the scale of the largest |g|, so the factor
 // is a power of two <= 1), which leaves dz^T[v, n] * hidden^T[h, n] in the scale s_all * s_hidden for every n.  A token
@@ -581,6 +581,21 @@ __device__ __forceinline__ float pow2_scale(float m) {
 }
 __device__ __forceinline__ float slot_scale(const uint32_t* slot, float mult) {
     return slot != nullptr ? pow2_scale(__uint_as_float(*slot) * mult) : 1.f;
+}
+// The weight's scale comes from a SAMPLE of it (every kSampleRows-th row), so that no pass over the whole weight is needed
+// before the one that converts it; that pass finds the true maximum on its way.  slots[0] is the sample's largest magnitude,
+// slots[1] that of the entries that exceed it (0 if none does).  The sample's scale leaves a factor of 4 to fp16's largest
+// value; only when the chunk reaches beyond it, or the sample holds nothing but zeros, is the chunk converted again
+// with the scale of its own maximum.
+constexpr int kSampleRows = 32;
+struct WeightScale {
+    float scale;
+    bool again;  // the chunk has to be converted (again) with `scale`
+};
+__device__ __forceinline__ WeightScale weight_scale(const uint32_t* sample, const uint32_t* beyond) {
+    const float m = __uint_as_float(*sample), top = __uint_as_float(max(*sample, *beyond)), s = pow2_scale(m);
+    if (top == 0.f || (m > 0.f && top * s <= 65504.f)) return {s, false};
+    return {pow2_scale(top), true};
 }
 
 // tanh for soft-capping: sign(x) (1 - t) / (1 + t) with t = exp(-2 |x|) from the hardware's exp2 and reciprocal (a
@@ -1121,6 +1136,7 @@ struct GemmArgs {
     int first;
     const uint32_t* max_a;
     const uint32_t* max_b;
+    const uint32_t* beyond_b;  // B is the weight: max_b and this are the two slots of weight_scale()
     const float* g_rows;
     float mult_a;
     // K-major A, epilogue 1: the contraction cut into `slices` pieces of `kslice` (a multiple of the k step), each
@@ -1159,7 +1175,7 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     if (idle && (AKM || (K & (BK - 1)) == 0)) return move_tiles_only(DirectLoader<AKM>(B, c0, A, r0, smem), K, false);
     gemm_tile_nt<DT, AKM>(B, c0, A, r0, K, acc, smem);
     if (idle) return;  // (no barrier follows)
-    const float inv_b = 1.f / slot_scale(a.max_b, 1.f);
+    const float inv_b = 1.f / (a.beyond_b != nullptr ? weight_scale(a.max_b, a.beyond_b).scale : slot_scale(a.max_b, 1.f));
     const float inv_common = inv_b / slot_scale(a.max_a, a.mult_a);
     const int g = lane >> 4;
     // The wave's 128 columns inside the output (nearly every tile), rows aligned for vector accesses: a row's 8 running
@@ -1297,24 +1313,28 @@ __global__ __launch_bounds__(256) void split_bf16x3_kernel(const float* in, int6
 }
 
 // Largest magnitudes of the backward's operands in one launch: out[0] of the fp32 vector g [n_g], out[1] of hidden, out[2]
-// of the weight (bf16 matrices of C8 * 8 columns; no workgroups are launched for them in an fp16 problem), as the bit
-// patterns of those floats (non-negative floats order like unsigned integers; the caller clears `out`).
+// of every kSampleRows-th row of the weight (bf16 matrices of C8 * 8 columns; no workgroups are launched for them in an
+// fp16 problem), as the bit patterns of those floats (non-negative floats order like unsigned integers; the caller clears
+// `out`).
 //
-// Bound by the read of the weight.  Workgroups of 1024 lanes, at most two per CU for a matrix, eight 16-byte loads in
-// flight per lane, one atomic per workgroup and only when it would raise the maximum: atomics on one address retire
-// about one per 15 ns, so one per wave of 4096 small workgroups took 250 us whatever the size of the matrix.
-// Weights of 206 / 525 / 1089 MB (50257 x 2048, 128256 x 2048, 151936 x 3584) with 1400 / 1400 / 9700 tokens: the three
-// launches 263 / 279 / 355 us -> 34 / 96 / 201 us (5.6-6.1 TB/s).
+// Bound by the read of hidden and of the sample.  Workgroups of 1024 lanes, at most two per CU for a matrix, eight 16-byte
+// loads in flight per lane, one atomic per workgroup and only when it would raise the maximum: atomics on one address
+// retire about one per 15 ns, so one per wave of 4096 small workgroups took 250 us whatever the size of the matrix.
 constexpr int kMaxThreads = 1024, kMaxBlocks = 512;
 struct MaxAbsArgs {
     const float* g;
     int64_t n_g;
     const uint16_t *hidden, *weight;
-    int64_t ld_hidden, ld_weight;
+    int64_t ld_hidden, ld_weight;       // (the weight's: between two rows of the sample)
     int n_hidden, n_weight, C8;         // rows; 16-byte vectors per row
     int blocks_g, blocks_h, blocks_w;   // workgroups of each
     uint32_t* out;
 };
+__device__ __forceinline__ uint32_t max_bits(uint32_t m, u32x4 q) {  // of the 8 bf16 in q, as fp32 bit patterns
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m = max(m, max((q[i] << 16) & 0x7fff0000u, q[i] & 0x7fff0000u));
+    return m;
+}
 __global__ __launch_bounds__(kMaxThreads) void head_maxabs_kernel(MaxAbsArgs a) {
     __shared__ uint32_t part[kMaxThreads / kWave];
     int block = blockIdx.x, slot;
@@ -1332,28 +1352,20 @@ __global__ __launch_bounds__(kMaxThreads) void head_maxabs_kernel(MaxAbsArgs a) 
         const uint16_t* in = is_w ? a.weight : a.hidden;
         const int64_t ld = is_w ? a.ld_weight : a.ld_hidden;
         const int R = is_w ? a.n_weight : a.n_hidden;
-        auto take = [&](u32x4 q) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) m = max(m, max((q[i] << 16) & 0x7fff0000u, q[i] & 0x7fff0000u));
+        const int64_t n = int64_t(R) * a.C8, step = int64_t(blocks) * kMaxThreads;
+        auto at = [&](int64_t v) {
+            const int64_t r = v / a.C8;
+            return *reinterpret_cast<const u32x4*>(in + r * ld + (v - r * a.C8) * 8);
         };
-        if (ld == int64_t(a.C8) * 8) {  // dense rows: one flat sweep
-            const u32x4* p = reinterpret_cast<const u32x4*>(in);
-            const int64_t n = int64_t(R) * a.C8, step = int64_t(blocks) * kMaxThreads;
-            int64_t v = int64_t(block) * kMaxThreads + threadIdx.x;
-            for (; v + 7 * step < n; v += 8 * step) {
-                u32x4 q[8];
+        int64_t v = int64_t(block) * kMaxThreads + threadIdx.x;
+        for (; v + 7 * step < n; v += 8 * step) {
+            u32x4 q[8];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) q[k] = p[v + k * step];
+            for (int k = 0; k < 8; ++k) q[k] = at(v + k * step);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) take(q[k]);
-            }
-            for (; v < n; v += step) take(p[v]);
-        } else {
-            for (int r = block; r < R; r += blocks) {
-                const u32x4* row = reinterpret_cast<const u32x4*>(in + int64_t(r) * ld);
-                for (int c = threadIdx.x; c < a.C8; c += kMaxThreads) take(row[c]);
-            }
+            for (int k = 0; k < 8; ++k) m = max_bits(m, q[k]);
         }
+        for (; v < n; v += step) m = max_bits(m, at(v));
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off, 64)));
@@ -1367,29 +1379,28 @@ __global__ __launch_bounds__(kMaxThreads) void head_maxabs_kernel(MaxAbsArgs a) 
     }
 }
 
-// [R, C] (ld) -> [C, ldo] with columns >= R zero-filled up to `fill`: 64 x 64 tiles through LDS.
-// TO_F16: the input is bf16 and the output fp16, multiplied by the power of two that `in_max` (the input's largest
-// magnitude) asks for.
+// One 64 x 64 tile of [R, C] (ld) -> [C, ldo] with columns >= R zero-filled up to `fill`, through LDS.
+// TO_F16: the input is bf16 and the output fp16, multiplied by the power of two `sc`.
 // ROW_G: input row r is also multiplied by s_all / pow2_scale(|row_g[r]| * zs) (0 where row_g[r] is 0), s_all from
 // `g_max`: what brings the columns of hidden^T into the scales of the d logits' columns (see above).
-template <bool TO_F16, bool ROW_G = false>
-__global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
-                                                          int64_t ldo, int64_t fill, const uint32_t* in_max,
-                                                          const float* row_g = nullptr, const uint32_t* g_max = nullptr,
-                                                          float zs = 1.f) {
+// Returns the largest magnitude (bit pattern) of what this lane read when TRACK is set.
+constexpr int kTransposeStride = 136;
+template <bool TO_F16, bool ROW_G, bool TRACK>
+__device__ __forceinline__ uint32_t transpose16_tile(uint16_t* tile, int c0, int r0, const uint16_t* in, int64_t ld, int R, int C,
+                                                     uint16_t* out, int64_t ldo, int64_t fill, float sc, const float* row_g,
+                                                     const uint32_t* g_max, float zs) {
     // C, ld, ldo and fill are multiples of 8 and both matrices 16-byte aligned (the callers' operands are): a lane
     // moves 8 elements at a time.  Tile rows are skewed by 8 elements per group of 8 rows, which spreads the
     // 2-byte column reads of the second phase over all banks.
-    constexpr int kStride = 136;
-    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kStride];
-    const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
+    constexpr int kStride = kTransposeStride;
     const int tid = threadIdx.x, hi = tid >> 3, lo = tid & 7;
-    const float sc = TO_F16 ? slot_scale(in_max, 1.f) : 1.f;
+    uint32_t m = 0;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const int row = hi + 32 * p, cc = lo * 8;
         u32x4 q = {0u, 0u, 0u, 0u};
         if (r0 + row < R && c0 + cc < C) q = *reinterpret_cast<const u32x4*>(in + int64_t(r0 + row) * ld + c0 + cc);
+        if (TRACK) m = max_bits(m, q);
         if (TO_F16 || ROW_G) {
             float f = sc;
             if (ROW_G) {
@@ -1420,6 +1431,47 @@ __global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* in, in
             const u32x4 q = {w[0], w[1], w[2], w[3]};
             *reinterpret_cast<u32x4*>(out + int64_t(c0 + c) * ldo + r0 + r8 * 8) = q;
         }
+    }
+    return m;
+}
+template <bool TO_F16, bool ROW_G = false>
+__global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
+                                                          int64_t ldo, int64_t fill, const uint32_t* in_max,
+                                                          const float* row_g = nullptr, const uint32_t* g_max = nullptr,
+                                                          float zs = 1.f) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kTransposeStride];
+    transpose16_tile<TO_F16, ROW_G, false>(tile, blockIdx.x * 64, blockIdx.y * 64, in, ld, R, C, out, ldo, fill,
+                                           TO_F16 ? slot_scale(in_max, 1.f) : 1.f, row_g, g_max, zs);
+}
+// W_chunk^T of a bf16 problem in the sample's scale.  The largest magnitude of what it converts is found on the way: a wave
+// whose entries all stay below the sample's maximum (nearly every one) spends one comparison on it, the others one atomic.
+// The separate pass over the whole weight that used to precede this one took 36 / 93 / 214 us for weights of 206 / 525 / 1089 MB
+// (50257 x 2048, 128256 x 2048, 151936 x 3584); the sample takes 7 / 10 / 15 us, a second launch with nothing to do 3-5 us.
+__global__ __launch_bounds__(256) void transpose_weight_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
+                                                               int64_t ldo, int64_t fill, const uint32_t* sample, uint32_t* beyond) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kTransposeStride];
+    uint32_t m = transpose16_tile<true, false, true>(tile, blockIdx.x * 64, blockIdx.y * 64, in, ld, R, C, out, ldo, fill,
+                                                     slot_scale(sample, 1.f), nullptr, nullptr, 1.f);
+    const uint32_t known = max(*sample, __hip_atomic_load(beyond, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (__any(m > known)) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off, 64)));
+        if ((threadIdx.x & (kWave - 1)) == 0) atomicMax(beyond, m);
+    }
+}
+// The same again in the scale of the chunk's own maximum, where the sample's does not do: returns at once everywhere else (few
+// workgroups that step through the tiles, so that a launch with nothing to do takes 3-5 us).
+constexpr int kAgainBlocks = 1024;
+__global__ __launch_bounds__(256) void transpose_weight_again_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
+                                                                     int64_t ldo, int64_t fill, const uint32_t* sample,
+                                                                     const uint32_t* beyond, int tiles_c, int tiles) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kTransposeStride];
+    const WeightScale w = weight_scale(sample, beyond);
+    if (!w.again) return;
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+        transpose16_tile<true, false, false>(tile, t % tiles_c * 64, t / tiles_c * 64, in, ld, R, C, out, ldo, fill, w.scale,
+                                             nullptr, nullptr, 1.f);
+        __syncthreads();  // (the next tile overwrites the LDS)
     }
 }
 
@@ -1505,7 +1557,7 @@ BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     l.slices = int((l.cpad + l.kslice - 1) / l.kslice);
     l.off_dh = take(size_t(l.slices) * N * H * 4);
     l.n_chunks = (V + l.cpad - 1) / l.cpad;
-    l.off_max = take(size_t(2 + l.n_chunks) * 4);  // largest magnitudes: g, hidden, each chunk of W
+    l.off_max = take(size_t(3 + l.n_chunks) * 4);  // largest magnitudes: g, hidden, sample of W, what exceeds it in each chunk
     l.total = o;
     return l;
 }
@@ -1737,19 +1789,19 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
     uint16_t* ht = reinterpret_cast<uint16_t*>(ws + l.off_ht);    // [H, npad], row stride ld_n
     uint16_t* dzt = reinterpret_cast<uint16_t*>(ws + l.off_dzt);  // [cpad, npad], row stride ld_n
     float* dh = reinterpret_cast<float*>(ws + l.off_dh);          // [slices][N, H]
-    uint32_t* maxima = reinterpret_cast<uint32_t*>(ws + l.off_max);  // [0] g, [1] hidden, [2] W
+    uint32_t* maxima = reinterpret_cast<uint32_t*>(ws + l.off_max);  // [0] g, [1] hidden, [2] sample of W, [3 + chunk] beyond it
     const int H = int(hidden_size), N = int(n_tokens), V = int(vocab);
     const bool from_bf16 = dtype == TRLK_BF16;  // the products' operands are fp16: bf16 inputs are converted on the way
     const uint32_t* max_g = maxima;
     const uint32_t* max_h = from_bf16 ? maxima + 1 : nullptr;
-    hipLaunchKernelGGL(head_fill_kernel, dim3(unsigned((2 + l.n_chunks + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<float*>(maxima), 2 + l.n_chunks, 0.f);
+    hipLaunchKernelGGL(head_fill_kernel, dim3(unsigned((3 + l.n_chunks + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<float*>(maxima), 3 + l.n_chunks, 0.f);
     MaxAbsArgs ma{};
     ma.g = d_g_logp;
     ma.n_g = n_tokens;
     ma.blocks_g = int(N < 32 * kMaxThreads ? (N + kMaxThreads - 1) / kMaxThreads : 32);
     ma.out = maxima;
-    if (from_bf16) {  // (one scale for the whole weight: a single sweep over it instead of one per chunk)
+    if (from_bf16) {
         const auto blocks = [&](int64_t rows) {
             const int64_t b = (rows * (H / 8) + 8 * kMaxThreads - 1) / (8 * kMaxThreads);
             return int(b < kMaxBlocks ? b : kMaxBlocks);
@@ -1757,12 +1809,12 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         ma.hidden = static_cast<const uint16_t*>(d_hidden);
         ma.weight = static_cast<const uint16_t*>(d_weight);
         ma.ld_hidden = hidden_stride;
-        ma.ld_weight = weight_stride;
+        ma.ld_weight = weight_stride * kSampleRows;
         ma.n_hidden = N;
-        ma.n_weight = V;
+        ma.n_weight = (V + kSampleRows - 1) / kSampleRows;
         ma.C8 = H / 8;
         ma.blocks_h = blocks(N);
-        ma.blocks_w = blocks(V);
+        ma.blocks_w = blocks(ma.n_weight);
     }
     hipLaunchKernelGGL(head_maxabs_kernel, dim3(unsigned(ma.blocks_w + ma.blocks_h + ma.blocks_g)), dim3(kMaxThreads), 0, s, ma);
     if (from_bf16) {
@@ -1837,13 +1889,17 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         // row stride of this operand as short as that of the other three
         const uint16_t* w_chunk = static_cast<const uint16_t*>(d_weight) + c0 * weight_stride;
         const uint32_t* max_w = from_bf16 ? maxima + 2 : nullptr;
+        uint32_t* beyond_w = from_bf16 ? maxima + 3 + c0 / chunk : nullptr;
         const dim3 tgrid((H + 63) / 64, unsigned((kpad + 63) / 64));
         if (from_bf16) {
-            hipLaunchKernelGGL(transpose16_kernel<true>, tgrid, dim3(256), 0, s, w_chunk, weight_stride, rows, H, wt, l.ld_c,
-                               int64_t(kpad), max_w);
+            hipLaunchKernelGGL(transpose_weight_kernel, tgrid, dim3(256), 0, s, w_chunk, weight_stride, rows, H, wt, l.ld_c,
+                               int64_t(kpad), max_w, beyond_w);
+            const int tiles = int(tgrid.x * tgrid.y);
+            hipLaunchKernelGGL(transpose_weight_again_kernel, dim3(tiles < kAgainBlocks ? tiles : kAgainBlocks), dim3(256), 0, s,
+                               w_chunk, weight_stride, rows, H, wt, l.ld_c, int64_t(kpad), max_w, beyond_w, int(tgrid.x), tiles);
         } else {
             hipLaunchKernelGGL(transpose16_kernel<false>, tgrid, dim3(256), 0, s, w_chunk, weight_stride, rows, H, wt, l.ld_c,
-                               int64_t(kpad), max_w);
+                               int64_t(kpad), nullptr);
         }
         if (int rc2 = launch_status("fused_head_bwd (W^T)")) return rc2;
         // dHidden[N, H] += dz[N, chunk] * (W_chunk^T[H, chunk])^T
@@ -1862,6 +1918,7 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         gh.g_rows = d_g_logp;
         gh.mult_a = zs;
         gh.max_b = max_w;
+        gh.beyond_b = beyond_w;
         gh.slices = l.slices;  // (of the last, possibly shorter chunk those that its rows reach)
         while (gh.slices > 1 && int64_t(gh.slices - 1) * l.kslice >= kpad) --gh.slices;
         gh.kslice = l.kslice;
