@@ -871,3 +871,48 @@ def test_dpo_log_of_two_processes(amd):
     assert got.keys() == want.keys() and got["num_tokens"] == want["num_tokens"]
     for k, v in want.items():
         assert abs(got[k] - v) <= 1e-6 * max(1.0, abs(v)), k
+
+
+def test_native_ops_under_tracers_and_on_errors(amd):
+    """The operators registered from C++: schema, shapes, gradients under fake tensors and ahead-of-time autograd, the window as a
+    symbolic size; the exception classes of bad arguments; what carries no gradient of its own says so."""
+    from trl_amd import _lib, ops
+
+    f = lambda *s: torch.rand(s, device=DEV)  # noqa: E731
+    B, L, T, V = 2, 6, 4, 40
+    logits, ids = f(B, L, V).bfloat16(), torch.randint(0, V, (B * T, 1), device=DEV)
+    leaf = lambda t: t.clone().requires_grad_(True)  # noqa: E731
+    grpo = (f(B, T), f(B, T), f(B), torch.ones(B, T, device=DEV))
+    loss_cfg = (_lib.GRPO, 0.2, 0.2, math.nan, 0.04, False, 1.0, 1.0, 1.0, 0.1)
+    traced = ("test_schema", "test_autograd_registration", "test_faketensor", "test_aot_dispatch_dynamic")
+    for op, args in (
+        (ops.logp_entropy_fwd, (leaf(logits), ids, 0.9, 1, T, None)),
+        (ops.logp_entropy_stats_fwd, (leaf(logits), ids, 0.9, 1, T, None)),
+        (ops.grpo_loss_op, (leaf(f(B, T)), grpo[0], grpo[1], leaf(f(B, T)), *grpo[2:], None, None, None, *loss_cfg)),
+        (ops.dpo_loss_op, (leaf(f(B, T)), grpo[3], f(1), f(1), 0.1)),
+    ):
+        torch.library.opcheck(op, args, test_utils=traced)
+    logp, ent, lse = ops.logp_entropy_fwd(logits, ids, 0.9, 1, T, None)
+    fused = (logits, ids.view(B, T), 0.9, 1, T, grpo[3], grpo[2], f(B), grpo[0], None, None, None, _lib.TERM_CLIP, 0.2, 0.2,
+             math.nan, 0.0, False, 1.0, 1.05)
+    for op, args in ((ops.logp_entropy_bwd, (logits, ids, 0.9, 1, T, lse, ent, logp, None)), (ops.grpo_fused_fwd_bwd, fused),
+                     (ops._scale_unless_one, (f(4, 8), f(1)))):
+        torch.library.opcheck(op, args, test_utils=("test_schema", "test_faketensor"))
+
+    with pytest.raises(_lib.TrlkArgumentError, match="trlk status"):
+        ops.logp_entropy_fwd(logits, ids, 0.0, 1, T, None)
+    with pytest.raises(ValueError, match="contiguous"):
+        ops.logp_entropy_fwd(logits.transpose(1, 2), ids, 1.0, 0, T, None)
+    with pytest.raises(ValueError, match="rows"):
+        ops.logp_entropy_fwd(logits, ids, 1.0, 3, T, None)
+    with pytest.raises(TypeError, match="float32, bfloat16 or float16"):
+        ops.logp_entropy_fwd(logits.double(), ids, 1.0, 1, T, None)
+    with pytest.raises(ValueError, match="old_logp"):
+        ops.grpo_loss_op(f(B, T), f(B, T + 1), None, None, grpo[2], grpo[3], None, None, None, *loss_cfg)
+    with pytest.raises(NotImplementedError):
+        ops.logp_entropy_fwd(logits.cpu(), ids.cpu(), 1.0, 1, T, None)
+    x = leaf(logits)
+    (g,) = torch.autograd.grad(ops.logp_entropy_fwd(x, ids, 1.0, 1, T, None)[0].sum(), x, create_graph=True)
+    if g.requires_grad:
+        with pytest.raises(RuntimeError, match="not implemented"):
+            g.float().sum().backward()

@@ -1,6 +1,6 @@
 """MI355X-native kernels for TRL's per-token log-probability, entropy and policy-loss path.
 
-Importing the package loads `trl_amd/lib/libtrlk.so`; there is no fallback if it is missing.
+Importing the package loads `trl_amd/lib/libtrlk.so` and `libtrlk_torch.so`; there is no fallback if one is missing.
 """
 from . import _lib, ops
 from .ops import check_device_errors

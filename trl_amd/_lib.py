@@ -11,10 +11,12 @@ import ctypes
 import os
 from ctypes import c_char_p, c_double, c_float, c_int32, c_int64, c_size_t, c_void_p
 
-import torch  # noqa: F401  (loads the HIP runtime the library binds to)
+import torch  # (loads the HIP runtime the library binds to)
 
+_LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 # TRLK_LIBRARY_PATH points at another build of the same library (kernel experiments)
-LIB_PATH = os.environ.get("TRLK_LIBRARY_PATH") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libtrlk.so")
+LIB_PATH = os.environ.get("TRLK_LIBRARY_PATH") or os.path.join(_LIB_DIR, "libtrlk.so")
+TORCH_LIB_PATH = os.path.join(_LIB_DIR, "libtrlk_torch.so")
 
 F32, BF16, F16 = 0, 1, 2
 GRPO, BNPO, DR_GRPO, DAPO, LUSPO = 0, 1, 2, 3, 4
@@ -152,7 +154,7 @@ def _load():
             f"{LIB_PATH} is missing: build the HIP kernels first (python trl_amd/build.py, or "
             "make -C trl_amd/csrc). There is no fallback implementation."
         )
-    lib = ctypes.CDLL(LIB_PATH)
+    lib = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_GLOBAL)  # (libtrlk_torch.so finds the entry points in it)
     for name, (restype, argtypes) in SIGNATURES.items():
         fn = getattr(lib, name)  # AttributeError here = the built library is stale
         fn.restype = restype
@@ -165,6 +167,17 @@ def _load():
 
 
 lib = _load()
+
+
+def _load_torch_ops() -> None:
+    """Registers the operators of csrc/torch_ops.cpp with torch (they call into the library that is loaded above)."""
+    if not os.path.exists(TORCH_LIB_PATH):
+        raise ImportError(f"{TORCH_LIB_PATH} is missing: build the package first (python trl_amd/build.py, or "
+                          "make -C trl_amd/csrc). There is no fallback implementation.")
+    torch.ops.load_library(TORCH_LIB_PATH)
+
+
+_load_torch_ops()
 
 
 def last_error() -> str:

@@ -1,7 +1,8 @@
 """PyTorch custom ops over the C ABI (include/trlk.h).
 
 Each op hands raw device pointers, sizes, strides and the current HIP stream to
-libtrlk.so; torch only owns the memory.  The ops exist for device tensors only
+libtrlk.so; torch only owns the memory.  The ops of the logits-level steps, which launch many small kernels, are registered
+from C++ (csrc/torch_ops.cpp), the others here.  The ops exist for device tensors only
 (`device_types="cuda"`, which is the ROCm device in a ROCm build): there is no CPU or
 eager fallback, a CPU tensor raises.
 
@@ -23,17 +24,11 @@ from . import _lib
 from ._lib import check, current_stream, dtype_code, lib, on_device, ptr
 
 _SYNC_CHECKS = os.environ.get("TRL_AMD_SYNC_CHECKS", "0") == "1"
-_error_flags: dict[int, Tensor] = {}
 
 
 def _error_flag(device: torch.device) -> Tensor:
     """Per-device int32 word the kernels OR error bits into (see `check_device_errors`)."""
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    flag = _error_flags.get(idx)
-    if flag is None:
-        flag = torch.zeros(1, dtype=torch.int32, device=device)
-        _error_flags[idx] = flag
-    return flag
+    return torch.ops.trl_amd.error_flag.default(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def check_device_errors() -> None:
@@ -44,7 +39,7 @@ def check_device_errors() -> None:
     the device, and this function (one device->host read, i.e. a synchronisation) reports it.
     Set TRL_AMD_SYNC_CHECKS=1 to run it after every forward call.
     """
-    for flag in _error_flags.values():
+    for flag in torch.ops.trl_amd.error_flags.default():
         bits = int(flag.item())
         if bits:
             flag.zero_()
@@ -69,11 +64,27 @@ def raise_for_error_bits(bits: float, device: torch.device) -> None:
         raise RuntimeError(f"trl_amd: device error flag {bits:#x}")
 
 
-# Ops without a gradient of their own (their callers' autograd functions have it) that run several times per step: no Python
-# autograd layer around them, as `custom_op` would put there.
 _library = torch.library.Library("trl_amd", "FRAGMENT")
 
 
+def _native_op(name: str, fake, syncs: bool = False):
+    """The operator `trl_amd::<name>` that the native library registers (csrc/torch_ops.cpp), with `fake` as its shapes for
+    tracers; `syncs`: it reads token ids, and TRL_AMD_SYNC_CHECKS=1 looks at the error word behind each call."""
+    torch.library.register_fake(f"trl_amd::{name}", fake, lib=_library)
+    op = getattr(torch.ops.trl_amd, name).default
+    if not (syncs and _SYNC_CHECKS):
+        return op
+
+    def checked(*args, **kwargs):
+        out = op(*args, **kwargs)
+        check_device_errors()
+        return out
+
+    return checked
+
+
+# Ops without a gradient of their own (their callers' autograd functions have it) that run several times per step: no Python
+# autograd layer around them, as `custom_op` would put there.
 def _plain_op(schema: str, fake):
     """Registers the decorated function as `trl_amd::<schema>` for GPU tensors, `fake` as its shapes for tracers; returns
     the op."""
@@ -98,127 +109,35 @@ def _check_logits3d(logits: Tensor) -> None:
         raise ValueError("the vocabulary axis of the logits must be contiguous")
 
 
-def _run_logp_entropy_fwd(logits, index, temperature, keep_start, keep_len, row_mask, with_stats, sum_p2=True):
-    _check_logits3d(logits)
-    n_seq, _, vocab = logits.shape
-    rows = n_seq * keep_len
-    k = index.shape[-1]
-    dev = logits.device
-    logp = torch.empty((rows, k), dtype=torch.float32, device=dev)
-    ent = torch.empty((rows,), dtype=torch.float32, device=dev)
-    lse = torch.empty((rows,), dtype=torch.float32, device=dev)
-    stats = torch.empty((rows, 4), dtype=torch.float32, device=dev) if with_stats else None
-    if rows == 0:
-        return logp, ent, lse, stats
-    index = index.contiguous()
-    view = logits[:, keep_start : keep_start + keep_len]
-    with on_device(dev):
-        check(
-            lib.trlk_logp_entropy_fwd(
-                view.data_ptr(), dtype_code(logits.dtype), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
-                ptr(index), k, temperature, ptr(row_mask), ptr(logp), ptr(ent), ptr(lse), ptr(stats),
-                int(bool(sum_p2)), ptr(_error_flag(dev)), current_stream(dev),
-            )
-        )
-    if _SYNC_CHECKS:
-        check_device_errors()
-    return logp, ent, lse, stats
+def _f32_like(t: Tensor, *sizes) -> Tensor:
+    return torch.empty(sizes, dtype=torch.float32, device=t.device)
 
 
-@torch.library.custom_op("trl_amd::logp_entropy_fwd", mutates_args=(), device_types="cuda")
-def logp_entropy_fwd(
-    logits: Tensor, index: Tensor, temperature: float, keep_start: int, keep_len: int, row_mask: Optional[Tensor]
-) -> tuple[Tensor, Tensor, Tensor]:
-    """logits [n_seq, L, V] (strided view, last axis contiguous); rows keep_start..keep_start+keep_len
-    of every sequence are processed.  index int64 [n_seq*keep_len, K].  Returns fp32
-    (logp [rows, K], entropy [rows], lse [rows])."""
-    return _run_logp_entropy_fwd(logits, index, temperature, keep_start, keep_len, row_mask, False)[:3]
-
-
-@logp_entropy_fwd.register_fake
-def _(logits, index, temperature, keep_start, keep_len, row_mask):
+# logits [n_seq, L, V] (strided view, last axis contiguous); rows keep_start..keep_start+keep_len of every sequence are
+# processed.  index int64 [n_seq*keep_len, K].  Returns fp32 (logp [rows, K], entropy [rows], lse [rows]).
+def _logp_entropy_fake(logits, index, temperature, keep_start, keep_len, row_mask):
     rows = logits.shape[0] * keep_len
-    f = lambda *s: torch.empty(s, dtype=torch.float32, device=logits.device)  # noqa: E731
-    return f(rows, index.shape[-1]), f(rows), f(rows)
+    return _f32_like(logits, rows, index.shape[-1]), _f32_like(logits, rows), _f32_like(logits, rows)
 
 
-@torch.library.custom_op("trl_amd::logp_entropy_stats_fwd", mutates_args=(), device_types="cuda")
-def logp_entropy_stats_fwd(
-    logits: Tensor, index: Tensor, temperature: float, keep_start: int, keep_len: int, row_mask: Optional[Tensor],
-    sum_p2: bool = True,
-) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    """As `logp_entropy_fwd`, plus the fp32 row statistics `[rows, 4]` of the same pass: mean logit,
-    log sum_v p_v^2 (0 without `sum_p2`: the kernel is bound by its arithmetic and runs 4 % faster without that
-    sum), whether index[:, 0] is the row's arg-max (first maximal position), 0."""
-    return _run_logp_entropy_fwd(logits, index, temperature, keep_start, keep_len, row_mask, True, sum_p2)
+logp_entropy_fwd = _native_op("logp_entropy_fwd", _logp_entropy_fake, syncs=True)
 
 
-@logp_entropy_stats_fwd.register_fake
-def _(logits, index, temperature, keep_start, keep_len, row_mask, sum_p2=True):
-    rows = logits.shape[0] * keep_len
-    f = lambda *s: torch.empty(s, dtype=torch.float32, device=logits.device)  # noqa: E731
-    return f(rows, index.shape[-1]), f(rows), f(rows), f(rows, 4)
+# As `logp_entropy_fwd`, plus the fp32 row statistics `[rows, 4]` of the same pass: mean logit, log sum_v p_v^2 (0 without
+# `sum_p2`: the kernel is bound by its arithmetic and runs 4 % faster without that sum), whether index[:, 0] is the row's
+# arg-max (first maximal position), 0.
+def _logp_entropy_stats_fake(logits, index, temperature, keep_start, keep_len, row_mask, sum_p2=True):
+    return (*_logp_entropy_fake(logits, index, temperature, keep_start, keep_len, row_mask),
+            _f32_like(logits, logits.shape[0] * keep_len, 4))
 
 
-@torch.library.custom_op("trl_amd::logp_entropy_bwd", mutates_args=(), device_types="cuda")
-def logp_entropy_bwd(
-    logits: Tensor, index: Tensor, temperature: float, keep_start: int, keep_len: int, lse: Tensor,
-    entropy: Optional[Tensor], g_logp: Optional[Tensor], g_entropy: Optional[Tensor],
-) -> Tensor:
-    """d(loss)/d(logits) for the whole [n_seq, L, V] input (contiguous, same dtype): rows outside
-    the kept window and rows whose upstream gradients are all zero are zero-filled."""
-    _check_logits3d(logits)
-    n_seq, length, vocab = logits.shape
-    dlogits = torch.empty((n_seq, length, vocab), dtype=logits.dtype, device=logits.device)
-    if dlogits.numel() == 0:
-        return dlogits
-    dev = logits.device
-    view = logits[:, keep_start : keep_start + keep_len]
-    k = index.shape[-1] if g_logp is not None else 0
-    index = index.contiguous()
-    g_logp = None if g_logp is None else g_logp.contiguous().float()
-    g_entropy = None if g_entropy is None else g_entropy.contiguous().float()
-    with on_device(dev):
-        check(
-            lib.trlk_logp_entropy_bwd(
-                view.data_ptr(), dtype_code(logits.dtype), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
-                ptr(index), k, temperature, ptr(lse), ptr(entropy if g_entropy is not None else None), ptr(g_logp),
-                ptr(g_entropy), ptr(dlogits), length, keep_start, dlogits.stride(0), dlogits.stride(1),
-                current_stream(dev),
-            )
-        )
-    return dlogits
+logp_entropy_stats_fwd = _native_op("logp_entropy_stats_fwd", _logp_entropy_stats_fake, syncs=True)
 
-
-@logp_entropy_bwd.register_fake
-def _(logits, index, temperature, keep_start, keep_len, lse, entropy, g_logp, g_entropy):
-    return torch.empty(logits.shape, dtype=logits.dtype, device=logits.device)
-
-
-def _lpe_setup(ctx, inputs, output):
-    logits, index, temperature, keep_start, keep_len, row_mask = inputs[:6]
-    ctx.n_inputs = len(inputs)
-    _, ent, lse = output[:3]
-    ctx.save_for_backward(logits, index, lse, ent)
-    ctx.cfg = (temperature, keep_start, keep_len)
-    ctx.set_materialize_grads(False)
-
-
-def _lpe_backward(ctx, g_logp, g_ent, g_lse, g_stats=None):
-    logits, index, lse, ent = ctx.saved_tensors
-    temperature, keep_start, keep_len = ctx.cfg
-    # the lse output only exists to be saved for this backward; a gradient arriving there is ignored
-    rest = (None,) * (ctx.n_inputs - 1)
-    if g_logp is None and g_ent is None:
-        return (None, *rest)
-    if g_logp is None and index.shape[-1] > 0:
-        g_logp = torch.zeros(index.shape, dtype=torch.float32, device=logits.device)
-    d = logp_entropy_bwd(logits, index, temperature, keep_start, keep_len, lse, ent, g_logp, g_ent)
-    return (d, *rest)
-
-
-logp_entropy_fwd.register_autograd(_lpe_backward, setup_context=_lpe_setup)
-logp_entropy_stats_fwd.register_autograd(_lpe_backward, setup_context=_lpe_setup)
+# d(loss)/d(logits) for the whole [n_seq, L, V] input (contiguous, same dtype): rows outside the kept window and rows whose
+# upstream gradients are all zero are zero-filled.
+logp_entropy_bwd = _native_op(
+    "logp_entropy_bwd", lambda logits, index, temperature, keep_start, keep_len, lse, entropy, g_logp, g_entropy:
+    torch.empty(logits.shape, dtype=logits.dtype, device=logits.device))
 
 
 # ---- the same pair for fp64 logits: double operands, arithmetic and outputs --------------------------------
@@ -298,7 +217,15 @@ def _lpe64_backward(ctx, g_logp, g_ent, g_lse):
     return d, None, None, None, None, None
 
 
-logp_entropy_fwd_f64.register_autograd(_lpe64_backward, setup_context=_lpe_setup)
+def _lpe64_setup(ctx, inputs, output):
+    logits, index, temperature, keep_start, keep_len, _ = inputs
+    _, ent, lse = output
+    ctx.save_for_backward(logits, index, lse, ent)
+    ctx.cfg = (temperature, keep_start, keep_len)
+    ctx.set_materialize_grads(False)
+
+
+logp_entropy_fwd_f64.register_autograd(_lpe64_backward, setup_context=_lpe64_setup)
 
 
 def logp_entropy_forward(logits: Tensor, index: Tensor, temperature: float, keep_start: int, keep_len: int,
@@ -359,90 +286,16 @@ def _f32c(t: Optional[Tensor]) -> Optional[Tensor]:
     return None if t is None else t.contiguous().float()
 
 
-@torch.library.custom_op("trl_amd::grpo_loss", mutates_args=(), device_types="cuda")
-def grpo_loss_op(
-    logp: Tensor, old_logp: Optional[Tensor], ref_logp: Optional[Tensor], entropy: Optional[Tensor],
-    advantages: Tensor, mask: Tensor, token_weight: Optional[Tensor], entropy_mask: Optional[Tensor],
-    dapo_normalizer: Optional[Tensor], loss_type: int, epsilon_low: float, epsilon_high: float, delta: float,
-    beta: float, use_bias_correction_kl: bool, grad_accum_steps: float, dr_grpo_denominator: float,
-    num_processes: float, entropy_coef: float, policy_term: int = 0, sequence_level: bool = False,
-    seq_coef: Optional[Tensor] = None, sapo_temperature_pos: float = 1.0, sapo_temperature_neg: float = 1.05,
-) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    """Returns (loss [], metrics [16], d loss/d logp [B,T], d loss/d entropy [B,T])."""
-    if logp.dim() != 2:
-        raise ValueError("grpo_loss: per-token log-probs must be [B, T]")
-    B, T = logp.shape
-    dev = logp.device
-    logp, old_logp, ref_logp, entropy = _f32c(logp), _f32c(old_logp), _f32c(ref_logp), _f32c(entropy)
-    mask, token_weight, entropy_mask = _f32c(mask), _f32c(token_weight), _f32c(entropy_mask)
-    advantages = _f32c(advantages)
-    if advantages.dim() == 1 or (advantages.dim() == 2 and advantages.shape[1] == 1):
-        if advantages.numel() != B:
-            raise ValueError("grpo_loss: advantages must have one entry per sequence")
-        sb, st = 1, 0
-    elif tuple(advantages.shape) == (B, T):
-        sb, st = T, 1
-    else:
-        raise ValueError(f"grpo_loss: advantages of shape {tuple(advantages.shape)} do not match [B]={B} or [B,T]")
-    for name, t in (("old_logp", old_logp), ("ref_logp", ref_logp), ("entropy", entropy), ("mask", mask),
-                    ("token_weight", token_weight), ("entropy_mask", entropy_mask)):
-        if t is not None and tuple(t.shape) != (B, T):
-            raise ValueError(f"grpo_loss: {name} has shape {tuple(t.shape)}, expected {(B, T)}")
-    dapo_normalizer = None if dapo_normalizer is None else dapo_normalizer.reshape(1).contiguous().float()
-    if seq_coef is not None:
-        if seq_coef.numel() != B:
-            raise ValueError("grpo_loss: seq_coef must have one entry per sequence")
-        seq_coef = seq_coef.reshape(B).contiguous().float()
-    loss = torch.empty((), dtype=torch.float32, device=dev)
-    metrics = torch.empty((_lib.GRPO_NUM_METRICS,), dtype=torch.float32, device=dev)
-    dlogp = torch.empty((B, T), dtype=torch.float32, device=dev)
-    dent = torch.empty((B, T), dtype=torch.float32, device=dev) if entropy_coef != 0.0 else None
-    ws_bytes = lib.trlk_grpo_workspace_bytes(B)
-    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
-    with on_device(dev):
-        check(
-            lib.trlk_grpo_loss(
-                ptr(logp), ptr(old_logp), ptr(ref_logp), ptr(entropy), ptr(advantages), sb, st, ptr(mask),
-                ptr(token_weight), ptr(entropy_mask), ptr(seq_coef), B, T, loss_type, policy_term,
-                int(sequence_level), epsilon_low, epsilon_high, delta, beta, int(use_bias_correction_kl),
-                grad_accum_steps, dr_grpo_denominator, ptr(dapo_normalizer), num_processes, entropy_coef,
-                sapo_temperature_pos, sapo_temperature_neg, ptr(loss), ptr(metrics), ptr(dlogp), ptr(dent), ptr(ws),
-                ws_bytes, current_stream(dev),
-            )
-        )
-    if dent is None:
-        dent = torch.zeros((0,), dtype=torch.float32, device=dev)
-    return loss, metrics, dlogp, dent
+# Returns (loss [], metrics [16], d loss/d logp [B,T], d loss/d entropy [B,T]); the first carries the gradient.
+def _grpo_loss_fake(logp, old_logp, ref_logp, entropy, advantages, mask, token_weight, entropy_mask, dapo_normalizer, loss_type,
+                    epsilon_low, epsilon_high, delta, beta, use_bias_correction_kl, grad_accum_steps, dr_grpo_denominator,
+                    num_processes, entropy_coef, policy_term=0, sequence_level=False, seq_coef=None, sapo_temperature_pos=1.0,
+                    sapo_temperature_neg=1.05):
+    return (_f32_like(logp), _f32_like(logp, _lib.GRPO_NUM_METRICS), _f32_like(logp, *logp.shape),
+            _f32_like(logp, *logp.shape) if entropy_coef != 0.0 else _f32_like(logp, 0))
 
 
-@grpo_loss_op.register_fake
-def _(logp, old_logp, ref_logp, entropy, advantages, mask, token_weight, entropy_mask, dapo_normalizer, loss_type,
-      epsilon_low, epsilon_high, delta, beta, use_bias_correction_kl, grad_accum_steps, dr_grpo_denominator,
-      num_processes, entropy_coef, policy_term=0, sequence_level=False, seq_coef=None, sapo_temperature_pos=1.0,
-      sapo_temperature_neg=1.05):
-    f = lambda *s: torch.empty(s, dtype=torch.float32, device=logp.device)  # noqa: E731
-    return f(), f(_lib.GRPO_NUM_METRICS), f(*logp.shape), (f(*logp.shape) if entropy_coef != 0.0 else f(0))
-
-
-def _grpo_setup(ctx, inputs, output):
-    _, _, dlogp, dent = output
-    ctx.save_for_backward(dlogp, dent)
-    ctx.logp_dtype = inputs[0].dtype
-    ctx.has_ent_grad = inputs[18] != 0.0 and inputs[3] is not None
-    ctx.set_materialize_grads(False)
-
-
-def _grpo_backward(ctx, g_loss, g_metrics, g_dlogp, g_dent):
-    dlogp, dent = ctx.saved_tensors
-    grads = [None] * 24
-    if g_loss is not None:
-        grads[0] = (g_loss * dlogp).to(ctx.logp_dtype)
-        if ctx.has_ent_grad:
-            grads[3] = g_loss * dent
-    return tuple(grads)
-
-
-grpo_loss_op.register_autograd(_grpo_backward, setup_context=_grpo_setup)
+grpo_loss_op = _native_op("grpo_loss", _grpo_loss_fake)
 
 
 def grpo_loss_static_max_seq() -> int:
@@ -517,112 +370,39 @@ def grpo_fused_max_vocab(dtype: torch.dtype) -> int:
     return int(lib.trlk_grpo_fused_max_vocab(dtype_code(dtype))) if dtype in (torch.bfloat16, torch.float16, torch.float32) else 0
 
 
-def grpo_fused_fwd_bwd(
-    logits: Tensor, index: Tensor, temperature: float, keep_start: int, keep_len: int, mask: Tensor, advantages: Tensor,
-    row_scale: Tensor, old_logp: Optional[Tensor], ref_logp: Optional[Tensor], token_weight: Optional[Tensor],
-    seq_coef: Optional[Tensor], policy_term: int, epsilon_low: float, epsilon_high: float, delta: float, beta: float,
-    use_bias_correction_kl: bool, sapo_temperature_pos: float, sapo_temperature_neg: float,
-    compute_masked_rows: bool = False, entropy_weight: Optional[Tensor] = None,
-) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    """One pass over `logits[:, keep_start : keep_start + keep_len]` (`[B, L, V]`, bf16 / fp16 / fp32): returns
-    `(logp [B, K], entropy [B, K], lse [B, K], dlogits [B, L, V])`, the gradient for an upstream gradient of 1 on
-    the loss whose per-sequence normalisation is `row_scale [B]`.  Rows with `mask == 0` are not read (outputs 0)
-    unless `compute_masked_rows`.  `entropy_weight [B, K]` is d loss / d entropy per token (entropy bonus)."""
-    _check_logits3d(logits)
-    n_seq, length, vocab = logits.shape
-    dev = logits.device
-    if tuple(index.shape) != (n_seq, keep_len) or tuple(mask.shape) != (n_seq, keep_len):
-        raise ValueError(f"grpo_fused: index and mask must be [{n_seq}, {keep_len}]")
-    index = index.contiguous()
-    if index.dtype != torch.int64:
-        index = index.long()
-    mask, old_logp, ref_logp, token_weight = _f32c(mask), _f32c(old_logp), _f32c(ref_logp), _f32c(token_weight)
-    entropy_weight = _f32c(entropy_weight)
-    for name, t in (("old_logp", old_logp), ("ref_logp", ref_logp), ("token_weight", token_weight),
-                    ("entropy_weight", entropy_weight)):
-        if t is not None and tuple(t.shape) != (n_seq, keep_len):
-            raise ValueError(f"grpo_fused: {name} has shape {tuple(t.shape)}, expected {(n_seq, keep_len)}")
-    advantages = _f32c(advantages)
-    if advantages.dim() == 1 or (advantages.dim() == 2 and advantages.shape[1] == 1):
-        if advantages.numel() != n_seq:
-            raise ValueError("grpo_fused: advantages must have one entry per sequence")
-        sb, st = 1, 0
-    elif tuple(advantages.shape) == (n_seq, keep_len):
-        sb, st = keep_len, 1
-    else:
-        raise ValueError(f"grpo_fused: advantages of shape {tuple(advantages.shape)} do not match [B] or [B, K]")
-    row_scale = row_scale.reshape(n_seq).contiguous().float()
-    seq_coef = None if seq_coef is None else seq_coef.reshape(n_seq).contiguous().float()
-    logp = torch.empty((n_seq, keep_len), dtype=torch.float32, device=dev)
-    ent = torch.empty_like(logp)
-    lse = torch.empty_like(logp)
-    dlogits = torch.empty((n_seq, length, vocab), dtype=logits.dtype, device=dev)
-    if dlogits.numel() == 0:
-        return logp, ent, lse, dlogits
-    view = logits[:, keep_start : keep_start + keep_len]
-    with on_device(dev):
-        check(
-            lib.trlk_grpo_fused_fwd_bwd(
-                view.data_ptr(), dtype_code(logits.dtype), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
-                ptr(index), temperature, ptr(old_logp), ptr(ref_logp), ptr(advantages), sb, st, ptr(mask),
-                ptr(token_weight), ptr(seq_coef), ptr(row_scale), ptr(entropy_weight), policy_term, epsilon_low, epsilon_high, delta, beta,
-                int(use_bias_correction_kl), sapo_temperature_pos, sapo_temperature_neg, ptr(logp), ptr(ent), ptr(lse),
-                ptr(dlogits), length, keep_start, dlogits.stride(0), dlogits.stride(1), int(compute_masked_rows),
-                ptr(_error_flag(dev)), current_stream(dev),
-            )
-        )
-    if _SYNC_CHECKS:
-        check_device_errors()
-    return logp, ent, lse, dlogits
+# One pass over `logits[:, keep_start : keep_start + keep_len]` (`[B, L, V]`, bf16 / fp16 / fp32): returns
+# `(logp [B, K], entropy [B, K], lse [B, K], dlogits [B, L, V])`, the gradient for an upstream gradient of 1 on the loss whose
+# per-sequence normalisation is `row_scale [B]`.  Rows with `mask == 0` are not read (outputs 0) unless
+# `compute_masked_rows`.  `entropy_weight [B, K]` is d loss / d entropy per token (entropy bonus).
+def _grpo_fused_fake(logits, index, temperature, keep_start, keep_len, *args, **kwargs):
+    tokens = (logits.shape[0], keep_len)
+    return (_f32_like(logits, *tokens), _f32_like(logits, *tokens), _f32_like(logits, *tokens),
+            torch.empty(logits.shape, dtype=logits.dtype, device=logits.device))
+
+
+grpo_fused_fwd_bwd = _native_op("grpo_fused", _grpo_fused_fake, syncs=True)
+
+_scale_unless_one = _native_op("scale_unless_one_", lambda data, scale: None)
 
 
 def scale_unless_one_(data: Tensor, scale: Tensor) -> Tensor:
     """In place `data *= scale` for a contiguous bf16 / fp16 / fp32 tensor and a one-element device scalar; when the
     scalar is exactly 1 the launched kernel touches nothing (no host synchronisation either way)."""
-    if not data.is_contiguous() or data.dtype not in (torch.bfloat16, torch.float16, torch.float32):
-        raise ValueError("scale_unless_one_: contiguous bf16 / fp16 / fp32 data expected")
-    scale = scale.reshape(1).to(device=data.device, dtype=torch.float32)
-    with on_device(data.device):
-        check(lib.trlk_scale_unless_one(data.data_ptr(), dtype_code(data.dtype), data.numel(), ptr(scale),
-                                        current_stream(data.device)))
+    _scale_unless_one(data, scale)
     return data
 
 
 # --------------------------------------------------------------------------------------------
 # DPO / RLOO sequence losses (K4)
 # --------------------------------------------------------------------------------------------
-@_plain_op("grpo_log_values(Tensor metrics) -> Tensor",
-           lambda metrics: metrics.new_empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32))
-def grpo_log_values(metrics):
-    """What `_compute_loss` logs of the loss kernel's `metrics`, as one fp32 device vector (`trlk_grpo_log_values`): nine
-    sums to be added over the processes, the smallest and the largest clip ratio, the policy loss, the error word."""
-    dev = metrics.device
-    out = torch.empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32, device=dev)
-    with on_device(dev):
-        check(lib.trlk_grpo_log_values(ptr(metrics), ptr(_error_flag(dev)), ptr(out), current_stream(dev)))
-    return out
+# What `_compute_loss` logs of the loss kernel's `metrics`, as one fp32 device vector (`trlk_grpo_log_values`): nine sums to be
+# added over the processes, the smallest and the largest clip ratio, the policy loss, the error word.
+grpo_log_values = _native_op("grpo_log_values",
+                             lambda metrics: metrics.new_empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32))
 
-
-@torch.library.custom_op("trl_amd::grpo_row_scale", mutates_args=(), device_types="cuda")
-def _grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Optional[Tensor], upstream: Optional[Tensor],
-                    with_mask: bool) -> tuple[Tensor, Tensor]:
-    B, T = mask.shape
-    dev = mask.device
-    if any(t is not None and t.device != dev for t in (n_items, upstream)):
-        raise ValueError("grpo_row_scale: the mask and the scalars must be on one GPU")
-    mask_f = torch.empty((B, T) if with_mask else (0,), dtype=torch.float32, device=dev)
-    scale = torch.empty((B,), dtype=torch.float32, device=dev)
-    with on_device(dev):
-        check(lib.trlk_grpo_row_scale(ptr(mask), _KEEP_TYPES[mask.dtype], B, T, mask.stride(0), mask.stride(1), loss_type,
-                                      numerator, ptr(n_items), ptr(upstream), ptr(mask_f) if with_mask else None, ptr(scale),
-                                      current_stream(dev)))
-    return mask_f, scale
-
-
-@_grpo_row_scale.register_fake
-def _(mask, loss_type, numerator, n_items, upstream, with_mask):
-    f = lambda *s: torch.empty(s, dtype=torch.float32, device=mask.device)  # noqa: E731
-    return (f(*mask.shape) if with_mask else f(0)), f(mask.shape[0])
+_grpo_row_scale = _native_op(
+    "grpo_row_scale", lambda mask, loss_type, numerator, n_items, upstream, with_mask:
+    (_f32_like(mask, *mask.shape) if with_mask else _f32_like(mask, 0), _f32_like(mask, mask.shape[0])))
 
 
 def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Optional[Tensor] = None,
@@ -636,84 +416,17 @@ def grpo_row_scale(mask: Tensor, loss_type: int, numerator: float, n_items: Opti
     return (mask if as_is else mask_f), scale
 
 
-@torch.library.custom_op("trl_amd::dpo_log_values", mutates_args=(), device_types="cuda")
-def dpo_log_values(entropy: Tensor, row_stats: Tensor, mask: Tensor, seq_logps: Tensor, ref_chosen: Tensor,
-                   ref_rejected: Tensor, beta: float) -> Tensor:
-    """What a DPO step logs, as one fp32 device vector `[8 + 4 P]` (`trlk_dpo_log_values`): `entropy`, `mask` `[2P, T]`,
-    `row_stats` `[2P, T, 4]`, `seq_logps` `[2P]`, the reference's log-probs `[P]` or broadcast to it."""
-    B, T = mask.shape
-    P, dev = B // 2, mask.device
-    if B % 2 or entropy.numel() != B * T or row_stats.numel() != 4 * B * T or seq_logps.numel() != B:
-        raise ValueError("dpo_log_values: the shapes do not match")
-    entropy, row_stats, mask, seq_logps = _f32c(entropy), _f32c(row_stats), _f32c(mask), _f32c(seq_logps)
-    ref_chosen, ref_rejected = _f32c(ref_chosen.expand(P)), _f32c(ref_rejected.expand(P))
-    out = torch.empty((8 + 2 * B,), dtype=torch.float32, device=dev)
-    if B == 0:
-        return out.zero_()
-    ws = torch.empty((4 * B,), dtype=torch.float32, device=dev)
-    with on_device(dev):
-        check(lib.trlk_dpo_log_values(ptr(entropy), ptr(row_stats), ptr(mask), B, T, ptr(seq_logps), ptr(ref_chosen),
-                                      ptr(ref_rejected), beta, ptr(_error_flag(dev)), ptr(out), ptr(ws),
-                                      current_stream(dev)))
-    return out
+# What a DPO step logs, as one fp32 device vector `[8 + 4 P]` (`trlk_dpo_log_values`): `entropy`, `mask` `[2P, T]`, `row_stats`
+# `[2P, T, 4]`, `seq_logps` `[2P]`, the reference's log-probs `[P]` or broadcast to it.
+dpo_log_values = _native_op(
+    "dpo_log_values", lambda entropy, row_stats, mask, seq_logps, ref_chosen, ref_rejected, beta:
+    _f32_like(mask, 8 + 2 * mask.shape[0]))
 
-
-@dpo_log_values.register_fake
-def _(entropy, row_stats, mask, seq_logps, ref_chosen, ref_rejected, beta):
-    return torch.empty((8 + 2 * mask.shape[0],), dtype=torch.float32, device=mask.device)
-
-
-@torch.library.custom_op("trl_amd::dpo_loss", mutates_args=(), device_types="cuda")
-def dpo_loss_op(token_logp: Tensor, mask: Tensor, ref_chosen: Tensor, ref_rejected: Tensor, beta: float
-                ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    """Returns (loss [], seq_logps [B], metrics [8], d loss/d token_logp [B,T])."""
-    if token_logp.dim() != 2:
-        raise ValueError("dpo_loss: per-token log-probs must be [B, T]")
-    B, T = token_logp.shape
-    if B % 2 or B < 2:
-        raise ValueError("dpo_loss: the batch must be [chosen; rejected], i.e. an even number of sequences")
-    dev = token_logp.device
-    token_logp, mask = _f32c(token_logp), _f32c(mask)
-    ref_chosen, ref_rejected = _f32c(ref_chosen), _f32c(ref_rejected)
-    if tuple(mask.shape) != (B, T) or ref_chosen.numel() != B // 2 or ref_rejected.numel() != B // 2:
-        raise ValueError("dpo_loss: mask must be [B, T] and the reference log-probs [B/2] each")
-    loss = torch.empty((), dtype=torch.float32, device=dev)
-    seq = torch.empty((B,), dtype=torch.float32, device=dev)
-    metrics = torch.empty((_lib.DPO_NUM_METRICS,), dtype=torch.float32, device=dev)
-    dlogp = torch.empty((B, T), dtype=torch.float32, device=dev)
-    with on_device(dev):
-        check(lib.trlk_dpo_loss(ptr(token_logp), ptr(mask), ptr(ref_chosen), ptr(ref_rejected), B, T, beta, ptr(seq),
-                                ptr(loss), ptr(metrics), ptr(dlogp), current_stream(dev)))
-    return loss, seq, metrics, dlogp
-
-
-@dpo_loss_op.register_fake
-def _(token_logp, mask, ref_chosen, ref_rejected, beta):
-    f = lambda *s: torch.empty(s, dtype=torch.float32, device=token_logp.device)  # noqa: E731
-    return f(), f(token_logp.shape[0]), f(_lib.DPO_NUM_METRICS), f(*token_logp.shape)
-
-
-def _seq_setup(ctx, inputs, output):
-    ctx.save_for_backward(output[3], inputs[1])
-    ctx.n_inputs = len(inputs)
-    ctx.logp_dtype = inputs[0].dtype
-    ctx.indicator = True
-    ctx.set_materialize_grads(False)
-
-
-def _seq_backward(ctx, g_loss, g_seq, g_metrics, g_dlogp):
-    dlogp, mask = ctx.saved_tensors
-    g = None
-    if g_loss is not None:
-        g = g_loss * dlogp
-    if g_seq is not None:
-        w = (mask != 0).float() if ctx.indicator else mask.float()
-        extra = g_seq.unsqueeze(1) * w
-        g = extra if g is None else g + extra
-    return (None if g is None else g.to(ctx.logp_dtype),) + (None,) * (ctx.n_inputs - 1)
-
-
-dpo_loss_op.register_autograd(_seq_backward, setup_context=_seq_setup)
+# Returns (loss [], seq_logps [B], metrics [8], d loss/d token_logp [B,T]); the first two carry the gradient.
+dpo_loss_op = _native_op(
+    "dpo_loss", lambda token_logp, mask, ref_chosen, ref_rejected, beta:
+    (_f32_like(token_logp), _f32_like(token_logp, token_logp.shape[0]), _f32_like(token_logp, _lib.DPO_NUM_METRICS),
+     _f32_like(token_logp, *token_logp.shape)))
 
 
 @torch.library.custom_op("trl_amd::rloo_loss", mutates_args=(), device_types="cuda")
@@ -745,11 +458,24 @@ def _(token_logp, mask, old_seq_logps, advantages, epsilon_low, epsilon_high):
 
 
 def _rloo_setup(ctx, inputs, output):
-    _seq_setup(ctx, inputs, output)
-    ctx.indicator = False
+    ctx.save_for_backward(output[3], inputs[1])
+    ctx.n_inputs = len(inputs)
+    ctx.logp_dtype = inputs[0].dtype
+    ctx.set_materialize_grads(False)
 
 
-rloo_loss_op.register_autograd(_seq_backward, setup_context=_rloo_setup)
+def _rloo_backward(ctx, g_loss, g_seq, g_metrics, g_dlogp):
+    dlogp, mask = ctx.saved_tensors
+    g = None
+    if g_loss is not None:
+        g = g_loss * dlogp
+    if g_seq is not None:
+        extra = g_seq.unsqueeze(1) * mask.float()
+        g = extra if g is None else g + extra
+    return (None if g is None else g.to(ctx.logp_dtype),) + (None,) * (ctx.n_inputs - 1)
+
+
+rloo_loss_op.register_autograd(_rloo_backward, setup_context=_rloo_setup)
 
 
 
