@@ -1,4 +1,5 @@
 """Shared pytest configuration: the `gpu` marker, repo root on sys.path, golden loader."""
+import gc
 import json
 import os
 import sys
@@ -17,6 +18,19 @@ GOLDEN_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+
+
+@pytest.fixture(autouse=True)
+def _no_collection_between_memory_readings(request):
+    """Tests that compare two readings of the allocator: what earlier tests left in reference cycles is collected before
+    them, and not between the readings."""
+    if request.module.__name__ != "test_zz_no_alloc":
+        yield
+        return
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()
 
 
 def load_golden(stem):
