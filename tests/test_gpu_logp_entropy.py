@@ -521,3 +521,34 @@ def test_rows_walked_from_their_first_line(amd, dtype, vocab):
         assert bool(((got.cpu().double() - w).abs() <= bound).all())
         assert _rel_l2(got, w) < (1e-5 if dtype == torch.float32 else 2.0**-8)
     amd.check_device_errors()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("groups,rest", [(0, 1), (0, -1), (1, 0), (1, 1), (1, -1), (2, 0), (2, 255), (2, -1), (3, 5)])
+def test_rows_around_whole_groups_of_loads(dtype, groups, rest):
+    """Rows of a whole number of the forward's load groups (256 lanes x 6 vectors), one entry more or less and far into the next
+    group, aligned and not, with statistics and without: log-prob, entropy, mean and arg-max against float64."""
+    import trl_amd
+    from trl_amd import ops
+
+    per_group = 256 * 6 * (4 if dtype == torch.float32 else 8)
+    V = groups * per_group + (rest if rest >= 0 else per_group + rest)
+    g = torch.Generator().manual_seed(V)
+    x = (2.0 * torch.randn(5, V + 3, generator=g)).to(dtype)
+    ids = torch.randint(0, V, (5, 1), generator=g)
+    for cut in (0, 3):  # (the second view starts at another alignment)
+        rows = x[:, cut : cut + V]
+        z = rows.double() / 0.9
+        lse = z.logsumexp(1)
+        lp = z.gather(1, ids)[:, 0] - lse
+        ent = lse - ((z - lse[:, None]).exp() * z).sum(1)
+        dev = x.to("cuda:0")[None][:, :, cut : cut + V]
+        got = ops.logp_entropy_fwd(dev, ids.to("cuda:0"), 0.9, 0, 5, None)
+        stats = ops.logp_entropy_stats_fwd(dev, ids.to("cuda:0"), 0.9, 0, 5, None)
+        assert all(torch.equal(a, b) for a, b in zip(got, stats[:3]))
+        # sums of V terms in fp32, pairwise across lanes: a few 1e-6 of values of about 10
+        torch.testing.assert_close(got[0][:, 0].double().cpu(), lp, rtol=0, atol=2e-5)
+        torch.testing.assert_close(got[1].double().cpu(), ent, rtol=0, atol=5e-5)
+        torch.testing.assert_close(stats[3][:, 0].double().cpu(), rows.double().mean(1), rtol=0, atol=1e-5)
+        assert torch.equal(stats[3][:, 2].cpu() == 1, rows.argmax(1) == ids[:, 0])
+    trl_amd.check_device_errors()

@@ -1,7 +1,7 @@
 // K1 / K3: streaming log-prob + entropy forward and its recompute backward.
 //
 // One workgroup owns one row (token position).  The row is streamed once with 16-byte
-// non-temporal loads, `UNR` loads in flight per lane; every lane keeps an online
+// non-temporal loads in groups of `UN` per lane, the next group in flight while one is summed; every lane keeps an online
 // (reference exponent r, sum 2^(x*c-r), sum 2^(x*c-r)*x) triple in fp32 and the triples are merged
 // across the workgroup through wave shuffles and LDS.  The temperature is folded into the
 // exponent multiplier (c = log2(e)/T), so no scaled copy of the row ever exists.
@@ -12,13 +12,13 @@ namespace trlk {
 namespace {
 
 // Tuning knobs (overridable with -D for experiments; the defaults are the measured best on the
-// [65536, 151936] bf16 workload).  Forward: 4 non-temporal 16-byte loads in flight per lane.
+// [65536, 151936] bf16 workload).  Forward: groups of 6 non-temporal 16-byte loads per lane, two groups in flight.
 // Backward: 8 KiB chunks (2 loads per lane), plain loads, non-temporal stores.
 #ifndef TRLK_THREADS
 #define TRLK_THREADS 256
 #endif
 #ifndef TRLK_FWD_UNROLL
-#define TRLK_FWD_UNROLL 4
+#define TRLK_FWD_UNROLL 6
 #endif
 #ifndef TRLK_BWD_UNROLL
 #define TRLK_BWD_UNROLL 2
@@ -34,7 +34,7 @@ namespace {
 #endif
 constexpr int kThreads = TRLK_THREADS;
 constexpr int kUnroll = TRLK_FWD_UNROLL;
-static_assert(kUnroll >= 2, "the row tail of the forward holds up to kUnroll - 1 vectors per lane");
+constexpr int kStatsUnroll = 4;  // (with statistics, whose tail costs more: 16384 rows of 32000 bf16 184 us against 193 with groups of 6)
 constexpr int kBwdUnroll = TRLK_BWD_UNROLL;
 
 // A 16-byte vector at any element alignment: rows whose length is no multiple of the vector width start at 2- or
@@ -146,10 +146,9 @@ __device__ __forceinline__ float max_of(const float* x) {
 // STATS: 1 or 2 also produce the row statistics of `out_stats`; only 2 accumulates the sum of squared probabilities
 // (one more multiply-add per logit in a loop that is bound by its arithmetic: 5.14 against 4.95 ms on 33.6 GB of bf16
 // logits), 1 reports 0 in its place.
-// TH lanes per row, UN 16-byte loads in flight per lane.
-template <int DT, bool VEC, int STATS, int TH = kThreads, int UN = kUnroll>
+// TH lanes per row, groups of UN 16-byte loads per lane.
+template <int DT, bool VEC, int STATS, int TH = kThreads, int UN = (STATS ? kStatsUnroll : kUnroll)>
 __global__ __launch_bounds__(TH) void logp_entropy_fwd_kernel(FwdArgs a) {
-    static_assert(UN >= 2, "the row tail holds up to UN - 1 vectors per lane");
     typedef Elem<DT> E;
     typedef typename E::type T;
     constexpr int NW = TH / kWave;
@@ -241,11 +240,24 @@ __global__ __launch_bounds__(TH) void logp_entropy_fwd_kernel(FwdArgs a) {
         }
         const u32x4* vp = reinterpret_cast<const u32x4*>(base + head);
         const int nvec = int((V - head) / EPV);
-        int v = tid;
-        for (; v + (UN - 1) * TH < nvec; v += UN * TH) {
-            u32x4 q[UN];
+        // Groups of UN vectors per lane, the next group's loads (or the row's tail's) in flight while one is summed.  A launch
+        // of few rows is bound by the chain of memory round trips along a row, a larger one by the memory.  Groups of 4
+        // loaded and summed in turn / groups of 4 with the next in flight / of 6, in us: 64 rows of 32000 bf16 9.2 / 6.5 / 6.3,
+        // of 151936 27 / 15 / 13, of 151936 fp32 45 / 25 / 20; 300 rows of 50257 fp32 17.6 / 15.2 / 14.9; 2048 rows of 32000
+        // fp32 46.3 / 44.7 / 43.3, of 151936 bf16 104 / 104 / 100; 8192 rows of 151936 bf16 383 / 381 / 382 (groups of 8: fp32
+        // 20 % behind on a single round of workgroups).  (The tail's loads go out together: one after the other
+        // they would cost a round trip each, at the end of every row.)
+        const int groups = nvec / (UN * TH);
+        auto fetch = [&](int g, u32x4(&q)[UN]) {
 #pragma unroll
-            for (int j = 0; j < UN; ++j) q[j] = stream_load<kFwdNt>(vp + v + j * TH);
+            for (int j = 0; j < UN; ++j) q[j] = stream_load<kFwdNt>(vp + (g * UN + j) * TH + tid);
+        };
+        auto fetch_tail = [&](u32x4(&q)[UN]) {
+#pragma unroll
+            for (int j = 0; j < UN; ++j)
+                if ((groups * UN + j) * TH + tid < nvec) q[j] = stream_load<kFwdNt>(vp + (groups * UN + j) * TH + tid);
+        };
+        auto sum_group = [&](int g, const u32x4(&q)[UN]) {
             if constexpr (STATS) {
 #pragma unroll
                 for (int j = 0; j < UN; ++j) stat_sum(q[j]);
@@ -264,29 +276,36 @@ __global__ __launch_bounds__(TH) void logp_entropy_fwd_kernel(FwdArgs a) {
                     st.vmax = bm;
                     int first = UN * EPV - 1;
                     for (int i = UN * EPV - 2; i >= 0; --i) first = x[i] == bm ? i : first;
-                    st.vpos = float(head + int64_t(v + (first / EPV) * TH) * EPV + first % EPV);
+                    st.vpos = float(head + int64_t((g * UN + first / EPV) * TH + tid) * EPV + first % EPV);
                 }
             }
+        };
+        u32x4 q[UN], next[UN];
+        if (groups > 0) {
+            fetch(0, q);
+            for (int g = 0; g + 1 < groups; ++g) {
+                fetch(g + 1, next);
+                sum_group(g, q);
+#pragma unroll
+                for (int j = 0; j < UN; ++j) q[j] = next[j];
+            }
+            fetch_tail(next);
+            sum_group(groups - 1, q);
+        } else {
+            fetch_tail(next);
         }
-        // the row's tail: fewer than UN vectors are left for this lane; their loads go out together
-        // (one after the other they would cost a memory round trip each, at the end of every row)
-        {
-            u32x4 q[UN - 1];
 #pragma unroll
-            for (int j = 0; j < UN - 1; ++j)
-                if (v + j * TH < nvec) q[j] = stream_load<kFwdNt>(vp + v + j * TH);
+        for (int j = 0; j < UN; ++j) {
+            const int v = (groups * UN + j) * TH + tid;
+            if (v < nvec) {
+                if constexpr (STATS) stat_sum(next[j]);
+                float x[EPV];
+                E::unpack(next[j], x);
+                const float bm = max_of<EPV>(x);
+                raise(bm);
 #pragma unroll
-            for (int j = 0; j < UN - 1; ++j) {
-                if (v + j * TH < nvec) {
-                    if constexpr (STATS) stat_sum(q[j]);
-                    float x[EPV];
-                    E::unpack(q[j], x);
-                    const float bm = max_of<EPV>(x);
-                    raise(bm);
-#pragma unroll
-                    for (int i = 0; i < EPV; ++i) add(x[i]);
-                    if constexpr (STATS) stat_vec(x, head + int64_t(v + j * TH) * EPV, EPV, bm);
-                }
+                for (int i = 0; i < EPV; ++i) add(x[i]);
+                if constexpr (STATS) stat_vec(x, head + int64_t(v) * EPV, EPV, bm);
             }
         }
         if constexpr (!VEC) {  // what is left of the row after its whole vectors (these positions come last for a lane)
@@ -545,7 +564,7 @@ int check_view(const char* what, const void* p, int dtype, int64_t n_seq, int64_
                  "%s: unsupported dtype code %d", what, dtype);
     TRLK_REQUIRE(n_seq >= 0 && rows_per_seq >= 0, TRLK_ERR_BAD_SHAPE, "%s: negative row count", what);
     TRLK_REQUIRE(vocab >= 1, TRLK_ERR_BAD_SHAPE, "%s: vocab must be >= 1 (got %lld)", what, (long long)vocab);
-    TRLK_REQUIRE(vocab < (int64_t(1) << 31) - 16 * kThreads * kUnroll, TRLK_ERR_BAD_SHAPE,
+    TRLK_REQUIRE(vocab < (int64_t(1) << 31) - 64 * kThreads, TRLK_ERR_BAD_SHAPE,
                  "%s: vocab %lld too large", what, (long long)vocab);
     TRLK_REQUIRE(n_seq * rows_per_seq < (int64_t(1) << 31), TRLK_ERR_BAD_SHAPE, "%s: too many rows (%lld)", what,
                  (long long)(n_seq * rows_per_seq));
