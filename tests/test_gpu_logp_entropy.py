@@ -526,12 +526,12 @@ def test_rows_walked_from_their_first_line(amd, dtype, vocab):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("groups,rest", [(0, 1), (0, -1), (1, 0), (1, 1), (1, -1), (2, 0), (2, 255), (2, -1), (3, 5)])
 def test_rows_around_whole_groups_of_loads(dtype, groups, rest):
-    """Rows of a whole number of the forward's load groups (256 lanes x 6 vectors), one entry more or less and far into the next
+    """Rows of a whole number of the forward's load groups (256 lanes x 4 vectors), one entry more or less and far into the next
     group, aligned and not, with statistics and without: log-prob, entropy, mean and arg-max against float64."""
     import trl_amd
     from trl_amd import ops
 
-    per_group = 256 * 6 * (4 if dtype == torch.float32 else 8)
+    per_group = 256 * 4 * (4 if dtype == torch.float32 else 8)
     V = groups * per_group + (rest if rest >= 0 else per_group + rest)
     g = torch.Generator().manual_seed(V)
     x = (2.0 * torch.randn(5, V + 3, generator=g)).to(dtype)

@@ -12,13 +12,13 @@ namespace trlk {
 namespace {
 
 // Tuning knobs (overridable with -D for experiments; the defaults are the measured best on the
-// [65536, 151936] bf16 workload).  Forward: groups of 6 non-temporal 16-byte loads per lane, two groups in flight.
+// [65536, 151936] bf16 workload).  Forward: groups of 4 non-temporal 16-byte loads per lane, two groups in flight.
 // Backward: 8 KiB chunks (2 loads per lane), plain loads, non-temporal stores.
 #ifndef TRLK_THREADS
 #define TRLK_THREADS 256
 #endif
 #ifndef TRLK_FWD_UNROLL
-#define TRLK_FWD_UNROLL 6
+#define TRLK_FWD_UNROLL 4
 #endif
 #ifndef TRLK_BWD_UNROLL
 #define TRLK_BWD_UNROLL 2
@@ -34,7 +34,6 @@ namespace {
 #endif
 constexpr int kThreads = TRLK_THREADS;
 constexpr int kUnroll = TRLK_FWD_UNROLL;
-constexpr int kStatsUnroll = 4;  // (with statistics, whose tail costs more: 16384 rows of 32000 bf16 184 us against 193 with groups of 6)
 constexpr int kBwdUnroll = TRLK_BWD_UNROLL;
 
 // A 16-byte vector at any element alignment: rows whose length is no multiple of the vector width start at 2- or
@@ -147,7 +146,7 @@ __device__ __forceinline__ float max_of(const float* x) {
 // (one more multiply-add per logit in a loop that is bound by its arithmetic: 5.14 against 4.95 ms on 33.6 GB of bf16
 // logits), 1 reports 0 in its place.
 // TH lanes per row, groups of UN 16-byte loads per lane.
-template <int DT, bool VEC, int STATS, int TH = kThreads, int UN = (STATS ? kStatsUnroll : kUnroll)>
+template <int DT, bool VEC, int STATS, int TH = kThreads, int UN = kUnroll>
 __global__ __launch_bounds__(TH) void logp_entropy_fwd_kernel(FwdArgs a) {
     typedef Elem<DT> E;
     typedef typename E::type T;
@@ -242,11 +241,12 @@ __global__ __launch_bounds__(TH) void logp_entropy_fwd_kernel(FwdArgs a) {
         const int nvec = int((V - head) / EPV);
         // Groups of UN vectors per lane, the next group's loads (or the row's tail's) in flight while one is summed.  A launch
         // of few rows is bound by the chain of memory round trips along a row, a larger one by the memory.  Groups of 4
-        // loaded and summed in turn / groups of 4 with the next in flight / of 6, in us: 64 rows of 32000 bf16 9.2 / 6.5 / 6.3,
-        // of 151936 27 / 15 / 13, of 151936 fp32 45 / 25 / 20; 300 rows of 50257 fp32 17.6 / 15.2 / 14.9; 2048 rows of 32000
-        // fp32 46.3 / 44.7 / 43.3, of 151936 bf16 104 / 104 / 100; 8192 rows of 151936 bf16 383 / 381 / 382 (groups of 8: fp32
-        // 20 % behind on a single round of workgroups).  (The tail's loads go out together: one after the other
-        // they would cost a round trip each, at the end of every row.)
+        // loaded and summed in turn -> with the next in flight, in us: 64 rows of 32000 bf16 9.2 -> 6.5, of 151936 27 -> 15, of
+        // 151936 fp32 45 -> 25; 300 rows of 50257 fp32 17.6 -> 15.2; 2048 rows of 32000 fp32 46.3 -> 44.7; 8192 rows of 151936
+        // bf16 383 -> 381.  Groups of 6 are 1 to 3 % ahead of that without statistics, but behind with them on short rows (16384
+        // rows of 32000 bf16 193 us against 184), and both must sum a row in one order: log-probs with and without
+        // statistics are equal to the last bit.  (The tail's loads go out together: one after the other they would cost a
+        // round trip each, at the end of every row.)
         const int groups = nvec / (UN * TH);
         auto fetch = [&](int g, u32x4(&q)[UN]) {
 #pragma unroll
