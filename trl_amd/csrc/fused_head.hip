@@ -1,16 +1,16 @@
 // K5 / K6: lm_head fused with the log-prob / entropy reduction (forward) and its backward.
 //
-// All contractions run on the matrix cores (v_mfma_f32_16x16x32_{bf16,f16}, fp32 accumulate)
-// through ONE "NT" tile loop: C[256 x 256] += A[256 x K] * B[256 x K]^T with both operands
+// All contractions run on the matrix cores (v_mfma_f32_16x16x32_{bf16,f16}, in the forward 32x32x16, fp32 accumulate) as
+// "NT" tiles: C[256 x 256] += A[256 x K] * B[256 x K]^T with both operands
 // row-major and K contiguous, which is the layout the MFMA A/B fragments want (a lane holds 8
 // consecutive k of one row), so fragments come straight out of LDS with 16-byte reads and nothing
 // is ever transposed on the fly.  512 threads = 8 waves, 2 along M x 4 along N; a wave owns 128 x 64 of
-// the tile = 8 x 4 MFMA blocks = 128 accumulator registers per lane.  Tiles go from memory
+// the tile = 8 x 4 (4 x 2) MFMA blocks = 128 accumulator registers per lane.  Tiles go from memory
 // straight into two LDS stages (global_load_lds_dwordx4) when K is a multiple of the k step,
 // through registers otherwise.
 //
 // Forward (K5): the tile is computed TRANSPOSED -- M = vocabulary rows of W, N = tokens -- so that
-// a lane of the accumulator layout holds 4 vocabulary entries of ONE token per block.  The online
+// a lane of the accumulator layout holds 16 vocabulary entries of ONE token per block.  The online
 // log-sum-exp state of a token therefore lives in the lane's own registers and the per-tile
 // epilogue needs no cross-lane traffic; a workgroup keeps 256 tokens and walks over its share of
 // the vocabulary tiles, the logits exist only as accumulators.
@@ -38,6 +38,7 @@ constexpr int kHeadThreads = WGM * WGN * 64;
 #define TRLK_HEAD_KERNEL __global__ __launch_bounds__(kHeadThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 constexpr int WM = BM / WGM, WN = BN / WGN;  // per-wave tile
 constexpr int MI = WM / 16, NI = WN / 16;    // MFMA blocks of it
+constexpr int MB = WM / 32, NB = WN / 32;    // ... in the forward
 constexpr int kLdsRow = BK + 8;  // register-staged loop: elements per LDS row (16 bytes of padding keep 16-byte reads conflict-free)
 constexpr int kCpr = BK / 8;                        // 16-byte chunks per tile row
 constexpr int kRowStep = kHeadThreads / kCpr;       // rows staged per pass of the workgroup
@@ -49,16 +50,22 @@ constexpr int kDenseA = BM * kRowBytes, kDenseStage = (BM + BN) * kRowBytes;
 constexpr int kDzLdsRow = BN * 2 + 16;     // bytes per vocabulary row of the dz tile staged in LDS by the backward
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 constexpr int kHeadLdsBytes = cmax(cmax(2 * kStageBytes, 2 * kDenseStage), BM * kDzLdsRow);
-static_assert(4 * WGM * BN * 4 * 4 <= kHeadLdsBytes && BN <= kHeadThreads, "merge scratch");
+static_assert(2 * WGM * BN * 4 * 4 <= kHeadLdsBytes && BN <= kHeadThreads, "merge scratch");
 static_assert(BM % kRowStep == 0 && BN % kRowStep == 0, "tile shape");
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // The 16x16x32 shape reads and writes half as many accumulators per multiply-add as 32x32x16 does.  The part is limited by
 // power under matrix load, so that shows as speed: a bare loop of MFMAs on random bf16 operands runs at 2020-2060 TFLOP/s
 // (2.05-2.12 GHz) against 1830-1880 TFLOP/s (1.87-1.90 GHz), on zeros both at 2450-2490 TFLOP/s (2.4 GHz).
+// The forward uses 32x32x16.  Its loop has registers for two sets of fragments there (nothing of the softmax state is
+// spilled) and takes, against the same loop as the products', 272 for 286 us with 1396 tokens, H = 2048, V = 50257 and
+// 302 for 330 us with 879 tokens, H = 1024, V = 151665; 8345 for 8240 us with 9664 tokens, H = 3584, V = 151936, where
+// power decides, is the other side.  And the log-probs of peaked rows hang on the last bits of the logits' sums: what a
+// run has stored of its old or its reference policy stays what it computes again.
 template <int DT>
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
     if constexpr (DT == TRLK_BF16)
@@ -78,6 +85,16 @@ __device__ __forceinline__ int fresh(int x) {
 
 // A value that is the same in every lane, in a scalar register.
 __device__ __forceinline__ float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+
+template <int DT>
+__device__ __forceinline__ f32x16 mfma_fwd(u32x4 a, u32x4 b, f32x16 c) {
+    if constexpr (DT == TRLK_BF16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                       0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+                                                      0, 0);
+}
 
 // Where a wave sits in the tile.  A SIMD runs waves w and w + 4: they differ in their columns (N) by half the tile, so
 // that a tile of at most 128 columns leaves every SIMD one wave with work, not two of them both.
@@ -215,11 +232,9 @@ __device__ __forceinline__ void move_tiles_only(const DirectLoader<BKM>& loader,
     }
 }
 
-// `prefetched`: the caller has already run DirectLoader::prologue for this tile (and nothing has
-// touched the LDS since).
 template <int DT, bool BKM = false>
 __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, const Operand B, int n0, int K,
-                                                    f32x4 (&acc)[MI][NI], char* smem, bool prefetched) {
+                                                    f32x4 (&acc)[MI][NI], char* smem) {
     const DirectLoader<BKM> loader(A, m0, B, n0, smem);
     constexpr int kStageLoads = DirectLoader<BKM>::kStageLoads;
     const int lane = threadIdx.x & 63, wave = loader.wave;
@@ -257,7 +272,7 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
     };
 
     const int nk = K / BK;
-    if (!prefetched) loader.prologue(K);
+    loader.prologue(K);
     loader.first_stage_landed(nk);
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -275,9 +290,10 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
     // the last fragments of the stage, read at the end of the first slice, have arrived.  The stage's refill follows
     // it, one transfer every other MFMA, and has until the same place of the next step to land.
     //
-    // Bound by power (clock 1.5-1.7 GHz) and the arrival of the tiles.  Whole steps, forward and both products, against
-    // the loop on 32x32x16 MFMAs with two sets of fragments: 9664 tokens, H = 3584, V = 151936 28.3 -> 26.8 ms; 1396 tokens,
-    // H = 2048, V = 50257 1128 -> 1054 us; forward alone of 459 tokens, H = 3584, V = 151936 532 -> 520 us.
+    // Bound by power (clock 1.5-1.7 GHz) and the arrival of the tiles.  Forward and backward, of which the two products are
+    // two thirds, against products on 32x32x16 MFMAs with two sets of fragments and the tile order of that time: 9664
+    // tokens, H = 3584, V = 151936 27.7 -> 26.4 ms; 1396 tokens, H = 2048, V = 50257 1115 -> 1020 us; 459 tokens, H = 3584,
+    // V = 151936 2554 -> 2300 us.
     constexpr int kBarAt = 4;
     static_assert(NI == 4 && 2 * kStageLoads <= 2 * (MI - kBarAt) + 2 * MI, "the refill fits behind the barrier");
     u32x4 a[MI], b[NI];
@@ -344,14 +360,12 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
     // every LDS read of this tile completed before the last barrier: the caller may reuse the LDS right away
 }
 
-// acc[i][j] = sum_k A[m0 + .., k] * B[n0 + .., k].  Rows beyond the operand's end are clamped to
+// The register-staged tile, sum_k A[m0 + .., k] * B[n0 + .., k].  Rows beyond the operand's end are clamped to
 // its last row (callers ignore those outputs); k beyond K reads as zero (K % 8 == 0).
-template <int DT>
-__device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, const Operand B, int n0, int K,
-                                             f32x4 (&acc)[MI][NI], char* smem) {
+// `compute(sa, sb)` multiplies one stage (rows of kLdsRow elements).
+template <typename Compute>
+__device__ __forceinline__ void staged_tile(const Operand A, int m0, const Operand B, int n0, int K, char* smem, Compute compute) {
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave_m(wave), wn = wave_n(wave);
     const int kc = tid % kCpr, r0 = tid / kCpr;  // this thread stages rows r0 + kRowStep*j, 16-byte chunk kc
 
     // uniform tile base + 32-bit per-lane byte offsets (a tile spans < 4 GiB)
@@ -371,13 +385,6 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
         bo[j] = uint32_t((int64_t(rb) * B.ld + kc * 8) * 2);
     }
     const int st_off = (r0 * kLdsRow + kc * 8) * 2;        // + j * kRowStep rows
-    const int fa_off = ((wm * WM + (lane & 15)) * kLdsRow + (lane >> 4) * 8) * 2;  // + i * 16 rows, + ks * 32
-    const int fb_off = ((wn * WN + (lane & 15)) * kLdsRow + (lane >> 4) * 8) * 2;
-
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const u32x4 zero = {0u, 0u, 0u, 0u};
     // full k steps load unconditionally; only the last, partial step (K % BK != 0) masks its chunks
@@ -405,9 +412,35 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
 #pragma unroll
         for (int j = 0; j < kLoadsB; ++j) *reinterpret_cast<u32x4*>(sb + st_off + j * kRowStep * kLdsRow * 2) = rb[j];
     };
-    auto compute = [&](int buf) {
-        const char* sa = smem + buf * kStageBytes;
-        const char* sb = sa + kTileABytes;
+    // Registers hold the tile of step kt+1 while step kt computes out of LDS; it is written to the
+    // other LDS buffer at the end of the step (one barrier per step).
+    const int nk = (K + BK - 1) / BK;
+    u32x4 ra[kLoadsA], rb[kLoadsB];
+    load_stage(ra, rb, 0);
+    store_stage(ra, rb, 0);
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+        const bool more = kt + 1 < nk;
+        if (more) load_stage(ra, rb, (kt + 1) * BK);
+        compute(smem + (kt & 1) * kStageBytes, smem + (kt & 1) * kStageBytes + kTileABytes);
+        if (more) store_stage(ra, rb, (kt + 1) & 1);
+        __syncthreads();
+    }
+}
+
+template <int DT>
+__device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, const Operand B, int n0, int K,
+                                                    f32x4 (&acc)[MI][NI], char* smem) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave_m(wave), wn = wave_n(wave);
+    const int fa_off = ((wm * WM + (lane & 15)) * kLdsRow + (lane >> 4) * 8) * 2;  // + i * 16 rows, + ks * 32
+    const int fb_off = ((wn * WN + (lane & 15)) * kLdsRow + (lane >> 4) * 8) * 2;
+
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    staged_tile(A, m0, B, n0, K, smem, [&](const char* sa, const char* sb) {
 #pragma unroll
         for (int ks = 0; ks < BK / 32; ++ks) {
             u32x4 fa[MI], fb[NI];
@@ -420,32 +453,177 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
 #pragma unroll
                 for (int j = 0; j < NI; ++j) acc[i][j] = mfma<DT>(fa[i], fb[j], acc[i][j]);
         }
+    });
+}
+
+// The forward's tile loop: 32x32x16 MFMAs (a fragment is 32 rows x 16 k), the logits' sums in that shape's order.  The caller
+// has run DirectLoader::prologue.
+template <int DT>
+__device__ __forceinline__ void fwd_tile_direct(const Operand A, int m0, const Operand B, int n0, int K, f32x16 (&acc)[MB][NB],
+                                                char* smem) {
+    const DirectLoader<> loader(A, m0, B, n0, smem);
+    const int lane = threadIdx.x & 63, wave = loader.wave;
+    const int wm = wave_m(wave), wn = wave_n(wave);
+
+    // --- fragment side (tile rows of a wave start at multiples of 32, so the swizzle depends on the lane only)
+    const int swz = tile_swizzle(lane & 31);
+    const int hl = lane >> 5;
+    const int fa_row = (wm * WM + (lane & 31)) * kRowBytes, fb_row = (wn * WN + (lane & 31)) * kRowBytes;
+    constexpr int KS = BK / 16;
+    int koff[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) koff[ks] = ((ks * 2 + hl) ^ swz) * 16;
+    auto read_a = [&](const char* sa, int mb, int ks) -> u32x4 {
+        return *reinterpret_cast<const u32x4*>(sa + fa_row + mb * 32 * kRowBytes + koff[ks]);
     };
 
-    // Registers hold the tile of step kt+1 while step kt computes out of LDS; it is written to the
-    // other LDS buffer at the end of the step (one barrier per step).
-    const int nk = (K + BK - 1) / BK;
-    u32x4 ra[kLoadsA], rb[kLoadsB];
-    load_stage(ra, rb, 0);
-    store_stage(ra, rb, 0);
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-        const bool more = kt + 1 < nk;
-        if (more) load_stage(ra, rb, (kt + 1) * BK);
-        compute(kt & 1);
-        if (more) store_stage(ra, rb, (kt + 1) & 1);
-        __syncthreads();
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
+
+    // Software pipeline.  Fragment loads run one 16-wide k slice ahead of the MFMAs that consume them,
+    // across the barrier too: the last slice of a stage is already in registers when the workgroup
+    // synchronises, so its MFMAs cover the refill of the freed stage and the first fragment reads of
+    // the next one.
+    constexpr int kStageLoads = DirectLoader<>::kStageLoads;
+    auto load_frags = [&](int buf, int ks, u32x4(&fa)[MB], u32x4(&fb)[NB]) {
+        const char* sa = smem + buf * kDenseStage;
+        const char* sb = sa + kDenseA;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) fa[mb] = read_a(sa, mb, ks);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+            fb[nb] = *reinterpret_cast<const u32x4*>(sb + fb_row + nb * 32 * kRowBytes + koff[ks]);
+    };
+    u32x4 fa[2][MB], fb[2][NB];
+    static_assert(KS % 2 == 0 && MB * NB > MB + NB, "pipeline shape");
+    constexpr std::true_type T{};
+    constexpr std::false_type F{};
+    const int nk = K / BK;
+    loader.first_stage_landed(nk);
+    constexpr int kLoadsPost = (kStageLoads + 1) / 2, kLoadsPre = kStageLoads - kLoadsPost;
+    load_frags(0, 0, fa[0], fb[0]);
+    // Exact issue order, pinned instruction by instruction (sched_barrier(0) between the groups):
+    // MFMA i of the slice, then at most one fragment read of the next slice and at most one tile
+    // transfer.  Fragments are read in the order the mb-major MFMA sequence needs them (fa0, fb*,
+    // fa1, ...), so every read has most of a slice between its issue and its first use.  The refill
+    // of a stage is split: the first half of its transfers goes behind the barrier that frees it, the
+    // second half into the first slice of the following step.
+    constexpr int M = MB * NB, R = MB + NB;
+    auto slice = [&](u32x4(&ca)[MB], u32x4(&cb)[NB], auto read_tag, int rbuf, int rks, u32x4(&na)[MB], u32x4(&nb_)[NB],
+                     auto nload_tag, int lbuf, int lk0, int lfirst) {
+        constexpr bool READ = decltype(read_tag)::value;
+        constexpr int NL = decltype(nload_tag)::value;
+        const char* sa = smem + rbuf * kDenseStage;
+        const char* sb = sa + kDenseA;
+        int issued = 0;
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+            const int mb = i / NB, nb = i % NB;
+            acc[mb][nb] = mfma_fwd<DT>(ca[mb], cb[nb], acc[mb][nb]);
+            if (READ && i < R) {
+                // read order: fa[0], fb[0..NB-1], fa[1..MB-1]
+                if (i == 0)
+                    na[0] = read_a(sa, 0, rks);
+                else if (i <= NB)
+                    nb_[i - 1] = *reinterpret_cast<const u32x4*>(sb + fb_row + (i - 1) * 32 * kRowBytes + koff[rks]);
+                else
+                    na[i - NB] = read_a(sa, i - NB, rks);
+            }
+            if (NL > 0 && (i + 1) * NL / M > i * NL / M) {
+                loader.issue_one(lbuf, lk0, lfirst + issued);
+                ++issued;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    typedef std::integral_constant<int, kLoadsPost> post_t;
+    typedef std::integral_constant<int, kLoadsPre> pre_t;
+    typedef std::integral_constant<int, 0> zero_t;
+    // POST / PRE: this step issues the first half of the refill of the stage it frees / the second
+    // half of the refill the previous step started.  NEXT: another step follows.
+    auto step = [&](int kt, auto post_tag, auto pre_tag, auto next_tag) {
+        constexpr bool POST = decltype(post_tag)::value, PRE = decltype(pre_tag)::value, NEXT = decltype(next_tag)::value;
+        const int cur = kt & 1, nxt = cur ^ 1;
+#pragma unroll
+        for (int ks = 0; ks + 1 < KS; ++ks) {
+            if (PRE && ks == 0)
+                slice(fa[ks & 1], fb[ks & 1], T, cur, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1], pre_t{}, nxt,
+                      (kt + 1) * BK, kLoadsPost);
+            else
+                slice(fa[ks & 1], fb[ks & 1], T, cur, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1], zero_t{}, 0, 0, 0);
+        }
+        // every fragment read of this stage has returned and the next stage has landed
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        // A bare s_barrier: __syncthreads() carries release/acquire fences, for which the compiler
+        // adds waits of its own.  The waits above are the ones this exchange needs; nothing may move across the barrier.
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        constexpr int L = (KS - 1) & 1;
+        if constexpr (NEXT && POST)
+            slice(fa[L], fb[L], T, nxt, 0, fa[0], fb[0], post_t{}, cur, (kt + 2) * BK, 0);
+        else if constexpr (NEXT)
+            slice(fa[L], fb[L], T, nxt, 0, fa[0], fb[0], zero_t{}, 0, 0, 0);
+        else
+            slice(fa[L], fb[L], F, 0, 0, fa[0], fb[0], zero_t{}, 0, 0, 0);
+    };
+    static_assert(((KS - 1) & 1) == 1, "the last slice of a stage sits in fragment buffer 1, the next stage's first in 0");
+    int kt = 0;
+    if (nk > 2) {
+        step(kt++, T, F, T);
+        for (; kt + 2 < nk; ++kt) step(kt, T, T, T);
+        step(kt++, F, T, T);  // kt = nk - 2: completes the last refill
+    } else if (nk == 2) {
+        step(kt++, F, F, T);
     }
+    for (; kt + 1 < nk; ++kt) step(kt, F, F, T);  // (no step is left; without the loop a register is spilled in the one above)
+    step(kt, F, F, F);
+    // every LDS read of this tile completed before the last barrier: the caller may reuse the LDS right away
+}
+
+template <int DT>
+__device__ __forceinline__ void fwd_tile_staged(const Operand A, int m0, const Operand B, int n0, int K, f32x16 (&acc)[MB][NB],
+                                                char* smem) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int fa_off = ((wave_m(wave) * WM + (lane & 31)) * kLdsRow + (lane >> 5) * 8) * 2;  // + mb * 32 rows, + ks * 16
+    const int fb_off = ((wave_n(wave) * WN + (lane & 31)) * kLdsRow + (lane >> 5) * 8) * 2;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
+    staged_tile(A, m0, B, n0, K, smem, [&](const char* sa, const char* sb) {
+#pragma unroll
+        for (int ks = 0; ks < BK / 16; ++ks) {
+            u32x4 fa[MB], fb[NB];
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                fa[mb] = *reinterpret_cast<const u32x4*>(sa + fa_off + (mb * 32 * kLdsRow + ks * 16) * 2);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                fb[nb] = *reinterpret_cast<const u32x4*>(sb + fb_off + (nb * 32 * kLdsRow + ks * 16) * 2);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mfma_fwd<DT>(fa[mb], fb[nb], acc[mb][nb]);
+        }
+    });
 }
 
 template <int DT, bool BKM = false>
 __device__ __forceinline__ void gemm_tile_nt(const Operand A, int m0, const Operand B, int n0, int K,
-                                             f32x4 (&acc)[MI][NI], char* smem, bool prefetched = false) {
+                                             f32x4 (&acc)[MI][NI], char* smem) {
     if constexpr (BKM) {  // (callers of this form pad K to whole steps)
-        gemm_tile_nt_direct<DT, true>(A, m0, B, n0, K, acc, smem, prefetched);
+        gemm_tile_nt_direct<DT, true>(A, m0, B, n0, K, acc, smem);
     } else {
         if ((K & (BK - 1)) == 0)
-            gemm_tile_nt_direct<DT>(A, m0, B, n0, K, acc, smem, prefetched);
+            gemm_tile_nt_direct<DT>(A, m0, B, n0, K, acc, smem);
         else
             gemm_tile_nt_staged<DT>(A, m0, B, n0, K, acc, smem);
     }
@@ -455,6 +633,11 @@ __device__ __forceinline__ void gemm_tile_nt(const Operand A, int m0, const Oper
 __device__ __forceinline__ int acc_row(int wm, int i, int r, int lane) { return wm * WM + i * 16 + (lane >> 4) * 4 + r; }
 // Column (N index) inside the workgroup tile of block j, for this lane.
 __device__ __forceinline__ int acc_col(int wn, int j, int lane) { return wn * WN + j * 16 + (lane & 15); }
+// The same in the forward: element r of block mb, block nb.
+__device__ __forceinline__ int fwd_row(int wm, int mb, int r, int lane) {
+    return wm * WM + mb * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+}
+__device__ __forceinline__ int fwd_col(int wn, int nb, int lane) { return wn * WN + nb * 32 + (lane & 31); }
 
 // Workgroup id -> (tile along axis `a`, tile along axis `b`) such that the workgroups that run
 // together on one XCD (ids congruent mod 8, dispatched round-robin) form patches of about 4 x 8 tiles: they share
@@ -630,18 +813,18 @@ TRLK_HEAD_KERNEL void fused_head_fwd_kernel(HeadArgs a) {
     const int vt0 = vs * a.tiles_per_split;
     const int vt1 = vt0 + a.tiles_per_split < n_vt ? vt0 + a.tiles_per_split : n_vt;
 
-    // per-lane online state of the NI tokens this lane owns (base-2, integer reference exponent)
-    float ref[NI], S[NI], U[NI], zmax[NI];
-    int tg[NI];
+    // per-lane online state of the NB tokens this lane owns (base-2, integer reference exponent)
+    float ref[NB], S[NB], U[NB], zmax[NB];
+    int tg[NB];
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-        ref[j] = -INFINITY;
-        zmax[j] = -INFINITY;
-        S[j] = 0.f;
-        U[j] = 0.f;
-        const int tok = n0 + acc_col(wn, j, tid & 63);
+    for (int nb = 0; nb < NB; ++nb) {
+        ref[nb] = -INFINITY;
+        zmax[nb] = -INFINITY;
+        S[nb] = 0.f;
+        U[nb] = 0.f;
+        const int tok = n0 + fwd_col(wn, nb, tid & 63);
         const int64_t t = tok < a.N ? a.targets[tok] : -1;
-        tg[j] = t >= 0 && t < a.V ? int(t) : -1;
+        tg[nb] = t >= 0 && t < a.V ? int(t) : -1;
     }
     const Operand W{a.weight, a.ldw, a.V}, Hd{a.hidden, a.ldh, a.N};
 
@@ -658,21 +841,22 @@ TRLK_HEAD_KERNEL void fused_head_fwd_kernel(HeadArgs a) {
     }
     for (int vt = vt0; vt < vt1 && !idle; ++vt) {
         const int m0 = vt * BM;
-        f32x4 acc[MI][NI];
+        f32x16 acc[MB][NB];
         if constexpr (STAGED) {
-            gemm_tile_nt_staged<DT>(W, m0, Hd, n0, a.H, acc, smem);
+            fwd_tile_staged<DT>(W, m0, Hd, n0, a.H, acc, smem);
         } else {
-            gemm_tile_nt_direct<DT>(W, m0, Hd, n0, a.H, acc, smem, true);
+            fwd_tile_direct<DT>(W, m0, Hd, n0, a.H, acc, smem);
             // What of the state did not fit beside the accumulators and fragments comes back from scratch here: behind the
-            // transfers below each reload would wait for them to land (5 of a tile's 96 us at H = 3584).
+            // transfers below each reload would wait for them to land.
 #pragma unroll
-            for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(ref[j]), "+v"(S[j]), "+v"(U[j]), "+v"(zmax[j]), "+v"(tg[j]));
+            for (int nb = 0; nb < NB; ++nb)
+                asm volatile("" : "+v"(ref[nb]), "+v"(S[nb]), "+v"(U[nb]), "+v"(zmax[nb]), "+v"(tg[nb]));
             // the next tile's first stages travel while this tile's logits are reduced (registers only)
             if (vt + 1 < vt1) DirectLoader<>(W, m0 + BM, Hd, n0, smem).prologue(a.H);
         }
-        const int lane = fresh(tid & 63), g = lane >> 4, l15 = lane & 15;
-        // Stash: for one accumulator quad (4 consecutive vocabulary rows of one token per lane) the 16 lanes of a
-        // group hold 16 consecutive tokens = 128 contiguous bytes per store.  The buffer is padded to whole tiles.
+        const int lane = fresh(tid & 63), half = lane >> 5;
+        // Stash: for one accumulator quad (4 consecutive vocabulary rows of one token per lane) the 32 lanes of a
+        // half-wave hold 32 consecutive tokens = 256 contiguous bytes per store.  The buffer is padded to whole tiles.
         // Addresses are a uniform pointer that walks down the quads (scalar registers, one addition per store) plus
         // the lane's byte offset (one vector register; the entry point bounds ld so that it fits 32 bits).
         char* stash_blk = nullptr;
@@ -682,50 +866,50 @@ TRLK_HEAD_KERNEL void fused_head_fwd_kernel(HeadArgs a) {
             const int col = n0 + wn * WN;
             stash_blk = reinterpret_cast<char*>(a.stash.quads() + int64_t(m0 / 4 + wm * (WM / 4)) * a.stash.ld + col);
             ref_blk = a.stash.refs() + int64_t(m0 / 128 + wm) * 2 * a.stash.ld + col;
-            ref_lane = uint32_t(g & 1) * uint32_t(a.stash.ld) + uint32_t(l15);
-            stash_lane = (uint32_t(g) * uint32_t(a.stash.ld) + uint32_t(l15)) * 8u;
+            ref_lane = uint32_t(half) * uint32_t(a.stash.ld) + uint32_t(lane & 31);
+            stash_lane = ref_lane * 8u;
         }
         const bool partial_tile = m0 + BM > a.V;
         constexpr bool plain = !GENERAL;
         // Before the reduction, only where needed (a bias, the general form of z, or the vocabulary's last tile, whose
         // rows beyond the vocabulary count as -inf): the accumulators become y + bias (usual head) or z itself
-        // (general form).  A lane's 4 accumulators of a block are consecutive vocabulary rows, so the bias
-        // comes as one 16-byte load per block row, four of them issued before the first is used.
+        // (general form).  A lane's 16 accumulators of a block are 4 quads of consecutive vocabulary rows, so the bias
+        // comes as one 16-byte load per quad, all of a block row's loads issued before the first is used.
         if (GENERAL || a.bias != nullptr || partial_tile) {
             const float inv_cap = a.softcap > 0.f ? 1.f / a.softcap : 0.f;
             typedef float f32x4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
 #pragma unroll
-            for (int i0 = 0; i0 < MI; i0 += 4) {
+            for (int mb = 0; mb < MB; ++mb) {
                 f32x4 bq[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int v0 = m0 + acc_row(wm, i0 + q, 0, lane);
+                    const int v0 = m0 + fwd_row(wm, mb, q * 4, lane);
                     bq[q] = f32x4{0.f, 0.f, 0.f, 0.f};
                     if (a.bias != nullptr) {
                         if (v0 + 3 < a.V) {
                             bq[q] = *reinterpret_cast<const f32x4_dword_aligned*>(a.bias + v0);
                         } else {
 #pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                if (v0 + r < a.V) bq[q][r] = a.bias[v0 + r];
+                            for (int i = 0; i < 4; ++i)
+                                if (v0 + i < a.V) bq[q][i] = a.bias[v0 + i];
                         }
                     }
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int v0 = m0 + acc_row(wm, i0 + q, 0, lane);
+                    const int v0 = m0 + fwd_row(wm, mb, q * 4, lane);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const bool beyond = partial_tile && v0 + r >= a.V;
+                    for (int i = 0; i < 4; ++i) {
+                        const bool beyond = partial_tile && v0 + i >= a.V;
 #pragma unroll
-                        for (int j = 0; j < NI; ++j) {
-                            float y = acc[i0 + q][j][r] + bq[q][r];
+                        for (int nb = 0; nb < NB; ++nb) {
+                            float y = acc[mb][nb][q * 4 + i] + bq[q][i];
                             if constexpr (GENERAL) {
                                 y *= a.logit_scale;
                                 if (a.softcap > 0.f) y = head_tanh(y * inv_cap) * a.softcap;
                                 y *= a.inv_t;
                             }
-                            acc[i0 + q][j][r] = beyond ? -INFINITY : y;
+                            acc[mb][nb][q * 4 + i] = beyond ? -INFINITY : y;
                         }
                     }
                 }
@@ -734,96 +918,96 @@ TRLK_HEAD_KERNEL void fused_head_fwd_kernel(HeadArgs a) {
         // (With a stash the numerators are stored as they are produced.  Packed into registers and stored in one run
         // at the end of the epilogue they cost more: 28.6 against 27.8 ms for the benchmark's forward.)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
+        for (int nb = 0; nb < NB; ++nb) {
             float bm = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
+            for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) bm = fmaxf(bm, acc[i][j][r]);
+                for (int r = 0; r < 16; ++r) bm = fmaxf(bm, acc[mb][nb][r]);
             if constexpr (plain) bm *= zs;
             // target logit: rarely inside this wave's 128 vocabulary rows.  It is selected into one register
             // and stored once: a conditional store per accumulator held the wave for about 20 us, and a
             // workgroup that falls behind the others no longer finds the tiles they share in the L2.
-            const int rel = tg[j] - (m0 + wm * WM);
-            if (tg[j] >= 0 && rel >= 0 && rel < WM) {
-                const int want = rel - g * 4;  // acc_row() without this lane's group offset
+            const int rel = tg[nb] - (m0 + wm * WM);
+            if (tg[nb] >= 0 && rel >= 0 && rel < WM) {
+                const int want = rel - half * 4;  // fwd_row() without this lane's half-wave offset
                 float tv = 0.f;
                 bool mine = false;
 #pragma unroll
-                for (int i = 0; i < MI; ++i)
+                for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const bool m = i * 16 + r == want;
-                        tv = m ? acc[i][j][r] : tv;
+                    for (int r = 0; r < 16; ++r) {
+                        const bool m = (mb * 32 + (r >> 2) * 8 + (r & 3)) == want;
+                        tv = m ? acc[mb][nb][r] : tv;
                         mine |= m;
                     }
-                if (mine) a.tgt[n0 + acc_col(wn, j, lane)] = plain ? tv * zs : tv;
+                if (mine) a.tgt[n0 + fwd_col(wn, nb, lane)] = plain ? tv * zs : tv;
             }
-            zmax[j] = fmaxf(zmax[j], bm);
-            // lanes l and l + 32 hold row quads of the same parity: they share a reference exponent (see StashView)
-            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(bm), __float_as_uint(bm), false, false);
-            const float need = ceilf(fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])) * kLog2e);
-            if (need > ref[j]) {
-                const float sc = fast_exp2(ref[j] - need);
-                S[j] *= sc;
-                U[j] *= sc;
-                ref[j] = need;
+            zmax[nb] = fmaxf(zmax[nb], bm);
+            const float need = ceilf(bm * kLog2e);
+            if (need > ref[nb]) {
+                const float sc = fast_exp2(ref[nb] - need);
+                S[nb] *= sc;
+                U[nb] *= sc;
+                ref[nb] = need;
             }
-            const float rr = ref[j] == -INFINITY ? 0.f : ref[j];
+            const float rr = ref[nb] == -INFINITY ? 0.f : ref[nb];
             // numerators times 2^15 (exact; S and U carry the factor until they are written out), with or without a
             // stash: the outputs must not depend on stashing
-            int64_t stash_off = j * 16 * 8;  // byte offset of this token block's column of quads (uniform)
-            if constexpr (STASH) ref_blk[j * 16 + ref_lane] = rr;
+            int64_t stash_off = nb * 32 * 8;  // byte offset of this token block's column of quads (uniform)
+            if constexpr (STASH) ref_blk[nb * 32 + ref_lane] = rr;
             const float rsub = rr - kStashExp;
             float s = 0.f, u = 0.f;
             auto sum_tile = [&](auto guard_tag) {
                 constexpr bool kGuard = decltype(guard_tag)::value;  // -inf among the logits (0 * -inf in sum(e * y))
                 const float mul = plain ? zs2 : kLog2e;  // general path: the accumulators hold z itself by now
 #pragma unroll
-                for (int i = 0; i < MI; ++i) {
-                    float e[4];
+                for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float y = acc[i][j][r];
-                        e[r] = fast_exp2(fmaf(y, mul, -rsub));
-                        s += e[r];
-                        u = (kGuard && y == -INFINITY) ? u : fmaf(e[r], y, u);
+                    for (int q = 0; q < 4; ++q) {
+                        float e[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float y = acc[mb][nb][q * 4 + i];
+                            e[i] = fast_exp2(fmaf(y, mul, -rsub));
+                            s += e[i];
+                            u = (kGuard && y == -INFINITY) ? u : fmaf(e[i], y, u);
+                        }
+                        if constexpr (STASH) {
+                            uint2 w;
+                            w.x = Elem<TRLK_F16>::pack2(e[0], e[1]);
+                            w.y = Elem<TRLK_F16>::pack2(e[2], e[3]);
+                            *reinterpret_cast<uint2*>(stash_blk + stash_off + stash_lane) = w;
+                            stash_off += a.stash.ld * 16;  // two quads down: the other parity is the other half-wave's
+                            // (one running offset, not 16 precomputed ones; an offset, because a pointer that
+                            // passed through here would no longer be known to point to global memory)
+                            asm volatile("" : "+s"(stash_off));
+                        }
                     }
-                    if constexpr (STASH) {
-                        uint2 w;
-                        w.x = Elem<TRLK_F16>::pack2(e[0], e[1]);
-                        w.y = Elem<TRLK_F16>::pack2(e[2], e[3]);
-                        *reinterpret_cast<uint2*>(stash_blk + stash_off + stash_lane) = w;
-                        stash_off += a.stash.ld * 32;  // four quads down: those between are the other lane groups'
-                        // (one running offset, not 8 precomputed ones; an offset, because a pointer that
-                        // passed through here would no longer be known to point to global memory)
-                        asm volatile("" : "+s"(stash_off));
-                    }
-                }
             };
             if (GENERAL || partial_tile)
                 sum_tile(std::true_type{});
             else
                 sum_tile(std::false_type{});
             if constexpr (plain) u *= zs;
-            S[j] += s;
-            U[j] += u;
+            S[nb] += s;
+            U[nb] += u;
         }
     }
 
-    // merge the partial states of every token (4 lane groups x WGM M-waves) through LDS
-    const int lane = tid & 63, g = lane >> 4;
-    constexpr int kParts = 4 * WGM;
+    // merge the partial states of every token (2 lane halves x WGM M-waves) through LDS
+    const int lane = tid & 63;
+    constexpr int kParts = 2 * WGM;
     float* sm = reinterpret_cast<float*>(smem);  // [kParts][BN tokens][4]
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-        const int col = acc_col(wn, j, lane);
-        const int part = wm * 4 + g;
+    for (int nb = 0; nb < NB; ++nb) {
+        const int col = fwd_col(wn, nb, lane);
+        const int part = wm * 2 + (lane >> 5);
         // (copies of their own: joined to a 16-byte store's registers, the state would be kept as vectors through the whole
         // tile loop, and spilled)
         float r, z;
-        asm volatile("v_mov_b32 %0, %2\n\tv_mov_b32 %1, %3" : "=&v"(r), "=v"(z) : "v"(ref[j]), "v"(zmax[j]));
-        *reinterpret_cast<f32x4*>(sm + (part * BN + col) * 4) = f32x4{r, S[j] * 0x1p-15f, U[j] * 0x1p-15f, z};
+        asm volatile("v_mov_b32 %0, %2\n\tv_mov_b32 %1, %3" : "=&v"(r), "=v"(z) : "v"(ref[nb]), "v"(zmax[nb]));
+        *reinterpret_cast<f32x4*>(sm + (part * BN + col) * 4) = f32x4{r, S[nb] * 0x1p-15f, U[nb] * 0x1p-15f, z};
     }
     __syncthreads();
     if (tid < BN && n0 + tid < a.N) {
