@@ -5,6 +5,8 @@ fp32 autograd on the same bf16-valued operands.
 Tolerances: the reference's own bf16 test uses 1e-2 (tests/test_utils.py:1212-1232).  Against
 fp32 op-math on the same stored values: log-probs / entropies 2e-3 abs; gradients 1e-2 relative L2 against the
 unrounded fp32 result, and 1.5e-3 (bf16) / 5e-4 (fp16) against that result rounded to the output dtype."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -928,3 +930,66 @@ def test_weight_scale_from_a_sample(amd, monkeypatch, kind, stash):
         assert not dh.any()
         rdh = dh.float()
     _check_beyond_output_rounding(dh, dw, rdh, rdw, torch.bfloat16)
+
+
+def _cancelling_operands(n, v, h, dtype, seed):
+    """hidden [n, h], weight [v, h] whose products make partial sums of some thousands that cancel to exactly 0 in the first h - n
+    columns; in the last n, column h - n + i belongs to token i and to row `targets[i]` alone and adds 14 to their logit."""
+    half = (h - n) // 2
+    g = torch.Generator().manual_seed(seed)
+    w_half = (torch.randn(v, half, generator=g) * torch.exp(torch.randn(v, half, generator=g))).to(dtype)
+    x_half = (8.0 * torch.randn(n, half, generator=g) * torch.exp(torch.randn(1, half, generator=g))).to(dtype)
+    targets = torch.randperm(v, generator=g)[:n]
+    own = torch.zeros(v, n, dtype=dtype)
+    own[targets, torch.arange(n)] = 8.0
+    rest = (h - n) % 2
+    weight = torch.cat([w_half, w_half, torch.zeros(v, rest, dtype=dtype), own], 1)
+    hidden = torch.cat([x_half, -x_half, torch.zeros(n, rest, dtype=dtype), torch.diag(torch.full((n,), 14.0 / 8.0)).to(dtype)], 1)
+    return hidden, weight, targets, 1.0 + torch.rand(n, generator=g)
+
+
+@pytest.mark.parametrize("h", [2048, 1096])  # (a multiple of the k step, and not)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_both_matrix_instructions_sum_a_logit_in_one_order(amd, dtype, h):
+    """The forward's tiles run on 32x32x16 MFMAs, the recompute's on 16x16x32.  The logits of the targets, which the forward
+    leaves in its stash, and the same products of the other loop are equal to the last bit, on sums that lose some hundred units
+    in the last place of their result to rounding."""
+    from trl_amd import ops
+
+    n, v = 64, 600
+    hidden, weight, targets, _ = _cancelling_operands(n, v, h, dtype, h)
+    hidden, weight, targets = hidden.to(DEV), weight.to(DEV), targets.to(DEV)
+    if dtype == torch.float32:
+        hidden, weight = ops.split_bf16x3(hidden, 0), ops.split_bf16x3(weight, 1)
+    all_z = ops.gemm_nt(hidden, weight)
+    assert float((all_z - all_z.double().round().float()).abs().max()) > 1e-5  # (exact would be 0 and 14)
+    for shift in range(0, v, 97):
+        t = (targets + shift) % v
+        stash = ops.fused_head_fwd(hidden, weight, t, 1.0, 0.0, 1.0, None, True)[4]
+        z = stash[-1].reshape(-1).view(torch.float32)[:n]
+        assert torch.equal(z, all_z.gather(1, t[:, None])[:, 0])
+
+
+@pytest.mark.parametrize("form", ["plain", "bias"])
+@pytest.mark.parametrize("h", [2048, 1096])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_recomputed_logits_are_those_of_the_forward(amd, monkeypatch, dtype, h, form):
+    """The gradient of a nearly certain token is 1 - p: with recomputed logits it is right only if their rounding errors (about
+    5e-4 here) cancel against those in log_z.  d hidden[i, h - n + i] is 8 times the target's entry of d logits."""
+    monkeypatch.setenv("TRL_AMD_HEAD_STASH_GIB", "0")
+    n, v = 64, 600
+    hidden, weight, targets, gout = _cancelling_operands(n, v, h, dtype, h)
+    hd, wd = hidden.to(DEV).requires_grad_(True), weight.to(DEV).requires_grad_(True)
+    bias = None if form == "plain" else torch.zeros(v, device=DEV)
+    lp, _ = amd._ChunkedLogProbFunction.apply(hd, wd, targets.to(DEV), 1.0, 256, None, 1.0, bias)
+    (lp * gout.to(DEV)).sum().backward()
+    got = hd.grad[torch.arange(n), h - n + torch.arange(n)].double().cpu() / (8.0 * gout.double())
+    want = (v - 1) / (math.exp(14.0) + v - 1)
+    # 1 - p itself moves with its logit's errors: a rounding of half a unit of 2^-12 (partial sums below 4096) in each of 256
+    # steps, rms 1.2e-4 / sqrt(3) * 16 = 1.1e-3, four times that in the worst of 64 rows; the 16-bit d logits and outputs round
+    # to 2^-12 + 2^-9 of it.  log_z and its product with log2(e) round below 16 and 32, 5e-7 + 7e-7; with a bias z passes through
+    # three more fp32 roundings in the recompute, 5e-7 each.
+    bound = want * (4.5e-3 + (2.0**-8 if dtype != torch.float32 else 0.0)) + (1.5e-6 if form == "plain" else 3e-6)
+    err = float((got - want).abs().max())
+    print(f"{dtype} H={h} {form}: 1 - p = {want:.3e}, largest error {err:.2e}, bound {bound:.2e}")
+    assert err <= bound

@@ -16,7 +16,8 @@
 // the vocabulary tiles, the logits exist only as accumulators.
 //
 // Backward (K6), per vocabulary chunk: (1) dz = dL/dlogits as scaled fp16 [chunk, tokens] (vocabulary-major, each
-// token's column in that token's own power-of-two scale) -- from a recompute of the chunk's logits (same tile loop),
+// token's column in that token's own power-of-two scale) -- from a recompute of the chunk's logits (equal to the forward's
+// to the last bit),
 // or, when the forward was asked to stash its softmax numerators, from one elementwise sweep over that stash;
 // (2) dHidden += dz * W_chunk: the tile loop with dz as a K-MAJOR operand (its k rows go to LDS as they lie in
 // memory and the MFMA fragments come out through the LDS transpose loads, ds_read_b64_tr_b16) against W_chunk^T;
@@ -64,8 +65,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // The forward uses 32x32x16.  Its loop has registers for two sets of fragments there (nothing of the softmax state is
 // spilled) and takes, against the same loop as the products', 272 for 286 us with 1396 tokens, H = 2048, V = 50257 and
 // 302 for 330 us with 879 tokens, H = 1024, V = 151665; 8345 for 8240 us with 9664 tokens, H = 3584, V = 151936, where
-// power decides, is the other side.  And the log-probs of peaked rows hang on the last bits of the logits' sums: what a
-// run has stored of its old or its reference policy stays what it computes again.
+// power decides, is the other side.  The logits come out the same, to the last bit, in both shapes (180000 compared, bf16
+// and fp16, sums that cancel and sums that do not): the backward's recompute may use the other one, and the rounding of z
+// still cancels against that in log_z.  But the layout of 16x16x32 spreads a token's exponentials over twice as many lanes,
+// which changes the order of THEIR sum and the last bits of log_z; with the forward's loop as it is, what a run has stored of
+// its old or its reference policy stays what it computes again.
 template <int DT>
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
     if constexpr (DT == TRLK_BF16)
@@ -456,8 +460,7 @@ __device__ __forceinline__ void gemm_tile_nt_staged(const Operand A, int m0, con
     });
 }
 
-// The forward's tile loop: 32x32x16 MFMAs (a fragment is 32 rows x 16 k), the logits' sums in that shape's order.  The caller
-// has run DirectLoader::prologue.
+// The forward's tile loop: 32x32x16 MFMAs (a fragment is 32 rows x 16 k).  The caller has run DirectLoader::prologue.
 template <int DT>
 __device__ __forceinline__ void fwd_tile_direct(const Operand A, int m0, const Operand B, int n0, int K, f32x16 (&acc)[MB][NB],
                                                 char* smem) {
