@@ -916,3 +916,22 @@ def test_native_ops_under_tracers_and_on_errors(amd):
     if g.requires_grad:
         with pytest.raises(RuntimeError, match="not implemented"):
             g.float().sum().backward()
+
+
+def test_ops_that_hand_out_a_gradient_carry_none(amd):
+    """`grpo_fused_fwd_bwd` returns the gradient itself and `scale_unless_one_` scales one in place: both take logits that
+    require grad, and neither ties its results to a graph."""
+    from trl_amd import _lib, ops
+
+    B, T, V = 2, 3, 64
+    f = lambda *s: torch.rand(s, device=DEV)  # noqa: E731
+    logits = f(B, T, V).requires_grad_(True)
+    args = (torch.zeros(B, T, dtype=torch.long, device=DEV), 0.9, 0, T, torch.ones(B, T, device=DEV), f(B), f(B), None, None, None,
+            None, _lib.TERM_CLIP, 0.2, 0.2, math.nan, 0.0, False, 1.0, 1.05)
+    outputs = ops.grpo_fused_fwd_bwd(logits, *args)
+    assert not any(t.requires_grad for t in outputs)
+    assert all(torch.equal(a, b) for a, b in zip(outputs, ops.grpo_fused_fwd_bwd(logits.detach(), *args)))
+    leaf = f(4, 8).requires_grad_(True)
+    want = leaf.detach() * 0.5
+    assert ops.scale_unless_one_(leaf, torch.tensor(0.5, device=DEV)) is leaf
+    assert leaf.is_leaf and leaf.grad_fn is None and torch.equal(leaf.detach(), want)

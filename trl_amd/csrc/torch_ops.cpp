@@ -528,6 +528,8 @@ TORCH_LIBRARY_IMPL(trl_amd, Autograd, m) {
     m.impl("logp_entropy_stats_fwd", logp_entropy_stats_fwd_autograd);
     m.impl("grpo_loss", grpo_loss_autograd);
     m.impl("dpo_loss", dpo_loss_autograd);
-    for (const char* name : {"logp_entropy_bwd", "grpo_fused", "grpo_log_values", "grpo_row_scale", "dpo_log_values"})
+    for (const char* name : {"logp_entropy_bwd", "grpo_row_scale", "dpo_log_values"})
         m.impl(name, torch::autograd::autogradNotImplementedFallback());
+    // (these hand out a gradient or scale one in place: their results belong to no graph, whatever the logits require)
+    for (const char* name : {"grpo_fused", "scale_unless_one_"}) m.impl(name, torch::CppFunction::makeFallthrough());
 }
