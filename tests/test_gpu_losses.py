@@ -2,6 +2,9 @@
 vectors written by the reference's own `_compute_loss` methods and against the CPU oracle.
 Tolerance: losses, metrics and gradients within 1e-3 relative (fp32 cases are far tighter)."""
 import math
+import os
+import subprocess
+import sys
 from collections import defaultdict
 from types import SimpleNamespace
 
@@ -935,3 +938,62 @@ def test_ops_that_hand_out_a_gradient_carry_none(amd):
     want = leaf.detach() * 0.5
     assert ops.scale_unless_one_(leaf, torch.tensor(0.5, device=DEV)) is leaf
     assert leaf.is_leaf and leaf.grad_fn is None and torch.equal(leaf.detach(), want)
+
+
+def _in_a_new_process(program, **env):
+    """The last word that `program` prints."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", program], cwd=root, capture_output=True, text=True, timeout=100,
+                          env=dict(os.environ, **env))
+    assert done.returncode == 0, done.stderr[-2000:]
+    return done.stdout.split()[-1]
+
+
+_SYNC_CHECKED = """
+import math, torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+import trl_amd
+from trl_amd import _lib, ops
+
+D = "cuda:0"
+B, T, V = 2, 3, 64
+logits, ids = torch.randn(B, T, V, device=D), torch.zeros(B, T, dtype=torch.long, device=D)
+bad = ids.clone()
+bad[1, 2] = V
+f = lambda *s: torch.rand(s, device=D)
+fused = lambda x, i: ops.grpo_fused_fwd_bwd(x, i, 0.9, 0, T, torch.ones(B, T, device=D), f(B), f(B), None, None, None, None,
+                                            _lib.TERM_CLIP, 0.2, 0.2, math.nan, 0.0, False, 1.0, 1.05)
+calls = {
+    "logp": lambda x, i: ops.logp_entropy_fwd(x, i.view(-1, 1), 1.0, 0, T, None),
+    "named": lambda x, i: torch.ops.trl_amd.logp_entropy_fwd(x, i.view(-1, 1), 1.0, 0, T, None),
+    "stats": lambda x, i: ops.logp_entropy_stats_fwd(x, i.view(-1, 1), 1.0, 0, T, None),
+    "grad": lambda x, i: trl_amd.selective_log_softmax(x.clone().requires_grad_(True), i),
+    "fused": fused,
+}
+for name, call in calls.items():
+    call(logits, ids)
+    try:
+        call(logits, bad)
+    except IndexError as e:
+        assert "outside [0, vocab)" in str(e)
+    else:
+        raise AssertionError(name + ": no IndexError behind the call")
+    call(logits, ids)  # (the report has cleared the word)
+for op in (ops.logp_entropy_fwd, ops.logp_entropy_stats_fwd, ops.grpo_fused_fwd_bwd):
+    assert isinstance(op, torch._ops.OpOverload)
+with FakeTensorMode() as mode:
+    out = ops.logp_entropy_fwd(mode.from_tensor(logits), mode.from_tensor(ids).view(-1, 1), 1.0, 0, T, None)
+    assert [tuple(t.shape) for t in out] == [(B * T, 1), (B * T,), (B * T,)]
+compiled = torch.compile(calls["named"], backend="aot_eager", fullgraph=True)
+compiled(logits, ids)
+try:
+    compiled(logits, bad)
+except IndexError:
+    print("checked")
+"""
+
+
+def test_sync_checks_sit_inside_the_operators(amd):
+    """TRL_AMD_SYNC_CHECKS=1 (read when the package is loaded: a process of its own): a bad token id is reported by the call that
+    met it, however the operator was reached, and the operators stay what tracers take."""
+    assert _in_a_new_process(_SYNC_CHECKED, TRL_AMD_SYNC_CHECKS="1") == "checked"

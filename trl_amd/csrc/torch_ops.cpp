@@ -15,8 +15,10 @@
 #include <torch/library.h>
 #include <torch/python.h>
 
+#include <cstdlib>
 #include <map>
 #include <mutex>
+#include <string>
 
 #include "trlk.h"
 
@@ -86,6 +88,17 @@ std::vector<Tensor> all_error_flags() {
 }
 int32_t* error_word(const Tensor& t) { return static_cast<int32_t*>(error_flag(t.device().index()).mutable_data_ptr()); }
 
+// With TRL_AMD_SYNC_CHECKS=1 the error words are looked at behind each launch that reads token ids (a synchronisation).
+const bool kSyncChecks = [] {
+    const char* value = std::getenv("TRL_AMD_SYNC_CHECKS");
+    return value != nullptr && std::string(value) == "1";
+}();
+void check_ids() {
+    if (!kSyncChecks) return;
+    pybind11::gil_scoped_acquire gil;
+    pybind11::module_::import("trl_amd.ops").attr("check_device_errors")();
+}
+
 void check_logits3d(const Tensor& logits) {
     TORCH_CHECK_VALUE(logits.dim() == 3, "expected [n_seq, rows, vocab] logits, got shape ", logits.sizes());
     TORCH_CHECK_VALUE(logits.size(2) <= 1 || logits.stride(2) == 1, "the vocabulary axis of the logits must be contiguous");
@@ -118,6 +131,7 @@ Tensor4 run_logp_entropy(const Tensor& logits, const Tensor& index_, double temp
                                 row_mask ? static_cast<const uint8_t*>(row_mask->const_data_ptr()) : nullptr, out(logp), out(ent),
                                 out(lse), with_stats ? out(stats) : nullptr, sum_p2 ? 1 : 0, error_word(logits),
                                 stream_of(logits)));
+    check_ids();
     return {logp, ent, lse, stats};
 }
 Tensor3 logp_entropy_fwd(const Tensor& logits, const Tensor& index, double temperature, int64_t keep_start, int64_t keep_len,
@@ -371,6 +385,7 @@ Tensor4 grpo_fused(const Tensor& logits, const Tensor& index_, double temperatur
         float(beta), bias_correction_kl ? 1 : 0, float(sapo_pos), float(sapo_neg), out(logp), out(ent), out(lse),
         dlogits.mutable_data_ptr(), length, keep_start, dlogits.stride(0), dlogits.stride(1), compute_masked_rows ? 1 : 0,
         error_word(logits), stream_of(logits)));
+    check_ids();
     return {logp, ent, lse, dlogits};
 }
 

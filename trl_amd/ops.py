@@ -67,20 +67,11 @@ def raise_for_error_bits(bits: float, device: torch.device) -> None:
 _library = torch.library.Library("trl_amd", "FRAGMENT")
 
 
-def _native_op(name: str, fake, syncs: bool = False):
+def _native_op(name: str, fake):
     """The operator `trl_amd::<name>` that the native library registers (csrc/torch_ops.cpp), with `fake` as its shapes for
-    tracers; `syncs`: it reads token ids, and TRL_AMD_SYNC_CHECKS=1 looks at the error word behind each call."""
+    tracers."""
     torch.library.register_fake(f"trl_amd::{name}", fake, lib=_library)
-    op = getattr(torch.ops.trl_amd, name).default
-    if not (syncs and _SYNC_CHECKS):
-        return op
-
-    def checked(*args, **kwargs):
-        out = op(*args, **kwargs)
-        check_device_errors()
-        return out
-
-    return checked
+    return getattr(torch.ops.trl_amd, name).default
 
 
 # Ops without a gradient of their own (their callers' autograd functions have it) that run several times per step: no Python
@@ -120,7 +111,7 @@ def _logp_entropy_fake(logits, index, temperature, keep_start, keep_len, row_mas
     return _f32_like(logits, rows, index.shape[-1]), _f32_like(logits, rows), _f32_like(logits, rows)
 
 
-logp_entropy_fwd = _native_op("logp_entropy_fwd", _logp_entropy_fake, syncs=True)
+logp_entropy_fwd = _native_op("logp_entropy_fwd", _logp_entropy_fake)
 
 
 # As `logp_entropy_fwd`, plus the fp32 row statistics `[rows, 4]` of the same pass: mean logit, log sum_v p_v^2 (0 without
@@ -131,7 +122,7 @@ def _logp_entropy_stats_fake(logits, index, temperature, keep_start, keep_len, r
             _f32_like(logits, logits.shape[0] * keep_len, 4))
 
 
-logp_entropy_stats_fwd = _native_op("logp_entropy_stats_fwd", _logp_entropy_stats_fake, syncs=True)
+logp_entropy_stats_fwd = _native_op("logp_entropy_stats_fwd", _logp_entropy_stats_fake)
 
 # d(loss)/d(logits) for the whole [n_seq, L, V] input (contiguous, same dtype): rows outside the kept window and rows whose
 # upstream gradients are all zero are zero-filled.
@@ -380,7 +371,7 @@ def _grpo_fused_fake(logits, index, temperature, keep_start, keep_len, *args, **
             torch.empty(logits.shape, dtype=logits.dtype, device=logits.device))
 
 
-grpo_fused_fwd_bwd = _native_op("grpo_fused", _grpo_fused_fake, syncs=True)
+grpo_fused_fwd_bwd = _native_op("grpo_fused", _grpo_fused_fake)
 
 _scale_unless_one = _native_op("scale_unless_one_", lambda data, scale: None)
 
