@@ -997,3 +997,21 @@ def test_sync_checks_sit_inside_the_operators(amd):
     """TRL_AMD_SYNC_CHECKS=1 (read when the package is loaded: a process of its own): a bad token id is reported by the call that
     met it, however the operator was reached, and the operators stay what tracers take."""
     assert _in_a_new_process(_SYNC_CHECKED, TRL_AMD_SYNC_CHECKS="1") == "checked"
+
+
+def test_error_word_made_in_inference_mode(amd):
+    """The word that the kernels report bad ids in is made by the first call on a device; one made in inference mode can be
+    cleared outside of it."""
+    assert _in_a_new_process("""
+import torch, trl_amd
+logits, ids = torch.randn(1, 3, 64, device="cuda:0"), torch.zeros(1, 3, dtype=torch.long, device="cuda:0")
+with torch.inference_mode():
+    trl_amd.selective_log_softmax(logits, ids)
+ids[0, 0] = 64
+trl_amd.selective_log_softmax(logits, ids)
+try:
+    trl_amd.check_device_errors()
+except IndexError:
+    trl_amd.check_device_errors()
+    print("cleared")
+""") == "cleared"

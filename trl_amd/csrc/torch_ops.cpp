@@ -10,6 +10,7 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/InferenceMode.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
@@ -75,8 +76,10 @@ Tensor error_flag(int64_t index) {
     ErrorFlags& flags = error_flags();
     std::lock_guard<std::mutex> lock(flags.mutex);
     auto it = flags.of_device.find(index);
-    if (it == flags.of_device.end())
+    if (it == flags.of_device.end()) {
+        const c10::InferenceMode off(false);  // (a word made in inference mode could not be cleared outside of it)
         it = flags.of_device.emplace(index, at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA, index))).first;
+    }
     return it->second;
 }
 std::vector<Tensor> all_error_flags() {
