@@ -11,7 +11,8 @@ CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 def build(clean: bool = True, jobs: int = 4) -> str:
     if clean:
         subprocess.run(["make", "-C", CSRC, "clean"], check=True, stdout=subprocess.DEVNULL)
-    subprocess.run(["make", "-C", CSRC, f"-j{jobs}"], check=True)
+    # (the torch to build against is the one of the interpreter that will load the result, whatever `python3` is on the path)
+    subprocess.run(["make", "-C", CSRC, f"-j{jobs}", f"PYTHON={sys.executable}"], check=True)
     # the same device code under a sanitized host build: what tests/test_abi_sanitized.py loads
     subprocess.run(["make", "-C", CSRC, f"-j{jobs}", "asan"], check=True)
     out = os.path.join(os.path.dirname(CSRC), "lib", "libtrlk.so")
