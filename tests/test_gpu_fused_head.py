@@ -896,7 +896,7 @@ def test_partly_filled_tiles(amd, monkeypatch, n, h, v, stash):
 
 
 @pytest.mark.parametrize("stash", [True, False])
-@pytest.mark.parametrize("kind", ["outlier", "outlier_of_one_chunk", "zero_sample", "zero_weight", "just_inside"])
+@pytest.mark.parametrize("kind", ["outlier", "outlier_of_one_chunk", "zero_sample", "zero_weight", "just_inside", "just_outside"])
 def test_weight_scale_from_a_sample(amd, monkeypatch, kind, stash):
     """The backward converts the bf16 weight to fp16 in a scale taken from every 32nd row; a chunk that reaches beyond what that
     scale leaves room for, or whose sample holds only zeros, is converted again in its own scale."""
@@ -906,7 +906,8 @@ def test_weight_scale_from_a_sample(amd, monkeypatch, kind, stash):
     g = torch.Generator().manual_seed(3)
     hidden = torch.randn(n, h, generator=g).bfloat16() * 0.01
     weight = torch.randn(v, h, generator=g) * 0.02
-    sample_max = weight[::32].abs().max()
+    # the scale puts the power of two at or below this magnitude at 2^13
+    octave = 2.0 ** torch.floor(torch.log2(weight[::32].bfloat16().float().abs().max()))
     if kind == "outlier":
         weight[5, 7] = 300.0
         weight[801, 0] = -2000.0
@@ -916,8 +917,10 @@ def test_weight_scale_from_a_sample(amd, monkeypatch, kind, stash):
         weight[::32] = 0.0
     elif kind == "zero_weight":
         weight.zero_()
-    else:  # the largest magnitude that the sample's scale still holds
-        weight[33, 1] = 3.9 * 2.0 ** torch.floor(torch.log2(sample_max))
+    elif kind == "just_inside":  # the largest bf16 value that the sample's scale still holds: 65280 in fp16
+        weight[33, 1] = 7.96875 * octave
+    else:  # the next one: infinite in fp16 unless the chunk is converted again
+        weight[33, 1] = 8.0 * octave
     weight = weight.bfloat16()
     labels = torch.randint(0, v, (n,), generator=g)
     labels[:4] = torch.tensor([5, 801, 300, 33])
