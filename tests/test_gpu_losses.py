@@ -916,9 +916,9 @@ def test_native_ops_under_tracers_and_on_errors(amd):
         ops.logp_entropy_fwd(logits.cpu(), ids.cpu(), 1.0, 1, T, None)
     x = leaf(logits)
     (g,) = torch.autograd.grad(ops.logp_entropy_fwd(x, ids, 1.0, 1, T, None)[0].sum(), x, create_graph=True)
-    if g.requires_grad:
-        with pytest.raises(RuntimeError, match="not implemented"):
-            g.float().sum().backward()
+    assert g.requires_grad  # (a gradient cut off from the graph would drop a penalty on it without a word)
+    with pytest.raises(RuntimeError, match="not implemented"):
+        g.float().sum().backward()
 
 
 def test_ops_that_hand_out_a_gradient_carry_none(amd):
