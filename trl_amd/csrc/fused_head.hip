@@ -584,7 +584,10 @@ __device__ __forceinline__ void fwd_tile_direct(const Operand A, int m0, const O
     } else if (nk == 2) {
         step(kt++, F, F, T);
     }
-    for (; kt + 1 < nk; ++kt) step(kt, F, F, T);  // (no step is left; without the loop a register is spilled in the one above)
+    // No step is left.  Without this loop, and with six other ways to write these lines, one or two registers of the kernel with
+    // a stash are spilled: 0.5 to 1 % more time (1396 tokens, H = 2048, V = 50257 259 -> 262 us; 9664 tokens, H = 3584, V = 151936
+    // 8415 -> 8441 us).
+    for (; kt + 1 < nk; ++kt) step(kt, F, F, T);
     step(kt, F, F, F);
     // every LDS read of this tile completed before the last barrier: the caller may reuse the LDS right away
 }
@@ -1621,14 +1624,21 @@ __device__ __forceinline__ uint32_t transpose16_tile(uint16_t* tile, int c0, int
     }
     return m;
 }
-template <bool TO_F16, bool ROW_G = false>
-__global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
-                                                          int64_t ldo, int64_t fill, const uint32_t* in_max,
-                                                          const float* row_g = nullptr, const uint32_t* g_max = nullptr,
-                                                          float zs = 1.f) {
+// hidden^T, its columns in the scales of the d logits' columns.
+template <bool TO_F16>
+__global__ __launch_bounds__(256) void transpose_hidden_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
+                                                               int64_t ldo, int64_t fill, const uint32_t* in_max,
+                                                               const float* row_g, const uint32_t* g_max, float zs) {
     __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kTransposeStride];
-    transpose16_tile<TO_F16, ROW_G, false>(tile, blockIdx.x * 64, blockIdx.y * 64, in, ld, R, C, out, ldo, fill,
-                                           TO_F16 ? slot_scale(in_max, 1.f) : 1.f, row_g, g_max, zs);
+    transpose16_tile<TO_F16, true, false>(tile, blockIdx.x * 64, blockIdx.y * 64, in, ld, R, C, out, ldo, fill,
+                                          TO_F16 ? slot_scale(in_max, 1.f) : 1.f, row_g, g_max, zs);
+}
+// W_chunk^T of an fp16 problem, as it is.
+__global__ __launch_bounds__(256) void transpose_weight_f16_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
+                                                                   int64_t ldo, int64_t fill) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kTransposeStride];
+    transpose16_tile<false, false, false>(tile, blockIdx.x * 64, blockIdx.y * 64, in, ld, R, C, out, ldo, fill, 1.f, nullptr,
+                                          nullptr, 1.f);
 }
 // W_chunk^T of a bf16 problem in the sample's scale.  The largest magnitude of what it converts is found on the way: a wave
 // whose entries all stay below the sample's maximum (nearly every one) spends one comparison on it, the others one atomic.
@@ -1647,7 +1657,10 @@ __global__ __launch_bounds__(256) void transpose_weight_kernel(const uint16_t* i
     }
 }
 // The same again in the scale of the chunk's own maximum, where the sample's does not do: returns at once everywhere else (few
-// workgroups that step through the tiles, so that a launch with nothing to do takes 3-5 us).
+// workgroups that step through the tiles, so that a launch with nothing to do takes 3-5 us).  One entry of 50 in a weight of
+// deviation 0.02, which makes every chunk that holds it convert again: whole backward 709 -> 780 us (1396 tokens, H = 2048, V =
+// 50257), 1676 -> 1842 us (1392 tokens, V = 128256), 1716 -> 1933 us (459 tokens, H = 3584, V = 151936) -- about what the separate
+// pass over the weight cost every call (772, 1857 and 1949 us).
 constexpr int kAgainBlocks = 1024;
 __global__ __launch_bounds__(256) void transpose_weight_again_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
                                                                      int64_t ldo, int64_t fill, const uint32_t* sample,
@@ -2005,11 +2018,11 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
     }
     hipLaunchKernelGGL(head_maxabs_kernel, dim3(unsigned(ma.blocks_w + ma.blocks_h + ma.blocks_g)), dim3(kMaxThreads), 0, s, ma);
     if (from_bf16) {
-        hipLaunchKernelGGL((transpose16_kernel<true, true>), dim3((H + 63) / 64, unsigned((l.npad + 63) / 64)), dim3(256), 0, s,
+        hipLaunchKernelGGL(transpose_hidden_kernel<true>, dim3((H + 63) / 64, unsigned((l.npad + 63) / 64)), dim3(256), 0, s,
                            static_cast<const uint16_t*>(d_hidden), hidden_stride, N, H, ht, l.ld_n, l.npad, max_h, d_g_logp,
                            max_g, logit_scale / temperature);
     } else {
-        hipLaunchKernelGGL((transpose16_kernel<false, true>), dim3((H + 63) / 64, unsigned((l.npad + 63) / 64)), dim3(256), 0, s,
+        hipLaunchKernelGGL(transpose_hidden_kernel<false>, dim3((H + 63) / 64, unsigned((l.npad + 63) / 64)), dim3(256), 0, s,
                            static_cast<const uint16_t*>(d_hidden), hidden_stride, N, H, ht, l.ld_n, l.npad, max_h, d_g_logp,
                            max_g, logit_scale / temperature);
     }
@@ -2085,8 +2098,8 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
             hipLaunchKernelGGL(transpose_weight_again_kernel, dim3(tiles < kAgainBlocks ? tiles : kAgainBlocks), dim3(256), 0, s,
                                w_chunk, weight_stride, rows, H, wt, l.ld_c, int64_t(kpad), max_w, beyond_w, int(tgrid.x), tiles);
         } else {
-            hipLaunchKernelGGL(transpose16_kernel<false>, tgrid, dim3(256), 0, s, w_chunk, weight_stride, rows, H, wt, l.ld_c,
-                               int64_t(kpad), nullptr);
+            hipLaunchKernelGGL(transpose_weight_f16_kernel, tgrid, dim3(256), 0, s, w_chunk, weight_stride, rows, H, wt, l.ld_c,
+                               int64_t(kpad));
         }
         if (int rc2 = launch_status("fused_head_bwd (W^T)")) return rc2;
         // dHidden[N, H] += dz[N, chunk] * (W_chunk^T[H, chunk])^T
