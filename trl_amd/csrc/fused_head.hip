@@ -1643,7 +1643,8 @@ __global__ __launch_bounds__(256) void transpose_weight_f16_kernel(const uint16_
 // W_chunk^T of a bf16 problem in the sample's scale.  The largest magnitude of what it converts is found on the way: a wave
 // whose entries all stay below the sample's maximum (nearly every one) spends one comparison on it, the others one atomic.
 // The separate pass over the whole weight that used to precede this one took 36 / 93 / 214 us for weights of 206 / 525 / 1089 MB
-// (50257 x 2048, 128256 x 2048, 151936 x 3584); the sample takes 7 / 10 / 15 us, a second launch with nothing to do 3-5 us.
+// (50257 x 2048, 128256 x 2048, 151936 x 3584); the launch that reads the sample takes 9 / 10 / 15 us with few tokens (28 with
+// the 69 MB of 9664 hidden states of 3584, which it reads too), a second launch with nothing to do 5 us.
 __global__ __launch_bounds__(256) void transpose_weight_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
                                                                int64_t ldo, int64_t fill, const uint32_t* sample, uint32_t* beyond) {
     __shared__ __attribute__((aligned(16))) uint16_t tile[64 * kTransposeStride];
@@ -1657,7 +1658,7 @@ __global__ __launch_bounds__(256) void transpose_weight_kernel(const uint16_t* i
     }
 }
 // The same again in the scale of the chunk's own maximum, where the sample's does not do: returns at once everywhere else (few
-// workgroups that step through the tiles, so that a launch with nothing to do takes 3-5 us).  One entry of 50 in a weight of
+// workgroups that step through the tiles, so that a launch with nothing to do takes 5 us).  One entry of 50 in a weight of
 // deviation 0.02, which makes every chunk that holds it convert again: whole backward 709 -> 780 us (1396 tokens, H = 2048, V =
 // 50257), 1676 -> 1842 us (1392 tokens, V = 128256), 1716 -> 1933 us (459 tokens, H = 3584, V = 151936) -- about what the separate
 // pass over the weight cost every call (772, 1857 and 1949 us).
