@@ -1015,3 +1015,49 @@ except IndexError:
     trl_amd.check_device_errors()
     print("cleared")
 """) == "cleared"
+
+
+def test_operands_in_host_memory_are_refused(amd):
+    """An operator runs on the GPU as soon as one of its tensors is there: each other one in turn in ordinary host memory raises
+    before a kernel is launched.  Pinned memory, which kernels can read, is taken as before."""
+    from trl_amd import _lib, ops
+
+    f = lambda *s: torch.rand(s, device=DEV)  # noqa: E731
+    B, T, V = 2, 3, 40
+    logits, ids, mask = f(B, T, V), torch.randint(0, V, (B * T, 1), device=DEV), torch.ones(B, T, device=DEV)
+    rows = torch.ones(B * T, dtype=torch.uint8, device=DEV)
+    logp, ent, lse = ops.logp_entropy_fwd(logits, ids, 0.9, 0, T, None)
+    logp64, ent64, lse64 = ops.logp_entropy_fwd_f64(logits.double(), ids, 0.9, 0, T, None)
+    loss = (_lib.DAPO, 0.2, 0.2, math.nan, 0.04, False, 1.0, 1.0, 1.0, 0.1, 0, False)
+    term = (_lib.TERM_CLIP, 0.2, 0.2, math.nan, 0.1, False, 1.0, 1.05, False)
+    hidden, weight, targets = f(4, 64).bfloat16(), f(100, 64).bfloat16(), torch.randint(0, 100, (4,), device=DEV)
+    log_z = ops.fused_head_fwd(hidden, weight, targets, 1.0, 0.0, 1.0)[2]
+    calls = [
+        (ops.logp_entropy_fwd, (logits, ids, 0.9, 0, T, rows)),
+        (ops.logp_entropy_stats_fwd, (logits, ids, 0.9, 0, T, rows)),
+        (ops.logp_entropy_bwd, (logits, ids, 0.9, 0, T, lse, ent, logp, ent)),
+        (ops.logp_entropy_fwd_f64, (logits.double(), ids, 0.9, 0, T, rows)),
+        (ops.logp_entropy_bwd_f64, (logits.double(), ids, 0.9, 0, T, lse64, ent64, logp64, ent64)),
+        (ops.grpo_loss_op, (f(B, T), f(B, T), f(B, T), f(B, T), f(B), mask, f(B, T), mask, f(1), *loss, f(B))),
+        (ops.grpo_fused_fwd_bwd, (logits, ids.view(B, T), 0.9, 0, T, mask, f(B), f(B), f(B, T), f(B, T), f(B, T), f(B), *term,
+                                  f(B, T))),
+        (ops._grpo_row_scale, (mask, _lib.DAPO, 1.0, f(1), f(1), True)),
+        (ops.dpo_loss_op, (f(B, T), mask, f(1), f(1), 0.1)),
+        (ops.dpo_log_values, (f(B, T), f(B, T, 4), mask, f(B), f(1), f(1), 0.1)),
+        (ops.rloo_loss_op, (f(B, T), mask, f(B), f(B), 0.2, 0.2)),
+        (ops.fused_head_fwd, (hidden, weight, targets, 1.0, 0.0, 1.0, f(100))),
+        (ops.fused_head_bwd, (hidden, weight, targets, 1.0, 0.0, 1.0, log_z, f(4), 256, f(100))),
+    ]
+    for op, args in calls:
+        op(*args)
+        for i, a in enumerate(args):
+            if isinstance(a, torch.Tensor):
+                with pytest.raises((RuntimeError, ValueError), match="device|GPU"):
+                    op(*args[:i], a.cpu(), *args[i + 1 :])
+    with pytest.raises(RuntimeError, match="device"):
+        ops.scale_unless_one_(torch.ones(8), f(1))
+    with pytest.raises(RuntimeError, match="device"):
+        amd.selective_log_softmax(logits, ids.view(B, T).cpu())
+    pinned = ids.cpu().pin_memory()
+    assert torch.equal(ops.logp_entropy_fwd(logits, pinned, 0.9, 0, T, None)[0], logp)
+    amd.check_device_errors()

@@ -200,7 +200,13 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else t.data_ptr()
+    """The data of an operand.  An op is dispatched to the GPU if ANY of its tensors is there: one in ordinary host memory among
+    them is an error and must not reach a kernel (pinned memory can be read)."""
+    if t is None:
+        return None
+    if not t.is_cuda and t.numel() and not t.is_pinned():
+        raise RuntimeError(f"Expected all tensors to be on the same device, but found one of shape {tuple(t.shape)} on {t.device}")
+    return t.data_ptr()
 
 
 def current_stream(device: torch.device) -> int:

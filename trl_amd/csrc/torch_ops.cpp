@@ -58,10 +58,17 @@ Tensor f32(const Tensor& like, at::IntArrayRef sizes) { return at::empty(sizes, 
 // fp32 and contiguous
 Tensor f32c(const Tensor& t) { return t.contiguous().to(at::kFloat); }
 optional<Tensor> f32c(const optional<Tensor>& t) { return t ? optional<Tensor>(f32c(*t)) : std::nullopt; }
-const float* fptr(const Tensor& t) { return static_cast<const float*>(t.const_data_ptr()); }
+// The data of an operand.  A call is dispatched here if ANY of its tensors is on a GPU: one in ordinary host memory among them
+// is an error and must not reach a kernel (pinned memory can be read).
+const void* operand(const Tensor& t) {
+    TORCH_CHECK(t.is_cuda() || t.numel() == 0 || t.is_pinned(),
+                "Expected all tensors to be on the same device, but found one of shape ", t.sizes(), " on ", t.device());
+    return t.const_data_ptr();
+}
+const float* fptr(const Tensor& t) { return static_cast<const float*>(operand(t)); }
 const float* fptr(const optional<Tensor>& t) { return t ? fptr(*t) : nullptr; }
 float* out(const Tensor& t) { return static_cast<float*>(t.mutable_data_ptr()); }
-const int64_t* iptr(const Tensor& t) { return static_cast<const int64_t*>(t.const_data_ptr()); }
+const int64_t* iptr(const Tensor& t) { return static_cast<const int64_t*>(operand(t)); }
 
 // The int32 word per device that the kernels OR error bits into.  It lives until the process ends.
 struct ErrorFlags {
@@ -105,6 +112,7 @@ void check_ids() {
 void check_logits3d(const Tensor& logits) {
     TORCH_CHECK_VALUE(logits.dim() == 3, "expected [n_seq, rows, vocab] logits, got shape ", logits.sizes());
     TORCH_CHECK_VALUE(logits.size(2) <= 1 || logits.stride(2) == 1, "the vocabulary axis of the logits must be contiguous");
+    (void)operand(logits);
 }
 // the rows from keep_start on of every sequence
 const char* window(const Tensor& logits, int64_t keep_start) {
@@ -131,7 +139,7 @@ Tensor4 run_logp_entropy(const Tensor& logits, const Tensor& index_, double temp
     const Tensor index = index_.contiguous();
     check(trlk_logp_entropy_fwd(window(logits, keep_start), dtype_code(logits), n_seq, keep_len, vocab, logits.stride(0),
                                 logits.stride(1), iptr(index), k, float(temperature),
-                                row_mask ? static_cast<const uint8_t*>(row_mask->const_data_ptr()) : nullptr, out(logp), out(ent),
+                                row_mask ? static_cast<const uint8_t*>(operand(*row_mask)) : nullptr, out(logp), out(ent),
                                 out(lse), with_stats ? out(stats) : nullptr, sum_p2 ? 1 : 0, error_word(logits),
                                 stream_of(logits)));
     check_ids();
@@ -398,6 +406,7 @@ void scale_unless_one_(const Tensor& data, const Tensor& scale_) {
                       "scale_unless_one_: contiguous bf16 / fp16 / fp32 data expected");
     const c10::DeviceGuard guard(data.device());
     const Tensor scale = scale_.reshape({1}).to(data.options().dtype(at::kFloat));
+    (void)operand(data);
     check(trlk_scale_unless_one(data.mutable_data_ptr(), dtype_code(data), data.numel(), fptr(scale), stream_of(data)));
 }
 
@@ -424,7 +433,7 @@ std::tuple<Tensor, Tensor> grpo_row_scale(const Tensor& mask, int64_t loss_type,
     }
     const c10::DeviceGuard guard(mask.device());
     const Tensor mask_f = with_mask ? f32(mask, {B, T}) : f32(mask, {0}), scale = f32(mask, {B});
-    check(trlk_grpo_row_scale(mask.const_data_ptr(), type, B, T, mask.stride(0), mask.stride(1), int(loss_type), float(numerator),
+    check(trlk_grpo_row_scale(operand(mask), type, B, T, mask.stride(0), mask.stride(1), int(loss_type), float(numerator),
                               fptr(n_items), fptr(upstream), with_mask ? out(mask_f) : nullptr, out(scale), stream_of(mask)));
     return {mask_f, scale};
 }
@@ -488,6 +497,7 @@ Tensor dpo_log_values(const Tensor& entropy_, const Tensor& row_stats_, const Te
     const int64_t B = mask_.size(0), T = mask_.size(1), P = B / 2;
     TORCH_CHECK_VALUE(B % 2 == 0 && entropy_.numel() == B * T && row_stats_.numel() == 4 * B * T && seq_logps_.numel() == B,
                       "dpo_log_values: the shapes do not match");
+    (void)operand(mask_);
     const c10::DeviceGuard guard(mask_.device());
     const Tensor entropy = f32c(entropy_), row_stats = f32c(row_stats_), mask = f32c(mask_), seq_logps = f32c(seq_logps_);
     const Tensor ref_chosen = f32c(ref_chosen_.expand({P})), ref_rejected = f32c(ref_rejected_.expand({P}));

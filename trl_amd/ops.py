@@ -151,7 +151,7 @@ def logp_entropy_fwd_f64(
     index = index.contiguous()
     view = logits[:, keep_start : keep_start + keep_len]
     with on_device(dev):
-        check(lib.trlk_logp_entropy_fwd_f64(view.data_ptr(), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
+        check(lib.trlk_logp_entropy_fwd_f64(ptr(view), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
                                             ptr(index), k, temperature, ptr(row_mask), ptr(logp), ptr(ent), ptr(lse),
                                             ptr(_error_flag(dev)), current_stream(dev)))
     if _SYNC_CHECKS:
@@ -184,7 +184,7 @@ def logp_entropy_bwd_f64(
     g_logp = None if g_logp is None else g_logp.contiguous().double()
     g_entropy = None if g_entropy is None else g_entropy.contiguous().double()
     with on_device(dev):
-        check(lib.trlk_logp_entropy_bwd_f64(view.data_ptr(), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
+        check(lib.trlk_logp_entropy_bwd_f64(ptr(view), n_seq, keep_len, vocab, view.stride(0), view.stride(1),
                                             ptr(index), k, temperature, ptr(lse),
                                             ptr(entropy if g_entropy is not None else None), ptr(g_logp), ptr(g_entropy),
                                             ptr(dlogits), length, keep_start, dlogits.stride(0), dlogits.stride(1),
