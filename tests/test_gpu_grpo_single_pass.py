@@ -1112,3 +1112,35 @@ def test_sums_of_peaked_rows(amd, V):
         wrong.append(torch.stack([logp[b] - lsm.gather(1, ids[b, :, None]).squeeze(1), ent[b] + (lsm.exp() * lsm).sum(1)]))
     rms = torch.cat(wrong, 1).square().mean(1).sqrt()
     assert float(rms[0]) < 8.5e-7 and float(rms[1]) < 4.2e-6, rms
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("B,K", [(1, 1), (3, 26), (5, 47), (9, 34), (2, 411), (300, 2), (4, 257)])
+def test_rows_dealt_to_the_xcds_in_runs(amd, dtype, B, K):
+    """Row counts around whole rounds of runs (a run is about an 80th of the rows): both gradient kernels write every row of the
+    output, those with a gradient as float64 has it, the others as zeros."""
+    V, T = 520, 0.9
+    logits, ids, mask, adv, _ = _inputs(B, K, V, dtype, seed=B + K, extra_rows=1)
+    mask[:, K // 2] = 1
+    coef = -adv.double()[:, None] * mask / (B * K)  # d loss / d log-prob of a dr_grpo step whose ratios are all 1
+    p = (logits[:, :K].double() / T).softmax(-1)
+    want = torch.zeros_like(logits, dtype=torch.float64)
+    want[:, :K] = (torch.zeros_like(p).scatter_(-1, ids[..., None], 1.0) - p) * coef[..., None] / T
+    # p in fp32 to 1e-5 of itself (entries of one row sum to 1), the one-hot's difference and the product a rounding each, and one to the dtype
+    bound = 2e-5 * (coef.abs() / T)[..., None] * (p + torch.zeros_like(p).scatter_(-1, ids[..., None], 1.0))
+    bound = torch.nn.functional.pad(bound, (0, 0, 0, 1)) + (0.0 if dtype == torch.float32 else 2.0**-8) * want.abs()
+
+    def poisoned_memory():  # (what the gradient's buffer is likely to hold beforehand)
+        torch.full_like(logits, float("nan"))
+
+    leaf = logits.clone().requires_grad_(True)
+    poisoned_memory()
+    loss, _, _, _ = amd.grpo_loss_from_logits(leaf, ids, adv, mask, temperature=T, loss_type="dr_grpo", max_completion_length=K)
+    loss.backward()
+    assert bool(((leaf.grad.double() - want).abs() <= bound).all())
+    leaf = logits.clone().requires_grad_(True)
+    lp, _ = amd.per_token_logps_and_entropies(leaf, ids, K, T, True)
+    loss = (lp * coef.float()).sum()
+    poisoned_memory()
+    (grad,) = torch.autograd.grad(loss, leaf)
+    assert bool(((grad.double() - want).abs() <= bound).all())

@@ -46,6 +46,15 @@ typedef __attribute__((address_space(1))) u32x4 GlobalVecOut;
 typedef u32x4 u32x4_u __attribute__((aligned(2)));  // a 16-byte vector at any element alignment
 typedef __attribute__((address_space(1))) u32x4_u GlobalVecOutU;
 
+// Bytes of rows that follow each other on one XCD (see xcd_run).  Against one contiguous eighth of the rows per XCD, two draws of
+// completions of 1/16 of the longest to the longest, bf16: [32, 1024, 151936] 2848 / 2730 -> 2689 / 2684 us, [16, 1024, 128256]
+// 1278 / 1285 -> 1148 / 1136, [8, 700, 262144] 980 / 982 -> 854 / 862, [16, 509, 50257] 251 / 255 -> 244 / 240,
+// [16, 2047, 40000] 785 / 794 -> 751 / 738, [8, 512, 50264] fp32 250 -> 228; [20, 585, 50264] loses, 339 / 331 -> 347 / 341.
+// Every row active: within 2 %; half of every sequence, which leaves no XCD with more: -4 to +5 %.  A narrow row (see
+// kNarrowVec) has neighbours on its CU, and an XCD twice to five times as many rows under way: runs of 4 MiB lose 3 to 5 %
+// there (50264 and 65536 entries), while wide rows of 256 KB lose 2 % in runs of 8 MiB and of 512 KB 5 % in runs of 39.
+constexpr int64_t kNarrowRunBytes = 12 << 20, kWideRunBytes = 6 << 20;
+
 struct FusedArgs {
     const void* logits;
     int64_t rows_per_seq, vocab, seq_stride, row_stride;
@@ -62,7 +71,8 @@ struct FusedArgs {
     void* dlogits;
     int64_t out_rows_per_seq, out_row_offset, out_seq_stride, out_row_stride;
     int32_t* error_flag;
-    int64_t total_rows;  // output rows: the grid is rounded up to a multiple of 8
+    int64_t total_rows;  // output rows
+    unsigned run, grid;  // rows of an XCD side by side (see xcd_piece), workgroups of the launch
     int all_rows;  // also read the rows with mask == 0 for their log-prob and entropy (their gradient is zero either way)
 };
 
@@ -130,12 +140,7 @@ __global__ __launch_bounds__(TH) void grpo_fused_kernel(FusedArgs a) {
     extern __shared__ __attribute__((aligned(16))) char overflow[];  // [NLDS][1024 lanes] 16-byte vectors
     __shared__ float red[7][(TH / kWave)];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
-    // The hardware deals consecutive workgroups to the eight XCDs in turn.  Each XCD takes one contiguous eighth of
-    // the rows and walks it in order, instead of every eighth row of the whole tensor: eight separate streams of reads
-    // and writes, one per XCD.  Measured on bf16 [64, 1024, 151936] with the benchmark's mask: 5.65 -> 5.24 ms
-    // (every row read: 7.25 -> 6.86 ms; every row active: 7.55 -> 7.28 ms).
-    const int64_t per_xcd = int64_t(gridDim.x) >> 3;  // (the grid is a multiple of 8)
-    const int64_t orow = int64_t(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    const int64_t orow = xcd_piece(blockIdx.x, a.run);
     if (orow >= a.total_rows) return;
     const int64_t b = orow / a.out_rows_per_seq;
     const int64_t to = orow - b * a.out_rows_per_seq;
@@ -511,27 +516,27 @@ int reserve_dtype() {
 }
 
 template <int DT, int NLDS, bool EXTRA, bool R>
-int launch_fused_wide(const FusedArgs& a, unsigned rows, hipStream_t s) {
+int launch_fused_wide(const FusedArgs& a, hipStream_t s) {
     constexpr int kBytes = NLDS * kFThreads * 16;
     if (int rc = reserve_overflow_lds(grpo_fused_kernel<DT, kWideVec, NLDS, EXTRA, R>, kBytes)) return rc;
-    hipLaunchKernelGGL((grpo_fused_kernel<DT, kWideVec, NLDS, EXTRA, R>), dim3((rows + 7) / 8 * 8), dim3(kFThreads), kBytes, s, a);
+    hipLaunchKernelGGL((grpo_fused_kernel<DT, kWideVec, NLDS, EXTRA, R>), dim3(a.grid), dim3(kFThreads), kBytes, s, a);
     return TRLK_OK;
 }
 
 // R: rows that are not whole aligned vectors
 template <int DT, bool R>
-int launch_fused(const FusedArgs& a, int vectors, unsigned rows, hipStream_t s) {
+int launch_fused(const FusedArgs& a, int vectors, hipStream_t s) {
     const int nvec = (vectors + kFThreads - 1) / kFThreads;  // per lane of a wide workgroup
-    if (nvec > kWideVec + kMaxLdsVec) return launch_fused_wide<DT, kMaxLdsVec, true, R>(a, rows, s);
+    if (nvec > kWideVec + kMaxLdsVec) return launch_fused_wide<DT, kMaxLdsVec, true, R>(a, s);
     if (nvec > kMaxVec) {
         switch ((nvec - kWideVec + kLdsStep - 1) / kLdsStep) {
-            case 1: return launch_fused_wide<DT, 3, false, R>(a, rows, s);
-            case 2: return launch_fused_wide<DT, 6, false, R>(a, rows, s);
-            default: return launch_fused_wide<DT, 9, false, R>(a, rows, s);
+            case 1: return launch_fused_wide<DT, 3, false, R>(a, s);
+            case 2: return launch_fused_wide<DT, 6, false, R>(a, s);
+            default: return launch_fused_wide<DT, 9, false, R>(a, s);
         }
     }
 #define TRLK_LAUNCH_FUSED(NVEC, TH) \
-    hipLaunchKernelGGL((grpo_fused_kernel<DT, NVEC, 0, false, R, TH>), dim3((rows + 7) / 8 * 8), dim3(TH), 0, s, a)
+    hipLaunchKernelGGL((grpo_fused_kernel<DT, NVEC, 0, false, R, TH>), dim3(a.grid), dim3(TH), 0, s, a)
     const int narrow = (vectors + kNarrowThreads - 1) / kNarrowThreads;
     switch (narrow <= kNarrowVec ? (narrow + kVecStep - 1) / kVecStep : 0) {
         case 1: TRLK_LAUNCH_FUSED(4, kNarrowThreads); return TRLK_OK;
@@ -555,8 +560,8 @@ int launch_fused(const FusedArgs& a, int vectors, unsigned rows, hipStream_t s) 
 }
 
 template <int DT>
-int launch_fused_any(const FusedArgs& a, int vectors, bool ragged, unsigned rows, hipStream_t s) {
-    return ragged ? launch_fused<DT, true>(a, vectors, rows, s) : launch_fused<DT, false>(a, vectors, rows, s);
+int launch_fused_any(const FusedArgs& a, int vectors, bool ragged, hipStream_t s) {
+    return ragged ? launch_fused<DT, true>(a, vectors, s) : launch_fused<DT, false>(a, vectors, s);
 }
 
 // data *= *scale over 16-byte vectors, unless the scale is exactly 1 (then nothing is read or written, and what the
@@ -737,9 +742,12 @@ extern "C" int trlk_grpo_fused_fwd_bwd(const void* d_logits, int dtype, int64_t 
     const bool lines = !ragged && reinterpret_cast<uintptr_t>(d_dlogits) % 128 == 0 && (out_seq_stride * es) % 128 == 0 &&
                        (out_row_stride * es) % 128 == 0;
     const int vectors = int(vocab / epv) + (lines ? 0 : kSkew);
-    if (int rc = dtype == TRLK_BF16  ? launch_fused_any<TRLK_BF16>(a, vectors, ragged, unsigned(orows), s)
-                 : dtype == TRLK_F16 ? launch_fused_any<TRLK_F16>(a, vectors, ragged, unsigned(orows), s)
-                                     : launch_fused_any<TRLK_F32>(a, vectors, ragged, unsigned(orows), s))
+    const int64_t run_bytes = vectors <= kNarrowVec * kNarrowThreads ? kNarrowRunBytes : kWideRunBytes;
+    a.run = xcd_run(orows, run_bytes / (vocab * es), out_rows_per_seq);
+    a.grid = xcd_grid(orows, a.run);
+    if (int rc = dtype == TRLK_BF16  ? launch_fused_any<TRLK_BF16>(a, vectors, ragged, s)
+                 : dtype == TRLK_F16 ? launch_fused_any<TRLK_F16>(a, vectors, ragged, s)
+                                     : launch_fused_any<TRLK_F32>(a, vectors, ragged, s))
         return rc;
     return launch_status("grpo_fused");
 }

@@ -409,6 +409,7 @@ struct BwdArgs {
     void* dlogits;
     int64_t out_rows_per_seq, out_row_offset, out_seq_stride, out_row_stride;
     int64_t total_chunks;  // rows x chunks per row
+    unsigned run;          // chunks of an XCD side by side (see xcd_piece)
 };
 
 // The backward has no reduction, so a row is cut into chunks of kChunkElems elements and one
@@ -416,6 +417,12 @@ struct BwdArgs {
 // (row-major), which keeps the read and write streams of the whole grid inside a narrow,
 // DRAM-page-friendly window instead of thousands of rows apart.
 constexpr int kChunkBytes = kThreads * kBwdUnroll * 16;
+// Chunks that follow each other on one XCD: 264 KiB.  bf16, completions of 1/16 of the longest to the longest, against one
+// contiguous eighth of the buffer per XCD: [16, 512, 151936] 680-699 -> 596-601 us, [16, 1024, 128257] 1132-1168 -> 1016-1032,
+// [32, 900, 32001] 491-498 -> 452, [8, 300, 32000] 47 -> 41, [8, 512, 202048] fp32 930 -> 823; every row active 782 -> 758 and
+// 1314 -> 1287.  Completions of one length (half of the rows), which leave no XCD with more: 594 -> 579, but 949 -> 986 at
+// 128257 entries, where a whole eighth makes all XCDs write zeros at the same time.  Runs of 31 to 255 chunks lie within 5 %.
+constexpr int kBwdRun = 33;
 
 template <int DT>
 constexpr int chunk_elems() {
@@ -430,12 +437,7 @@ __global__ __launch_bounds__(kThreads) void logp_entropy_bwd_kernel(BwdArgs a, i
     constexpr int CE = chunk_elems<DT>();
 
     const int tid = threadIdx.x;
-    // The hardware deals consecutive workgroups to the eight XCDs in turn.  Each XCD walks one contiguous eighth of the
-    // chunks (address-linear inside it) instead of every eighth chunk of the whole buffer: eight narrow write windows,
-    // one per XCD.  Measured on bf16 [64, 1024, 151936]: zero-filled rows 3.39 -> 2.97 ms, the benchmark's prefix mask
-    // 5.20 -> 4.95 ms, every row active 6.3 -> 6.5 ms; 16, 32 or 64 such regions are slower than either.
-    const int64_t per_xcd = int64_t(gridDim.x) >> 3;  // (the grid is a multiple of 8)
-    const int64_t linear = int64_t(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    const int64_t linear = xcd_piece(blockIdx.x, a.run);
     if (linear >= a.total_chunks) return;
     const int64_t orow = linear / chunks_per_row;
     const int chunk = int(linear - orow * chunks_per_row);
@@ -685,7 +687,8 @@ extern "C" int trlk_logp_entropy_bwd(const void* d_logits, int dtype, int64_t n_
                  "logp_entropy_bwd: %lld rows x %lld chunks exceed the grid limit", (long long)orows,
                  (long long)chunks_per_row);
     a.total_chunks = orows * chunks_per_row;
-    const dim3 grid((unsigned)(((a.total_chunks + 7) / 8) * 8)), block(kThreads);
+    a.run = xcd_run(a.total_chunks, kBwdRun, out_rows_per_seq * chunks_per_row);
+    const dim3 grid(xcd_grid(a.total_chunks, a.run)), block(kThreads);
     const int cpr = int(chunks_per_row);
 #define TRLK_LAUNCH_BWD(DT)                                                                              \
     if (vec && has_h)                                                                                    \
