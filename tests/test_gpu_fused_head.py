@@ -996,3 +996,36 @@ def test_recomputed_logits_are_those_of_the_forward(amd, monkeypatch, dtype, h, 
     err = float((got - want).abs().max())
     print(f"{dtype} H={h} {form}: 1 - p = {want:.3e}, largest error {err:.2e}, bound {bound:.2e}")
     assert err <= bound
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,h,v", [(1, 8, 64), (65, 72, 63), (200, 264, 65), (257, 136, 1000), (129, 520, 9001), (2304, 64, 300),
+                                   (2305, 64, 300)])
+def test_weight_read_as_it_lies_in_memory(amd, dtype, n, h, v):
+    """One vocabulary chunk and at most 2304 tokens: the dHidden product reads the weight itself, converting a bf16 one on the way
+    (in two scales where the sampled one does not hold it).  Ragged columns and vocabularies inside a buffer of NaN, against
+    float64 and the copy of the weight that several chunks or more tokens take."""
+    g = torch.Generator().manual_seed(n + h + v)
+    hidden = (0.1 * torch.randn(n, h, generator=g)).to(dtype)
+    for outlier in (0.0, 300.0):
+        values = torch.randn(v, h, generator=g) * (0.5 / h**0.5)
+        if outlier:
+            values[v // 2 | 1, h - 1] = outlier  # (the sample has rows 0, 32, ...)
+        weight = torch.full((v + 1, h + 8), float("nan"), dtype=dtype, device=DEV)[:v, :h]
+        weight.copy_(values)
+        labels = torch.randint(0, v, (n,), generator=g)
+        gout = torch.randn(n, generator=g)
+        hd, wd = hidden.double(), weight.double().cpu()
+        p = (hd @ wd.t() / 0.9).softmax(-1)
+        dz = (torch.zeros_like(p).scatter_(1, labels[:, None], 1.0) - p) * gout.double()[:, None] / 0.9
+        want_h, want_w = dz @ wd, dz.t() @ hd
+        args = (hidden.to(DEV), weight, labels.to(DEV), 0.9, 0.0, 1.0)
+        out = amd.ops.fused_head_fwd(*args, None, True)
+        # the outputs round to their type, every term of a sum to fp16 twice (its numerator and its d logit), independently: at
+        # most 2^-12 each, so four times 2 * 2^-12 of the terms' root sum of squares is out of reach
+        unit = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
+        for chunk in (v, max(1, v // 2)):
+            got_h, got_w, _ = amd.ops.fused_head_bwd(*args, out[2], gout.to(DEV), chunk, None, out[4])
+            for got, want, squares in ((got_h, want_h, dz.square() @ wd.square()), (got_w, want_w, dz.square().t() @ hd.square())):
+                err, bound = (got.cpu().double() - want).norm(), unit * want.norm() + 2.0**-9 * squares.sum().sqrt()
+                assert err < bound, (outlier, chunk, float(err), float(bound))

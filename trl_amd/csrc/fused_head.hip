@@ -20,7 +20,8 @@
 // to the last bit),
 // or, when the forward was asked to stash its softmax numerators, from one elementwise sweep over that stash;
 // (2) dHidden += dz * W_chunk: the tile loop with dz as a K-MAJOR operand (its k rows go to LDS as they lie in
-// memory and the MFMA fragments come out through the LDS transpose loads, ds_read_b64_tr_b16) against W_chunk^T;
+// memory and the MFMA fragments come out through the LDS transpose loads, ds_read_b64_tr_b16) against W_chunk, which with few
+// tokens is read k-major too and otherwise comes as a transposed copy;
 // (3) dW_chunk = dz^T * hidden as an NT product against hidden^T, whose columns carry the inverse of the tokens'
 // scales; all on fp16 operands (bf16 inputs are converted while they are transposed).  Both are computed transposed too
 // (M = columns of the output), so that a lane of the accumulator layout holds 4 consecutive columns of one output row.  The contraction of (2)/(3)
@@ -135,17 +136,18 @@ __device__ __forceinline__ int tile_swizzle(int r) { return (r & 7) ^ ((r >> 3) 
 // BKM: the right operand is k-major.  Its stage is then 64 k rows of 512 bytes (256 columns); one transfer fills two
 // k rows; the 16-byte unit at physical position pu of k row r holds logical unit pu ^ ((r & 3) << 1) ^ (r & 8), which
 // spreads the eight k rows that two neighbouring groups of 16 lanes read with a transpose load over all banks.
-template <bool BKM = false>
+// LEFT: the left operand travels this way too (otherwise LeftKm moves it).
+template <bool BKM = false, bool LEFT = true>
 struct DirectLoader {
     static constexpr int kWaves = kHeadThreads / 64, kRowsPerBlk = 1024 / kRowBytes;
-    static constexpr int kBlkA = BM / kRowsPerBlk / kWaves, kBlkB = BN / kRowsPerBlk / kWaves;  // per wave and stage
+    static constexpr int kBlkA = LEFT ? BM / kRowsPerBlk / kWaves : 0, kBlkB = BN / kRowsPerBlk / kWaves;  // per wave and stage
     static constexpr int kStageLoads = kBlkA + kBlkB;
     static_assert(BM % (kRowsPerBlk * kWaves) == 0 && BN % (kRowsPerBlk * kWaves) == 0 && BN == 256, "blocks per wave");
     const char *abase, *bbase;
     char* smem;
     int wave;
     int64_t bkstep;  // bytes between two k of the right operand
-    uint32_t ao[kBlkA], bo[kBlkB];
+    uint32_t ao[LEFT ? kBlkA : 1], bo[kBlkB];
 
     __device__ __forceinline__ DirectLoader(const Operand A, int m0, const Operand B, int n0, char* lds) : smem(lds) {
         const int lane = fresh(threadIdx.x & 63);
@@ -219,28 +221,117 @@ struct DirectLoader {
     }
 };
 
+// The left operand of the dHidden product straight from the weight: k-major (A.p is [krows, A.rows], K = krows rounded up to
+// the k step) and, with CONVERT, bf16 that becomes fp16 times a power of two.  A stage is 64 k rows of 256 columns, laid out
+// like a k-major right operand's; it goes through registers, because the conversion is done on the way: a lane holds 4 vectors
+// of 8 columns, of k rows 16 apart, loaded one step before they are converted and written to the LDS.  k rows beyond the last
+// are read as the last (the other operand is zero there), columns beyond the last as the last 8 (nobody stores them).
+// The conversion is what this costs beside the plain loop: 1392 tokens, H = 2048, V = 128256, backward of a bf16 problem 1562 us,
+// of an fp16 problem (nothing to convert) 1555; behind every MFMA of the refill instead of behind two of three 1577.
+template <bool CONVERT>
+struct LeftKm {
+    static constexpr int kVecs = 4;
+    const char* base;
+    char* lds;
+    uint32_t row_bytes, col;  // (a tile spans less than 4 GiB)
+    int row0, krows;
+    float scale, top;  // top: the largest magnitude converted so far, times the scale
+    __device__ __forceinline__ LeftKm(const Operand A, int m0, int krows_, float scale_, char* smem)
+        : krows(krows_), scale(scale_), top(0.f) {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        base = reinterpret_cast<const char*>(A.p + m0);
+        row_bytes = uint32_t(A.ld * 2);
+        row0 = wave * 2 + (lane >> 5);
+        const int unit = (lane & 31) ^ ((row0 & 3) << 1) ^ (row0 & 8);  // the logical 16-byte unit of this lane, as in DirectLoader
+        col = uint32_t(min(unit * 8, A.rows - m0 - 8)) * 2u;
+        lds = smem + wave * 1024 + lane * 16;
+    }
+    __device__ __forceinline__ void load(int k0, int j, u32x4& w) const {
+        const int row = min(row0 + 16 * j, krows - 1 - k0);
+        w = *reinterpret_cast<const u32x4*>(base + int64_t(k0) * row_bytes + (uint32_t(row) * row_bytes + col));
+    }
+    // two neighbouring columns; exact wherever fp16 holds the scaled value (one rounding to nearest elsewhere)
+    __device__ __forceinline__ void convert(uint32_t& w) {
+        if constexpr (CONVERT) {
+            const float lo = __uint_as_float(w << 16) * scale, hi = __uint_as_float(w & 0xffff0000u) * scale;
+            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(lo), "v"(hi));
+            w = Elem<TRLK_F16>::pack2(lo, hi);
+        }
+    }
+    __device__ __forceinline__ void store(int buf, int j, u32x4 w) const {
+        *reinterpret_cast<u32x4*>(lds + buf * kDenseStage + j * 8192) = w;
+    }
+    // the first two stages into the LDS, the third (or, where there is none, the last) into `w`
+    __device__ __forceinline__ void prologue(int nk, u32x4 (&w)[kVecs]) {
+        u32x4 first[2][kVecs];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < kVecs; ++j) load(min(s, nk - 1) * BK, j, first[s][j]);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < kVecs; ++j) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    uint32_t x = first[s][j][i];
+                    convert(x);
+                    first[s][j][i] = x;
+                }
+                store(s, j, first[s][j]);
+            }
+#pragma unroll
+        for (int j = 0; j < kVecs; ++j) load(min(2, nk - 1) * BK, j, w[j]);
+    }
+};
+struct NoLeftKm {};
+
 // What a wave whose rows or columns all lie beyond the operands does in place of the tile loop: it moves its share of the
 // tiles (exactly the transfers, waits and barriers of the loop) and spends nothing on matrix work.
-template <bool BKM>
-__device__ __forceinline__ void move_tiles_only(const DirectLoader<BKM>& loader, int K, bool prefetched) {
+template <bool BKM, bool LEFT, typename Left = NoLeftKm>
+__device__ __forceinline__ void move_tiles_only(const DirectLoader<BKM, LEFT>& loader, int K, bool prefetched, Left left = {}) {
     const int nk = K / BK;
+    u32x4 w[4];
     if (!prefetched) loader.prologue(K);
-    loader.first_stage_landed(nk);
+    if constexpr (LEFT) {
+        loader.first_stage_landed(nk);
+    } else {
+        left.prologue(nk, w);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+    }
 #pragma unroll 1
     for (int kt = 0; kt < nk; ++kt) {
         __builtin_amdgcn_s_waitcnt(0);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (kt + 2 < nk) loader.issue(kt & 1, (kt + 2) * BK);
+        if (kt + 2 < nk) {
+            loader.issue(kt & 1, (kt + 2) * BK);
+            if constexpr (!LEFT) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        uint32_t x = w[j][i];
+                        left.convert(x);
+                        w[j][i] = x;
+                    }
+                    left.store(kt & 1, j, w[j]);
+                    left.load(min(kt + 3, nk - 1) * BK, j, w[j]);
+                }
+            }
+        }
     }
 }
 
-template <int DT, bool BKM = false>
+// `left`: a LeftKm, where the left operand is k-major.
+template <int DT, bool BKM = false, typename Left = NoLeftKm>
 __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, const Operand B, int n0, int K,
-                                                    f32x4 (&acc)[MI][NI], char* smem) {
-    const DirectLoader<BKM> loader(A, m0, B, n0, smem);
-    constexpr int kStageLoads = DirectLoader<BKM>::kStageLoads;
+                                                    f32x4 (&acc)[MI][NI], char* smem, Left&& left = {}) {
+    constexpr bool AKM = !std::is_same_v<std::decay_t<Left>, NoLeftKm>;
+    const DirectLoader<BKM, !AKM> loader(A, m0, B, n0, smem);
+    constexpr int kStageLoads = DirectLoader<BKM, !AKM>::kStageLoads;
     const int lane = threadIdx.x & 63, wave = loader.wave;
     const int wm = wave_m(wave), wn = wave_n(wave);
 
@@ -259,25 +350,63 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
         for (int j = 0; j < NI; ++j)
             fb_km[j] = (8 * g + (l15 >> 2)) * (BN * 2) + (((wn * WN + j * 16) / 8 + ((l15 & 3) >> 1)) ^ f) * 16 + (l15 & 1) * 8;
     }
+    int fa_km[MI];  // the same for a k-major left operand
+    if constexpr (AKM) {
+        const int f = ((l15 >> 2) << 1) ^ ((g & 1) << 3);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+            fa_km[i] = (8 * g + (l15 >> 2)) * (BM * 2) + (((wm * WM + i * 16) / 8 + ((l15 & 3) >> 1)) ^ f) * 16 + (l15 & 1) * 8;
+    }
+    // (absolute LDS addresses of the stage that is read next, changed over once a step)
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
+    uint32_t at_a[MI], at_b[NI];
+    if constexpr (AKM)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) at_a[i] = lds0 + fa_km[i];
+    if constexpr (BKM)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) at_b[j] = lds0 + kDenseA + fb_km[j];
+    auto other_stage = [&] {
+        static_assert(kDenseStage == 65536, "one address bit tells the stages apart");
+        if constexpr (AKM)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) at_a[i] ^= kDenseStage;
+        if constexpr (BKM)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) at_b[j] ^= kDenseStage;
+    };
+    auto read_tr = [&](uint32_t base, int ks) -> u32x4 {
+        static_assert(BM == BN, "k rows of both operands have one length");
+        const uint32_t at = base + uint32_t(ks * 32 * (BN * 2));
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at + 4 * (BN * 2)));
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        return __builtin_bit_cast(u32x4, both);
+    };
     auto read_a = [&](const char* sa, int i, int ks) -> u32x4 {
-        return *reinterpret_cast<const u32x4*>(sa + fa_row + i * 16 * kRowBytes + koff[ks]);
+        if constexpr (AKM)
+            return read_tr(at_a[i], ks);
+        else
+            return *reinterpret_cast<const u32x4*>(sa + fa_row + i * 16 * kRowBytes + koff[ks]);
     };
     auto read_b = [&](const char* sb, int j, int ks) -> u32x4 {
-        if constexpr (BKM) {
-            const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(sb)) + uint32_t(fb_km[j] + ks * 32 * (BN * 2));
-            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_s16x4*>(at + 4 * (BN * 2)));
-            typedef short s16x8 __attribute__((ext_vector_type(8)));
-            const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            return __builtin_bit_cast(u32x4, both);
-        } else {
+        if constexpr (BKM)
+            return read_tr(at_b[j], ks);
+        else
             return *reinterpret_cast<const u32x4*>(sb + fb_row + j * 16 * kRowBytes + koff[ks]);
-        }
     };
 
     const int nk = K / BK;
+    u32x4 lw[4];  // the left operand's stage kt + 2 at the start of step kt
     loader.prologue(K);
-    loader.first_stage_landed(nk);
+    if constexpr (AKM) {
+        left.prologue(nk, lw);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+    } else {
+        loader.first_stage_landed(nk);
+    }
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -320,6 +449,7 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
             const char* nb = na + kDenseA;
             const bool load = ks == 0 || NEXT;
             int issued = 0, slot = 0;
+            if (ks == 1) other_stage();
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -327,7 +457,12 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
                     if (ks == 1 && half == 0 && i == kBarAt) {
                         // Every fragment read of this stage has returned and the next stage has landed.  A bare s_barrier:
                         // __syncthreads() carries release / acquire fences; nothing may move across it.
-                        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                        // (with a left operand in registers the wait is one that the compiler counts: it need not wait for them again)
+                        if constexpr (AKM)
+                            __builtin_amdgcn_s_waitcnt(0);
+                        else
+                            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                        asm volatile("" ::: "memory");
                         __builtin_amdgcn_sched_barrier(0);
                         __builtin_amdgcn_s_barrier();
                         __builtin_amdgcn_sched_barrier(0);
@@ -343,9 +478,24 @@ __device__ __forceinline__ void gemm_tile_nt_direct(const Operand A, int m0, con
                             if (i == MI - 1) b[j] = read_b(nb, j, ks ^ 1);
                         }
                         if (REFILL && ks == 1 && (half == 1 || i >= kBarAt)) {
-                            if ((slot & 1) && issued < kStageLoads) {
+                            if ((AKM ? slot % 3 == 2 : (slot & 1)) && issued < kStageLoads) {
                                 loader.issue_one(kt & 1, (kt + 2) * BK, issued);
                                 ++issued;
+                            }
+                            // a pair of columns behind two of three MFMAs (its six instructions keep the vector unit as busy as
+                            // three MFMAs of the SIMD's two waves do the matrix unit); a vector that is whole makes room
+                            // for the next stage's
+                            if constexpr (AKM) {
+                                if (slot % 3 != 2) {
+                                    const int pair = slot - slot / 3;
+                                    uint32_t x = lw[pair >> 2][pair & 3];
+                                    left.convert(x);
+                                    lw[pair >> 2][pair & 3] = x;
+                                    if ((pair & 3) == 3) {
+                                        left.store(kt & 1, pair >> 2, lw[pair >> 2]);
+                                        left.load(min(kt + 3, nk - 1) * BK, pair >> 2, lw[pair >> 2]);
+                                    }
+                                }
                             }
                             ++slot;
                         }
@@ -622,11 +772,11 @@ __device__ __forceinline__ void fwd_tile_staged(const Operand A, int m0, const O
     });
 }
 
-template <int DT, bool BKM = false>
+template <int DT, bool BKM = false, typename Left = NoLeftKm>
 __device__ __forceinline__ void gemm_tile_nt(const Operand A, int m0, const Operand B, int n0, int K,
-                                             f32x4 (&acc)[MI][NI], char* smem) {
+                                             f32x4 (&acc)[MI][NI], char* smem, Left&& left = {}) {
     if constexpr (BKM) {  // (callers of this form pad K to whole steps)
-        gemm_tile_nt_direct<DT, true>(A, m0, B, n0, K, acc, smem);
+        gemm_tile_nt_direct<DT, true>(A, m0, B, n0, K, acc, smem, left);
     } else {
         if ((K & (BK - 1)) == 0)
             gemm_tile_nt_direct<DT>(A, m0, B, n0, K, acc, smem);
@@ -1327,6 +1477,10 @@ struct GemmArgs {
     const uint32_t* max_a;
     const uint32_t* max_b;
     const uint32_t* beyond_b;  // B is the weight: max_b and this are the two slots of weight_scale()
+    // B is the weight itself, [b_krows, N] as it lies in memory, not a transposed copy (bf16: converted on its way in the scale
+    // of the sample, what exceeds it is left in beyond_out).
+    int b_krows;
+    uint32_t* beyond_out;
     const float* g_rows;
     float mult_a;
     // K-major A, epilogue 1: the contraction cut into `slices` pieces of `kslice` (a multiple of the k step), each
@@ -1336,13 +1490,14 @@ struct GemmArgs {
 };
 
 // DT: dtype of the operands (the matrix-core instruction), ODT: storage dtype of `out_lp`.
-// AKM: A is given k-major ([K, M], leading dimension A.ld).
-template <int DT, int MODE, int ODT, bool AKM = false>
+// AKM: A is given k-major ([K, M], leading dimension A.ld).  BW: B is the weight in its own layout and dtype (ODT); AGAIN: the
+// sample's scale did not do, it is converted in that of its largest entry.
+template <int DT, int MODE, int ODT, bool AKM = false, bool BW = false, bool AGAIN = false>
 __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char* smem) {
     typedef Elem<ODT> E;
     const int n_mt = (a.M + BN - 1) / BN, n_nt = (a.N + BM - 1) / BM;
     Operand A = a.A, B = a.B;
-    int K = a.K;
+    int K = a.K, b_krows = a.b_krows;
     float* out_f32 = a.out_f32;
     constexpr bool kSlices = AKM && MODE == 1;
     const int n_cols = kSlices ? n_nt * a.slices : n_nt;
@@ -1353,7 +1508,8 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
         const int slice = tn / n_nt, k0 = slice * a.kslice;
         tn -= slice * n_nt;
         A.p += int64_t(k0) * A.ld;
-        B.p += k0;
+        B.p += BW ? int64_t(k0) * B.ld : int64_t(k0);
+        b_krows -= k0;
         K = min(a.kslice, K - k0);
         out_f32 += int64_t(slice) * a.M * a.ld_f32;
     }
@@ -1362,10 +1518,34 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     const int r0 = tm * BN, c0 = tn * BM;  // the tile's first row and column of the output
     f32x4 acc[MI][NI];
     const bool idle = r0 + wn * WN >= a.M || c0 + wm * WM >= a.N;  // all of this wave's rows or columns lie beyond the output
-    if (idle && (AKM || (K & (BK - 1)) == 0)) return move_tiles_only(DirectLoader<AKM>(B, c0, A, r0, smem), K, false);
-    gemm_tile_nt<DT, AKM>(B, c0, A, r0, K, acc, smem);
-    if (idle) return;  // (no barrier follows)
-    const float inv_b = 1.f / (a.beyond_b != nullptr ? weight_scale(a.max_b, a.beyond_b).scale : slot_scale(a.max_b, 1.f));
+    float inv_b;
+    if constexpr (BW) {
+        constexpr bool kConvert = ODT == TRLK_BF16;
+        const float scale = uniform(!kConvert ? 1.f : AGAIN ? weight_scale(a.max_b, a.beyond_out).scale : slot_scale(a.max_b, 1.f));
+        typedef LeftKm<kConvert> Left;
+        Left left(B, c0, b_krows, scale, smem);
+        if (idle)
+            move_tiles_only<true, false, Left&>(DirectLoader<true, false>(B, c0, A, r0, smem), K, false, left);
+        else
+            gemm_tile_nt<DT, true>(B, c0, A, r0, K, acc, smem, left);
+        if (kConvert && !AGAIN) {
+            uint32_t m = __float_as_uint(left.top / scale);
+            const uint32_t known = max(*a.max_b, __hip_atomic_load(a.beyond_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if (__any(m > known)) {
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off, 64)));
+                if (lane == 0) atomicMax(a.beyond_out, m);
+            }
+        }
+        if (idle) return;  // (no barrier follows)
+        inv_b = 1.f / scale;
+    } else {
+        if (idle && (AKM || (K & (BK - 1)) == 0))
+            return move_tiles_only(DirectLoader<AKM>(B, c0, A, r0, smem), K, false);
+        gemm_tile_nt<DT, AKM>(B, c0, A, r0, K, acc, smem);
+        if (idle) return;  // (no barrier follows)
+        inv_b = 1.f / (a.beyond_b != nullptr ? weight_scale(a.max_b, a.beyond_b).scale : slot_scale(a.max_b, 1.f));
+    }
     const float inv_common = inv_b / slot_scale(a.max_a, a.mult_a);
     const int g = lane >> 4;
     // The wave's 128 columns inside the output (nearly every tile), rows aligned for vector accesses: a row's 8 running
@@ -1436,13 +1616,20 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
 // Two independent products in one launch: workgroups [0, grid_a) take `a` (epilogue MODE_A; its left operand is
 // k-major), the rest take `b` (epilogue 0).  When the tile count of one product is not a multiple of the CU count, the other product's
 // tiles fill the CUs its last round leaves idle.  grid_a is a multiple of 8 (the XCD mapping of `b` is kept).
-template <int MODE_A, int ODT>
+template <int MODE_A, int ODT, bool BW>
 TRLK_HEAD_KERNEL void gemm_nt_pair_kernel(GemmArgs a, int grid_a, GemmArgs b) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     if (int(blockIdx.x) < grid_a)
-        gemm_nt_body<TRLK_F16, MODE_A, ODT, true>(a, blockIdx.x, smem);
+        gemm_nt_body<TRLK_F16, MODE_A, ODT, true, BW>(a, blockIdx.x, smem);
     else
         gemm_nt_body<TRLK_F16, 0, ODT>(b, int(blockIdx.x) - grid_a, smem);
+}
+// The first of the two once more, where the sample's scale did not hold all of a bf16 weight: returns at once everywhere else.
+template <int MODE_A>
+TRLK_HEAD_KERNEL void gemm_nt_again_kernel(GemmArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    if (!weight_scale(a.max_b, a.beyond_out).again) return;
+    gemm_nt_body<TRLK_F16, MODE_A, TRLK_BF16, true, true, true>(a, blockIdx.x, smem);
 }
 
 // dHidden from the sums of the slices of its contraction, in slice order: out[i] = sum_s parts[s][i], 8 values per lane
@@ -1711,6 +1898,7 @@ struct BwdLayout {
     int64_t ld_v, ld_n, ld_c;    // row strides of [*, vpad], [*, npad], [*, cpad] matrices
     size_t off_wt, off_ht, off_dzt, off_dh, off_max, total;
     int64_t n_chunks;
+    bool direct;         // the dHidden product reads the weight itself: no transposed copy
     int slices, kslice;  // of the dHidden product's contraction over a chunk
 };
 // Slices of the contraction of the dHidden product.  Its tiles (token blocks x hidden tiles) contract over the whole
@@ -1736,6 +1924,15 @@ int dh_slices(int64_t n_tb, int64_t n_ht, int64_t kpad, int64_t npad) {
     }
     return best;
 }
+// Up to this many tokens the dHidden product takes the weight as it lies in memory (LeftKm) and not a transposed fp16 copy.  The
+// copy costs the same for every token count (525 MB read, 525 written: 193 us of a backward for V = 128256, H = 2048; 390 us for
+// 151936 x 3584), the conversion in the tile loop 5 to 10 % of the product.  Whole backward with the copy -> without, in us:
+// 100 tokens, H = 3584, V = 151936 1341 -> 859; 459 the same 1712 -> 1263; 300, H = 1024, V = 128256 506 -> 388; 900, H = 2560,
+// V = 151665 1784 -> 1557; 1396, H = 2048, V = 50257 710 -> 648; 1392, V = 128256 1662 -> 1562; 2300, H = 4096, V = 50264
+// 1800 -> 1760; from there on it loses: 2600, H = 3584, V = 151936 5298 -> 5340, 3300, H = 2048, V = 128256 3305 -> 3325, 7000,
+// V = 50264 2653 -> 2735.  Only with the whole vocabulary in one chunk: a product that has to be done again (weight_scale) then
+// overwrites what the first attempt left, and never a sum over several chunks.
+constexpr int64_t kDirectTokens = 2304;
 BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     BwdLayout l;
     l.vpad = round_up(V, BK);
@@ -1750,7 +1947,8 @@ BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
         o += (bytes + 255) / 256 * 256;
         return at;
     };
-    l.off_wt = take(size_t(H) * l.ld_c * 2);
+    l.direct = l.cpad >= V && N <= kDirectTokens;
+    l.off_wt = take(l.direct ? 0 : size_t(H) * l.ld_c * 2);
     l.off_ht = take(size_t(H) * l.ld_n * 2);
     l.off_dzt = take(size_t(l.cpad) * l.ld_n * 2);
     const int want = dh_slices(l.npad / BN, (H + BN - 1) / BN, l.cpad, l.npad);
@@ -2092,7 +2290,8 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         const uint32_t* max_w = from_bf16 ? maxima + 2 : nullptr;
         uint32_t* beyond_w = from_bf16 ? maxima + 3 + c0 / chunk : nullptr;
         const dim3 tgrid((H + 63) / 64, unsigned((kpad + 63) / 64));
-        if (from_bf16) {
+        if (l.direct) {
+        } else if (from_bf16) {
             hipLaunchKernelGGL(transpose_weight_kernel, tgrid, dim3(256), 0, s, w_chunk, weight_stride, rows, H, wt, l.ld_c,
                                int64_t(kpad), max_w, beyond_w);
             const int tiles = int(tgrid.x * tgrid.y);
@@ -2120,8 +2319,14 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         gh.mult_a = zs;
         gh.max_b = max_w;
         gh.beyond_b = beyond_w;
+        if (l.direct) {
+            gh.B = Operand{w_chunk, weight_stride, H};
+            gh.K = int(round_up(rows, BK));
+            gh.b_krows = rows;
+            gh.beyond_out = beyond_w;
+        }
         gh.slices = l.slices;  // (of the last, possibly shorter chunk those that its rows reach)
-        while (gh.slices > 1 && int64_t(gh.slices - 1) * l.kslice >= kpad) --gh.slices;
+        while (gh.slices > 1 && int64_t(gh.slices - 1) * l.kslice >= gh.K) --gh.slices;
         gh.kslice = l.kslice;
         const int ghgrid = xcd_patch_grid(n_tb, n_ht * gh.slices);
         // dW[chunk, H] = dz^T[chunk, N] * (hidden^T[H, N])^T
@@ -2141,12 +2346,21 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         // both products of the chunk in one launch (dHidden's workgroups first)
         const int gwgrid = xcd_patch_grid(n_vt, n_ht);
         const char* what = "fused_head_bwd (dHidden, dW)";
+        auto launch_pair = [&](auto mode_tag, auto bw_tag) {
+            constexpr int kMode = decltype(mode_tag)::value;
+            constexpr bool kBW = decltype(bw_tag)::value;
+            int rc2 = from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<kMode, TRLK_BF16, kBW>, ghgrid, gh, gwgrid, gw, s, what)
+                                : launch_head_pair(gemm_nt_pair_kernel<kMode, TRLK_F16, kBW>, ghgrid, gh, gwgrid, gw, s, what);
+            if (kBW && from_bf16 && rc2 == TRLK_OK)
+                rc2 = launch_head(gemm_nt_again_kernel<kMode>, ghgrid, gh, s, "fused_head_bwd (dHidden again)");
+            return rc2;
+        };
+        typedef std::integral_constant<int, 1> accumulate_t;
+        typedef std::integral_constant<int, 2> round_t;
         if (last && l.slices == 1)
-            rc = from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<2, TRLK_BF16>, ghgrid, gh, gwgrid, gw, s, what)
-                           : launch_head_pair(gemm_nt_pair_kernel<2, TRLK_F16>, ghgrid, gh, gwgrid, gw, s, what);
+            rc = l.direct ? launch_pair(round_t{}, std::true_type{}) : launch_pair(round_t{}, std::false_type{});
         else
-            rc = from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<1, TRLK_BF16>, ghgrid, gh, gwgrid, gw, s, what)
-                           : launch_head_pair(gemm_nt_pair_kernel<1, TRLK_F16>, ghgrid, gh, gwgrid, gw, s, what);
+            rc = l.direct ? launch_pair(accumulate_t{}, std::true_type{}) : launch_pair(accumulate_t{}, std::false_type{});
         if (rc) return rc;
     }
     if (l.slices > 1) {

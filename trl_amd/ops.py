@@ -775,10 +775,15 @@ def mean_logits(hidden, weight):
 # raised to what this much scratch holds, and the vocabulary is cut into equal chunks.  1396 tokens, H = 2048, V = 50257,
 # chunk_size 8192: one chunk instead of seven, products 1136 -> 575 us (with the slices of the dHidden product), sweeps
 # and transposes 189 -> 126 us.  Where that scratch cannot be allocated, the caller's own size is what it can have.
+# With few tokens one chunk needs no copy of the weight at all (`trlk_fused_head_bwd` decides) and fits where two with a copy
+# were needed: 459 tokens, H = 3584, V = 151936, whole backward 1712 -> 1263 us.
 _HEAD_SCRATCH_BYTES = 1 << 30
 
 
 def _backward_chunk(n_tokens: int, vocab: int, hidden_size: int, chunk_size: int) -> int:
+    hidden_size = (hidden_size + 7) // 8 * 8
+    if lib.trlk_fused_head_bwd_workspace_bytes(n_tokens, vocab, hidden_size, vocab) <= _HEAD_SCRATCH_BYTES:
+        return vocab
     rows = max(int(chunk_size), _HEAD_SCRATCH_BYTES // (2 * ((n_tokens + 255) // 256 * 256 + hidden_size)))
     return -(-vocab // -(-vocab // rows))
 
