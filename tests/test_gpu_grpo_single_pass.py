@@ -1144,3 +1144,50 @@ def test_rows_dealt_to_the_xcds_in_runs(amd, dtype, B, K):
     poisoned_memory()
     (grad,) = torch.autograd.grad(loss, leaf)
     assert bool(((grad.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("upstream", [None, 0.25], ids=["whole", "announced"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+def test_native_node_of_the_loss(amd, dtype, upstream, monkeypatch):
+    """The loss's native backward node against the Python one that traced calls take: the same loss and gradient to the bit, also
+    with a factor between loss and backward and with saved-tensor hooks; and what the Python node refuses stays refused."""
+    from trl_amd.trainer import grpo_trainer
+
+    logits, ids, mask, adv, _ = _inputs(3, 9, 4096, dtype, seed=5)
+
+    def step(leaf, **kw):
+        return amd.grpo_loss_from_logits(leaf, ids, adv, mask, num_items_in_batch=20.0, upstream_scale=upstream, **kw)
+
+    grads, losses = [], []
+    for native in (True, False):
+        with monkeypatch.context() as m:
+            if not native:
+                m.setattr(torch.compiler, "is_compiling", lambda: True)
+            leaf = logits.clone().requires_grad_(True)
+            packed = []
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.clone()) or len(packed) - 1, lambda i: packed[i]):
+                loss, metrics, logp, ent = step(leaf)
+            assert ("GradientInHand" in loss.grad_fn.name()) == native and any(t.shape == leaf.shape for t in packed)
+            assert not any(t.requires_grad for t in (metrics, logp, ent))
+            losses.append(loss.detach().clone())
+            loss *= 0.25  # (in place)
+            loss.backward()
+            grads.append(leaf.grad)
+    assert torch.equal(*losses) and torch.equal(*grads) and float(grads[0].abs().sum()) > 0
+
+    leaf = logits.clone().requires_grad_(True)
+    loss = step(leaf)[0]
+    loss.backward(retain_graph=True)
+    with pytest.raises(RuntimeError, match="can run only once"):
+        loss.backward()
+    factor = torch.ones((), device=DEV, requires_grad=True)
+    (grad,) = torch.autograd.grad(step(leaf)[0] * factor, leaf, create_graph=True)
+    with pytest.raises(RuntimeError, match="differentiate twice"):
+        grad.float().sum().backward()
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(leaf, torch.ones_like(leaf))
+        with pytest.raises(RuntimeError, match="forward AD|jvp|forward mode"):
+            step(dual)
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: step(x)[0])(logits)
+    assert grpo_trainer.forward_ad._current_level == -1

@@ -388,6 +388,8 @@ def scale_unless_one_(data: Tensor, scale: Tensor) -> Tensor:
 # --------------------------------------------------------------------------------------------
 # What `_compute_loss` logs of the loss kernel's `metrics`, as one fp32 device vector (`trlk_grpo_log_values`): nine sums to be
 # added over the processes, the smallest and the largest clip ratio, the policy loss, the error word.
+gradient_in_hand = torch.ops.trl_amd.gradient_in_hand.default
+
 grpo_log_values = _native_op("grpo_log_values",
                              lambda metrics: metrics.new_empty((_lib.GRPO_LOG_VALUES,), dtype=torch.float32))
 

@@ -15,6 +15,7 @@ import math
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from .. import _lib, ops
 from .utils import logps_and_entropies, nanmax, nanmin  # noqa: F401  (re-exported for callers that patch)
@@ -264,77 +265,85 @@ def grpo_single_pass_supported(logits: Tensor, loss_type: str = "dapo", importan
     return vocab >= (per_vector if whole else 2 * per_vector)
 
 
+def _one_pass(logits, completion_ids, advantages, mask, temperature, kw):
+    """`(loss, metrics, log-probs, entropies, d logits, upstream factor or None)`, all outside any graph: loss and gradient
+    from one pass over the logits."""
+    length = logits.shape[1]
+    if kw["keep_start"] is None:
+        keep_len = min(completion_ids.shape[1], length - 1)
+        keep_start = length - 1 - keep_len
+    else:
+        keep_len, keep_start = completion_ids.shape[1], int(kw["keep_start"])
+        if keep_start < 0 or keep_start + keep_len > length:
+            raise ValueError("grpo_loss_from_logits: keep_start + K exceeds the logits' rows")
+    ids = completion_ids[:, -keep_len:] if keep_len > 0 else completion_ids[:, :0]
+    mask = mask[:, -keep_len:] if keep_len > 0 else mask[:, :0]
+    n_seq = logits.shape[0]
+    reduce_code, term_code = ops.LOSS_TYPES[kw["loss_type"]]
+    ga = 1.0 if reduce_code == _lib.DAPO else float(kw["grad_accum_steps"])
+    up = kw.get("upstream_scale")
+    if up is not None:
+        # the caller will multiply the loss by this factor before backward (a gradient scaler's scale, a loss
+        # divisor): the gradient is written already scaled -- before its single rounding to the logits dtype --
+        # and `backward` has nothing left to do
+        up = (up.to(device=logits.device, dtype=torch.float32).reshape(()) if torch.is_tensor(up)
+              else torch.tensor(float(up), dtype=torch.float32, device=logits.device))
+    n_items = kw["num_items_in_batch"]
+    # d loss / d (masked token loss of sequence b), times the announced factor: what the loss kernel's second pass
+    # applies to its rows
+    if reduce_code == _lib.DAPO:
+        n_items = (n_items.to(device=logits.device, dtype=torch.float32).reshape(()) if torch.is_tensor(n_items)
+                   else torch.tensor(float(n_items), dtype=torch.float32, device=logits.device))
+        numerator = float(kw["num_processes"])
+    elif reduce_code == _lib.DR_GRPO:
+        numerator = 1.0 / float(n_seq * kw["max_completion_length"]) / ga
+    else:
+        numerator = 1.0 / (n_seq if reduce_code == _lib.GRPO else 1) / ga
+    mask_f, row_scale = ops.grpo_row_scale(mask, reduce_code, numerator, n_items if reduce_code == _lib.DAPO else None, up)
+    ent_weight = None
+    if kw["entropy_coef"] != 0.0:  # d loss / d entropy = -coef * mask / normaliser (grpo_trainer.py:3155-3181)
+        if reduce_code == _lib.DAPO:
+            ent_weight = mask_f * (-float(kw["entropy_coef"]) * row_scale[0])
+        else:
+            ent_weight = mask_f * (-float(kw["entropy_coef"]) / mask_f.sum().clamp(min=1.0) / ga)
+            if up is not None:
+                ent_weight = ent_weight * up
+    delta = kw["delta"]
+    logp, ent, _, dlogits = ops.grpo_fused_fwd_bwd(
+        logits, ids, float(temperature), keep_start, keep_len, mask_f, advantages, row_scale,
+        kw["old_per_token_logps"], kw["ref_per_token_logps"] if kw["beta"] != 0.0 else None, kw["token_weight"],
+        None, term_code, float(kw["epsilon_low"]), float(kw["epsilon_high"]),
+        math.nan if delta is None else float(delta), float(kw["beta"]), bool(kw["use_bias_correction_kl"]),
+        float(kw["sapo_temperature_pos"]), float(kw["sapo_temperature_neg"]), False, ent_weight)
+    if not kw["skip_masked_rows"] and keep_len > 0:
+        # the outputs of the rows without gradient come from the streaming forward kernel, which reads them
+        # faster than the one-workgroup-per-CU kernel would (its `compute_masked_rows` mode)
+        rest = mask_f == 0
+        lp0, ent0, _ = ops.logp_entropy_fwd(logits.detach(), ids.reshape(-1, 1), float(temperature), keep_start,
+                                            keep_len, rest.view(torch.uint8).reshape(-1))
+        logp = torch.where(rest, lp0.view_as(logp), logp)
+        ent = torch.where(rest, ent0.view_as(ent), ent)
+    # loss value and every metric from the [B, K]-sized kernel, on the log-probs of the same pass
+    loss, metrics = grpo_loss(
+        logp, advantages, mask_f, entropies=ent, old_per_token_logps=kw["old_per_token_logps"],
+        ref_per_token_logps=kw["ref_per_token_logps"], loss_type=kw["loss_type"], epsilon_low=kw["epsilon_low"],
+        epsilon_high=kw["epsilon_high"], beta=kw["beta"], delta=delta,
+        max_completion_length=kw["max_completion_length"], num_items_in_batch=n_items,
+        num_processes=kw["num_processes"], grad_accum_steps=kw["grad_accum_steps"],
+        use_bias_correction_kl=kw["use_bias_correction_kl"], token_weight=kw["token_weight"],
+        entropy_coef=kw["entropy_coef"],
+        sapo_temperature_pos=kw["sapo_temperature_pos"], sapo_temperature_neg=kw["sapo_temperature_neg"])
+    return loss, metrics, logp, ent, dlogits, up
+
+
 class _GRPOFromLogits(torch.autograd.Function):
     """loss (and the detached log-probs / entropies) from the logits; the gradient w.r.t. the logits was
-    written by the same pass and is only scaled by the upstream gradient in `backward`."""
+    written by the same pass and is only scaled by the upstream gradient in `backward`.  For calls that are traced or
+    transformed; others take the native node (`gradient_in_hand`), which neither tracers nor transforms follow."""
 
     @staticmethod
     def forward(ctx, logits, completion_ids, advantages, mask, temperature, kw):
-        length = logits.shape[1]
-        if kw["keep_start"] is None:
-            keep_len = min(completion_ids.shape[1], length - 1)
-            keep_start = length - 1 - keep_len
-        else:
-            keep_len, keep_start = completion_ids.shape[1], int(kw["keep_start"])
-            if keep_start < 0 or keep_start + keep_len > length:
-                raise ValueError("grpo_loss_from_logits: keep_start + K exceeds the logits' rows")
-        ids = completion_ids[:, -keep_len:] if keep_len > 0 else completion_ids[:, :0]
-        mask = mask[:, -keep_len:] if keep_len > 0 else mask[:, :0]
-        n_seq = logits.shape[0]
-        reduce_code, term_code = ops.LOSS_TYPES[kw["loss_type"]]
-        ga = 1.0 if reduce_code == _lib.DAPO else float(kw["grad_accum_steps"])
-        up = kw.get("upstream_scale")
-        if up is not None:
-            # the caller will multiply the loss by this factor before backward (a gradient scaler's scale, a loss
-            # divisor): the gradient is written already scaled -- before its single rounding to the logits dtype --
-            # and `backward` has nothing left to do
-            up = (up.to(device=logits.device, dtype=torch.float32).reshape(()) if torch.is_tensor(up)
-                  else torch.tensor(float(up), dtype=torch.float32, device=logits.device))
-        n_items = kw["num_items_in_batch"]
-        # d loss / d (masked token loss of sequence b), times the announced factor: what the loss kernel's second pass
-        # applies to its rows
-        if reduce_code == _lib.DAPO:
-            n_items = (n_items.to(device=logits.device, dtype=torch.float32).reshape(()) if torch.is_tensor(n_items)
-                       else torch.tensor(float(n_items), dtype=torch.float32, device=logits.device))
-            numerator = float(kw["num_processes"])
-        elif reduce_code == _lib.DR_GRPO:
-            numerator = 1.0 / float(n_seq * kw["max_completion_length"]) / ga
-        else:
-            numerator = 1.0 / (n_seq if reduce_code == _lib.GRPO else 1) / ga
-        mask_f, row_scale = ops.grpo_row_scale(mask, reduce_code, numerator, n_items if reduce_code == _lib.DAPO else None, up)
-        ent_weight = None
-        if kw["entropy_coef"] != 0.0:  # d loss / d entropy = -coef * mask / normaliser (grpo_trainer.py:3155-3181)
-            if reduce_code == _lib.DAPO:
-                ent_weight = mask_f * (-float(kw["entropy_coef"]) * row_scale[0])
-            else:
-                ent_weight = mask_f * (-float(kw["entropy_coef"]) / mask_f.sum().clamp(min=1.0) / ga)
-                if up is not None:
-                    ent_weight = ent_weight * up
-        delta = kw["delta"]
-        logp, ent, _, dlogits = ops.grpo_fused_fwd_bwd(
-            logits, ids, float(temperature), keep_start, keep_len, mask_f, advantages, row_scale,
-            kw["old_per_token_logps"], kw["ref_per_token_logps"] if kw["beta"] != 0.0 else None, kw["token_weight"],
-            None, term_code, float(kw["epsilon_low"]), float(kw["epsilon_high"]),
-            math.nan if delta is None else float(delta), float(kw["beta"]), bool(kw["use_bias_correction_kl"]),
-            float(kw["sapo_temperature_pos"]), float(kw["sapo_temperature_neg"]), False, ent_weight)
-        if not kw["skip_masked_rows"] and keep_len > 0:
-            # the outputs of the rows without gradient come from the streaming forward kernel, which reads them
-            # faster than the one-workgroup-per-CU kernel would (its `compute_masked_rows` mode)
-            rest = mask_f == 0
-            lp0, ent0, _ = ops.logp_entropy_fwd(logits.detach(), ids.reshape(-1, 1), float(temperature), keep_start,
-                                                keep_len, rest.view(torch.uint8).reshape(-1))
-            logp = torch.where(rest, lp0.view_as(logp), logp)
-            ent = torch.where(rest, ent0.view_as(ent), ent)
-        # loss value and every metric from the [B, K]-sized kernel, on the log-probs of the same pass
-        loss, metrics = grpo_loss(
-            logp, advantages, mask_f, entropies=ent, old_per_token_logps=kw["old_per_token_logps"],
-            ref_per_token_logps=kw["ref_per_token_logps"], loss_type=kw["loss_type"], epsilon_low=kw["epsilon_low"],
-            epsilon_high=kw["epsilon_high"], beta=kw["beta"], delta=delta,
-            max_completion_length=kw["max_completion_length"], num_items_in_batch=n_items,
-            num_processes=kw["num_processes"], grad_accum_steps=kw["grad_accum_steps"],
-            use_bias_correction_kl=kw["use_bias_correction_kl"], token_weight=kw["token_weight"],
-            entropy_coef=kw["entropy_coef"],
-            sapo_temperature_pos=kw["sapo_temperature_pos"], sapo_temperature_neg=kw["sapo_temperature_neg"])
+        loss, metrics, logp, ent, dlogits, up = _one_pass(logits, completion_ids, advantages, mask, temperature, kw)
         ctx.save_for_backward(dlogits, *(() if up is None else (up,)))
         ctx.mark_non_differentiable(metrics, logp, ent)
         ctx.set_materialize_grads(False)  # (no zero tensors for the outputs that carry no gradient)
@@ -442,7 +451,12 @@ def grpo_loss_from_logits(
               use_bias_correction_kl=use_bias_correction_kl, token_weight=token_weight, entropy_coef=entropy_coef,
               sapo_temperature_pos=sapo_temperature_pos, sapo_temperature_neg=sapo_temperature_neg,
               skip_masked_rows=skip_masked_rows, keep_start=keep_start, upstream_scale=upstream_scale)
-    return _GRPOFromLogits.apply(logits, completion_ids, advantages, mask, temperature, kw)
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0):
+        return _GRPOFromLogits.apply(logits, completion_ids, advantages, mask, temperature, kw)
+    with torch.no_grad():
+        loss, metrics, logp, ent, dlogits, up = _one_pass(logits, completion_ids, advantages, mask, temperature, kw)
+    return ops.gradient_in_hand(loss, logits, dlogits, up), metrics, logp, ent
 
 
 class GRPOLossMixin:
@@ -695,14 +709,12 @@ class GRPOLossMixin:
         # (the kernels' error word rides along: a token id outside the vocabulary raises here, as the reference's
         # gather would, instead of surfacing as a NaN loss)
         values = ops.grpo_log_values(metrics.detach())
-        sums, low_min, high_max = values[:9], values[9:10], values[10:11]
         if self.accelerator.num_processes == 1:  # (accelerate's `reduce` would return a copy)
-            lows, highs, host = low_min, high_max, values.tolist()
+            n, host = 1, values.tolist()
         else:
-            totals = self.accelerator.reduce(sums, reduction="sum")
-            lows, highs = self.accelerator.gather(low_min), self.accelerator.gather(high_max)
-            host = torch.cat([totals, lows.reshape(-1), highs.reshape(-1), values[11:]]).tolist()
-        n = lows.numel()
+            totals = self.accelerator.reduce(values[:9], reduction="sum")
+            lows, highs = self.accelerator.gather(values[9:10]), self.accelerator.gather(values[10:11])
+            n, host = lows.numel(), torch.cat([totals, lows.reshape(-1), highs.reshape(-1), values[11:]]).tolist()
         kl_sum, ent_sum, cnt, clip_cnt, aux_sum, aux_cnt, low, high, region = host[:9]
         lmin = min((x for x in host[9 : 9 + n] if x == x), default=math.nan)
         hmax = max((x for x in host[9 + n : -2] if x == x), default=math.nan)
