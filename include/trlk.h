@@ -340,6 +340,14 @@ int trlk_scatter_rows(const void* d_src, int64_t row_bytes, const int32_t* d_pos
 int trlk_scatter_values(const float* d_a, const float* d_b, const int32_t* d_position, int64_t n, float* d_out_a,
                         float* d_out_b, trlk_stream_t stream);
 
+/* The fine-tuning loss of n tokens (trl/trainer/sft_trainer.py:196-234): *d_out_loss = -sum(logp) / denominator, the sums of the
+ * entropies and of the arg-max hits; denominator = *d_denominator unless that is null.  trlk_nll_grad: d loss / d logp of every
+ * token, -*d_grad_loss / denominator. */
+int trlk_nll_sums(const float* d_logp, const float* d_entropy, const float* d_hit, int64_t n, const float* d_denominator,
+                  float denominator, float* d_out_loss, float* d_out_entropy, float* d_out_hits, trlk_stream_t stream);
+int trlk_nll_grad(const float* d_grad_loss, int64_t n, const float* d_denominator, float denominator, float* d_out,
+                  trlk_stream_t stream);
+
 /* What a trainer logs of trlk_grpo_loss's metrics, in one vector of TRLK_GRPO_LOG_VALUES floats: the sums that processes add
  * up (KL, entropy, mask, clip count, aux, aux count, and the low / high / region clip sums), the smallest low and the largest
  * high clip ratio of a sequence, the policy loss, the error word (trl/trainer/grpo_trainer.py:3212-3258). */

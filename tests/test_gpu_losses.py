@@ -1061,3 +1061,43 @@ def test_operands_in_host_memory_are_refused(amd):
     pinned = ids.cpu().pin_memory()
     assert torch.equal(ops.logp_entropy_fwd(logits, pinned, 0.9, 0, T, None)[0], logp)
     amd.check_device_errors()
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 9001])
+@pytest.mark.parametrize("divisor", ["count", "tensor", "number"])
+def test_fine_tuning_sums(n, divisor):
+    """Loss, entropy sum and hits of one launch, and the loss's gradient, against float64.  The sums are rounded once, the quotient
+    once more: 2^-24 each.  Through `_chunked_cross_entropy_loss` the divisors agree with the torch expression that other types
+    of divisor take (sums of n terms in fp32: n / 1024 + 10 additions deep)."""
+    from trl_amd import ops
+    from trl_amd.trainer.sft_trainer import _chunked_cross_entropy_loss
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    logp, ent = -5 * torch.rand(n, generator=g, device=DEV), 3 * torch.rand(n, generator=g, device=DEV)
+    hit = (torch.rand(n, generator=g, device=DEV) < 0.3).float()
+    value = {"count": float(n), "tensor": 37.0, "number": 12.5}[divisor]
+    per = torch.tensor(value, device=DEV) if divisor == "tensor" else None
+    loss, entropies, hits = ops.nll_sums(logp, ent, hit, per, 1.0 if divisor == "tensor" else value)
+    assert float(loss) == pytest.approx(-float(logp.double().sum()) / value, rel=2 * 2**-24)
+    assert float(entropies) == pytest.approx(float(ent.double().sum()), rel=2**-24) and float(hits) == float(hit.double().sum())
+    up, by = torch.tensor(0.3, device=DEV), torch.tensor(value, device=DEV)  # (by a plain number torch multiplies by its inverse)
+    assert torch.equal(ops.nll_grad(up, n, per, 1.0 if divisor == "tensor" else value), (-(up / by)).expand(n))
+
+    if n > 1024:
+        return
+    H, V = 64, 512
+    hidden = torch.randn((1, n + 1, H), generator=g, device=DEV).bfloat16().requires_grad_(True)
+    weight = (0.1 * torch.randn((V, H), generator=g, device=DEV)).bfloat16().requires_grad_(True)
+    labels = torch.randint(0, V, (1, n + 1), generator=g, device=DEV)
+    fast = {"count": None, "tensor": torch.tensor(37, device=DEV), "number": 12.5}[divisor]
+    other = torch.tensor(float(n) if fast is None else float(fast), dtype=torch.float32, device=DEV).requires_grad_(True)
+    results = []
+    for items in (fast, other):
+        out = _chunked_cross_entropy_loss(hidden, weight, 8192, labels=labels, num_items_in_batch=items)
+        results.append((out, torch.autograd.grad(3.0 * out[0], (hidden, weight))))
+    (a, ga), (b, gb) = results
+    for x, y in zip(a, b):
+        assert x.shape == y.shape and x.dtype == y.dtype
+        assert float(x.detach()) == pytest.approx(float(y.detach()), rel=12 * 2**-24)
+    assert not a[1].requires_grad and not a[2].requires_grad
+    assert all(torch.equal(x, y) for x, y in zip(ga, gb))

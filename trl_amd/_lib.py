@@ -111,6 +111,11 @@ SIGNATURES = {
     ),
     "trlk_scatter_rows": (c_int32, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
     "trlk_scatter_values": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
+    "trlk_nll_sums": (
+        c_int32,
+        [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
+    "trlk_nll_grad": (c_int32, [c_void_p, c_int64, c_void_p, c_float, c_void_p, c_void_p]),
     "trlk_grpo_log_values": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "trlk_dpo_log_values": (
         c_int32,

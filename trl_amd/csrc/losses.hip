@@ -447,6 +447,44 @@ __global__ __launch_bounds__(kThreads) void dpo_finish_kernel(const float* __res
     for (int64_t t = tid; t < T; t += kThreads) out_dlogp[off + t] = (mask[off + t] != 0.f) ? g : 0.f;
 }
 
+// Loss and logged sums of a fine-tuning step, and the loss's gradient for every token.  One launch each where torch takes five
+// and three, 4 to 5 us of the device apiece: a step of 1396 tokens, H = 2048, V = 50257 927 -> 906 us.  The sums are fp64 on the chip, rounded once; one workgroup,
+// whose lanes have several loads in flight, is enough for the tokens that enter a head (a few thousand to 1e5).
+constexpr int kNllThreads = 1024;
+__global__ __launch_bounds__(kNllThreads) void nll_sums_kernel(const float* logp, const float* entropy, const float* hit, int64_t n,
+                                                               const float* d_denominator, float denominator, float* loss,
+                                                               float* entropy_sum, float* hits) {
+    __shared__ double parts[3][kNllThreads / kWave];
+    double v[3] = {0., 0., 0.};
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i < n; i += kNllThreads) {
+        v[0] += double(logp[i]);
+        v[1] += double(entropy[i]);
+        v[2] += double(hit[i]);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) v[j] += __shfl_xor(v[j], o);
+        if ((threadIdx.x & (kWave - 1)) == 0) parts[j][threadIdx.x / kWave] = v[j];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        v[j] = 0.;
+        for (int w = 0; w < kNllThreads / kWave; ++w) v[j] += parts[j][w];
+    }
+    *loss = -float(v[0]) / (d_denominator ? *d_denominator : denominator);
+    *entropy_sum = float(v[1]);
+    *hits = float(v[2]);
+}
+__global__ __launch_bounds__(kThreads) void nll_grad_kernel(const float* grad_loss, int64_t n, const float* d_denominator,
+                                                            float denominator, float* out) {
+    const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+    if (i < n) out[i] = -(*grad_loss / (d_denominator ? *d_denominator : denominator));
+}
+
 // The logged DPO values: masked sums of the entropies, the mean logits and the arg-max hits, one workgroup per sequence,
 // then their sums per half of the batch and the rewards, in one vector for one copy to the host.  Two launches in place
 // of two dozen [2P, T]-sized ones.
@@ -809,6 +847,29 @@ extern "C" int trlk_dpo_log_values(const float* d_entropy, const float* d_row_st
     hipLaunchKernelGGL(dpo_log_finish_kernel, dim3(1), dim3(kThreads), 0, s, d_workspace, d_seq_logps, d_ref_chosen,
                        d_ref_rejected, n_seq / 2, beta, d_error_flag, d_out);
     return launch_status("dpo_log_values");
+}
+
+extern "C" int trlk_nll_sums(const float* d_logp, const float* d_entropy, const float* d_hit, int64_t n,
+                             const float* d_denominator, float denominator, float* d_out_loss, float* d_out_entropy,
+                             float* d_out_hits, trlk_stream_t stream) {
+    clear_error();
+    TRLK_REQUIRE(n >= 0, TRLK_ERR_BAD_SHAPE, "nll_sums: negative token count %lld", (long long)n);
+    TRLK_REQUIRE((n == 0 || (d_logp && d_entropy && d_hit)) && d_out_loss && d_out_entropy && d_out_hits, TRLK_ERR_NULL_POINTER,
+                 "nll_sums: a required pointer is null");
+    hipLaunchKernelGGL(nll_sums_kernel, dim3(1), dim3(kNllThreads), 0, static_cast<hipStream_t>(stream), d_logp, d_entropy, d_hit,
+                       n, d_denominator, denominator, d_out_loss, d_out_entropy, d_out_hits);
+    return launch_status("nll_sums");
+}
+
+extern "C" int trlk_nll_grad(const float* d_grad_loss, int64_t n, const float* d_denominator, float denominator, float* d_out,
+                             trlk_stream_t stream) {
+    clear_error();
+    TRLK_REQUIRE(n >= 0 && n < (int64_t(1) << 31), TRLK_ERR_BAD_SHAPE, "nll_grad: bad token count %lld", (long long)n);
+    if (n == 0) return TRLK_OK;
+    TRLK_REQUIRE(d_grad_loss && d_out, TRLK_ERR_NULL_POINTER, "nll_grad: a required pointer is null");
+    hipLaunchKernelGGL(nll_grad_kernel, dim3(unsigned((n + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                       static_cast<hipStream_t>(stream), d_grad_loss, n, d_denominator, denominator, d_out);
+    return launch_status("nll_grad");
 }
 
 extern "C" int trlk_rloo_loss(const float* d_token_logp, const float* d_mask, const float* d_old_seq_logps,

@@ -750,6 +750,28 @@ def scatter_values(a, b, position, shape):
     return out_a, out_b
 
 
+@_plain_op("nll_sums(Tensor logp, Tensor entropy, Tensor hit, Tensor? denominator, float value) -> (Tensor, Tensor, Tensor)",
+           lambda logp, entropy, hit, denominator, value: tuple(_f32_like(logp) for _ in range(3)))
+def nll_sums(logp, entropy, hit, denominator, value):
+    """`(-logp.sum() / denominator, entropy.sum(), hit.sum())` of fp32 `[n]` vectors (`trlk_nll_sums`); the denominator is a
+    0-d fp32 tensor, or `value` without one."""
+    loss, entropies, hits = (_f32_like(logp) for _ in range(3))
+    with on_device(logp.device):
+        check(lib.trlk_nll_sums(ptr(logp), ptr(entropy), ptr(hit), logp.numel(), ptr(denominator), value, ptr(loss),
+                                ptr(entropies), ptr(hits), current_stream(logp.device)))
+    return loss, entropies, hits
+
+
+@_plain_op("nll_grad(Tensor grad_loss, SymInt n, Tensor? denominator, float value) -> Tensor",
+           lambda grad_loss, n, denominator, value: _f32_like(grad_loss, n))
+def nll_grad(grad_loss, n, denominator, value):
+    """`[n]` times `-grad_loss / denominator`: the gradient of `nll_sums`' loss (`trlk_nll_grad`)."""
+    out = _f32_like(grad_loss, n)
+    with on_device(out.device):
+        check(lib.trlk_nll_grad(ptr(grad_loss), n, ptr(denominator), value, ptr(out), current_stream(out.device)))
+    return out
+
+
 @_plain_op("mean_logits(Tensor hidden, Tensor weight) -> Tensor",
            lambda hidden, weight: hidden.new_empty((hidden.shape[0],), dtype=torch.float32))
 def mean_logits(hidden, weight):

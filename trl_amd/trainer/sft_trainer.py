@@ -42,9 +42,19 @@ def _chunked_cross_entropy_loss(
         hidden, targets = hidden_states.reshape(1, -1, h), shift_labels.reshape(1, -1)
     else:  # (labels of another shape that leave one label per remaining position)
         hidden, targets = hidden_states[..., :-1, :].reshape(1, -1, h), labels[..., 1:].reshape(1, -1)
+    # what the loss is divided by, where the head's own function can do it
+    mean_of = "count"
+    if isinstance(num_items_in_batch, Tensor):
+        mean_of = None
+        if (num_items_in_batch.dim() == 0 and num_items_in_batch.dtype in (torch.int64, torch.int32, torch.float32)
+                and not num_items_in_batch.requires_grad):
+            mean_of = num_items_in_batch.to(device=hidden.device, dtype=torch.float32)
+    elif num_items_in_batch is not None:
+        mean_of = num_items_in_batch if type(num_items_in_batch) in (int, float) else None
     try:
         logp, ent, hit, n_valid = _masked_head(hidden, lm_head_weight, targets, targets, 1.0, chunk_size,
-                                               final_logit_softcapping, logit_scale, lm_head_bias, -100, True, False, shifted)
+                                               final_logit_softcapping, logit_scale, lm_head_bias, -100, True, False, shifted,
+                                               mean_of)
     except (ValueError, TypeError, NotImplementedError):
         if bool((targets != -100).any()):
             raise
@@ -56,6 +66,8 @@ def _chunked_cross_entropy_loss(
             loss = loss + lm_head_bias.float().sum() * 0.0
         zero = hidden.new_zeros((), dtype=torch.float32)
         return loss, zero, zero.clone(), n_valid
+    if mean_of is not None:
+        return logp, hit, ent, n_valid
     loss = -logp.sum()
     if num_items_in_batch is None:
         loss = loss / n_valid

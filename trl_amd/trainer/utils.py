@@ -259,16 +259,22 @@ class _MaskedHeadFunction(torch.autograd.Function):
     """The head on some of the positions of `hidden` `[B, S, H]`: `targets` `[B, T]` (T <= S) belong to its first T
     positions, those whose `keep` `[B, T]` is not `skip` go through it.  Returns fp32 log-probs, entropies (both `[B, T]`,
     0 at the other positions, or packed `[n]` with `packed`) and argmax hits (packed), and the count as a device scalar.
-    Only the log-probs are differentiable."""
+    With `mean_of` (a number, a 0-d fp32 tensor, or "count" for the positions that went through) the first three come summed:
+    the negative log-probs divided by it, the entropies, the hits.  Only the log-probs, or their mean, are differentiable."""
 
     @staticmethod
-    def forward(ctx, hidden, weight, bias, targets, keep, skip, cfg, packed, may_clip, with_grad):
+    def forward(ctx, hidden, weight, bias, targets, keep, skip, cfg, packed, may_clip, with_grad, mean_of):
         index, position, count = ops.select_rows(keep, skip)
         n = int(count)  # (the one synchronisation: the packed tensors' size)
         rows, picked = ops.gather_rows(hidden, targets, index, n)
         logp, ent, log_z, hit, saved = _head_forward(rows, weight, picked, bias, cfg,
                                                      with_grad and any(ctx.needs_input_grad[:2]))
-        ctx.save_for_backward(rows, weight, picked, log_z, bias, saved, index, position)
+        ctx.mean_of = None
+        per = mean_of if torch.is_tensor(mean_of) else None
+        if mean_of is not None and n:
+            ctx.mean_of = 1.0 if per is not None else float(n if mean_of == "count" else mean_of)
+            logp, ent, hit = ops.nll_sums(logp, ent, hit, per, ctx.mean_of)
+        ctx.save_for_backward(rows, weight, picked, log_z, bias, saved, per, index, position)
         ctx.cfg, ctx.shape, ctx.cols, ctx.packed = cfg, tuple(hidden.shape), targets.shape[1], packed
         # Tokens without gradient (masked ones are not among the packed rows) are those that a loss clipped and, far more
         # of them, whole groups whose rewards are all equal.  The search costs a synchronisation, 35 to 80 us, and packing
@@ -286,18 +292,21 @@ class _MaskedHeadFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_logp, g_ent, g_hit, g_count):
         if g_logp is None:
-            return (None,) * 10
-        *operands, index, position = ctx.saved_tensors
+            return (None,) * 11
+        *operands, per, index, position = ctx.saved_tensors
         n = operands[0].shape[0]
-        g = g_logp if ctx.packed else g_logp.reshape(-1).index_select(0, index[:n])
+        if ctx.mean_of is not None:
+            g = ops.nll_grad(g_logp, n, per, ctx.mean_of)
+        else:
+            g = g_logp if ctx.packed else g_logp.reshape(-1).index_select(0, index[:n])
         d_rows, d_weight, d_bias = _head_backward(*operands, ctx.cfg, g, *ctx.drop)
         d_hidden = ops.scatter_rows(d_rows, position, ctx.shape, ctx.cols) if ctx.needs_input_grad[0] else None
-        return d_hidden, d_weight, d_bias, None, None, None, None, None, None, None
+        return d_hidden, d_weight, d_bias, None, None, None, None, None, None, None, None
 
 
 def _masked_head(hidden: Tensor, weight: Tensor, targets: Tensor, keep: Tensor, temperature: float, chunk_size: int,
                  softcap: float | None = None, logit_scale: float = 1.0, bias: Tensor | None = None, skip: int = 0,
-                 packed: bool = False, may_clip: bool = True, shifted: bool = False):
+                 packed: bool = False, may_clip: bool = True, shifted: bool = False, mean_of=None):
     """See `_MaskedHeadFunction`; every position has a target, or with `shifted` all but the last one of a sequence.  The
     products are kept for a backward only where one can follow (under `no_grad` the operands may still be parameters).
     `may_clip=False`: the loss gives every token that enters a gradient."""
@@ -314,7 +323,7 @@ def _masked_head(hidden: Tensor, weight: Tensor, targets: Tensor, keep: Tensor, 
     cap = 0.0 if softcap is None else float(softcap)
     return _MaskedHeadFunction.apply(hidden, weight, bias, targets, keep, skip,
                                      (float(temperature), int(chunk_size), cap, float(logit_scale)), packed,
-                                     may_clip, torch.is_grad_enabled())
+                                     may_clip, torch.is_grad_enabled(), mean_of)
 
 
 def chunked_logprobs_from_hidden(hidden_states: Tensor, lm_head_weight: Tensor, labels: Tensor,
