@@ -172,17 +172,20 @@ __global__ __launch_bounds__(256) void scatter_values_kernel(const float* a, con
 
 // ---- mean logits of whole sequences without logits: mean over t and v of hidden[b, t] . weight[v] =
 // (sum_t hidden[b, t] . wsum) / (T V) with wsum = sum_v weight[v].  Bound by the read of the weight (525 MB and 2048 hidden
-// rows: 89 us, 5.9 TB/s, of 113 us for all three launches; the same with fp32 sums); converting it to fp32 first and summing
-// that copy moved five times the bytes, 470 us.
+// rows: 86 us, 6.1 TB/s, of 96 us for all three launches; 90 of 113 with one set of eight rows in flight, four rows to a wave of
+// the dot products and the partial sums read one by one; all three after a flush of the caches, with their gaps: 173 -> 108;
+// 32000 x 4096 150 -> 89; 50257 x 1024 67 -> 40); converting it to fp32 first and summing that copy moved five times the bytes,
+// 470 us.
 //
 // A mean logit is small against the terms it is made of, and a chain of 250 fp32 additions per column (what 128256 rows in
 // 512 partial sums make) left it four times as far from 64 bits as the torch product (5e-7 against 1.3e-7 of its value on
 // [2, 512] positions).  So sums are exact or in fp64 on the chip and rounded to fp32 once on their way to memory: in 2^-24 of
 // the size that such a sum of random terms has, 0.7 to 1.3 where the torch product is 2.7 to 3.6 away (32000 to 202048 rows).
 //
-// Column sums: workgroup (x, y) sums rows y, y + gridDim.y, ... of 2048 columns, 8 columns per lane, eight rows in flight:
-// those are added up in pairs in fp32 (their 16-bit values leave 13 bits and more to spare), then to the fp64 sum; the
-// partial sums of the gridDim.y row sets are added in order by the second kernel.
+// Column sums: workgroup (x, y) sums rows y, y + gridDim.y, ... of 2048 columns, 8 columns per lane, eight rows in flight
+// while the eight before them are summed (1024 row sets with half as much work each: 108 -> 142 us): those are added up in
+// pairs in fp32 (their 16-bit values leave 13 bits and more to spare), then to the fp64 sum; the partial sums of the gridDim.y
+// row sets are added in order by the second kernel.
 constexpr int kColBlock = 256, kColParts = 512;
 template <int DT>
 __global__ __launch_bounds__(kColBlock) void column_sum_kernel(const uint16_t* w, int64_t ld, int rows, int cols8, float* parts) {
@@ -192,16 +195,28 @@ __global__ __launch_bounds__(kColBlock) void column_sum_kernel(const uint16_t* w
     const int64_t ld8 = ld / 8;
     double acc[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
     int r = blockIdx.y;
-    for (; r + 7 * step < rows; r += 8 * step) {
-        u32x4 q[8];
+    u32x4 q[8], next[8];
+    auto fetch = [&](int from, u32x4(&to)[8]) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) q[k] = p[int64_t(r + k * step) * ld8];
+        for (int k = 0; k < 8; ++k) to[k] = __builtin_nontemporal_load(p + int64_t(from + k * step) * ld8);
+    };
+    auto add_rows = [&] {
         float x[8][8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) Elem<DT>::unpack(q[k], x[k]);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             acc[i] += double(((x[0][i] + x[1][i]) + (x[2][i] + x[3][i])) + ((x[4][i] + x[5][i]) + (x[6][i] + x[7][i])));
+    };
+    if (r + 7 * step < rows) {
+        fetch(r, q);
+        for (r += 8 * step; r + 7 * step < rows; r += 8 * step) {
+            fetch(r, next);
+            add_rows();
+#pragma unroll
+            for (int k = 0; k < 8; ++k) q[k] = next[k];
+        }
+        add_rows();
     }
     for (; r < rows; r += step) {
         float x[8];
@@ -219,6 +234,7 @@ __global__ __launch_bounds__(1024) void column_sum_finish_kernel(const float* pa
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, c = blockIdx.x * kWave + lane;
     double s = 0.;
     if (c < cols)
+#pragma unroll 8
         for (int p = wave; p < n_parts; p += 16) s += double(parts[int64_t(p) * cols + c]);
     sum[wave][lane] = s;
     __syncthreads();
@@ -229,17 +245,18 @@ __global__ __launch_bounds__(1024) void column_sum_finish_kernel(const float* pa
         out[c] = float(t);
     }
 }
-// out[b][chunk] = scale * sum over the chunk's rows of hidden[b, t] . wsum, one wave per row at a time.
+// out[b][chunk] = scale * sum over the chunk's rows of hidden[b, t] . wsum, one wave per row.
 constexpr int kDotRows = 16;  // rows per workgroup
 template <int DT>
-__global__ __launch_bounds__(256) void row_dot_kernel(const uint16_t* hidden, int64_t seq_stride, int64_t row_stride, int T,
+__global__ __launch_bounds__(kDotRows * kWave) void row_dot_kernel(const uint16_t* hidden, int64_t seq_stride, int64_t row_stride, int T,
                                                       int cols8, const float* wsum, double scale, float* out) {
-    __shared__ double part[4];
+    __shared__ double part[kDotRows];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int t0 = blockIdx.x * kDotRows, t1 = min(T, t0 + kDotRows);
+    const int t = blockIdx.x * kDotRows + wave;
     double s = 0.;
-    for (int t = t0 + wave; t < t1; t += 4) {
+    if (t < T) {
         const u32x4* row = reinterpret_cast<const u32x4*>(hidden + int64_t(blockIdx.y) * seq_stride + int64_t(t) * row_stride);
+#pragma unroll 4
         for (int c = lane; c < cols8; c += kWave) {
             float x[8];
             Elem<DT>::unpack(row[c], x);
@@ -251,8 +268,12 @@ __global__ __launch_bounds__(256) void row_dot_kernel(const uint16_t* hidden, in
     for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane == 0) part[wave] = s;
     __syncthreads();
-    if (threadIdx.x == 0)
-        out[int64_t(blockIdx.y) * gridDim.x + blockIdx.x] = float(scale * (part[0] + part[1] + part[2] + part[3]));
+    if (threadIdx.x == 0) {
+        double sum = 0.;
+#pragma unroll
+        for (int w = 0; w < kDotRows; ++w) sum += part[w];
+        out[int64_t(blockIdx.y) * gridDim.x + blockIdx.x] = float(scale * sum);
+    }
 }
 
 bool whole_pieces(const void* a, const void* b, int64_t bytes) {
@@ -395,7 +416,7 @@ extern "C" int trlk_mean_logits(const void* d_hidden, const void* d_weight, int 
                            dim3(kColBlock), 0, s, static_cast<const uint16_t*>(d_weight), weight_stride, int(vocab), cols8, parts);
         hipLaunchKernelGGL(column_sum_finish_kernel, dim3(unsigned((hidden_size + kWave - 1) / kWave)), dim3(1024), 0, s, parts,
                            n_parts, int(hidden_size), wsum);
-        hipLaunchKernelGGL(row_dot_kernel<DT>, dim3(unsigned(trlk_mean_logits_chunks(rows_per_seq)), unsigned(n_seq)), dim3(256), 0,
+        hipLaunchKernelGGL(row_dot_kernel<DT>, dim3(unsigned(trlk_mean_logits_chunks(rows_per_seq)), unsigned(n_seq)), dim3(kDotRows * kWave), 0,
                            s, static_cast<const uint16_t*>(d_hidden), seq_stride, row_stride, int(rows_per_seq), cols8, wsum, scale,
                            d_out);
     };
