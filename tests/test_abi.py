@@ -161,3 +161,24 @@ def test_cpu_tensors_fail_loudly():
 
     with pytest.raises((NotImplementedError, RuntimeError)):
         trl_amd.selective_log_softmax(torch.randn(2, 3, 16), torch.zeros(2, 3, dtype=torch.long))
+
+
+def test_slices_of_the_dhidden_product():
+    """The slices that the backward's workspace holds are a number into which the contraction can be cut: the vocabulary's k steps
+    (of 64 rows) in slices of a whole number of steps, the last of them not empty.  Few tokens, so that the weight is read as it
+    lies in memory."""
+    from trl_amd import _lib
+
+    def up(x, m):
+        return (x + m - 1) // m * m
+
+    for v in range(16321, 65536, 64):
+        steps = up(v, 64) // 64
+        for blocks in range(1, 10):
+            n = 256 * blocks
+            for h in (64, 256, 512, 1024, 1536, 2048, 3584):
+                total = _lib.lib.trlk_fused_head_bwd_workspace_bytes(n, v, h, v)
+                fixed = up(h * (n + 64) * 2, 256) + up(v, 256) * (n + 64) * 2  # hidden^T and the d logits; then the slices, [n, h] in fp32
+                slices = (total - fixed) // (n * h * 4)
+                length = -(-steps // slices)
+                assert -(-steps // length) == slices, (n, h, v, slices)

@@ -1029,3 +1029,31 @@ def test_weight_read_as_it_lies_in_memory(amd, dtype, n, h, v):
             for got, want, squares in ((got_h, want_h, dz.square() @ wd.square()), (got_w, want_w, dz.square().t() @ hd.square())):
                 err, bound = (got.cpu().double() - want).norm(), unit * want.norm() + 2.0**-9 * squares.sum().sqrt()
                 assert err < bound, (outlier, chunk, float(err), float(bound))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,h,v", [(200, 1024, 18433), (256, 1152, 32300), (700, 512, 32300), (1000, 512, 49500), (40, 72, 61441)])
+def test_only_slices_that_were_written_are_summed(amd, dtype, n, h, v, monkeypatch):
+    """Vocabularies whose last 64 to 192 rows up to a multiple of 256 would be a slice of the dHidden product by themselves: in a
+    workspace full of NaN, dHidden is as float64 has it.  (The bound: see test_weight_read_as_it_lies_in_memory.)"""
+    g = torch.Generator(device=DEV).manual_seed(n + v)
+    hidden = (0.1 * torch.randn(n, h, generator=g, device=DEV)).to(dtype)
+    weight = (torch.randn(v, h, generator=g, device=DEV) * (0.5 / h**0.5)).to(dtype)
+    labels = torch.randint(0, v, (n,), generator=g, device=DEV)
+    gout = torch.randn(n, generator=g, device=DEV)
+    args = (hidden, weight, labels, 0.9, 0.0, 1.0)
+    out = amd.ops.fused_head_fwd(*args, None, True)
+    empty = torch.empty
+
+    def poisoned(*a, **kw):
+        t = empty(*a, **kw)
+        return t.fill_(255) if t.dtype == torch.uint8 else t  # (all bits set: NaN in both types)
+
+    monkeypatch.setattr(torch, "empty", poisoned)
+    got, _, _ = amd.ops.fused_head_bwd(*args, out[2], gout, v, None, out[4])
+    p = (hidden.double() @ weight.double().t() / 0.9).softmax(-1)
+    dz = (torch.zeros_like(p).scatter_(1, labels[:, None], 1.0) - p) * gout.double()[:, None] / 0.9
+    want = dz @ weight.double()
+    unit = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
+    err, terms = (got.double() - want).norm(), (dz.square() @ weight.double().square()).sum().sqrt()
+    assert float(err) < float(unit * want.norm() + 2.0**-9 * terms)

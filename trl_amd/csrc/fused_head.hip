@@ -1899,7 +1899,11 @@ struct BwdLayout {
     size_t off_wt, off_ht, off_dzt, off_dh, off_max, total;
     int64_t n_chunks;
     bool direct;         // the dHidden product reads the weight itself: no transposed copy
-    int slices, kslice;  // of the dHidden product's contraction over a chunk
+    int64_t dh_k;        // length of the dHidden product's contraction over a whole chunk
+    int slices, kslice;  // of that contraction
+    // Slices that a contraction of length k reaches: `slices` of a whole chunk, fewer of a shorter last one.  What is launched and
+    // what is summed both come from here; a slice that is summed and not launched would add what the workspace held before.
+    int reached(int64_t k) const { return int((k + kslice - 1) / kslice); }
 };
 // Slices of the contraction of the dHidden product.  Its tiles (token blocks x hidden tiles) contract over the whole
 // chunk, tens of times longer than the dW tiles of the same launch, and they are few when there are few tokens: 48 tiles of
@@ -1952,8 +1956,9 @@ BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     l.off_ht = take(size_t(H) * l.ld_n * 2);
     l.off_dzt = take(size_t(l.cpad) * l.ld_n * 2);
     const int want = dh_slices(l.npad / BN, (H + BN - 1) / BN, l.cpad, l.npad);
-    l.kslice = int(round_up((l.cpad + want - 1) / want, BK));
-    l.slices = int((l.cpad + l.kslice - 1) / l.kslice);
+    l.dh_k = l.direct ? l.vpad : l.cpad;  // (a transposed copy is padded to whole tiles, the weight is read in whole k steps)
+    l.kslice = int(round_up((l.dh_k + want - 1) / want, BK));
+    l.slices = l.reached(l.dh_k);
     l.off_dh = take(size_t(l.slices) * N * H * 4);
     l.n_chunks = (V + l.cpad - 1) / l.cpad;
     l.off_max = take(size_t(3 + l.n_chunks) * 4);  // largest magnitudes: g, hidden, sample of W, what exceeds it in each chunk
@@ -2321,12 +2326,11 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         gh.beyond_b = beyond_w;
         if (l.direct) {
             gh.B = Operand{w_chunk, weight_stride, H};
-            gh.K = int(round_up(rows, BK));
+            gh.K = int(l.dh_k);
             gh.b_krows = rows;
             gh.beyond_out = beyond_w;
         }
-        gh.slices = l.slices;  // (of the last, possibly shorter chunk those that its rows reach)
-        while (gh.slices > 1 && int64_t(gh.slices - 1) * l.kslice >= gh.K) --gh.slices;
+        gh.slices = l.reached(gh.K);
         gh.kslice = l.kslice;
         const int ghgrid = xcd_patch_grid(n_tb, n_ht * gh.slices);
         // dW[chunk, H] = dz^T[chunk, N] * (hidden^T[H, N])^T
