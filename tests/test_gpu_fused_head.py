@@ -1057,3 +1057,49 @@ def test_only_slices_that_were_written_are_summed(amd, dtype, n, h, v, monkeypat
     unit = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
     err, terms = (got.double() - want).norm(), (dz.square() @ weight.double().square()).sum().sqrt()
     assert float(err) < float(unit * want.norm() + 2.0**-9 * terms)
+
+
+@pytest.mark.parametrize("kind", ["entry", "row", "third", "sample"])
+@pytest.mark.parametrize("n,h,v", [(1, 8, 64), (65, 72, 63), (257, 136, 1000), (129, 520, 9001), (200, 1024, 18433), (2304, 264, 300)])
+def test_entries_beyond_the_sampled_scale(amd, kind, n, h, v):
+    """bf16 weights with entries far above those of the sampled rows: one of 1e15 in a column where hidden is zero, a whole row,
+    a third of the rows, and a sample of nothing but zeros.  dHidden as float64 has it, in the columns of such entries and, where
+    the product reads the weight itself, in those without, and the same in a second run to the bit.  (The bound: see test_weight_read_as_it_lies_in_memory.)"""
+    g = torch.Generator().manual_seed(n + h + v)
+    hidden = (0.1 * torch.randn(n, h, generator=g)).bfloat16()
+    weight = torch.randn(v, h, generator=g) * (0.5 / h**0.5)
+    groups = torch.arange((v + 31) // 32)
+    sampled = torch.zeros(v, dtype=torch.bool)  # one row of every 32
+    sampled[(32 * groups + ((groups * 2654435761) % 2**32 >> 27)).clamp(max=v - 1)] = True
+    large = torch.zeros(h, dtype=torch.bool)  # columns with entries beyond the sample's scale
+    if kind == "entry":
+        large[h - 1] = True
+        hidden[:, h - 1] = 0
+        weight[int((~sampled).nonzero()[-1]), h - 1] = 1e15
+    elif kind == "row":
+        large[: h // 2] = True
+        weight[int((~sampled).nonzero()[len(sampled) // 3]), large] *= 100.0
+    elif kind == "third":
+        large[: h // 2] = True
+        weight[(torch.arange(v) % 3 == 1) & ~sampled, : h // 2] *= 20.0
+    else:
+        large[:] = True
+        weight[sampled] = 0
+    weight = weight.bfloat16()
+    labels = torch.randint(0, v, (n,), generator=g)
+    gout = torch.randn(n, generator=g)
+    hd, wd = hidden.double(), weight.double()
+    p = (hd @ wd.t() / 0.9).softmax(-1)
+    dz = (torch.zeros_like(p).scatter_(1, labels[:, None], 1.0) - p) * gout.double()[:, None] / 0.9
+    want, squares = dz @ wd, dz.square() @ wd.square()
+    args = (hidden.to(DEV), weight.to(DEV), labels.to(DEV), 0.9, 0.0, 1.0)
+    out = amd.ops.fused_head_fwd(*args, None, True)
+    for chunk, groups in ((v, (large, ~large)), (v // 2, (large,))):
+        runs = [amd.ops.fused_head_bwd(*args, out[2], gout.to(DEV), chunk, None, out[4])[0] for _ in range(2)]
+        assert torch.equal(*runs)
+        got = runs[0].cpu().double()
+        for columns in groups:
+            if bool(columns.any()):
+                err = (got - want)[:, columns].norm()
+                bound = 2.0**-9 * want[:, columns].norm() + 2.0**-9 * squares[:, columns].sum().sqrt()
+                assert err <= bound, (chunk, float(err), float(bound))

@@ -228,6 +228,7 @@ struct DirectLoader {
 // are read as the last (the other operand is zero there), columns beyond the last as the last 8 (nobody stores them).
 // The conversion is what this costs beside the plain loop: 1392 tokens, H = 2048, V = 128256, backward of a bf16 problem 1562 us,
 // of an fp16 problem (nothing to convert) 1555; behind every MFMA of the refill instead of behind two of three 1577.
+// An entry whose scaled value fp16 does not hold counts as fp16's largest (see direct_scale).
 template <bool CONVERT>
 struct LeftKm {
     static constexpr int kVecs = 4;
@@ -238,6 +239,9 @@ struct LeftKm {
     float scale, top;  // top: the largest magnitude converted so far, times the scale
     __device__ __forceinline__ LeftKm(const Operand A, int m0, int krows_, float scale_, char* smem)
         : krows(krows_), scale(scale_), top(0.f) {
+        // FP16_OVFL: what overflows fp16 becomes its largest value (infinities stay), for the rest of the wave's life.  A bit of
+        // the mode register, where a clamp would be two instructions more per pair of columns in the tile loop.
+        if constexpr (CONVERT) asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 1" ::: "memory");
         const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         base = reinterpret_cast<const char*>(A.p + m0);
         row_bytes = uint32_t(A.ld * 2);
@@ -250,7 +254,7 @@ struct LeftKm {
         const int row = min(row0 + 16 * j, krows - 1 - k0);
         w = *reinterpret_cast<const u32x4*>(base + int64_t(k0) * row_bytes + (uint32_t(row) * row_bytes + col));
     }
-    // two neighbouring columns; exact wherever fp16 holds the scaled value (one rounding to nearest elsewhere)
+    // two neighbouring columns; exact wherever fp16 holds the scaled value (below its range one rounding to nearest)
     __device__ __forceinline__ void convert(uint32_t& w) {
         if constexpr (CONVERT) {
             const float lo = __uint_as_float(w << 16) * scale, hi = __uint_as_float(w & 0xffff0000u) * scale;
@@ -921,12 +925,18 @@ __device__ __forceinline__ float pow2_scale(float m) {
 __device__ __forceinline__ float slot_scale(const uint32_t* slot, float mult) {
     return slot != nullptr ? pow2_scale(__uint_as_float(*slot) * mult) : 1.f;
 }
-// The weight's scale comes from a SAMPLE of it (every kSampleRows-th row), so that no pass over the whole weight is needed
+// The weight's scale comes from a SAMPLE of it (one of every kSampleRows rows, see sample_row), so that no pass over the whole weight is needed
 // before the one that converts it; that pass finds the true maximum on its way.  slots[0] is the sample's largest magnitude,
 // slots[1] that of the entries that exceed it (0 if none does).  The sample's scale leaves a factor of 4 to fp16's largest
 // value; only when the chunk reaches beyond it, or the sample holds nothing but zeros, is the chunk converted again
 // with the scale of its own maximum.
 constexpr int kSampleRows = 32;
+// The row that stands for rows 32 i to 32 i + 31 of V: not the same one of every 32, so that a period in the weight (large entries in
+// every other row) does not hide from the sample.
+__device__ __forceinline__ int sample_row(int i, int V) {
+    static_assert(kSampleRows == 32, "5 bits of the product");
+    return min(i * kSampleRows + int((uint32_t(i) * 2654435761u) >> 27), V - 1);
+}
 struct WeightScale {
     float scale;
     bool again;  // the chunk has to be converted (again) with `scale`
@@ -935,6 +945,17 @@ __device__ __forceinline__ WeightScale weight_scale(const uint32_t* sample, cons
     const float m = __uint_as_float(*sample), top = __uint_as_float(max(*sample, *beyond)), s = pow2_scale(m);
     if (top == 0.f || (m > 0.f && top * s <= 65504.f)) return {s, false};
     return {pow2_scale(top), true};
+}
+
+// The scale in which the dHidden product converts a weight that it reads itself: the sample's, whatever the other entries are.
+// What exceeds fp16 there (|w| * scale > kF16Max, four to eight times the sample's maximum) counts as kF16Max in the product; the
+// rest of it is added by the pass that sums the product's slices, from the rows in which beyond_rows_kernel finds such
+// entries.  So one large entry neither makes the product be done again nor takes bits from the others.  (2^60, also for a sample
+// of nothing but zeros: w * scale is finite up to |w| = 2^68.)
+constexpr float kF16Max = 65504.f;
+__device__ __forceinline__ float direct_scale(const uint32_t* sample) {
+    const float m = __uint_as_float(*sample);
+    return m > 0.f ? fminf(pow2_scale(m), 0x1p60f) : 0x1p60f;
 }
 
 // tanh for soft-capping: sign(x) (1 - t) / (1 + t) with t = exp(-2 |x|) from the hardware's exp2 and reciprocal (a
@@ -1477,8 +1498,8 @@ struct GemmArgs {
     const uint32_t* max_a;
     const uint32_t* max_b;
     const uint32_t* beyond_b;  // B is the weight: max_b and this are the two slots of weight_scale()
-    // B is the weight itself, [b_krows, N] as it lies in memory, not a transposed copy (bf16: converted on its way in the scale
-    // of the sample, what exceeds it is left in beyond_out).
+    // B is the weight itself, [b_krows, N] as it lies in memory, not a transposed copy (bf16: converted on its way, see
+    // direct_scale; *beyond_out becomes 1 where fp16 does not hold all of it).
     int b_krows;
     uint32_t* beyond_out;
     const float* g_rows;
@@ -1490,9 +1511,8 @@ struct GemmArgs {
 };
 
 // DT: dtype of the operands (the matrix-core instruction), ODT: storage dtype of `out_lp`.
-// AKM: A is given k-major ([K, M], leading dimension A.ld).  BW: B is the weight in its own layout and dtype (ODT); AGAIN: the
-// sample's scale did not do, it is converted in that of its largest entry.
-template <int DT, int MODE, int ODT, bool AKM = false, bool BW = false, bool AGAIN = false>
+// AKM: A is given k-major ([K, M], leading dimension A.ld).  BW: B is the weight in its own layout and dtype (ODT).
+template <int DT, int MODE, int ODT, bool AKM = false, bool BW = false>
 __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char* smem) {
     typedef Elem<ODT> E;
     const int n_mt = (a.M + BN - 1) / BN, n_nt = (a.N + BM - 1) / BM;
@@ -1521,22 +1541,15 @@ __device__ __forceinline__ void gemm_nt_body(const GemmArgs& a, int block, char*
     float inv_b;
     if constexpr (BW) {
         constexpr bool kConvert = ODT == TRLK_BF16;
-        const float scale = uniform(!kConvert ? 1.f : AGAIN ? weight_scale(a.max_b, a.beyond_out).scale : slot_scale(a.max_b, 1.f));
+        const float scale = uniform(kConvert ? direct_scale(a.max_b) : 1.f);
         typedef LeftKm<kConvert> Left;
         Left left(B, c0, b_krows, scale, smem);
         if (idle)
             move_tiles_only<true, false, Left&>(DirectLoader<true, false>(B, c0, A, r0, smem), K, false, left);
         else
             gemm_tile_nt<DT, true>(B, c0, A, r0, K, acc, smem, left);
-        if (kConvert && !AGAIN) {
-            uint32_t m = __float_as_uint(left.top / scale);
-            const uint32_t known = max(*a.max_b, __hip_atomic_load(a.beyond_out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            if (__any(m > known)) {
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) m = max(m, uint32_t(__shfl_xor(int(m), off, 64)));
-                if (lane == 0) atomicMax(a.beyond_out, m);
-            }
-        }
+        if (kConvert && __any(left.top > kF16Max) && lane == 0)
+            __hip_atomic_store(a.beyond_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (idle) return;  // (no barrier follows)
         inv_b = 1.f / scale;
     } else {
@@ -1624,31 +1637,127 @@ TRLK_HEAD_KERNEL void gemm_nt_pair_kernel(GemmArgs a, int grid_a, GemmArgs b) {
     else
         gemm_nt_body<TRLK_F16, 0, ODT>(b, int(blockIdx.x) - grid_a, smem);
 }
-// The first of the two once more, where the sample's scale did not hold all of a bf16 weight: returns at once everywhere else.
-template <int MODE_A>
-TRLK_HEAD_KERNEL void gemm_nt_again_kernel(GemmArgs a) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    if (!weight_scale(a.max_b, a.beyond_out).again) return;
-    gemm_nt_body<TRLK_F16, MODE_A, TRLK_BF16, true, true, true>(a, blockIdx.x, smem);
+
+__device__ __forceinline__ uint32_t max_bits(uint32_t m, u32x4 q) {  // of the 8 bf16 in q, as fp32 bit patterns
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m = max(m, max((q[i] << 16) & 0x7fff0000u, q[i] & 0x7fff0000u));
+    return m;
+}
+
+// The rows of a weight in which entries exceed fp16 in the scale of direct_scale, a bit each: returns at once where the product
+// met none.  Bound by the read of the weight where it did.  One workgroup per CU, which makes a launch with nothing to do cheap.
+constexpr int kBeyondThreads = 1024, kBeyondBlocks = 256;
+__global__ __launch_bounds__(kBeyondThreads) void beyond_rows_kernel(const uint16_t* w, int64_t ld, int rows, int cols8,
+                                                                     const uint32_t* sample, const uint32_t* any,
+                                                                     uint32_t* row_bits) {
+    if (*any == 0u) return;
+    const float scale = direct_scale(sample);
+    const int lane = threadIdx.x & (kWave - 1), step = int(gridDim.x) * (kBeyondThreads / kWave);
+    for (int row = blockIdx.x * (kBeyondThreads / kWave) + threadIdx.x / kWave; row < rows; row += step) {
+        const u32x4* p = reinterpret_cast<const u32x4*>(w + int64_t(row) * ld);
+        uint32_t m = 0;
+#pragma unroll 4
+        for (int c = lane; c < cols8; c += kWave) m = max_bits(m, p[c]);
+        if (__any(__uint_as_float(m) * scale > kF16Max) && lane == 0) atomicOr(row_bits + (row >> 5), 1u << (row & 31));
+    }
+}
+
+// What the dHidden product left out of a weight that it converted itself: sum over v of dz[v, n] * (w[v, h] -+ kF16Max / scale) over
+// the entries that exceed fp16, in fp32 and in the order of the rows.
+struct BeyondArgs {
+    const uint32_t* any;       // null: the product left nothing out
+    const uint32_t* row_bits;  // see beyond_rows_kernel
+    const uint32_t* sample;
+    const uint16_t *weight, *dzt;
+    int64_t ldw, ldzt;
+    const float* g;
+    float zs;
+    int n_words, H;
+};
+constexpr int kSumThreads = 256;
+// Adds it for the 8 outputs from i on (token i / H); every lane of the workgroup takes part.  8192 rows at a time: their numbers are
+// put in a list in LDS, sixteen of them are in flight.  Whole backward, weight of deviation 0.02 -> one entry of 50 -> 300 rows times 100
+// (a sample of 1/32 of the rows misses all of 300 once in 1e4 weights): 1396 tokens, H = 2048, V = 50257 715 -> 690 -> 837 us; 1392 tokens, V =
+// 128256 1578 -> 1640 -> 1727; 459 tokens, H = 3584, V = 151936 1241 -> 1415 -> 1520; 64 tokens, H = 1024, V = 32000 100 -> 112 -> 163.
+// With the whole product done again in another scale, one entry: 1029, 2590, 1967 and 124 us.
+__device__ __forceinline__ void add_beyond(const BeyondArgs& b, int64_t i, bool live, float (&x)[8]) {
+    constexpr int kInFlight = 16;
+    __shared__ uint16_t list[32 * kSumThreads];
+    __shared__ int counts[kSumThreads / kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const float most = kF16Max / direct_scale(b.sample);
+    const int n = live ? int(i / b.H) : 0, h = live ? int(i - int64_t(n) * b.H) : 0;
+    float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int w0 = 0; w0 < b.n_words; w0 += kSumThreads) {
+        uint32_t bits = w0 + tid < b.n_words ? b.row_bits[w0 + tid] : 0u;
+        const int mine = __popc(bits);
+        int at = mine;  // inclusive sum over the wave's lanes
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int below = __shfl_up(at, o);
+            if (lane >= o) at += below;
+        }
+        if (lane == kWave - 1) counts[wave] = at;
+        __syncthreads();
+        at -= mine;
+        int total = 0;
+#pragma unroll
+        for (int k = 0; k < kSumThreads / kWave; ++k) {
+            if (k < wave) at += counts[k];
+            total += counts[k];
+        }
+        for (; bits != 0u; bits &= bits - 1u) list[at++] = uint16_t(tid * 32 + __ffs(bits) - 1);
+        __syncthreads();
+        for (int k0 = 0; k0 < total; k0 += kInFlight) {
+            int at[kInFlight];
+            uint16_t dz[kInFlight];
+            u32x4 row[kInFlight];
+#pragma unroll
+            for (int k = 0; k < kInFlight; ++k) at[k] = list[min(k0 + k, total - 1)];  // (beyond the last one: the last one, times 0)
+#pragma unroll
+            for (int k = 0; k < kInFlight; ++k) {
+                dz[k] = b.dzt[int64_t(w0 * 32 + at[k]) * b.ldzt + n];
+                row[k] = *reinterpret_cast<const u32x4*>(b.weight + int64_t(w0 * 32 + at[k]) * b.ldw + h);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < kInFlight; ++k) {
+                const float d = k0 + k < total ? Elem<TRLK_F16>::to_float(dz[k]) : 0.f;
+                float w[8];
+                Elem<TRLK_BF16>::unpack(row[k], w);
+#pragma unroll
+                for (int q = 0; q < 8; ++q)  // (0 for an entry that fp16 holds)
+                    sum[q] = fmaf(d, w[q] - __builtin_amdgcn_fmed3f(w[q], -most, most), sum[q]);
+            }
+        }
+        __syncthreads();  // (the next rows overwrite the list)
+    }
+    const float inv = live ? 1.f / pow2_scale(fabsf(b.g[n]) * b.zs) : 0.f;  // (token n's d logits are in its own scale)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = fmaf(sum[q], inv, x[q]);
 }
 
 // dHidden from the sums of the slices of its contraction, in slice order: out[i] = sum_s parts[s][i], 8 values per lane
-// (n is a multiple of 8).
+// (n is a multiple of 8), and what the product left out.
 template <int ODT>
-__global__ __launch_bounds__(256) void sum_slices_kernel(const float* parts, int slices, int64_t n, uint16_t* out) {
-    const int64_t i = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 8;
-    if (i >= n) return;
+__global__ __launch_bounds__(kSumThreads) void sum_slices_kernel(const float* parts, int slices, int64_t n, uint16_t* out,
+                                                                 BeyondArgs beyond) {
+    const int64_t i = (int64_t(blockIdx.x) * kSumThreads + threadIdx.x) * 8;
+    const bool live = i < n;
     float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < slices; ++s) {
-        const f32x4 lo = *reinterpret_cast<const f32x4*>(parts + s * n + i);
-        const f32x4 hi = *reinterpret_cast<const f32x4*>(parts + s * n + i + 4);
+    if (live)
+        for (int s = 0; s < slices; ++s) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(parts + s * n + i);
+            const f32x4 hi = *reinterpret_cast<const f32x4*>(parts + s * n + i + 4);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            x[k] += lo[k];
-            x[4 + k] += hi[k];
+            for (int k = 0; k < 4; ++k) {
+                x[k] += lo[k];
+                x[4 + k] += hi[k];
+            }
         }
-    }
-    *reinterpret_cast<u32x4*>(out + i) = Elem<ODT>::pack(x);
+    if constexpr (ODT == TRLK_BF16)
+        if (beyond.any != nullptr && *beyond.any != 0u) add_beyond(beyond, i, live, x);
+    if (live) *reinterpret_cast<u32x4*>(out + i) = Elem<ODT>::pack(x);
 }
 
 // A single product (epilogue 1: fp32 output, overwritten or accumulated into).
@@ -1690,7 +1799,7 @@ __global__ __launch_bounds__(256) void split_bf16x3_kernel(const float* in, int6
 }
 
 // Largest magnitudes of the backward's operands in one launch: out[0] of the fp32 vector g [n_g], out[1] of hidden, out[2]
-// of every kSampleRows-th row of the weight (bf16 matrices of C8 * 8 columns; no workgroups are launched for them in an
+// of a sample of the weight's rows (bf16 matrices of C8 * 8 columns; no workgroups are launched for them in an
 // fp16 problem), as the bit patterns of those floats (non-negative floats order like unsigned integers; the caller clears
 // `out`).
 //
@@ -1702,16 +1811,12 @@ struct MaxAbsArgs {
     const float* g;
     int64_t n_g;
     const uint16_t *hidden, *weight;
-    int64_t ld_hidden, ld_weight;       // (the weight's: between two rows of the sample)
-    int n_hidden, n_weight, C8;         // rows; 16-byte vectors per row
+    int64_t ld_hidden, ld_weight;
+    int n_hidden, n_weight, C8;         // rows (of the weight those in the sample); 16-byte vectors per row
+    int vocab;
     int blocks_g, blocks_h, blocks_w;   // workgroups of each
     uint32_t* out;
 };
-__device__ __forceinline__ uint32_t max_bits(uint32_t m, u32x4 q) {  // of the 8 bf16 in q, as fp32 bit patterns
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m = max(m, max((q[i] << 16) & 0x7fff0000u, q[i] & 0x7fff0000u));
-    return m;
-}
 __global__ __launch_bounds__(kMaxThreads) void head_maxabs_kernel(MaxAbsArgs a) {
     __shared__ uint32_t part[kMaxThreads / kWave];
     int block = blockIdx.x, slot;
@@ -1731,8 +1836,8 @@ __global__ __launch_bounds__(kMaxThreads) void head_maxabs_kernel(MaxAbsArgs a) 
         const int R = is_w ? a.n_weight : a.n_hidden;
         const int64_t n = int64_t(R) * a.C8, step = int64_t(blocks) * kMaxThreads;
         auto at = [&](int64_t v) {
-            const int64_t r = v / a.C8;
-            return *reinterpret_cast<const u32x4*>(in + r * ld + (v - r * a.C8) * 8);
+            const int64_t r = v / a.C8, row = is_w ? sample_row(int(r), a.vocab) : r;
+            return *reinterpret_cast<const u32x4*>(in + row * ld + (v - r * a.C8) * 8);
         };
         int64_t v = int64_t(block) * kMaxThreads + threadIdx.x;
         for (; v + 7 * step < n; v += 8 * step) {
@@ -1846,9 +1951,8 @@ __global__ __launch_bounds__(256) void transpose_weight_kernel(const uint16_t* i
 }
 // The same again in the scale of the chunk's own maximum, where the sample's does not do: returns at once everywhere else (few
 // workgroups that step through the tiles, so that a launch with nothing to do takes 5 us).  One entry of 50 in a weight of
-// deviation 0.02, which makes every chunk that holds it convert again: whole backward 709 -> 780 us (1396 tokens, H = 2048, V =
-// 50257), 1676 -> 1842 us (1392 tokens, V = 128256), 1716 -> 1933 us (459 tokens, H = 3584, V = 151936) -- about what the separate
-// pass over the weight cost every call (772, 1857 and 1949 us).
+// deviation 0.02, which makes the chunk that holds it convert again: whole backward 1336-1375 -> 1396 us (3300 tokens, H = 2048, V =
+// 50257, one chunk), 3255 -> 3258 (V = 128256, one of two chunks), 5255 -> 5390 (2600 tokens, H = 3584, V = 151936, one of two).
 constexpr int kAgainBlocks = 1024;
 __global__ __launch_bounds__(256) void transpose_weight_again_kernel(const uint16_t* in, int64_t ld, int R, int C, uint16_t* out,
                                                                      int64_t ldo, int64_t fill, const uint32_t* sample,
@@ -1897,7 +2001,7 @@ struct BwdLayout {
     int64_t vpad, npad, cpad;    // padded extents (zero-filled)
     int64_t ld_v, ld_n, ld_c;    // row strides of [*, vpad], [*, npad], [*, cpad] matrices
     size_t off_wt, off_ht, off_dzt, off_dh, off_max, total;
-    int64_t n_chunks;
+    int64_t n_chunks, n_maxima;
     bool direct;         // the dHidden product reads the weight itself: no transposed copy
     int64_t dh_k;        // length of the dHidden product's contraction over a whole chunk
     int slices, kslice;  // of that contraction
@@ -1934,8 +2038,9 @@ int dh_slices(int64_t n_tb, int64_t n_ht, int64_t kpad, int64_t npad) {
 // 100 tokens, H = 3584, V = 151936 1341 -> 859; 459 the same 1712 -> 1263; 300, H = 1024, V = 128256 506 -> 388; 900, H = 2560,
 // V = 151665 1784 -> 1557; 1396, H = 2048, V = 50257 710 -> 648; 1392, V = 128256 1662 -> 1562; 2300, H = 4096, V = 50264
 // 1800 -> 1760; from there on it loses: 2600, H = 3584, V = 151936 5298 -> 5340, 3300, H = 2048, V = 128256 3305 -> 3325, 7000,
-// V = 50264 2653 -> 2735.  Only with the whole vocabulary in one chunk: a product that has to be done again (weight_scale) then
-// overwrites what the first attempt left, and never a sum over several chunks.
+// V = 50264 2653 -> 2735.  Only with the whole vocabulary in one chunk: there is one product to add left-out entries to
+// (direct_scale).  A bf16 problem's sums are left in fp32 for that even where one slice would do (tiles of dHidden enough for the whole
+// chip): 2304 tokens, H = 4096, V = 50257 1740 -> 1762 us, 1792 tokens, H = 5120, V = 128256 4378 -> 4400.
 constexpr int64_t kDirectTokens = 2304;
 BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     BwdLayout l;
@@ -1961,7 +2066,10 @@ BwdLayout bwd_layout(int64_t N, int64_t V, int64_t H, int64_t chunk) {
     l.slices = l.reached(l.dh_k);
     l.off_dh = take(size_t(l.slices) * N * H * 4);
     l.n_chunks = (V + l.cpad - 1) / l.cpad;
-    l.off_max = take(size_t(3 + l.n_chunks) * 4);  // largest magnitudes: g, hidden, sample of W, what exceeds it in each chunk
+    // largest magnitudes: g, hidden, sample of W, what exceeds it in each chunk -- or whether fp16 does not hold all of W, and
+    // a bit for each row of it
+    l.n_maxima = 3 + l.n_chunks + (l.direct ? (V + 31) / 32 : 0);
+    l.off_max = take(size_t(l.n_maxima) * 4);
     l.total = o;
     return l;
 }
@@ -2193,13 +2301,13 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
     uint16_t* ht = reinterpret_cast<uint16_t*>(ws + l.off_ht);    // [H, npad], row stride ld_n
     uint16_t* dzt = reinterpret_cast<uint16_t*>(ws + l.off_dzt);  // [cpad, npad], row stride ld_n
     float* dh = reinterpret_cast<float*>(ws + l.off_dh);          // [slices][N, H]
-    uint32_t* maxima = reinterpret_cast<uint32_t*>(ws + l.off_max);  // [0] g, [1] hidden, [2] sample of W, [3 + chunk] beyond it
+    uint32_t* maxima = reinterpret_cast<uint32_t*>(ws + l.off_max);  // [0] g, [1] hidden, [2] sample of W, the rest: see bwd_layout
     const int H = int(hidden_size), N = int(n_tokens), V = int(vocab);
     const bool from_bf16 = dtype == TRLK_BF16;  // the products' operands are fp16: bf16 inputs are converted on the way
     const uint32_t* max_g = maxima;
     const uint32_t* max_h = from_bf16 ? maxima + 1 : nullptr;
-    hipLaunchKernelGGL(head_fill_kernel, dim3(unsigned((3 + l.n_chunks + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<float*>(maxima), 3 + l.n_chunks, 0.f);
+    hipLaunchKernelGGL(head_fill_kernel, dim3(unsigned((l.n_maxima + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<float*>(maxima), l.n_maxima, 0.f);
     MaxAbsArgs ma{};
     ma.g = d_g_logp;
     ma.n_g = n_tokens;
@@ -2213,7 +2321,8 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         ma.hidden = static_cast<const uint16_t*>(d_hidden);
         ma.weight = static_cast<const uint16_t*>(d_weight);
         ma.ld_hidden = hidden_stride;
-        ma.ld_weight = weight_stride * kSampleRows;
+        ma.ld_weight = weight_stride;
+        ma.vocab = V;
         ma.n_hidden = N;
         ma.n_weight = (V + kSampleRows - 1) / kSampleRows;
         ma.C8 = H / 8;
@@ -2255,6 +2364,8 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
     const float zs = logit_scale / temperature;  // |dz[n, v]| <= |g[n]| * zs
     const int n_tb = int((n_tokens + BN - 1) / BN);
     const int n_ht = (H + BN - 1) / BN;
+    const bool converts = l.direct && from_bf16;   // the dHidden product may leave something out (see direct_scale)
+    const bool sums = l.slices > 1 || converts;  // dHidden is left in fp32 and rounded by a pass of its own
     for (int64_t c0 = 0; c0 < vocab; c0 += chunk) {
         const int64_t c1 = c0 + chunk < vocab ? c0 + chunk : vocab;
         const int rows = int(c1 - c0);
@@ -2353,28 +2464,31 @@ extern "C" int trlk_fused_head_bwd(const void* d_hidden, const void* d_weight, c
         auto launch_pair = [&](auto mode_tag, auto bw_tag) {
             constexpr int kMode = decltype(mode_tag)::value;
             constexpr bool kBW = decltype(bw_tag)::value;
-            int rc2 = from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<kMode, TRLK_BF16, kBW>, ghgrid, gh, gwgrid, gw, s, what)
-                                : launch_head_pair(gemm_nt_pair_kernel<kMode, TRLK_F16, kBW>, ghgrid, gh, gwgrid, gw, s, what);
-            if (kBW && from_bf16 && rc2 == TRLK_OK)
-                rc2 = launch_head(gemm_nt_again_kernel<kMode>, ghgrid, gh, s, "fused_head_bwd (dHidden again)");
-            return rc2;
+            return from_bf16 ? launch_head_pair(gemm_nt_pair_kernel<kMode, TRLK_BF16, kBW>, ghgrid, gh, gwgrid, gw, s, what)
+                             : launch_head_pair(gemm_nt_pair_kernel<kMode, TRLK_F16, kBW>, ghgrid, gh, gwgrid, gw, s, what);
         };
         typedef std::integral_constant<int, 1> accumulate_t;
         typedef std::integral_constant<int, 2> round_t;
-        if (last && l.slices == 1)
+        if (last && !sums)
             rc = l.direct ? launch_pair(round_t{}, std::true_type{}) : launch_pair(round_t{}, std::false_type{});
         else
             rc = l.direct ? launch_pair(accumulate_t{}, std::true_type{}) : launch_pair(accumulate_t{}, std::false_type{});
         if (rc) return rc;
     }
-    if (l.slices > 1) {
+    if (sums) {
+        BeyondArgs beyond{};
+        if (converts) {
+            beyond = BeyondArgs{maxima + 3, maxima + 4, maxima + 2, a.weight, dzt, weight_stride, l.ld_n, d_g_logp, zs, int((vocab + 31) / 32), H};
+            hipLaunchKernelGGL(beyond_rows_kernel, dim3(kBeyondBlocks), dim3(kBeyondThreads), 0, s, a.weight, weight_stride, V, H / 8,
+                               maxima + 2, maxima + 3, maxima + 4);
+        }
         const int64_t n = int64_t(N) * H;
-        const dim3 grid(unsigned((n / 8 + 255) / 256));
+        const dim3 grid(unsigned((n / 8 + kSumThreads - 1) / kSumThreads)), block(kSumThreads);
         uint16_t* out = static_cast<uint16_t*>(d_out_dhidden);
         if (from_bf16)
-            hipLaunchKernelGGL(sum_slices_kernel<TRLK_BF16>, grid, dim3(256), 0, s, dh, l.slices, n, out);
+            hipLaunchKernelGGL(sum_slices_kernel<TRLK_BF16>, grid, block, 0, s, dh, l.slices, n, out, beyond);
         else
-            hipLaunchKernelGGL(sum_slices_kernel<TRLK_F16>, grid, dim3(256), 0, s, dh, l.slices, n, out);
+            hipLaunchKernelGGL(sum_slices_kernel<TRLK_F16>, grid, block, 0, s, dh, l.slices, n, out, beyond);
         return launch_status("fused_head_bwd (dHidden)");
     }
     return TRLK_OK;
