@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "trlk.h"
+#include "xcd_order.hpp"
 
 namespace trlk {
 
@@ -163,38 +164,6 @@ struct Elem<TRLK_F16> {
         *p = __builtin_bit_cast(uint16_t, _Float16(v));
     }
 };
-
-// Pieces of a large buffer in address order, dealt to the workgroups of a launch.  The hardware deals consecutive workgroups to
-// the eight XCDs in turn; workgroup w of XCD w mod 8 takes the XCD's pieces in order, and those are runs of `run` neighbouring
-// pieces, every eighth run of the buffer: what an XCD reads and writes at a time is one narrow window, and eight neighbouring
-// windows move through the buffer together.  (Single pieces in turn have no such windows.  One contiguous eighth of the buffer
-// per XCD has, but gives each XCD whole sequences: with completions of 1/16 of the longest to the longest an XCD gets up to a
-// fifth more bytes than the mean, and the launch waits for it.)
-__device__ __forceinline__ int64_t xcd_piece(unsigned w, unsigned run) {
-    const unsigned q = w >> 3, k = q / run;
-    return (int64_t(k) * 8 + (w & 7)) * run + (q - k * run);
-}
-// The length of a run for `total` pieces, `period` of them per sequence, where `want` is wanted: short enough for 10 runs per XCD,
-// and such that an XCD does not meet the same part of every sequence, one XCD the padding and another none.  That happens when
-// the 8 runs of a round are about a sequence, or half of one: 1025 rows of 151936 16-bit logits per sequence, runs of 17 to
-// 25 rows 2665-2680 us, 32 2716-2732, 64 2793, 128 2934-2950.  Rounds far shorter than a sequence cannot do it; longer ones
-// are brought to a whole number of sequences and 0.382 or 0.618 of one (the golden section: the part of the sequence that
-// an XCD meets keeps moving).
-inline unsigned xcd_run(int64_t total, int64_t want, int64_t period) {
-    const int64_t most = total < (int64_t(1) << 30) ? total / 80 : 1, run = want < most ? want : most;
-    if (run <= 1) return 1u;
-    const double round = 8.0 * double(run) / double(period), whole = double(int64_t(round));  // in sequences
-    if (round <= 0.382) return unsigned(run);
-    double best = 0.382;
-    for (double c : {whole - 0.382, whole + 0.382, whole + 0.618, whole + 1.382}) {
-        const double is = c < round ? round / c : c / round, was = best < round ? round / best : best / round;
-        if (c > 0.0 && is < was) best = c;
-    }
-    const int64_t adjusted = int64_t(best * double(period) / 8.0 + 0.5);
-    return adjusted > 1 ? unsigned(adjusted) : 1u;
-}
-// Workgroups of the launch: whole rounds of runs; the pieces from `total` on do not exist.
-inline unsigned xcd_grid(int64_t total, unsigned run) { return unsigned((total + 8 * run - 1) / (8 * run) * (8 * run)); }
 
 inline size_t elem_size(int dtype) { return dtype == TRLK_F32 ? 4 : 2; }
 

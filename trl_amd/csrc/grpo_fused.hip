@@ -49,8 +49,9 @@ typedef __attribute__((address_space(1))) u32x4_u GlobalVecOutU;
 // Bytes of rows that follow each other on one XCD (see xcd_run).  Against one contiguous eighth of the rows per XCD, two draws of
 // completions of 1/16 of the longest to the longest, bf16: [32, 1024, 151936] 2848 / 2730 -> 2689 / 2684 us, [16, 1024, 128256]
 // 1278 / 1285 -> 1148 / 1136, [8, 700, 262144] 980 / 982 -> 854 / 862, [16, 509, 50257] 251 / 255 -> 244 / 240,
-// [16, 2047, 40000] 785 / 794 -> 751 / 738, [8, 512, 50264] fp32 250 -> 228; [20, 585, 50264] loses, 339 / 331 -> 347 / 341.
-// Every row active: within 2 %; half of every sequence, which leaves no XCD with more: -4 to +5 %.  A narrow row (see
+// [16, 2047, 40000] 785 / 794 -> 751 / 738, [8, 512, 50264] fp32 250 -> 228; nothing gained at [20, 585, 50264], whole operator 405-408 /
+// 411-415 -> 408-410 / 410-412, and [12, 600, 50264], 248-254 / 279 -> 255-257 / 280.  Every row active: within 2 %.  Half of every
+// sequence, which leaves no XCD with more: -4 to +5 %, and 61 -> 68 us at [8, 300, 32000], where an eighth is one sequence.  A narrow row (see
 // kNarrowVec) has neighbours on its CU, and an XCD twice to five times as many rows under way: runs of 4 MiB lose 3 to 5 %
 // there (50264 and 65536 entries), while wide rows of 256 KB lose 2 % in runs of 8 MiB and of 512 KB 5 % in runs of 39.
 constexpr int64_t kNarrowRunBytes = 12 << 20, kWideRunBytes = 6 << 20;

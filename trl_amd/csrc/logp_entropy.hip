@@ -420,8 +420,8 @@ constexpr int kChunkBytes = kThreads * kBwdUnroll * 16;
 // Chunks that follow each other on one XCD: 264 KiB.  bf16, completions of 1/16 of the longest to the longest, against one
 // contiguous eighth of the buffer per XCD: [16, 512, 151936] 680-699 -> 596-601 us, [16, 1024, 128257] 1132-1168 -> 1016-1032,
 // [32, 900, 32001] 491-498 -> 452, [8, 300, 32000] 47 -> 41, [8, 512, 202048] fp32 930 -> 823; every row active 782 -> 758 and
-// 1314 -> 1287.  Completions of one length (half of the rows), which leave no XCD with more: 594 -> 579, but 949 -> 986 at
-// 128257 entries, where a whole eighth makes all XCDs write zeros at the same time.  Runs of 31 to 255 chunks lie within 5 %.
+// 1314 -> 1287.  Completions of one length (half of the rows), which leave no XCD with more: 594 -> 579, at 128257 entries
+// 949 -> 986 and in later runs 987 -> 967, [8, 300, 32000] 42 -> 46.  Runs of 31 to 255 chunks lie within 5 %.
 constexpr int kBwdRun = 33;
 
 template <int DT>
