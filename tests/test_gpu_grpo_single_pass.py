@@ -1191,3 +1191,37 @@ def test_native_node_of_the_loss(amd, dtype, upstream, monkeypatch):
     with pytest.raises(RuntimeError):
         torch.func.grad(lambda x: step(x)[0])(logits)
     assert grpo_trainer.forward_ad._current_level == -1
+
+
+@pytest.mark.parametrize("missing", [None, "_len_torch_dispatch_stack", "_current_level"])
+def test_python_node_where_torch_does_not_tell(amd, missing, monkeypatch):
+    """A traced call (`torch.jit.trace`), and any call on a torch without one of the questions that the choice of the node asks,
+    takes the Python node: loss and gradient as with the native one, also of the traced function on other logits.  (The third
+    question, for function transforms, torch's own `Function.apply` asks too.)"""
+    from trl_amd.trainer import grpo_trainer
+
+    logits, ids, mask, adv, _ = _inputs(3, 9, 4096, torch.float32, seed=6)
+    nodes = []
+
+    def step(x):
+        loss = amd.grpo_loss_from_logits(x, ids, adv, mask, num_items_in_batch=20.0)[0]
+        nodes.append(loss.grad_fn.name())
+        return loss
+
+    def gradient(f, x):
+        leaf = x.clone().requires_grad_(True)
+        loss = f(leaf)
+        loss.backward()
+        return loss.detach(), leaf.grad
+
+    want = gradient(step, 1.5 * logits)
+    assert "GradientInHand" in nodes[-1]
+    with monkeypatch.context() as m:
+        if missing is None:
+            function = torch.jit.trace(step, (logits.clone().requires_grad_(True),), check_trace=False)
+        else:
+            function = step
+            m.delattr(grpo_trainer.forward_ad if missing == "_current_level" else torch._C, missing)
+        got = gradient(function, 1.5 * logits)
+    assert "GradientInHand" not in nodes[-1]
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and float(want[1].abs().sum()) > 0

@@ -336,6 +336,18 @@ def _one_pass(logits, completion_ids, advantages, mask, temperature, kw):
     return loss, metrics, logp, ent, dlogits, up
 
 
+def _traced_or_transformed() -> bool:
+    """Whether something looks on that follows a Python autograd function but not a native node: a tracer, a dispatch mode, a function
+    transform, forward mode.  A torch that does not answer one of these questions counts as one where something does."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return True
+    modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+    transforms = getattr(torch._C, "_are_functorch_transforms_active", None)
+    if modes is None or transforms is None:
+        return True
+    return modes() > 0 or transforms() or getattr(forward_ad, "_current_level", 0) >= 0
+
+
 class _GRPOFromLogits(torch.autograd.Function):
     """loss (and the detached log-probs / entropies) from the logits; the gradient w.r.t. the logits was
     written by the same pass and is only scaled by the upstream gradient in `backward`.  For calls that are traced or
@@ -451,8 +463,7 @@ def grpo_loss_from_logits(
               use_bias_correction_kl=use_bias_correction_kl, token_weight=token_weight, entropy_coef=entropy_coef,
               sapo_temperature_pos=sapo_temperature_pos, sapo_temperature_neg=sapo_temperature_neg,
               skip_masked_rows=skip_masked_rows, keep_start=keep_start, upstream_scale=upstream_scale)
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0):
+    if _traced_or_transformed():
         return _GRPOFromLogits.apply(logits, completion_ids, advantages, mask, temperature, kw)
     with torch.no_grad():
         loss, metrics, logp, ent, dlogits, up = _one_pass(logits, completion_ids, advantages, mask, temperature, kw)
