@@ -950,8 +950,9 @@ __device__ __forceinline__ WeightScale weight_scale(const uint32_t* sample, cons
 // The scale in which the dHidden product converts a weight that it reads itself: the sample's, whatever the other entries are.
 // What exceeds fp16 there (|w| * scale > kF16Max, four to eight times the sample's maximum) counts as kF16Max in the product; the
 // rest of it is added by the pass that sums the product's slices, from the rows in which beyond_rows_kernel finds such
-// entries.  So one large entry neither makes the product be done again nor takes bits from the others.  (2^60, also for a sample
-// of nothing but zeros: w * scale is finite up to |w| = 2^68.)
+// entries.  So one large entry neither makes the product be done again nor takes bits from the others.  (At most 2^60, also
+// for a sample of nothing but zeros.  w * scale has to be finite in fp32: an entry of 2^113 times the sample's maximum, and of 2^68
+// beside such a sample, counts as infinite.)
 constexpr float kF16Max = 65504.f;
 __device__ __forceinline__ float direct_scale(const uint32_t* sample) {
     const float m = __uint_as_float(*sample);
@@ -1675,13 +1676,14 @@ struct BeyondArgs {
     int n_words, H;
 };
 constexpr int kSumThreads = 256;
-// Adds it for the 8 outputs from i on (token i / H); every lane of the workgroup takes part.  8192 rows at a time: their numbers are
-// put in a list in LDS, sixteen of them are in flight.  Whole backward, weight of deviation 0.02 -> one entry of 50 -> 300 rows times 100
-// (a sample of 1/32 of the rows misses all of 300 once in 1e4 weights): 1396 tokens, H = 2048, V = 50257 715 -> 690 -> 837 us; 1392 tokens, V =
-// 128256 1578 -> 1640 -> 1727; 459 tokens, H = 3584, V = 151936 1241 -> 1415 -> 1520; 64 tokens, H = 1024, V = 32000 100 -> 112 -> 163.
-// With the whole product done again in another scale, one entry: 1029, 2590, 1967 and 124 us.
+// Adds it for the 8 outputs from i on (token i / H); every lane of the workgroup takes part.  8192 rows at a time: their numbers
+// are put in a list in LDS, eight of them are in flight (sixteen take no less time, and their registers leave the launch with no such
+// rows four waves per SIMD: 7.4 for 7.0 us).  Whole backward, weight of deviation 0.02 -> one entry of 50 -> 300 rows times 100 (a
+// sample of 1/32 of the rows misses all of 300 once in 1e4 weights): 1396 tokens, H = 2048, V = 50257 715 -> 690 -> 837 us; 1392
+// tokens, V = 128256 1578 -> 1640 -> 1727; 459 tokens, H = 3584, V = 151936 1241 -> 1415 -> 1520; 64 tokens, H = 1024, V = 32000 100 ->
+// 112 -> 163.  With the whole product done again in another scale, one entry: 1029, 2590, 1967 and 124 us.
 __device__ __forceinline__ void add_beyond(const BeyondArgs& b, int64_t i, bool live, float (&x)[8]) {
-    constexpr int kInFlight = 16;
+    constexpr int kInFlight = 8;
     __shared__ uint16_t list[32 * kSumThreads];
     __shared__ int counts[kSumThreads / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
